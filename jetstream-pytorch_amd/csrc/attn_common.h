@@ -17,6 +17,12 @@ int32_t attn_fast_launch(const jpt_attn_args& a, AttnMode mode, hipStream_t stre
 int64_t attn_fast_workspace_bytes(const jpt_attn_args& a);
 int32_t attn_plan_launch(const jpt_attn_args& a, bool paged, hipStream_t stream);
 
+// Many query rows (prefill) over bf16 keys and values: attn_prefill.hip.  The workspace it can use lies
+// behind the state block and need not be cleared.
+bool attn_prefill_supported(const jpt_attn_args& a, AttnMode mode);
+int64_t attn_prefill_workspace_bytes(const jpt_attn_args& a);
+int32_t attn_prefill_launch(const jpt_attn_args& a, hipStream_t stream);
+
 int32_t attn_generic_launch(const jpt_attn_args& a, AttnMode mode, hipStream_t stream);
 
 }  // namespace jpt

@@ -626,8 +626,8 @@ bool attn_fast_supported(const jpt_attn_args& a, AttnMode mode) {
 int64_t attn_fast_workspace_bytes(const jpt_attn_args& a) {
   const int rows = a.q_heads / a.kv_heads * a.q_rows;
   // shapes the streaming kernel never takes (prefill-shaped queries, huge
-  // batches) run on the generic kernel, which uses neither plan nor partials
-  if (rows > kMaxRows || a.batch > kMaxPlanBatch) return JPT_ATTN_WS_STATE_BYTES;
+  // batches) run on kernels that use neither plan nor partials
+  if (rows > kMaxRows || a.batch > kMaxPlanBatch) return JPT_ATTN_WS_STATE_BYTES + attn_prefill_workspace_bytes(a);
   return make_layout(a.batch, a.kv_heads, rows).total;
 }
 
@@ -731,6 +731,7 @@ static int32_t attn_entry(const jpt_attn_args* args, jpt::AttnMode mode, void* s
     if (attn_fast_supported(a, mode)) return attn_fast_launch(a, mode, s);
   }
   JPT_REQUIRE(!a.new_to_pages, "new_to_pages needs head_dim 128, a bf16 query and page_size a multiple of 32");
+  if (attn_prefill_supported(a, mode)) return attn_prefill_launch(a, s);
   return attn_generic_launch(a, mode, s);
 }
 

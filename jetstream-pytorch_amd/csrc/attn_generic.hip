@@ -2,9 +2,9 @@
 // rows, bf16/f32/int8 keys, optional scales, additive mask, page table and
 // fused new-token term.  One wavefront per (slot, q head, q row); scores of a
 // tile of positions go through LDS, the online softmax is carried in
-// registers.  It is the path for shapes the MFMA kernel does not take (tiny
-// test shapes, prefill-shaped calls, f32 caches) and is not tuned; it also
-// serves as a second implementation to cross-check the MFMA kernel on the GPU.
+// registers.  It is the path for shapes the MFMA kernels do not take (tiny
+// test shapes, f32 caches) and is not tuned; it also
+// serves as a second implementation to cross-check the MFMA kernels on the GPU.
 #include <math.h>
 
 #include "attn_common.h"

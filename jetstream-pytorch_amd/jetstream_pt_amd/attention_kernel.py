@@ -288,7 +288,10 @@ def _attend(mode, xq, keys, values, *, lengths=None, page_table=None, mask=None,
 
   ws = None
   if not _streaming_kernel_may_run(hq // hkv * t, d, xq.dtype, keys.dtype) or force_generic:
-    pass  # prefill-shaped and other calls of the generic kernel: no workspace, no plan
+    # prefill-shaped and other calls: no plan; what is live in a large mask is noted in a workspace
+    nbytes = _ffi.lib.jpt_attn_workspace_bytes(a) if mask is not None and not force_generic else 0
+    if nbytes > _ffi.ATTN_WS_STATE_BYTES:
+      ws = _shared_workspace(nbytes, device)
   elif plan is not None and plan.key == (b, hq, hkv, t, a.seq or None, a.page_size or None,
                                          a.max_pages or None) and lengths is not None \
       and plan.lengths.data_ptr() == lengths.data_ptr():

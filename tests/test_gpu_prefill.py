@@ -1,0 +1,87 @@
+"""GPU parity: attention of many query rows (prefill) on the matrix cores, against
+the float64 closed form, at the edges of its tiles: 128 query rows and 32 a wave,
+64 positions a tile, mask blocks of 32 rows x 64 positions, heads folded below 128
+rows.  Softmax weights carry 16 bits, so below 2 (where the output's rounding is at
+most 2^-8) the error stays under 6e-3: half an ulp, 2^-8, plus a score's float32
+sums and exp2, far below it."""
+
+import math
+
+import pytest
+import torch
+
+from conftest import attention_bound
+from oracle import attention as OA
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def rnd(g, shape, dtype=torch.bfloat16):
+  return torch.randn(shape, generator=g).to(dtype)
+
+
+def make_mask(kind, g, b, hq, t, s):
+  if kind is None:
+    return None
+  if kind == "causal":  # the last rows of a causal mask over s positions
+    return torch.full((t, s), -math.inf).triu(1 + s - t).reshape(1, 1, t, s).to(torch.bfloat16)
+  m = torch.randn((b, hq, t, s), generator=g)
+  m[:, :, :, : s // 2] = 0.0                              # blocks of zeros
+  m[:, :, t // 3:, s // 3: 2 * s // 3] = -math.inf        # dead blocks with ragged edges
+  m[0, 0, 0] = -math.inf                                  # a row with nothing to attend
+  m[-1, -1, t // 2:] = -math.inf
+  return m
+
+
+CASES = [  # b, hq, hkv, d, t, s, mask, scale heads (None: no scales), scale dtype
+    (1, 4, 4, 128, 17, 17, "causal", None, None),
+    (2, 8, 2, 128, 31, 65, "causal", None, None),
+    (1, 8, 2, 128, 127, 127, "causal", 1, torch.bfloat16),
+    (1, 4, 2, 128, 128, 256, "causal", None, None),
+    (1, 4, 2, 128, 129, 257, "causal", 1, torch.float32),
+    (2, 4, 2, 64, 300, 300, "causal", None, None),
+    (1, 2, 1, 256, 321, 321, "causal", 1, torch.bfloat16),
+    (1, 28, 4, 128, 259, 259, "causal", None, None),
+    (2, 4, 2, 128, 200, 330, "any", 2, torch.float32),
+    (2, 2, 2, 256, 130, 384, "any", None, None),
+    (2, 4, 1, 64, 33, 400, "any", 1, torch.float32),
+    (1, 8, 2, 128, 64, 63, None, 2, torch.bfloat16),
+    (1, 2, 2, 64, 1, 77, None, None, None),
+    (3, 4, 2, 256, 5, 1, None, None, None),
+]
+
+
+@pytest.mark.parametrize("case", CASES, ids=lambda c: "-".join(str(x).replace("torch.", "") for x in c))
+def test_many_query_rows(case):
+  from jetstream_pt_amd import attention_kernel as ak
+  b, hq, hkv, d, t, s, kind, hs, sdt = case
+  g = torch.Generator().manual_seed(900 + t)
+  q, k, v = rnd(g, (b, hq, t, d)), rnd(g, (b, hkv, s, d)), rnd(g, (b, hkv, s, d))
+  mask = make_mask(kind, g, b, hq, t, s)
+  ks = vs = None
+  if hs:
+    ks, vs = ((torch.rand((b, hs, s, 1), generator=g) + 0.5).to(sdt) for _ in range(2))
+  rows = None if mask is None else mask.expand(b, hq, t, s).reshape(b, hkv, hq // hkv * t, s)
+  want, wm, wl = OA.closed_form(q, k, v, mask=rows, k_scale=ks, v_scale=vs)
+  dev = [None if x is None else x.to(DEV) for x in (q, k, v, ks, vs, mask)]
+  got, (m, l) = ak.flash_attention(*dev[:3], 0, dev[3], dev[4], dev[5])
+  err = (got.double().cpu() - want).abs()
+  assert torch.all(err <= torch.where(want.abs() < 2.0, torch.full_like(err, 6e-3), attention_bound(want))), float(err.max())
+  live = wl > 0
+  assert torch.allclose(m.double().cpu()[live], wm[live], rtol=1e-3, atol=1e-4)
+  assert torch.allclose(l.double().cpu()[live], wl[live], rtol=1e-3)
+  assert torch.all(torch.isneginf(m.cpu()[~live])) and torch.all(l.cpu()[~live] == 0) and torch.all(got.cpu()[(~live).expand_as(got)] == 0)
+
+
+def test_many_query_rows_with_lengths():
+  """Left-aligned slots of their own lengths, empty and full ones among them."""
+  from jetstream_pt_amd import attention_kernel as ak
+  g = torch.Generator().manual_seed(940)
+  b, hq, hkv, d, t, s = 5, 8, 4, 128, 20, 192
+  q, k, v = rnd(g, (b, hq, t, d)), rnd(g, (b, hkv, s, d)), rnd(g, (b, hkv, s, d))
+  end = torch.tensor([0, 1, 64, 65, 192], dtype=torch.int32)
+  want, _, _ = OA.closed_form(q, k, v, lengths=end)
+  got, _ = ak.ragged_mha(q.to(DEV), k.to(DEV), v.to(DEV), 0, None, end.to(DEV))
+  err = (got.double().cpu().reshape(want.shape) - want).abs()
+  assert torch.all(err <= 6e-3), float(err.max())
