@@ -21,7 +21,7 @@ BUILD = os.path.join(HERE, "build")
 # the units that hold the streaming attention kernel, one per cache type and way the new token comes
 STREAMING = ["attn_decode_i8_raw.hip", "attn_decode_i8_raw_wide.hip", "attn_decode_i8_raw_rope.hip", "attn_decode_i8_raw_wide_rope.hip",
              "attn_decode_i8_none.hip", "attn_decode_i8_given.hip", "attn_decode_bf16_given.hip", "attn_decode_bf16_none.hip"]
-SOURCES = STREAMING + ["api.cpp", "pam.cpp", "kv_lines.hip", "prefill_insert.hip", "paged_kv.hip", "device_pages.hip", "attn_generic.hip", "attn_prefill.hip",
+SOURCES = STREAMING + ["api.cpp", "pam.cpp", "kv_lines.hip", "prefill_insert.hip", "paged_kv.hip", "device_pages.hip", "attn_generic.hip", "attn_prefill.hip", "attn_split.hip",
                        "attn_decode.hip"]
 
 HIPCC = os.environ.get("HIPCC", "/opt/rocm/bin/hipcc")

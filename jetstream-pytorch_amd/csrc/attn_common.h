@@ -15,7 +15,14 @@ int32_t check_attn_args(const jpt_attn_args& a, AttnMode mode);
 bool attn_fast_supported(const jpt_attn_args& a, AttnMode mode);
 int32_t attn_fast_launch(const jpt_attn_args& a, AttnMode mode, hipStream_t stream);
 int64_t attn_fast_workspace_bytes(const jpt_attn_args& a);
+int64_t attn_partials_offset(const jpt_attn_args& a);  // in the workspace: behind the plan
 int32_t attn_plan_launch(const jpt_attn_args& a, bool paged, hipStream_t stream);
+
+// Few query rows over caches the streaming kernel is not built for: attn_split.hip.  Needs a workspace
+// (its state block zero before the first use; the rest need not be cleared).
+bool attn_split_supported(const jpt_attn_args& a, AttnMode mode);
+int64_t attn_split_workspace_bytes(const jpt_attn_args& a);
+int32_t attn_split_launch(const jpt_attn_args& a, hipStream_t stream);
 
 // Many query rows (prefill) over bf16 keys and values: attn_prefill.hip.  The workspace it can use lies
 // behind the state block and need not be cleared.

@@ -631,6 +631,11 @@ int64_t attn_fast_workspace_bytes(const jpt_attn_args& a) {
   return make_layout(a.batch, a.kv_heads, rows).total;
 }
 
+int64_t attn_partials_offset(const jpt_attn_args& a) {
+  if (a.batch > kMaxPlanBatch) return JPT_ATTN_WS_STATE_BYTES;  // never planned
+  return make_layout(a.batch, a.kv_heads, 1).partials;
+}
+
 int32_t attn_plan_launch(const jpt_attn_args& a, bool paged, hipStream_t stream) {
   const int rows = a.q_heads / a.kv_heads * a.q_rows;
   if (rows > kMaxRows || a.batch > kMaxPlanBatch) return JPT_OK;  // generic kernel: nothing to plan
@@ -696,7 +701,11 @@ int64_t jpt_attn_workspace_bytes(const jpt_attn_args* args) {
   if (args == nullptr || args->batch <= 0 || args->kv_heads <= 0 || args->q_heads <= 0 ||
       args->q_rows <= 0)
     return JPT_ATTN_WS_STATE_BYTES;
-  return jpt::attn_fast_workspace_bytes(*args);
+  const int64_t planned = jpt::attn_fast_workspace_bytes(*args);
+  const int64_t rows = static_cast<int64_t>(args->q_heads) / args->kv_heads * args->q_rows;
+  if ((args->dim != 64 && args->dim != 256) || rows > jpt::kMaxRows) return planned;
+  const int64_t split = jpt::attn_split_workspace_bytes(*args);
+  return split > planned ? split : planned;
 }
 
 static int32_t attn_entry(const jpt_attn_args* args, jpt::AttnMode mode, void* stream) {
@@ -731,6 +740,7 @@ static int32_t attn_entry(const jpt_attn_args* args, jpt::AttnMode mode, void* s
     if (attn_fast_supported(a, mode)) return attn_fast_launch(a, mode, s);
   }
   JPT_REQUIRE(!a.new_to_pages, "new_to_pages needs head_dim 128, a bf16 query and page_size a multiple of 32");
+  if (attn_split_supported(a, mode)) return attn_split_launch(a, s);
   if (attn_prefill_supported(a, mode)) return attn_prefill_launch(a, s);
   return attn_generic_launch(a, mode, s);
 }

@@ -59,6 +59,7 @@ _workspaces = {}
 _dense_workspaces = collections.OrderedDict()  # most recently used last
 _MAX_DENSE_WORKSPACES = 8
 _FAST_MAX_ROWS = 16  # query rows per KV head (rep * T) the streaming kernel takes
+_MATRIX_CORE_DIMS = (64, 128, 256)  # head dims of the kernels beside it
 
 
 def _streaming_kernel_may_run(rows, dim, q_dtype, kv_dtype):
@@ -288,10 +289,11 @@ def _attend(mode, xq, keys, values, *, lengths=None, page_table=None, mask=None,
 
   ws = None
   if not _streaming_kernel_may_run(hq // hkv * t, d, xq.dtype, keys.dtype) or force_generic:
-    # prefill-shaped and other calls: no plan; what is live in a large mask is noted in a workspace
-    nbytes = _ffi.lib.jpt_attn_workspace_bytes(a) if mask is not None and not force_generic else 0
-    if nbytes > _ffi.ATTN_WS_STATE_BYTES:
-      ws = _shared_workspace(nbytes, device)
+    # other kernels, which need no plan: the split kernel's partials, or what is live in a prefill's mask
+    if not force_generic and d in _MATRIX_CORE_DIMS and xq.dtype == torch.bfloat16 and mode != "paged":
+      nbytes = _ffi.lib.jpt_attn_workspace_bytes(a)
+      if nbytes > _ffi.ATTN_WS_STATE_BYTES:
+        ws = _shared_workspace(nbytes, device)
   elif plan is not None and plan.key == (b, hq, hkv, t, a.seq or None, a.page_size or None,
                                          a.max_pages or None) and lengths is not None \
       and plan.lengths.data_ptr() == lengths.data_ptr():

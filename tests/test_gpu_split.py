@@ -1,0 +1,93 @@
+"""GPU parity: decode attention over head dims of 64 and 256 and over cache lengths and masks the
+streaming kernel does not take, against the float64 closed form, where shares and tiles end: slots
+of 0, 1, 31..33 positions, fewer tiles than groups, sequences over many groups, more slots than a
+workgroup has threads.  Softmax weights carry 16 bits and more, so below 2 (where the output's
+rounding is at most 2^-8) the error stays under 6e-3."""
+
+import math
+
+import pytest
+import torch
+
+from conftest import attention_bound
+from oracle import attention as OA
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def make(g, kind, b, hkv, s, d, hs):
+  if kind == "bf16":
+    return [torch.randn((b, hkv, s, d), generator=g).to(torch.bfloat16) for _ in range(2)] + [None, None]
+  sdt = torch.float32 if kind == "int8_f32" else torch.bfloat16
+  kv = [torch.randint(-127, 128, (b, hkv, s, d), generator=g, dtype=torch.int8) for _ in range(2)]
+  return kv + [(torch.rand((b, hs, s, 1), generator=g) * 0.015 + 0.005).to(sdt) for _ in range(2)]
+
+
+def check(got, want, m, l, wm, wl):
+  err = (got.double().cpu().reshape(want.shape) - want).abs()
+  assert torch.all(err <= torch.where(want.abs() < 2.0, torch.full_like(err, 6e-3), attention_bound(want))), float(err.max())
+  m, l, live = m.double().cpu().reshape(wm.shape), l.double().cpu().reshape(wl.shape), wl > 0
+  assert torch.allclose(m[live], wm[live], rtol=1e-3, atol=1e-4) and torch.allclose(l[live], wl[live], rtol=1e-3)
+  assert torch.all(torch.isneginf(m[~live])) and torch.all(l[~live] == 0)
+
+
+@pytest.mark.parametrize("kind", ["bf16", "int8_f32", "int8_bf16"])
+@pytest.mark.parametrize("d,hq,hkv,s,lens", [
+    (64, 4, 4, 96, [0, 1, 31, 32, 33, 96]),
+    (256, 16, 2, 64, [64, 0, 63]),
+    (256, 8, 8, 4096, [4096, 3000, 17, 2049]),
+    (128, 32, 2, 333, [333, 5, 100, 0, 64]),
+    (64, 28, 4, 2048, [2047]),
+    (256, 2, 1, 40, [(7 * i) % 41 for i in range(300)]),
+    (64, 1, 1, 4, [i % 5 for i in range(4200)]),
+])
+@pytest.mark.parametrize("token", [False, True])
+def test_lengths(token, d, hq, hkv, s, lens, kind):
+  from jetstream_pt_amd import attention_kernel as ak
+  g = torch.Generator().manual_seed(1000 + d + s)
+  b = len(lens)
+  end = torch.tensor(lens, dtype=torch.int32)
+  q = torch.randn((b, hq, 1, d), generator=g).to(torch.bfloat16)
+  k, v, ks, vs = make(g, kind, b, hkv, s, d, hkv if kind == "int8_bf16" else 1)
+  new = {}
+  fk, fv, fks, fvs = k, v, ks, vs
+  if token:  # one more position, number `len` of a longer cache
+    nk, nv, nks, nvs = make(g, kind, b, hkv, 1, d, hkv if kind == "int8_bf16" else 1)
+    new = dict(new_key=nk.to(DEV), new_value=nv.to(DEV))
+    if nks is not None:
+      new.update(new_k_scaler=nks.to(DEV), new_v_scaler=nvs.to(DEV))
+    def longer(x, n):
+      if x is None:
+        return None
+      y = torch.cat([x, torch.zeros_like(x[:, :, :1])], 2)
+      for i, at in enumerate(lens):
+        y[i, :, at] = n[i, :, 0]
+      return y
+    fk, fv, fks, fvs = longer(k, nk), longer(v, nv), longer(ks, nks), longer(vs, nvs)
+  want, wm, wl = OA.closed_form(q, fk, fv, lengths=end + (1 if token else 0), k_scale=fks, v_scale=fvs)
+  dev = [None if x is None else x.to(DEV) for x in (q, k, v, end, ks, vs)]
+  o, (m, l) = ak.ragged_mha(*dev[:3], 0, None, dev[3], None, None, dev[4], dev[5], **new)
+  check(o, want, m, l, wm, wl)
+  o2, _ = ak.ragged_mha(*dev[:3], 0, None, dev[3], None, None, dev[4], dev[5], **new)
+  assert torch.equal(o, o2), "the counters are not back at zero, or the order of a sum changed"
+
+
+@pytest.mark.parametrize("kind", ["bf16", "int8_bf16"])
+@pytest.mark.parametrize("d,hq,hkv,t,s,per_head", [(64, 8, 2, 1, 160, False), (256, 4, 4, 3, 90, True), (128, 8, 4, 2, 77, True), (256, 16, 16, 1, 1024, False)])
+def test_masks(d, hq, hkv, t, s, per_head, kind):
+  from jetstream_pt_amd import attention_kernel as ak
+  g = torch.Generator().manual_seed(1100 + d)
+  b = 3
+  q = torch.randn((b, hq, t, d), generator=g).to(torch.bfloat16)
+  k, v, ks, vs = make(g, kind, b, hkv, s, d, 1)
+  mask = torch.where(torch.rand((b, hq if per_head else 1, t, s), generator=g) < 0.5, 0.0, -math.inf)
+  mask += torch.randn(mask.shape, generator=g)
+  mask[1, :, :, : s // 2] = -math.inf
+  mask[2] = -math.inf
+  mask = mask.to(torch.bfloat16 if per_head else torch.float32)
+  rows = mask.expand(b, hq, t, s).reshape(b, hkv, hq // hkv * t, s)
+  want, wm, wl = OA.closed_form(q, k, v, mask=rows, k_scale=ks, v_scale=vs)
+  dev = [None if x is None else x.to(DEV) for x in (q, k, v, ks, vs, mask)]
+  o, (m, l) = ak.flash_attention(*dev[:3], 0, dev[3], dev[4], dev[5])
+  check(o, want, m, l, wm, wl)
