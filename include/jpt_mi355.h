@@ -71,6 +71,12 @@ int32_t jpt_kv_scatter_lines(const jpt_line_tensor* tensors, int32_t n_tensors,
                              int32_t n_layers, int32_t batch, int32_t seq,
                              void* stream);
 
+/* The step's K and V rows into their stash (KVCacheGenerate.update with
+ * lazy_cache_update, cache_manager.py:250-266): `bytes` from src_k to dst_k and
+ * from src_v to dst_v, one launch. */
+int32_t jpt_kv_stash_lines(void* dst_k, const void* src_k, void* dst_v,
+                           const void* src_v, int64_t bytes, void* stream);
+
 /* ------------------------------------------------------------------------
  * Fused per-token absmax int8 quantisation + append.
  *
@@ -407,6 +413,9 @@ int64_t jpt_attn_workspace_bytes(const jpt_attn_args* args);
  * computes its per-step block tables the same way, once per decode step for
  * all layers (precompute_ragged_block_indices, engine.py:674-729). */
 int32_t jpt_attn_plan(const jpt_attn_args* args, int32_t paged, void* stream);
+/* The same for a workspace that has not been used before and need not be
+ * zero: what has to start at zero is cleared by the planning launch. */
+int32_t jpt_attn_plan_fresh(const jpt_attn_args* args, int32_t paged, void* stream);
 int32_t jpt_attn_ragged(const jpt_attn_args* args, void* stream);
 int32_t jpt_attn_dense(const jpt_attn_args* args, void* stream);
 int32_t jpt_attn_paged(const jpt_attn_args* args, void* stream);
@@ -548,6 +557,16 @@ int32_t jpt_decode_advance(void* mask, int32_t mask_dtype, int64_t mask_stride,
                            int32_t seq, int32_t ring_buffer,
                            int32_t current_position, int32_t update_mask,
                            int32_t advance, void* stream);
+
+/* A prompt's row of the decode state (Engine.insert, engine.py:371-626): the mask
+ * row of `slot` becomes 0 where lo <= x < hi (wrap: x >= lo or x < hi) and -inf
+ * elsewhere, start[slot] = first, input_pos[slot] = position, lens[slot] = length.
+ * mask (batch, seq) f32 or bf16; any of the four may be NULL. */
+int32_t jpt_insert_state(void* mask, int32_t mask_dtype, int64_t seq,
+                         int32_t* start, int32_t* input_pos, int32_t* lens,
+                         int32_t slot, int32_t first, int32_t position,
+                         int32_t length, int32_t lo, int32_t hi, int32_t wrap,
+                         void* stream);
 
 /* ------------------------------------------------------------------------
  * Engine.precompute_ragged_block_indices (engine.py:674-729): for every grid

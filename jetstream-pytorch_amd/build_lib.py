@@ -15,6 +15,7 @@ CSRC = os.path.join(HERE, "csrc")
 INCLUDE = os.path.join(os.path.dirname(HERE), "include")
 OUT_DIR = os.path.join(HERE, "jetstream_pt_amd")
 LIB = os.path.join(OUT_DIR, "libjpt_mi355.so")
+HOST_MODULE = os.path.join(OUT_DIR, "_host.so")  # the Python mirror's host side (csrc/py_host.cpp)
 TIMELINE_LIB = os.path.join(OUT_DIR, "libjpt_mi355_timeline.so")
 BUILD = os.path.join(HERE, "build")
 
@@ -55,6 +56,28 @@ def _link(objs, lib):
   os.replace(tmp, lib)
 
 
+def _build_host_module():
+  """An extension module against the installed torch; host code only."""
+  import sysconfig
+
+  import torch
+  from torch.utils import cpp_extension
+  rocm = os.path.dirname(os.path.dirname(HIPCC))
+  tmp = HOST_MODULE + ".tmp"
+  cmd = [os.environ.get("CXX", "g++"), "-O2", "-std=c++17", "-fPIC", "-shared", "-D__HIP_PLATFORM_AMD__=1", "-DUSE_ROCM",
+         f"-D_GLIBCXX_USE_CXX11_ABI={int(torch._C._GLIBCXX_USE_CXX11_ABI)}", "-I", INCLUDE]
+  for d in cpp_extension.include_paths() + [os.path.join(rocm, "include"), sysconfig.get_paths()["include"]]:
+    cmd += ["-isystem", d]
+  cmd += [os.path.join(CSRC, "py_host.cpp"), "-o", tmp]
+  for d in cpp_extension.library_paths():
+    cmd += [f"-L{d}"]
+  cmd += ["-ltorch_python", "-ltorch", "-ltorch_cpu", "-lc10", "-lc10_hip"]
+  r = subprocess.run(cmd, capture_output=True, text=True)
+  if r.returncode != 0:
+    raise RuntimeError(f"g++ failed on py_host.cpp:\n{r.stderr}")
+  os.replace(tmp, HOST_MODULE)
+
+
 def build(verbose=True, timeline=True):
   """The product library, and (timeline) its development twin libjpt_mi355_timeline.so, whose
   decode-attention kernel records when its waves start, stream and end (attn_timeline.py);
@@ -63,13 +86,15 @@ def build(verbose=True, timeline=True):
   # the twin's own units: what attn_timeline.py launches (int8 cache, raw token or none); the rest are the product's
   traced = ["attn_decode_i8_raw.hip", "attn_decode_i8_none.hip"]
   with concurrent.futures.ThreadPoolExecutor(max_workers=min(8, os.cpu_count() or 1)) as ex:
+    host = ex.submit(_build_host_module)
     plain = [ex.submit(_compile, src) for src in SOURCES]
     twin = [ex.submit(_compile, src, ("-DJPT_ATTN_TIMELINE",), "_timeline") for src in traced] if timeline else []
     objs = [f.result() for f in plain]
     twin = [f.result() for f in twin]
+    host.result()
   _link(objs, LIB)
   if verbose:
-    print(f"built {LIB}")
+    print(f"built {LIB} and {HOST_MODULE}")
   if timeline:
     swapped = [o for o, src in zip(objs, SOURCES) if src not in traced] + twin
     _link(swapped, TIMELINE_LIB)

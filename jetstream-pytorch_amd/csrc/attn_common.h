@@ -16,7 +16,7 @@ bool attn_fast_supported(const jpt_attn_args& a, AttnMode mode);
 int32_t attn_fast_launch(const jpt_attn_args& a, AttnMode mode, hipStream_t stream);
 int64_t attn_fast_workspace_bytes(const jpt_attn_args& a);
 int64_t attn_partials_offset(const jpt_attn_args& a);  // in the workspace: behind the plan
-int32_t attn_plan_launch(const jpt_attn_args& a, bool paged, hipStream_t stream);
+int32_t attn_plan_launch(const jpt_attn_args& a, bool paged, bool fresh, hipStream_t stream);
 
 // Few query rows over caches the streaming kernel is not built for: attn_split.hip.  Needs a workspace
 // (its state block zero before the first use; the rest need not be cleared).

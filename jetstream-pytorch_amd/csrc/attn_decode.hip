@@ -260,7 +260,7 @@ __device__ __forceinline__ int deal_longest_first_in_steps(int n, int per_round,
 
 __global__ void __launch_bounds__(256)
 plan_kernel(const int32_t* lengths, int batch, int seq_cap, int kv_heads, int target, int workers,
-            PlanEntry* entries, int32_t* arrivals, int max_entries, int32_t* status) {
+            PlanEntry* entries, int32_t* arrivals, int max_entries, int32_t* status, int fresh) {
   // An entry that does not fit the plan's array would be positions nobody attends: the capacity
   // (make_layout) is sized so that this cannot happen, and if it ever does the launch says so.
   auto overflow = [&]() { atomicOr(status, JPT_ATTN_STATUS_PLAN_OVERFLOW); };
@@ -284,6 +284,11 @@ plan_kernel(const int32_t* lengths, int batch, int seq_cap, int kv_heads, int ta
     s_positions = 0;
     s_pairs = 0;
     s_sizes = 0;
+  }
+  if (fresh) {  // a workspace nobody has used: what must start at zero
+    for (int i = tid; i < kSplitCounters; i += blockDim.x) status[kStateSplitCounters + i] = 0;
+    if (tid == 0) status[kStateStatus] = 0;
+    __threadfence_block();  // before the status bits below
   }
   for (int i = tid; i < kKeys; i += blockDim.x) s_hist[i] = 0;
   for (int i = tid; i < batch * kv_heads; i += blockDim.x) arrivals[i] = 0;
@@ -599,6 +604,10 @@ plan_kernel(const int32_t* lengths, int batch, int seq_cap, int kv_heads, int ta
   }
 }
 
+__global__ void __launch_bounds__(256) clear_state_kernel(int32_t* state) {
+  state[blockIdx.x * 256 + threadIdx.x] = 0;
+}
+
 }  // namespace
 
 bool attn_fast_supported(const jpt_attn_args& a, AttnMode mode) {
@@ -636,9 +645,15 @@ int64_t attn_partials_offset(const jpt_attn_args& a) {
   return make_layout(a.batch, a.kv_heads, 1).partials;
 }
 
-int32_t attn_plan_launch(const jpt_attn_args& a, bool paged, hipStream_t stream) {
+int32_t attn_plan_launch(const jpt_attn_args& a, bool paged, bool fresh, hipStream_t stream) {
   const int rows = a.q_heads / a.kv_heads * a.q_rows;
-  if (rows > kMaxRows || a.batch > kMaxPlanBatch) return JPT_OK;  // generic kernel: nothing to plan
+  if (rows > kMaxRows || a.batch > kMaxPlanBatch) {  // not the streaming kernel: nothing to plan
+    if (!fresh) return JPT_OK;
+    JPT_REQUIRE(a.workspace != nullptr && a.workspace_bytes >= JPT_ATTN_WS_STATE_BYTES && aligned(a.workspace, 256),
+                "a 256-byte aligned workspace of %d bytes needed", JPT_ATTN_WS_STATE_BYTES);
+    hipLaunchKernelGGL(clear_state_kernel, dim3(JPT_ATTN_WS_STATE_BYTES / 1024), dim3(256), 0, stream, static_cast<int32_t*>(a.workspace));
+    return launch_status("clear_state_kernel");
+  }
   const Layout l = make_layout(a.batch, a.kv_heads, rows);
   JPT_REQUIRE(a.workspace != nullptr && a.workspace_bytes >= l.total,
               "workspace of %lld bytes needed, %lld given", static_cast<long long>(l.total),
@@ -650,7 +665,7 @@ int32_t attn_plan_launch(const jpt_attn_args& a, bool paged, hipStream_t stream)
   hipLaunchKernelGGL(plan_kernel, dim3(1), dim3(256), 0, stream, a.lengths, a.batch, cap,
                      a.kv_heads, target_items(), persistent_blocks(), reinterpret_cast<PlanEntry*>(ws + l.entries),
                      reinterpret_cast<int32_t*>(ws + l.arrivals), l.max_entries,
-                     reinterpret_cast<int32_t*>(ws));
+                     reinterpret_cast<int32_t*>(ws), fresh ? 1 : 0);
   return launch_status("plan_kernel");
 }
 
@@ -673,7 +688,7 @@ int32_t attn_fast_launch(const jpt_attn_args& a, AttnMode mode, hipStream_t stre
   p.total_items = l.max_entries * a.kv_heads;
   p.status = reinterpret_cast<int32_t*>(ws);
   if (!a.reuse_plan) {
-    int32_t st = attn_plan_launch(a, mode == kPaged, stream);
+    int32_t st = attn_plan_launch(a, mode == kPaged, false, stream);
     if (st != JPT_OK) return st;
   }
   int32_t blocks = persistent_blocks();
@@ -745,13 +760,16 @@ static int32_t attn_entry(const jpt_attn_args* args, jpt::AttnMode mode, void* s
   return attn_generic_launch(a, mode, s);
 }
 
-int32_t jpt_attn_plan(const jpt_attn_args* args, int32_t paged, void* stream) {
+static int32_t plan_entry(const jpt_attn_args* args, int32_t paged, bool fresh, void* stream) {
   using namespace jpt;
   JPT_REQUIRE(args != nullptr, "args is NULL");
   JPT_REQUIRE(args->batch > 0 && args->kv_heads > 0 && args->q_heads > 0 && args->q_rows > 0 &&
                   args->q_heads % args->kv_heads == 0, "batch, heads and q_rows must be positive");
-  return attn_plan_launch(*args, paged != 0, static_cast<hipStream_t>(stream));
+  return attn_plan_launch(*args, paged != 0, fresh, static_cast<hipStream_t>(stream));
 }
+
+int32_t jpt_attn_plan(const jpt_attn_args* args, int32_t paged, void* stream) { return plan_entry(args, paged, false, stream); }
+int32_t jpt_attn_plan_fresh(const jpt_attn_args* args, int32_t paged, void* stream) { return plan_entry(args, paged, true, stream); }
 
 // ---- jpt_attn_ragged_static: the workspace is a device array of this library ----
 // Device memory that exists from the moment the code object is loaded on a GPU

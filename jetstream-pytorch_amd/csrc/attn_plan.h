@@ -34,6 +34,9 @@ constexpr int kStateArrivalsCount = 5;
 constexpr int kStateHandOut = 16;
 constexpr int kStateHandOutStride = 16;
 constexpr int kHandOutCounters = 8;
+// arrival counters of the split kernel (attn_split.hip), the end of the state block, zero between launches
+constexpr int kSplitCounters = 1024;
+constexpr int kStateSplitCounters = (JPT_ATTN_WS_STATE_BYTES - kSplitCounters * 4) / 4;
 
 struct FastParams {
   jpt_attn_args a;

@@ -32,9 +32,7 @@ namespace {
 
 constexpr int kSplitWaves = 4;
 constexpr int kSplitThreads = 64 * kSplitWaves;
-constexpr int kMaxGroups = 1024;
-// the groups' arrival counters: the end of the state block, zero between launches
-constexpr int kCountersAt = (JPT_ATTN_WS_STATE_BYTES - kMaxGroups * 4) / 4;
+constexpr int kMaxGroups = kSplitCounters;
 
 struct SplitParams {
   jpt_attn_args a;
@@ -572,7 +570,7 @@ int32_t attn_split_launch(const jpt_attn_args& a, hipStream_t stream) {
   p.a = a;
   p.rep = a.q_heads / a.kv_heads;
   p.rows = p.rep * a.q_rows;
-  p.counters = static_cast<int32_t*>(a.workspace) + decode::kCountersAt;
+  p.counters = static_cast<int32_t*>(a.workspace) + kStateSplitCounters;
   p.partials = reinterpret_cast<float*>(static_cast<char*>(a.workspace) + attn_partials_offset(a));
   const dim3 grid(static_cast<unsigned>(decode::split_groups(a)));
   if (a.dim == 64) decode::launch_split_dim<64>(p, grid, stream);

@@ -247,6 +247,23 @@ decode_advance_kernel(T* mask, int64_t mask_stride, int32_t* input_pos, int32_t*
   }
 }
 
+// One slot's row of the decode state after a prompt's insert.
+template <typename T>
+__global__ void __launch_bounds__(kThreads)
+insert_state_kernel(T* mask, int64_t seq, int32_t* start, int32_t* input_pos, int32_t* lens, int slot, int first,
+                    int position, int length, int lo, int hi, int wrap) {
+  const int64_t x = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
+  if (mask && x < seq) {
+    const bool live = wrap ? (x >= lo || x < hi) : (x >= lo && x < hi);
+    mask[slot * seq + x] = live ? static_cast<T>(0) : sizeof(T) == 2 ? static_cast<T>(0xff80u) : static_cast<T>(0xff800000u);
+  }
+  if (x == 0) {
+    if (start) start[slot] = first;
+    if (input_pos) input_pos[slot] = position;
+    if (lens) lens[slot] = length;
+  }
+}
+
 // One thread per cell (slot b, block i) of the reference's block-index tables:
 // the block the ring-aware ragged kernel of the reference would work on from
 // that grid cell (engine.py:674-729).  end = (start + input_pos) % cache_len.
@@ -358,6 +375,24 @@ int32_t jpt_decode_advance(void* mask, int32_t mask_dtype, int64_t mask_stride, 
     hipLaunchKernelGGL(decode_advance_kernel<float>, grid, dim3(kThreads), 0, s, static_cast<float*>(mask),
                        mask_stride, input_pos, lens, batch, seq, ring_buffer, current_position, update_mask, advance);
   return launch_status("decode_advance_kernel");
+}
+
+int32_t jpt_insert_state(void* mask, int32_t mask_dtype, int64_t seq, int32_t* start, int32_t* input_pos, int32_t* lens,
+                         int32_t slot, int32_t first, int32_t position, int32_t length, int32_t lo, int32_t hi, int32_t wrap,
+                         void* stream) {
+  using namespace jpt;
+  JPT_REQUIRE(slot >= 0, "slot %d out of range", slot);
+  JPT_REQUIRE(!mask || (seq > 0 && seq < (1ll << 31)), "seq out of range");
+  JPT_REQUIRE(!mask || mask_dtype == JPT_F32 || mask_dtype == JPT_BF16, "mask_dtype must be f32 or bf16");
+  const dim3 grid(static_cast<unsigned>(mask ? (seq + kThreads - 1) / kThreads : 1));
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  if (mask_dtype == JPT_BF16)
+    hipLaunchKernelGGL(insert_state_kernel<uint16_t>, grid, dim3(kThreads), 0, s, static_cast<uint16_t*>(mask), seq, start,
+                       input_pos, lens, slot, first, position, length, lo, hi, wrap);
+  else
+    hipLaunchKernelGGL(insert_state_kernel<uint32_t>, grid, dim3(kThreads), 0, s, static_cast<uint32_t*>(mask), seq, start,
+                       input_pos, lens, slot, first, position, length, lo, hi, wrap);
+  return launch_status("insert_state_kernel");
 }
 
 int32_t jpt_ragged_block_indices(const int32_t* start, const int32_t* input_pos, int32_t batch, int32_t cache_len,

@@ -56,6 +56,16 @@ int vector_bytes(const jpt_line_tensor& t) {
   return 1;
 }
 
+// The two tensors of a stash copy side by side: grid.y = K or V.
+template <typename V>
+__global__ void __launch_bounds__(256)
+stash_lines_kernel(V* dst_k, const V* src_k, V* dst_v, const V* src_v, int64_t n) {
+  const int64_t i = blockIdx.x * static_cast<int64_t>(blockDim.x) + threadIdx.x;
+  if (i >= n) return;
+  if (blockIdx.y == 0) dst_k[i] = src_k[i];
+  else dst_v[i] = src_v[i];
+}
+
 // ---- fused quantiser -------------------------------------------------------
 
 struct QuantParams {
@@ -397,6 +407,24 @@ int32_t jpt_kv_scatter_lines(const jpt_line_tensor* tensors, int32_t n_tensors,
   dim3 grid(static_cast<unsigned>(blocks), n_tensors);
   hipLaunchKernelGGL(scatter_lines_kernel, grid, dim3(256), 0, static_cast<hipStream_t>(stream), p);
   return launch_status("scatter_lines_kernel");
+}
+
+int32_t jpt_kv_stash_lines(void* dst_k, const void* src_k, void* dst_v, const void* src_v, int64_t bytes, void* stream) {
+  using namespace jpt;
+  JPT_REQUIRE(dst_k && src_k && dst_v && src_v, "NULL argument");
+  JPT_REQUIRE(bytes >= 0 && bytes < (1ll << 38), "bytes out of range");
+  if (bytes == 0) return JPT_OK;
+  hipStream_t s = static_cast<hipStream_t>(stream);
+  const bool wide = bytes % 16 == 0 && aligned(dst_k, 16) && aligned(src_k, 16) && aligned(dst_v, 16) && aligned(src_v, 16);
+  const int64_t n = wide ? bytes / 16 : bytes;
+  const dim3 grid(static_cast<unsigned>((n + 255) / 256), 2);
+  if (wide)
+    hipLaunchKernelGGL(stash_lines_kernel<uint4>, grid, dim3(256), 0, s, static_cast<uint4*>(dst_k), static_cast<const uint4*>(src_k),
+                       static_cast<uint4*>(dst_v), static_cast<const uint4*>(src_v), n);
+  else
+    hipLaunchKernelGGL(stash_lines_kernel<uint8_t>, grid, dim3(256), 0, s, static_cast<uint8_t*>(dst_k),
+                       static_cast<const uint8_t*>(src_k), static_cast<uint8_t*>(dst_v), static_cast<const uint8_t*>(src_v), n);
+  return launch_status("stash_lines_kernel");
 }
 
 int32_t jpt_kv_append_quant_i8(const jpt_quant_append_args* args, void* stream) {

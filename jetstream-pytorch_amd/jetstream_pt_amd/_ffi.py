@@ -13,13 +13,17 @@ import torch
 _HERE = os.path.dirname(os.path.abspath(__file__))
 LIB_PATH = os.environ.get("JPT_MI355_LIB") or os.path.join(_HERE, "libjpt_mi355.so")
 
-if not os.path.exists(LIB_PATH):
+_HOST_PATH = os.path.join(_HERE, "_host.so")
+
+if not (os.path.exists(LIB_PATH) and os.path.exists(_HOST_PATH)):
   raise ImportError(
-      f"{LIB_PATH} is missing: build it with `python jetstream-pytorch_amd/build_lib.py` "
+      f"{LIB_PATH} or {_HOST_PATH} is missing: build it with `python jetstream-pytorch_amd/build_lib.py` "
       "(hipcc, gfx950). jetstream_pt_amd has no CPU or PyTorch fallback."
   )
 
 lib = ctypes.CDLL(LIB_PATH)
+
+from . import _host  # noqa: E402  (the host side of the hot calls, csrc/py_host.cpp)
 
 OK, E_BADARG, E_NOPAGES, E_PAGE_OVERFLOW, E_HIP = 0, -1, -2, -3, -4
 BF16, F32, I8 = 0, 1, 2
@@ -122,6 +126,7 @@ def _sig(name, restype, *argtypes):
 _sig("jpt_version", _i32)
 _sig("jpt_last_error", _c.c_char_p)
 _sig("jpt_kv_scatter_lines", _i32, _c.POINTER(LineTensor), _i32, _vp, _i32, _i32, _i32, _i32, _vp)
+_sig("jpt_kv_stash_lines", _i32, _vp, _vp, _vp, _vp, _i64, _vp)
 _sig("jpt_kv_append_quant_i8", _i32, _c.POINTER(QuantAppendArgs), _vp)
 _sig("jpt_rope", _i32, _vp, _vp, _vp, _i32, _i32, _i32, _i32, _vp)
 _sig("jpt_paged_insert", _i32, _vp, _vp, _vp, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _i32, _vp)
@@ -134,6 +139,7 @@ _sig("jpt_prefill_insert_layers", _i32, _c.POINTER(PrefillInsertArgs), _c.POINTE
 _sig("jpt_prefill_insert_prompts", _i32, _c.POINTER(PrefillInsertArgs), _c.POINTER(InsertPrompt), _i32, _vp)
 _sig("jpt_attn_workspace_bytes", _i64, _c.POINTER(AttnArgs))
 _sig("jpt_attn_plan", _i32, _c.POINTER(AttnArgs), _i32, _vp)
+_sig("jpt_attn_plan_fresh", _i32, _c.POINTER(AttnArgs), _i32, _vp)
 _sig("jpt_attn_ragged", _i32, _c.POINTER(AttnArgs), _vp)
 _sig("jpt_attn_dense", _i32, _c.POINTER(AttnArgs), _vp)
 _sig("jpt_attn_paged", _i32, _c.POINTER(AttnArgs), _vp)
@@ -154,6 +160,7 @@ _sig("jpt_dpam_reserve_insert", _i32, _c.POINTER(Dpam), _vp, _vp, _i32, _i32, _i
 _sig("jpt_dpam_free", _i32, _c.POINTER(Dpam), _vp, _i32, _i32, _vp)
 _sig("jpt_dpam_decode_step", _i32, _c.POINTER(Dpam), _vp, _vp)
 _sig("jpt_decode_advance", _i32, _vp, _i32, _i64, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _i32, _vp)
+_sig("jpt_insert_state", _i32, _vp, _i32, _i64, _vp, _vp, _vp, _i32, _i32, _i32, _i32, _i32, _i32, _i32, _vp)
 _sig("jpt_ragged_block_indices", _i32, _vp, _vp, _i32, _i32, _i32, _vp, _vp, _vp)
 
 EXPORTS = (
@@ -167,7 +174,7 @@ EXPORTS = (
     "jpt_pam_free_count", "jpt_paged_append_dev", "jpt_dpam_init", "jpt_dpam_reserve_insert",
     "jpt_dpam_free", "jpt_dpam_decode_step", "jpt_decode_advance", "jpt_rope",
     "jpt_ragged_block_indices", "jpt_prefill_insert_layers", "jpt_prefill_insert_prompts",
-    "jpt_attn_status", "jpt_attn_ragged_static",
+    "jpt_attn_status", "jpt_attn_ragged_static", "jpt_attn_plan_fresh", "jpt_kv_stash_lines", "jpt_insert_state",
 )
 
 
@@ -228,13 +235,28 @@ def ptr(t):
   return None if t is None else _vp(t.data_ptr())
 
 
+def raw_stream():
+  """The current device's current stream, as an integer (torch.cuda.current_stream()
+  builds two objects and costs some microseconds)."""
+  return torch._C._cuda_getCurrentRawStream(torch._C._cuda_getDevice())
+
+
 def stream():
-  return _vp(torch.cuda.current_stream().cuda_stream)
+  return _vp(raw_stream())
+
+
+def addresses():
+  """The library's entry points as integers, for the native host side (_host)."""
+  return {name: _c.cast(getattr(lib, name), _vp).value for name in EXPORTS}
 
 
 def as_i32(x, device, n=None):
   """Positions / lengths as an int32 device tensor (accepts lists, numpy, any int dtype)."""
   if isinstance(x, torch.Tensor):
+    if x.dtype is torch.int32 and x.dim() == 1 and x.is_contiguous() and x.device == torch.device(device):
+      if n is not None and x.numel() != n:
+        raise ValueError(f"expected {n} entries, got {x.numel()}")
+      return x
     t = x.to(device=device, dtype=torch.int32).reshape(-1)
   else:
     import numpy as np

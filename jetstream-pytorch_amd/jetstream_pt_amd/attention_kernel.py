@@ -33,7 +33,7 @@ import weakref
 
 import torch
 
-from . import _ffi
+from . import _ffi, _host
 from .quantize import _rounding_code
 
 
@@ -44,10 +44,15 @@ _live_workspaces = weakref.WeakSet()  # every workspace still in use, for check_
 
 
 class _Workspace:
-  """Device scratch for the split-KV kernel; the leading state block stays zero."""
+  """Device scratch for the split-KV kernels; the leading state block starts at
+  zero (what lies behind it is written before it is read).  `buf`: a workspace
+  that a planning launch has already been given."""
 
-  def __init__(self, nbytes, device):
-    self.buf = torch.zeros(nbytes, dtype=torch.uint8, device=device)
+  def __init__(self, nbytes, device, buf=None):
+    if buf is None:
+      buf = torch.empty(nbytes, dtype=torch.uint8, device=device)
+      buf[:_ffi.ATTN_WS_STATE_BYTES].zero_()
+    self.buf = buf
     _live_workspaces.add(self)
 
   @property
@@ -106,12 +111,43 @@ def check_status(plan=None):
 
 def _shared_workspace(nbytes, device):
   # one per (device, stream): calls that share a workspace must not overlap
-  key = (torch.device(device), torch.cuda.current_stream(device).cuda_stream)
+  index = device if isinstance(device, int) else torch.device(device).index
+  index = torch._C._cuda_getDevice() if index is None else index
+  key = (index, torch._C._cuda_getCurrentRawStream(index))
   ws = _workspaces.get(key)
   if ws is None or ws.nbytes < nbytes:
-    ws = _Workspace(nbytes, device)
+    ws = _Workspace(nbytes, torch.device("cuda", index))
     _workspaces[key] = ws
   return ws
+
+
+def _dense_workspace(index, batch, q_heads, kv_heads, q_rows, seq):
+  """The workspace of a dense call without lengths and whether it holds a plan.
+  Every slot attends all `seq` positions: the split depends on the shape only,
+  so it is planned once per (stream, shape) into a workspace of its own; the
+  least recently used of these is dropped when there are too many."""
+  key = (index, torch._C._cuda_getCurrentRawStream(index), batch, q_heads, kv_heads, q_rows, seq)
+  ws = _dense_workspaces.get(key)
+  if ws is not None:
+    _dense_workspaces.move_to_end(key)
+    return ws, True
+  a = _ffi.AttnArgs(batch=batch, q_heads=q_heads, kv_heads=kv_heads, q_rows=q_rows, seq=seq)
+  ws = _Workspace(_ffi.lib.jpt_attn_workspace_bytes(a), torch.device("cuda", index))
+  a.workspace, a.workspace_bytes = _ffi.ptr(ws.buf), ws.nbytes
+  planned = _ffi.lib.jpt_attn_plan(a, 0, _ffi.stream()) == _ffi.OK
+  if planned:
+    _dense_workspaces[key] = ws
+    while len(_dense_workspaces) > _MAX_DENSE_WORKSPACES:
+      _dense_workspaces.popitem(last=False)
+  return ws, planned
+
+
+def _dense_workspace_buf(*shape):
+  ws, planned = _dense_workspace(*shape)
+  return ws.buf, planned
+
+
+_host.bind(_ffi.addresses(), _ffi.check, lambda nbytes, index: _shared_workspace(nbytes, index).buf, _dense_workspace_buf)
 
 
 class DecodePlan:
@@ -123,19 +159,29 @@ class DecodePlan:
     self.lengths = _ffi.dev(lengths, "lengths")
     self.paged = page_size is not None
     self.key = (batch, q_heads, kv_heads, q_rows, seq, page_size, max_pages)
-    args = _ffi.AttnArgs(
-        lengths=_ffi.ptr(lengths), batch=batch, q_heads=q_heads, kv_heads=kv_heads,
-        q_rows=q_rows, seq=seq or 0, page_size=page_size or 0, max_pages=max_pages or 0)
-    nbytes = _ffi.lib.jpt_attn_workspace_bytes(args)
-    self.workspace = _Workspace(nbytes, lengths.device)
-    args.workspace = _ffi.ptr(self.workspace.buf)
-    args.workspace_bytes = nbytes
-    self._args = args
+    self._shape = (batch, q_heads, kv_heads, q_rows, seq or 0, page_size or 0, max_pages or 0)
+    buf = _host.plan(lengths, *self._shape, None)
+    if buf is not None:
+      self.workspace = _Workspace(0, None, buf)
+      self.buf = buf
+      return
+    args = self._args()
+    self.workspace = _Workspace(_ffi.lib.jpt_attn_workspace_bytes(args), lengths.device)
+    self.buf = self.workspace.buf
     self.replan()
+
+  def _args(self):
+    b, hq, hkv, t, seq, ps, mp = self._shape
+    return _ffi.AttnArgs(lengths=_ffi.ptr(self.lengths), batch=b, q_heads=hq, kv_heads=hkv, q_rows=t, seq=seq,
+                         page_size=ps, max_pages=mp)
 
   def replan(self):
     """Plans again for the current contents of `lengths` (same tensor, same workspace)."""
-    _ffi.check(_ffi.lib.jpt_attn_plan(self._args, int(self.paged), _ffi.stream()))
+    if _host.plan(self.lengths, *self._shape, self.buf) is not None:
+      return
+    args = self._args()
+    args.workspace, args.workspace_bytes = _ffi.ptr(self.buf), self.buf.numel()
+    _ffi.check(_ffi.lib.jpt_attn_plan(args, int(self.paged), _ffi.stream()))
 
 
 def paged_decode_plan(pam, lengths, batch, q_heads, kv_heads, page_size, max_pages):
@@ -179,13 +225,25 @@ def _scale_tensor(s, paged):
   return _ffi.dev(s, "scaler"), s.shape[0 if paged else 1]
 
 
+_MODES = {"ragged": 0, "dense": 1, "paged": 2}
+
+
 def _attend(mode, xq, keys, values, *, lengths=None, page_table=None, mask=None,
             k_scaler=None, v_scaler=None, sm_scale=None, new_key=None,
             new_value=None, new_k_scaler=None, new_v_scaler=None, new_key_raw=None,
             new_value_raw=None, new_rounding="trunc", new_key_rope=None, new_to_pages=False,
-            want_stats=False, plan=None, force_generic=False):
-  """xq (B, Hq, T, D); keys/values (B, Hkv, S, D) or pages (Hkv, P, ps, D).
+            want_stats=False, plan=None, force_generic=False, layer=-1):
+  """xq (B, Hq, T, D); keys/values (B, Hkv, S, D), or stacks of them with `layer`
+  picking one, or pages (Hkv, P, ps, D).
   Returns (o (B, Hq, T, D), max (B, Hq, T) | None, denom (B, Hq, T) | None)."""
+  if not force_generic:
+    r = _host.attend(_MODES[mode], xq, keys, values, layer, lengths, page_table, mask, k_scaler, v_scaler, sm_scale,
+                     new_key, new_value, new_k_scaler, new_v_scaler, new_key_raw, new_value_raw,
+                     0 if new_key_raw is None else _rounding_code(new_rounding), new_key_rope, new_to_pages, want_stats, plan)
+    if r is not None:
+      return r
+  # not the ordinary case (contiguous device tensors of the library's dtypes): converted, or refused, here
+  keys, values, k_scaler, v_scaler = _pick_layer(keys, values, layer, k_scaler, v_scaler)
   xq = _ffi.dev(xq, "xq")
   keys, values = _ffi.dev(keys, "keys"), _ffi.dev(values, "values")
   b, hq, t, d = xq.shape
@@ -299,23 +357,8 @@ def _attend(mode, xq, keys, values, *, lengths=None, page_table=None, mask=None,
       and plan.lengths.data_ptr() == lengths.data_ptr():
     ws, a.reuse_plan = plan.workspace, 1
   elif lengths is None and mode == "dense":
-    # every slot attends all `seq` positions: the split depends on the shape
-    # only, so it is planned once per (stream, shape) into a workspace of its
-    # own; the least recently used of these is dropped when there are too many
-    key = (torch.device(device), torch.cuda.current_stream(device).cuda_stream, b, hq, hkv, t, a.seq)
-    ws = _dense_workspaces.get(key)
-    if ws is None:
-      ws = _Workspace(_ffi.lib.jpt_attn_workspace_bytes(a), device)
-      pa = _ffi.AttnArgs(batch=b, q_heads=hq, kv_heads=hkv, q_rows=t, seq=a.seq,
-                         workspace=_ffi.ptr(ws.buf), workspace_bytes=ws.nbytes)
-      if _ffi.lib.jpt_attn_plan(pa, 0, _ffi.stream()) == _ffi.OK:
-        _dense_workspaces[key] = ws
-        a.reuse_plan = 1
-        while len(_dense_workspaces) > _MAX_DENSE_WORKSPACES:
-          _dense_workspaces.popitem(last=False)
-    else:
-      _dense_workspaces.move_to_end(key)
-      a.reuse_plan = 1
+    ws, planned = _dense_workspace(device.index, b, hq, hkv, t, a.seq)
+    a.reuse_plan = int(planned)
   else:
     ws = _shared_workspace(_ffi.lib.jpt_attn_workspace_bytes(a), device)
   if ws is not None:
@@ -372,10 +415,9 @@ def flash_attention(xq, keys, values, layer, k_scaler=None, v_scaler=None, mask=
                     normalize_var=True):
   """Same attention, also returning the row max and the softmax denominator:
   o (B, Hq, T, D), (max, denom) each (B, Hq, T, 1)."""
-  keys, values, k_scaler, v_scaler = _pick_layer(keys, values, layer, k_scaler, v_scaler)
   sm = None if normalize_var else 1.0
   out, mx, den = _attend("dense", xq, keys, values, mask=mask, k_scaler=k_scaler,
-                         v_scaler=v_scaler, sm_scale=sm, want_stats=True)
+                         v_scaler=v_scaler, sm_scale=sm, want_stats=True, layer=layer)
   return out, (mx.unsqueeze(-1), den.unsqueeze(-1))
 
 
@@ -393,14 +435,13 @@ def ragged_mha(q, k, v, layer, start, end, ragged_batch_index=None,
   carry a DecodePlan (see precompute_ragged_block_indices).
   """
   del start, ragged_block_index, bk, mask_value, q_shard_axis, kv_shard_axis, testing
-  k, v, k_scaler, v_scaler = _pick_layer(k, v, layer, k_scaler, v_scaler)
   plan = ragged_batch_index if isinstance(ragged_batch_index, DecodePlan) else None
   out, mx, den = _attend(
       "ragged", q, k, v, lengths=end, k_scaler=k_scaler, v_scaler=v_scaler,
       sm_scale=None if normalize_var else 1.0, new_key=new_key, new_value=new_value,
       new_k_scaler=new_k_scaler, new_v_scaler=new_v_scaler, new_key_raw=new_key_raw,
       new_value_raw=new_value_raw, new_rounding=new_rounding, new_key_rope=new_key_rope,
-      want_stats=True, plan=plan)
+      want_stats=True, plan=plan, layer=layer)
   bq, hq, tq, dq = q.shape
   hkv = k.shape[-3]
   rows = hq // hkv * tq

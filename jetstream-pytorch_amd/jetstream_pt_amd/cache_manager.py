@@ -20,7 +20,7 @@ Keyword-only additions on Int8KVCacheGenerate, defaults reference-literal:
 
 import torch
 
-from . import _ffi
+from . import _ffi, _host
 from .page_attention_manager import DeviceTokenIndices, PageAttentionManager
 from .quantize import _rounding_code
 
@@ -61,6 +61,8 @@ class KVCachePrefill:
 
 def _scatter_lines(pairs, pos, pos_count, n_layers, batch, seq):
   """pairs: [(dst (L?, B, H, S, X), src (L?, B, H, 1, X))]; one launch."""
+  if _host.scatter_lines(tuple(d for d, _ in pairs), tuple(s for _, s in pairs), pos, pos_count, n_layers, batch, seq):
+    return
   arr = (_ffi.LineTensor * len(pairs))()
   for i, (dst, src) in enumerate(pairs):
     _ffi.dev(dst, "cache"), _ffi.dev(src, "new line")

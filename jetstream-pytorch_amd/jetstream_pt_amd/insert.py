@@ -13,11 +13,14 @@ the prompt's dtype.
 
 import torch
 
-from . import _ffi
+from . import _ffi, _host
+
+
+_ROUNDING = {"trunc": _ffi.ROUND_TRUNC, "rne": _ffi.ROUND_RNE}
 
 
 def _rounding_code(rounding):
-  return {"trunc": _ffi.ROUND_TRUNC, "rne": _ffi.ROUND_RNE}[rounding]
+  return _ROUNDING[rounding]
 
 
 def _layer_views(cache, layer, n_layers):
@@ -41,6 +44,8 @@ def insert_prefix_caches(prefix_caches, caches, cache_scales, slot, start, *, ro
   each (B, Hs, S, 1) / (L, B, Hs, S, 1).  int8 caches are quantised into;
   float caches take a copy (cast to the cache dtype first).
   """
+  if _host.insert_layers(prefix_caches, caches, cache_scales, None, int(slot), int(start), _ROUNDING.get(rounding)):
+    return
   n_layers = len(prefix_caches)
   layers, keep, common, shape = [], [], None, None
   for layer, (newk, newv) in enumerate(prefix_caches):
@@ -120,6 +125,8 @@ def insert_prefix_pages_copy(prefix_caches, decode_caches, page_ids):
   83-142).  Needs head_dim % 4 == 0 and layers of one shape and dtype; returns
   False, having done nothing, when that does not hold."""
   ids = _ffi.as_i32(page_ids, decode_caches[0][0].device)
+  if _host.insert_layers(prefix_caches, decode_caches, None, ids, 0, 0, 0):
+    return True
   layers, keep, common, shape = [], [ids], None, None
   for (newk, newv), (pk, pv) in zip(prefix_caches, decode_caches):
     if not (pk.is_cuda and pk.is_contiguous() and pv.is_contiguous()) or pk.dtype not in (torch.bfloat16, torch.float32):
@@ -216,21 +223,17 @@ def insert(env, prefix_caches, prefix_seq_len, caches, cache_scales, slot, *, cu
     cur = current_position
   else:
     wrap, cur = False, prefix_seq_len
-  if not wrap:
-    pos = cur - prefix_seq_len
-    insert_prefix_caches(prefix_caches, caches, cache_scales, slot, pos)
-    first = pos % seq
-    if mask is not None:
-      x = torch.arange(seq, device=mask.device)
-      mask[slot] = torch.where((x < cur) & (x >= pos), 0.0, float("-inf")).to(mask.dtype)
-  else:
-    first = (current_position - prefix_seq_len) % seq
-    insert_prefix_caches(prefix_caches, caches, cache_scales, slot, first)
-    if mask is not None:
-      x = torch.arange(seq, device=mask.device)
-      cond = ((x >= first) & (x < current_position)) if current_position > first else \
-          ((x >= first) | (x < current_position))
-      mask[slot] = torch.where(cond, 0.0, float("-inf")).to(mask.dtype)
+  first = (cur - prefix_seq_len) % seq if not wrap else (current_position - prefix_seq_len) % seq
+  insert_prefix_caches(prefix_caches, caches, cache_scales, slot, cur - prefix_seq_len if not wrap else first)
+  # the slot's live positions: [lo, hi), or with `over_end` [lo, seq) and [0, hi)
+  lo, hi = (cur - prefix_seq_len, cur) if not wrap else (first, current_position)
+  over_end = wrap and not current_position > first
+  if _host.insert_state(mask, start, input_pos, lens, slot, first, prefix_seq_len, lo, hi, over_end):
+    return first
+  if mask is not None:
+    x = torch.arange(seq, device=mask.device)
+    live = ((x >= lo) | (x < hi)) if over_end else ((x >= lo) & (x < hi))
+    mask[slot] = torch.where(live, 0.0, float("-inf")).to(mask.dtype)
   if start is not None:
     start[slot] = first
   if input_pos is not None:

@@ -18,10 +18,11 @@ projections, RoPE and norms are outside the KV path.
 
 import torch
 
-from . import _ffi
+from . import _ffi, _host, scopes
 from . import attention_kernel as ak
+from .cache_manager import Int8KVCacheGenerate, Int8PageKVCacheGenerate, KVCacheGenerate, PageKVCacheGenerate
+from .quantize import _rounding_code
 from .scopes import scoped
-from .cache_manager import Int8KVCacheGenerate
 
 
 def apply_rotary_emb(xq, xk, freqs_cis):
@@ -107,11 +108,51 @@ class AttentionKernel:
     return (self.fuse_new_token and env.lazy_cache_update and seqlen == 1 and env.ragged_mha
             and keys.shape[-2] > 1)
 
+  def _native_step(self, xq, xk, xv, mask, cache, end, plan, freqs_cis):
+    """A decode step's layer in one native call - cache update, attention, the token
+    merged - in the modes a serving loop runs: the stacked lazy cache with ragged
+    attention, the eagerly written cache under a mask, pages with the device
+    allocator.  None, with nothing returned yet, where the call is anything else:
+    it then goes the general way below, launch by launch."""
+    env = self.env
+    kind = type(cache)
+    if kind is KVCacheGenerate or kind is Int8KVCacheGenerate:
+      int8 = kind is Int8KVCacheGenerate
+      ks, vs, rounding = (cache.k_scaler, cache.v_scaler, _rounding_code(cache.rounding)) if int8 else (None, None, 0)
+      if env.lazy_cache_update:
+        if not (env.ragged_mha and env.generate_cache_stacked and env.new_cache_stacked and self.fuse_new_token):
+          return None
+        if int8 and not self.fuse_quantize:
+          return None
+        return _host.lazy_step(xq, xk, xv, cache.cache_k, cache.cache_v, ks, vs, cache.new_ks, cache.new_vs,
+                               cache.new_k_scaler if int8 else None, cache.new_v_scaler if int8 else None, self.layer_id,
+                               end, plan if isinstance(plan, ak.DecodePlan) else None, rounding, freqs_cis)
+      if env.ragged_mha or env.flash_attention or env.generate_cache_stacked or env.new_cache_stacked:
+        return None
+      return _host.eager_step(xq, xk, xv, mask, cache.cache_k, cache.cache_v, ks, vs, cache.input_pos, env.ring_buffer,
+                              rounding, freqs_cis)
+    if kind is PageKVCacheGenerate or kind is Int8PageKVCacheGenerate:
+      pam = cache.page_attention_manager
+      lens = getattr(pam, "step_lens", None)
+      if lens is None or not (env.page_attention and self.fuse_new_token) or env.ragged_mha or env.flash_attention:
+        return None
+      pages, table = cache.cache_k, pam.page_indices
+      step_plan = ak.paged_decode_plan(pam, lens, xq.shape[0], xq.shape[1], pages.shape[0], pages.shape[2], table.shape[1])
+      int8 = kind is Int8PageKVCacheGenerate
+      return _host.paged_step(xq, xk, xv, pages, cache.cache_v, cache.k_scaler if int8 else None,
+                              cache.v_scaler if int8 else None, lens, table, step_plan, self.sm_scale_paged,
+                              _rounding_code(cache.rounding) if int8 else 0, freqs_cis)
+    return None
+
   def __call__(self, xq, xk, xv, mask, cache, start=None, end=None, ragged_batch_index=None,
                ragged_block_index=None):
     """xq (batch, heads, seqlen, head_dim); xk, xv (batch, kv_heads, seqlen, head_dim);
     mask additive 0/-inf or None; cache a CacheInterface object."""
     seqlen = xq.shape[2]
+    if seqlen == 1 and not scopes.ENABLED:
+      out = self._native_step(xq, xk, xv, mask, cache, end, ragged_batch_index, None)
+      if out is not None:
+        return out
     args = (cache, start, end, ragged_batch_index, ragged_block_index)
     if hasattr(cache, "page_attention_manager") and self._will_append_in_launch(xq, cache, cache.cache_k):
       keys, values = scoped("attn_insert_cache", cache.update, xk, xv, self.layer_id, defer_append=True)
@@ -143,6 +184,10 @@ class Int8KVAttentionKernel(AttentionKernel):
     through apply_rotary_emb; the launch that quantises the key rotates it first
     (xq must come rotated).  One token per slot only."""
     seqlen = xq.shape[2]
+    if seqlen == 1 and not scopes.ENABLED:
+      out = self._native_step(xq, xk, xv, mask, cache, end, ragged_batch_index, freqs_cis)
+      if out is not None:
+        return out
     if freqs_cis is not None and (xk.shape[2] != 1 or not hasattr(cache, "rounding")):
       # no quantiser launch to fold the rotation into: rotate here
       xk = apply_rotary_emb(None, xk.transpose(1, 2), freqs_cis)[1].transpose(1, 2)

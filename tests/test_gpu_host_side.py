@@ -1,0 +1,95 @@
+"""The native host side (jetstream_pt_amd._host) against the general Python way: the same call with
+inputs it does not take (which go the general way) and with inputs it does gives the same bits; and
+the small launches it uses, at their edges."""
+
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+DEV = "cuda"
+
+
+def _step(int8, ring, strided, dim):
+  """One layer of a decode step; `strided`: the token's rows are not contiguous."""
+  from jetstream_pt_amd import attention_kernel as ak
+  from jetstream_pt_amd import cache_manager as cm
+  from jetstream_pt_amd import layers
+  from jetstream_pt_amd.environment import JetEngineEnvironment, JetEngineEnvironmentData
+  g = torch.Generator().manual_seed(31)
+  b, hq, hkv, s, nl = 3, 8, 2, 96, 2
+  env = JetEngineEnvironment(JetEngineEnvironmentData(batch_size=b, num_layers=nl, ring_buffer=ring))
+  kind = cm.Int8KVCacheGenerate if int8 else cm.KVCacheGenerate
+  cache = kind.empty((b, hkv, s, dim) if ring else (nl, b, hkv, s, dim), DEV, env)
+  for t in (cache.cache_k, cache.cache_v):
+    t.copy_(torch.randint(-100, 100, t.shape, generator=g) if int8 else torch.randn(t.shape, generator=g))
+  rows = lambda h: torch.randn((b, h, dim, 2), generator=g).to(torch.bfloat16).to(DEV)[..., 0].unsqueeze(2)
+  xq, xk, xv = rows(hq).contiguous(), rows(hkv), rows(hkv)
+  if not strided:
+    xk, xv = xk.contiguous(), xv.contiguous()
+  kern = (layers.Int8KVAttentionKernel if int8 else layers.AttentionKernel)(env, 1)
+  if ring:
+    cache.input_pos = torch.tensor([40], dtype=torch.int32, device=DEV)
+    mask = torch.zeros((b, 1, 1, s), device=DEV)
+    mask[:, :, :, 41:] = float("-inf")
+    out = kern(xq, xk, xv, mask, cache)
+  else:
+    pos = torch.tensor([0, 33, 95], dtype=torch.int32, device=DEV)
+    cache.input_pos = pos
+    plan, _ = ak.precompute_ragged_block_indices(pos, b, hq, hkv, s)
+    out = kern(xq, xk, xv, None, cache, start=None, end=plan.lengths, ragged_batch_index=plan)
+    cache.finalize()
+  return [out, cache.cache_k, cache.cache_v] + ([cache.k_scaler, cache.v_scaler] if int8 else [])
+
+
+@pytest.mark.parametrize("dim", [128, 64])
+@pytest.mark.parametrize("ring", [False, True])
+@pytest.mark.parametrize("int8", [False, True])
+def test_a_step_is_the_same_bits_whichever_way_it_goes(int8, ring, dim):
+  for a, b in zip(_step(int8, ring, False, dim), _step(int8, ring, True, dim)):
+    assert torch.equal(a, b)
+
+
+@pytest.mark.parametrize("n,skip", [(1, 0), (15, 1), (16, 0), (4096, 0), (4100, 0), (65552, 16), (1000, 3)])
+def test_stash_lines(n, skip):
+  from jetstream_pt_amd import _ffi
+  src = torch.arange(2 * (n + skip), device=DEV).to(torch.uint8)
+  dst = torch.full((2, n + skip + 64), 77, dtype=torch.uint8, device=DEV)
+  _ffi.check(_ffi.lib.jpt_kv_stash_lines(dst[0, skip:].data_ptr(), src[skip:].data_ptr(), dst[1, skip:].data_ptr(),
+                                         src[n + skip:].data_ptr(), n, _ffi.stream()))
+  assert torch.equal(dst[0, skip:skip + n], src[skip:skip + n]) and torch.equal(dst[1, skip:skip + n], src[n + skip:][:n])
+  assert bool((dst[:, :skip] == 77).all() and (dst[:, skip + n:] == 77).all())
+
+
+@pytest.mark.parametrize("dtype", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("seq,lo,hi,wrap", [(1, 0, 1, False), (300, 0, 300, False), (300, 17, 256, False), (300, 290, 5, True), (512, 100, 100, True)])
+def test_insert_state(seq, lo, hi, wrap, dtype):
+  from jetstream_pt_amd import _host
+  mask = torch.ones((3, seq), dtype=dtype, device=DEV)
+  rows = [torch.full((3,), -5, dtype=torch.int32, device=DEV) for _ in range(3)]
+  assert _host.insert_state(mask, *rows, 1, 7, 9, lo, hi, wrap)
+  x = torch.arange(seq)
+  live = ((x >= lo) | (x < hi)) if wrap else ((x >= lo) & (x < hi))
+  assert torch.equal(mask[1].cpu(), torch.where(live, 0.0, float("-inf")).to(dtype))
+  assert bool((mask[0] == 1).all() and (mask[2] == 1).all())
+  assert [r.tolist() for r in rows] == [[-5, 7, -5], [-5, 9, -5], [-5, 1, -5]]
+
+
+@pytest.mark.parametrize("dim,seq", [(128, 256), (128, 250), (64, 256)])
+def test_a_fresh_plan_needs_no_cleared_workspace(dim, seq):
+  """torch hands out used memory: a plan on a workspace full of other data gives the same outputs
+  and no status bit (seq 250 and dim 64 run on the kernel whose counters lie in the state block)."""
+  from jetstream_pt_amd import attention_kernel as ak
+  g = torch.Generator().manual_seed(7)
+  b, hq, hkv = 5, 8, 4
+  q = torch.randn((b, hq, 1, dim), generator=g).to(torch.bfloat16).to(DEV)
+  k, v = (torch.randn((b, hkv, seq, dim), generator=g).to(torch.bfloat16).to(DEV) for _ in range(2))
+  end = torch.tensor([seq - 1, 0, 31, 100, 129], dtype=torch.int32, device=DEV)
+  outs = []
+  for fill in (0, 255, 1):
+    torch.cuda.synchronize()
+    junk = torch.full((64 << 20,), fill, dtype=torch.uint8, device=DEV)
+    del junk  # the next allocation is cut from it
+    plan, _ = ak.precompute_ragged_block_indices(end, b, hq, hkv, seq)
+    outs.append(ak.ragged_mha(q, k, v, 0, None, plan.lengths, plan)[0])
+    assert ak.check_status(plan) == 0
+  assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
