@@ -84,9 +84,10 @@ __device__ __forceinline__ uint32_t pack_bf16(float lo, float hi) {
 
 // 16 bytes a lane from memory to LDS at `lds` + 16 * lane, not known to the
 // compiler as an LDS write: it would make every later LDS read wait for all
-// such loads, the next tile's among them.
+// such loads, the next tile's among them.  A write of M0 needs one wait state
+// before the load that uses it, which the compiler does not see to inside asm.
 __device__ __forceinline__ void load_to_lds(const char* base, uint32_t lane_off, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %2\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(lane_off), "s"(base), "s"(lds) : "memory");
+  asm volatile("s_mov_b32 m0, %2\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, %1" : : "v"(lane_off), "s"(base), "s"(lds) : "memory");
 }
 
 // Where 16-byte piece p of row t lies in its row: p ^ swizzle(t).  Sixteen

@@ -164,9 +164,10 @@ template <int D, typename KV>
 constexpr int split_waves_per_simd() { return D == 256 && sizeof(KV) == 2 ? 1 : 2; }
 
 // 16 bytes a lane from memory to LDS at `lds` + 16 * lane, not known to the compiler as an LDS write
-// (which would make every later LDS access wait for all loads in flight).
+// (which would make every later LDS access wait for all loads in flight).  A write of M0 needs one
+// wait state before the load that uses it, which the compiler does not see to inside asm.
 __device__ __forceinline__ void stage_to_lds(const char* from, uint32_t lds) {
-  asm volatile("s_mov_b32 m0, %1\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(from), "s"(lds) : "memory");
+  asm volatile("s_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %0, off" : : "v"(from), "s"(lds) : "memory");
 }
 
 template <int D, typename KV, int SCALE, bool MASK, int RC>
