@@ -729,9 +729,20 @@ static int32_t attn_entry(const jpt_attn_args* args, jpt::AttnMode mode, void* s
   int32_t st = check_attn_args(*args, mode);
   if (st != JPT_OK) return st;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  if (attn_fast_supported(*args, mode)) return attn_fast_launch(*args, mode, s);
+  // The attention launch can quantise the step's token itself, but every KV head's item then does
+  // the slot's whole token (its scale spans the heads), key rotation included, while the rest of its
+  // tiles wait in the ring: batch * kv_heads * kv_heads rows.  A launch of its own in front does each
+  // token once and costs a layer about 4 us.  Rotated keys, us a layer in one launch / in two:
+  // 32 KV heads, bf16 scales: 96 slots 174 / 139, 32 slots 43 / 39, 8 slots 29 / 28, 4 slots 25 / 25;
+  // 16 heads: 192 slots 158 / 138, 8 slots 22 / 25; 8 heads: 384 slots 143 / 133, 128 ragged slots
+  // 41 / 38, 16 slots 24 / 25; 4 heads, 384 slots 107 / 106.  Keys that come rotated: one launch is
+  // the better one, or as good, throughout (32 heads: 96 slots 139 / 139, 32 slots 34 / 38).
+  constexpr int64_t kRotateFirst = 8192;
+  const bool quantise_first = args->new_k_raw && args->new_k_rope &&
+                              static_cast<int64_t>(args->batch) * args->kv_heads * args->kv_heads >= kRotateFirst;
+  if (!quantise_first && attn_fast_supported(*args, mode)) return attn_fast_launch(*args, mode, s);
   jpt_attn_args a = *args;
-  if (a.new_k_raw) {  // no fused quantiser on this route: quantise first, then attend the codes
+  if (a.new_k_raw) {  // quantise first, then attend the codes
     jpt_quant_append_args q{};
     q.new_k = a.new_k_raw;
     q.new_v = a.new_v_raw;

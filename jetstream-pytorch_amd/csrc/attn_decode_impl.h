@@ -953,8 +953,8 @@ __global__ void __launch_bounds__(kThreads, kWavesPerSimd) attn_decode_kernel(Fa
           tv = static_cast<const char*>(a.new_v_raw) + raw;
         }
         // float32 scales of the new token come through the ring like any
-        // tile's; bf16 ones are read by the consumer, and the tile loads the
-        // head of the scale tensors only to keep its load count
+        // tile's; bf16 ones are read by the consumers at the item's start, and the
+        // tile loads the head of the scale tensors only to keep its load count
         const char* sc = scale_lane;
         if (SCALE == kScaleF32) sc = new_scale_lane + (static_cast<int64_t>(cur.slot) * a.scale_heads + hs) * kEs;
         const float* mk = MASK ? static_cast<const float*>(a.mask) + cur.slot * a.mask_stride_b : nullptr;
@@ -1152,6 +1152,9 @@ __global__ void __launch_bounds__(kThreads, kWavesPerSimd) attn_decode_kernel(Fa
   uint32_t keep_k = 0, keep_v = 0;
   float keep_ks = 0.f, keep_vs = 0.f;
   bool keep = false;
+  // bf16 scales of a token that comes quantised (float32 ones travel through the ring)
+  constexpr bool given_scales = SCALE == kScaleBF16 && has_new && !quant_new;
+  uint16_t given_ks = 0, given_vs = 0;
   // Chunks of split slots.  A chunk's partial must be in memory, where the
   // workgroups of every XCD see it, before the chunk is counted as arrived; the
   // wave that parked it does not wait for that: it sends the count after its
@@ -1204,10 +1207,8 @@ __global__ void __launch_bounds__(kThreads, kWavesPerSimd) attn_decode_kernel(Fa
       const float4 k0 = sk[g], k1 = sk[4 + g], v0 = sk[8 + g], v1 = sk[12 + g];
       ks[0] = k0.x; ks[1] = k0.y; ks[2] = k0.z; ks[3] = k0.w; ks[4] = k1.x; ks[5] = k1.y; ks[6] = k1.z; ks[7] = k1.w;
       vs[0] = v0.x; vs[1] = v0.y; vs[2] = v0.z; vs[3] = v0.w; vs[4] = v1.x; vs[5] = v1.y; vs[6] = v1.z; vs[7] = v1.w;
-    } else if (SCALE == kScaleBF16 && is_new) {
-      const int64_t si = static_cast<int64_t>(cur_slot) * a.scale_heads + (a.scale_heads == 1 ? 0 : cur_h);
-      const float nks = load_as_f32(a.new_k_scale, si, JPT_BF16);
-      const float nvs = load_as_f32(a.new_v_scale, si, JPT_BF16);
+    } else if (SCALE == kScaleBF16 && is_new && !quant_new) {  // asked for at the item's start
+      const float nks = bf16_bits_to_f32(given_ks), nvs = bf16_bits_to_f32(given_vs);
 #pragma unroll
       for (int i = 0; i < 8; ++i) { ks[i] = nks; vs[i] = nvs; }
     } else if (SCALE == kScaleBF16) {
@@ -1435,6 +1436,11 @@ __global__ void __launch_bounds__(kThreads, kWavesPerSimd) attn_decode_kernel(Fa
     const bool dst_room = cur.len < a.max_pages * a.page_size;
     if (to_pages && cur.start == 0 && cur.len > 0 && dst_room)
       dst_page = a.page_table[static_cast<int64_t>(cur.slot) * a.max_pages + cur.len / a.page_size];
+    if (given_scales && nt > n_cache) {
+      const int64_t si = static_cast<int64_t>(cur.slot) * a.scale_heads + (a.scale_heads == 1 ? 0 : cur.h);
+      given_ks = static_cast<const uint16_t*>(a.new_k_scale)[si];
+      given_vs = static_cast<const uint16_t*>(a.new_v_scale)[si];
+    }
 #pragma unroll
     for (int j = 0; j < 8; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
     accw = f32x4{0.f, 0.f, 0.f, 0.f};

@@ -93,6 +93,32 @@ def test_attention_launch_rotates_and_quantises_the_new_token(sdt, per_head, hq,
   assert torch.equal(got[3].cpu(), wc) and torch.equal(got[5].cpu().reshape(-1), ws.to(sdt).reshape(-1))
 
 
+@pytest.mark.parametrize("b,hq,hkv", [(8, 32, 32), (33, 16, 16), (128, 32, 8)])
+@pytest.mark.parametrize("sdt,per_head", [(torch.float32, False), (torch.bfloat16, False), (torch.bfloat16, True)])
+def test_many_rotated_tokens_are_quantised_ahead_of_the_launch(sdt, per_head, b, hq, hkv):
+  """From batch * kv_heads^2 = 8192 on the token is rotated and quantised by a launch of its own: codes and
+  scales are the quantiser's, the outputs those of the call that is given them, bit for bit."""
+  from jetstream_pt_amd import attention_kernel as ak
+  from jetstream_pt_amd.quantize import quantize_kv
+  s, d = 96, 128
+  g = torch.Generator().manual_seed(5)
+  xq, xk, xv, freqs = step_inputs(b, hq, hkv, d, 5)
+  end = torch.randint(0, s + 1, (b,), generator=g, dtype=torch.int32).to(DEV)
+  hs = hkv if per_head else 1
+  k, v = (torch.randint(-127, 128, (b, hkv, s, d), generator=g, dtype=torch.int8).to(DEV) for _ in range(2))
+  ks, vs = ((torch.rand((b, hs, s, 1), generator=g) * 0.045 + 0.005).to(sdt).to(DEV) for _ in range(2))
+  gq, raw_k, raw_v = (x.transpose(1, 2).contiguous().to(DEV) for x in (xq, xk, xv))
+  want = quantize_kv(raw_k, raw_v, rounding="trunc", scale_heads=hs, scale_dtype=sdt, freqs_cis=freqs.to(DEV))
+  got = [torch.zeros_like(raw_k, dtype=torch.int8) for _ in range(2)] + [torch.zeros((b, hs, 1, 1), dtype=sdt, device=DEV) for _ in range(2)]
+  names = ("new_key", "new_value", "new_k_scaler", "new_v_scaler")
+  out, stats = ak.ragged_mha(gq, k, v, 0, None, end, None, None, ks, vs, **dict(zip(names, got)), new_key_raw=raw_k,
+                             new_value_raw=raw_v, new_key_rope=freqs.to(DEV))
+  for a, w, name in zip(got, want, names):
+    assert torch.equal(a.reshape(-1), w.reshape(-1)), name
+  given, given_stats = ak.ragged_mha(gq, k, v, 0, None, end, None, None, ks, vs, **dict(zip(names, got)))
+  assert torch.equal(out, given) and all(torch.equal(a, w) for a, w in zip(stats, given_stats))
+
+
 def test_orchestration_with_unrotated_keys():
   """Int8KVAttentionKernel(freqs_cis=...) on raw keys == the same kernel on keys
   rotated beforehand, in lazy ragged (fused), eager dense and paged int8 modes;
