@@ -97,7 +97,9 @@ def test_attention_launch_rotates_and_quantises_the_new_token(sdt, per_head, hq,
 @pytest.mark.parametrize("sdt,per_head", [(torch.float32, False), (torch.bfloat16, False), (torch.bfloat16, True)])
 def test_many_rotated_tokens_are_quantised_ahead_of_the_launch(sdt, per_head, b, hq, hkv):
   """From batch * kv_heads^2 = 8192 on the token is rotated and quantised by a launch of its own: codes and
-  scales are the quantiser's, the outputs those of the call that is given them, bit for bit."""
+  scales are the quantiser's, the outputs those of the call that is given them on the same plan, bit for bit
+  (two plans of the same lengths may deal equally long slots out in another order, and with it the order of
+  a row's float32 sums)."""
   from jetstream_pt_amd import attention_kernel as ak
   from jetstream_pt_amd.quantize import quantize_kv
   s, d = 96, 128
@@ -111,11 +113,13 @@ def test_many_rotated_tokens_are_quantised_ahead_of_the_launch(sdt, per_head, b,
   want = quantize_kv(raw_k, raw_v, rounding="trunc", scale_heads=hs, scale_dtype=sdt, freqs_cis=freqs.to(DEV))
   got = [torch.zeros_like(raw_k, dtype=torch.int8) for _ in range(2)] + [torch.zeros((b, hs, 1, 1), dtype=sdt, device=DEV) for _ in range(2)]
   names = ("new_key", "new_value", "new_k_scaler", "new_v_scaler")
-  out, stats = ak.ragged_mha(gq, k, v, 0, None, end, None, None, ks, vs, **dict(zip(names, got)), new_key_raw=raw_k,
+  plan, _ = ak.precompute_ragged_block_indices(end, b, hq, hkv, s)
+  end = plan.lengths
+  out, stats = ak.ragged_mha(gq, k, v, 0, None, end, plan, None, ks, vs, **dict(zip(names, got)), new_key_raw=raw_k,
                              new_value_raw=raw_v, new_key_rope=freqs.to(DEV))
   for a, w, name in zip(got, want, names):
     assert torch.equal(a.reshape(-1), w.reshape(-1)), name
-  given, given_stats = ak.ragged_mha(gq, k, v, 0, None, end, None, None, ks, vs, **dict(zip(names, got)))
+  given, given_stats = ak.ragged_mha(gq, k, v, 0, None, end, plan, None, ks, vs, **dict(zip(names, got)))
   assert torch.equal(out, given) and all(torch.equal(a, w) for a, w in zip(stats, given_stats))
 
 
