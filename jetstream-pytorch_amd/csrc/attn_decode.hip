@@ -636,7 +636,7 @@ int64_t attn_fast_workspace_bytes(const jpt_attn_args& a) {
   const int rows = a.q_heads / a.kv_heads * a.q_rows;
   // shapes the streaming kernel never takes (prefill-shaped queries, huge
   // batches) run on kernels that use neither plan nor partials
-  if (rows > kMaxRows || a.batch > kMaxPlanBatch) return JPT_ATTN_WS_STATE_BYTES + attn_prefill_workspace_bytes(a);
+  if (rows > kMaxRows || a.batch > kMaxPlanBatch) return JPT_ATTN_WS_STATE_BYTES;
   return make_layout(a.batch, a.kv_heads, rows).total;
 }
 
@@ -718,7 +718,9 @@ int64_t jpt_attn_workspace_bytes(const jpt_attn_args* args) {
     return JPT_ATTN_WS_STATE_BYTES;
   const int64_t planned = jpt::attn_fast_workspace_bytes(*args);
   const int64_t rows = static_cast<int64_t>(args->q_heads) / args->kv_heads * args->q_rows;
-  if ((args->dim != 64 && args->dim != 256) || rows > jpt::kMaxRows) return planned;
+  // (the prefill kernel can do without; jpt_attn_ragged_static takes what its array has room for)
+  if (rows > jpt::kMaxRows) return planned + jpt::attn_prefill_workspace_bytes(*args);
+  if (args->dim != 64 && args->dim != 256) return planned;
   const int64_t split = jpt::attn_split_workspace_bytes(*args);
   return split > planned ? split : planned;
 }

@@ -187,7 +187,8 @@ __global__ void __launch_bounds__(64 * kWavesPerGroup, D == 256 ? 1 : 2) attn_pr
   const char* const v_base = static_cast<const char*>(a.v) + kv0;
   const uint32_t lds0 = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_char_ptr)&sm[0][0]));
   auto issue = [&](int tile, int buf) {
-    const int left = S - 1 - tile * kCols;  // rows past the cache's end repeat its last row
+    // rows past the slot's end repeat its last: what lies there may be anything, and 0 times NaN is NaN
+    const int left = len - 1 - tile * kCols;
     const char* kt = k_base + static_cast<int64_t>(tile) * kTileBytes;
     const char* vt = v_base + static_cast<int64_t>(tile) * kTileBytes;
 #pragma unroll
@@ -418,7 +419,9 @@ Classes mask_classes(const jpt_attn_args& a) {
 // Is a pass over the mask worth its launch (3 us)?  Where it can leave out tiles: with one row
 // tile and a handful of key tiles there is nothing to leave out that would pay for it.
 bool classes_pay(const jpt_attn_args& a) {
-  return a.mask != nullptr && a.q_rows >= kRowsPerGroup && a.seq >= 256 && a.seq <= kMaxTiles * kCols;
+  if (a.mask == nullptr || a.q_rows < kRowsPerGroup || a.seq < 256 || a.seq > kMaxTiles * kCols) return false;
+  const Classes c = mask_classes(a);
+  return c.row_blocks <= 65535 && static_cast<int64_t>(c.batches) * c.heads <= 65535;  // what a grid can count
 }
 
 template <int D, int SCALE>
@@ -474,7 +477,6 @@ int32_t attn_prefill_launch(const jpt_attn_args& a, hipStream_t stream) {
       p.class_stride_h = c.heads > 1 ? one : 0;
       p.class_stride_b = c.batches > 1 ? one * c.heads : 0;
       const dim3 grid((a.seq + 255) / 256, c.row_blocks, c.batches * c.heads);
-      JPT_REQUIRE(grid.y <= 65535 && grid.z <= 65535, "mask too large");
       if (a.mask_dtype == JPT_F32)
         hipLaunchKernelGGL(mask_class_kernel<uint32_t>, grid, dim3(256), 0, stream, static_cast<const uint32_t*>(a.mask),
                            a.mask_stride_b, a.mask_stride_h, a.mask_stride_t, a.q_rows, a.seq, c.heads, classes,
