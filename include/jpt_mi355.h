@@ -417,6 +417,10 @@ int32_t jpt_attn_plan(const jpt_attn_args* args, int32_t paged, void* stream);
  * zero: what has to start at zero is cleared by the planning launch. */
 int32_t jpt_attn_plan_fresh(const jpt_attn_args* args, int32_t paged, void* stream);
 int32_t jpt_attn_ragged(const jpt_attn_args* args, void* stream);
+/* jpt_attn_ragged with the step's token given as bf16 rows (new_k, new_v), which are also
+ * left at stash_k and stash_v, (batch, kv_heads, 1, dim) bf16 each: attention and
+ * jpt_kv_stash_lines in one launch where the streaming kernel takes the call. */
+int32_t jpt_attn_ragged_stash(const jpt_attn_args* args, void* stash_k, void* stash_v, void* stream);
 int32_t jpt_attn_dense(const jpt_attn_args* args, void* stream);
 int32_t jpt_attn_paged(const jpt_attn_args* args, void* stream);
 /* jpt_attn_ragged with the workspace inside the library: a device array of

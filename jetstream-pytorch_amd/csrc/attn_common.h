@@ -13,7 +13,8 @@ int32_t check_attn_args(const jpt_attn_args& a, AttnMode mode);
 // JPT_E_BADARG (without setting the message) when the shape is outside what
 // it handles and the generic kernel must run.
 bool attn_fast_supported(const jpt_attn_args& a, AttnMode mode);
-int32_t attn_fast_launch(const jpt_attn_args& a, AttnMode mode, hipStream_t stream);
+// stash_k, stash_v: see FastParams
+int32_t attn_fast_launch(const jpt_attn_args& a, AttnMode mode, hipStream_t stream, void* stash_k = nullptr, void* stash_v = nullptr);
 int64_t attn_fast_workspace_bytes(const jpt_attn_args& a);
 int64_t attn_partials_offset(const jpt_attn_args& a);  // in the workspace: behind the plan
 int32_t attn_plan_launch(const jpt_attn_args& a, bool paged, bool fresh, hipStream_t stream);

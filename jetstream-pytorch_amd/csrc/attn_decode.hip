@@ -669,7 +669,7 @@ int32_t attn_plan_launch(const jpt_attn_args& a, bool paged, bool fresh, hipStre
   return launch_status("plan_kernel");
 }
 
-int32_t attn_fast_launch(const jpt_attn_args& a, AttnMode mode, hipStream_t stream) {
+int32_t attn_fast_launch(const jpt_attn_args& a, AttnMode mode, hipStream_t stream, void* stash_k, void* stash_v) {
   const int rep = a.q_heads / a.kv_heads;
   const int rows = rep * a.q_rows;
   const Layout l = make_layout(a.batch, a.kv_heads, rows);
@@ -687,6 +687,8 @@ int32_t attn_fast_launch(const jpt_attn_args& a, AttnMode mode, hipStream_t stre
   p.rep = rep;
   p.total_items = l.max_entries * a.kv_heads;
   p.status = reinterpret_cast<int32_t*>(ws);
+  p.stash_k = stash_k;
+  p.stash_v = stash_v;
   if (!a.reuse_plan) {
     int32_t st = attn_plan_launch(a, mode == kPaged, false, stream);
     if (st != JPT_OK) return st;
@@ -783,6 +785,21 @@ static int32_t plan_entry(const jpt_attn_args* args, int32_t paged, bool fresh, 
 
 int32_t jpt_attn_plan(const jpt_attn_args* args, int32_t paged, void* stream) { return plan_entry(args, paged, false, stream); }
 int32_t jpt_attn_plan_fresh(const jpt_attn_args* args, int32_t paged, void* stream) { return plan_entry(args, paged, true, stream); }
+
+int32_t jpt_attn_ragged_stash(const jpt_attn_args* args, void* stash_k, void* stash_v, void* stream) {
+  using namespace jpt;
+  JPT_REQUIRE(args != nullptr && stash_k != nullptr && stash_v != nullptr, "args, stash_k and stash_v must not be NULL");
+  JPT_REQUIRE(args->kv_dtype == JPT_BF16 && args->new_k != nullptr && args->new_v != nullptr && args->new_k_raw == nullptr,
+              "a token given as bf16 rows is needed");
+  const int32_t st = check_attn_args(*args, kRagged);
+  if (st != JPT_OK) return st;
+  if (attn_fast_supported(*args, kRagged) && aligned(stash_k, 4) && aligned(stash_v, 4))
+    return attn_fast_launch(*args, kRagged, static_cast<hipStream_t>(stream), stash_k, stash_v);
+  const int32_t at = jpt_attn_ragged(args, stream);
+  if (at != JPT_OK) return at;
+  const int64_t bytes = static_cast<int64_t>(args->batch) * args->kv_heads * args->dim * 2;
+  return jpt_kv_stash_lines(stash_k, args->new_k, stash_v, args->new_v, bytes, stream);
+}
 
 // ---- jpt_attn_ragged_static: the workspace is a device array of this library ----
 // Device memory that exists from the moment the code object is loaded on a GPU

@@ -47,6 +47,7 @@ struct FastParams {
   int32_t rep;
   int32_t total_items;  // max_entries * kv_heads
   int32_t* status;      // the workspace's state block (kState* words)
+  void *stash_k, *stash_v;  // NULL, or where a given bf16 token's rows are left too: (batch, kv_heads, 128)
 };
 
 // How the step's new token reaches the streaming kernel (a template argument of it).

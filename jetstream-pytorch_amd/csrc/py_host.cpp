@@ -35,7 +35,7 @@ struct Library {
   int32_t (*plan[2])(const jpt_attn_args*, int32_t, void*);  // again, on a fresh workspace
   AttnFn attn[3];  // ragged, dense, paged
   int32_t (*scatter_lines)(const jpt_line_tensor*, int32_t, const int32_t*, int32_t, int32_t, int32_t, int32_t, void*);
-  int32_t (*stash_lines)(void*, const void*, void*, const void*, int64_t, void*);
+  int32_t (*ragged_stash)(const jpt_attn_args*, void*, void*, void*);
   int32_t (*append_quant)(const jpt_quant_append_args*, void*);
   int32_t (*insert_layers)(const jpt_prefill_insert_args*, const jpt_insert_layer*, int32_t, void*);
   int32_t (*insert_state)(void*, int32_t, int64_t, int32_t*, int32_t*, int32_t*, int32_t, int32_t, int32_t, int32_t, int32_t, int32_t,
@@ -127,6 +127,7 @@ struct Token {
   const float* rope = nullptr;
   int rounding = 0;
   bool to_pages = false;
+  void *stash_k = nullptr, *stash_v = nullptr;  // bf16 rows: where they are left too (kRagged)
 };
 
 struct Attended {
@@ -276,7 +277,8 @@ Attended attend(Mode mode, const Tensor& q, const Tensor& keys, const Tensor& va
     }
     if (a.workspace == nullptr) use_shared(lib.workspace_bytes(&a));
   }
-  check(lib.attn[mode](&a, stream()));
+  if (token != nullptr && token->stash_k != nullptr) check(lib.ragged_stash(&a, token->stash_k, token->stash_v, stream()));
+  else check(lib.attn[mode](&a, stream()));
   return r;
 }
 
@@ -400,12 +402,11 @@ PyObject* py_lazy_step(PyObject*, PyObject* const* x, Py_ssize_t n) {
       token.rope = rope_of(opt(x[15]), b, d);
     } else {
       need(code == JPT_BF16 && ks == nullptr && x[15] == Py_None);
+      token.stash_k = static_cast<char*>(nk.data_ptr()) + layer * row * 2;
+      token.stash_v = static_cast<char*>(nv.data_ptr()) + layer * row * 2;
     }
     need(is_int32(end, b));
     const Attended r = attend(kRagged, q, ck, cv, layer, &end, nullptr, nullptr, ks, vs, NAN, &token, false, x[13]);
-    if (code == JPT_BF16)
-      check(lib.stash_lines(static_cast<char*>(nk.data_ptr()) + layer * row * 2, xk.data_ptr(),
-                            static_cast<char*>(nv.data_ptr()) + layer * row * 2, xv.data_ptr(), row * 2, stream()));
     return wrap(r.out);
   });
 }
@@ -694,7 +695,7 @@ PyObject* py_bind(PyObject*, PyObject* args) {
   lib.attn[kDense] = reinterpret_cast<AttnFn>(get("jpt_attn_dense"));
   lib.attn[kPaged] = reinterpret_cast<AttnFn>(get("jpt_attn_paged"));
   lib.scatter_lines = reinterpret_cast<decltype(lib.scatter_lines)>(get("jpt_kv_scatter_lines"));
-  lib.stash_lines = reinterpret_cast<decltype(lib.stash_lines)>(get("jpt_kv_stash_lines"));
+  lib.ragged_stash = reinterpret_cast<decltype(lib.ragged_stash)>(get("jpt_attn_ragged_stash"));
   lib.append_quant = reinterpret_cast<decltype(lib.append_quant)>(get("jpt_kv_append_quant_i8"));
   lib.plan[0] = reinterpret_cast<int32_t (*)(const jpt_attn_args*, int32_t, void*)>(get("jpt_attn_plan"));
   lib.plan[1] = reinterpret_cast<int32_t (*)(const jpt_attn_args*, int32_t, void*)>(get("jpt_attn_plan_fresh"));

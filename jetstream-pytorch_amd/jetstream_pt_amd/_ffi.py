@@ -141,6 +141,7 @@ _sig("jpt_attn_workspace_bytes", _i64, _c.POINTER(AttnArgs))
 _sig("jpt_attn_plan", _i32, _c.POINTER(AttnArgs), _i32, _vp)
 _sig("jpt_attn_plan_fresh", _i32, _c.POINTER(AttnArgs), _i32, _vp)
 _sig("jpt_attn_ragged", _i32, _c.POINTER(AttnArgs), _vp)
+_sig("jpt_attn_ragged_stash", _i32, _c.POINTER(AttnArgs), _vp, _vp, _vp)
 _sig("jpt_attn_dense", _i32, _c.POINTER(AttnArgs), _vp)
 _sig("jpt_attn_paged", _i32, _c.POINTER(AttnArgs), _vp)
 _sig("jpt_attn_status", _i32, _vp, _vp, _i32p)
@@ -175,6 +176,7 @@ EXPORTS = (
     "jpt_dpam_free", "jpt_dpam_decode_step", "jpt_decode_advance", "jpt_rope",
     "jpt_ragged_block_indices", "jpt_prefill_insert_layers", "jpt_prefill_insert_prompts",
     "jpt_attn_status", "jpt_attn_ragged_static", "jpt_attn_plan_fresh", "jpt_kv_stash_lines", "jpt_insert_state",
+    "jpt_attn_ragged_stash",
 )
 
 

@@ -93,3 +93,32 @@ def test_a_fresh_plan_needs_no_cleared_workspace(dim, seq):
     outs.append(ak.ragged_mha(q, k, v, 0, None, plan.lengths, plan)[0])
     assert ak.check_status(plan) == 0
   assert torch.equal(outs[0], outs[1]) and torch.equal(outs[0], outs[2])
+
+
+@pytest.mark.parametrize("b,hq,hkv,d,s", [(1, 32, 8, 128, 2048), (5, 8, 8, 128, 512), (3, 8, 1, 128, 4096), (300, 16, 1, 128, 64),
+                                          (4, 8, 4, 64, 256), (3, 4, 2, 128, 333)])
+def test_lazy_bf16_step_leaves_the_token_in_the_stash(b, hq, hkv, d, s):
+  """The attention launch leaves the rows it was given in the layer's stash and nowhere else: empty, full and
+  cut slots, and shapes of the kernels beside the streaming one; outputs as without it, on the same plan."""
+  from jetstream_pt_amd import attention_kernel as ak, cache_manager as cm, layers
+  from jetstream_pt_amd.environment import JetEngineEnvironment, JetEngineEnvironmentData
+  g = torch.Generator().manual_seed(70 + b)
+  env = JetEngineEnvironment(JetEngineEnvironmentData(batch_size=b, num_layers=3, cache_sequence_length=s, ring_buffer=False))
+  cache = cm.KVCacheGenerate.empty((3, b, hkv, s, d), DEV, env)
+  for t in (cache.cache_k, cache.cache_v):
+    t.copy_(torch.randn(t.shape, generator=g).to(torch.bfloat16))
+  q, k, v = (torch.randn((b, h, 1, d), generator=g).to(torch.bfloat16).to(DEV) for h in (hq, hkv, hkv))
+  lens = torch.randint(0, s + 1, (b,), generator=g, dtype=torch.int32)
+  lens[0] = s
+  if b > 1:
+    lens[1] = 0
+  cache.input_pos = lens.to(DEV)
+  for t in (cache.new_ks, cache.new_vs):
+    t.fill_(7.0)
+  plan, _ = ak.precompute_ragged_block_indices(cache.input_pos, b, hq, hkv, s)
+  want, _ = ak.ragged_mha(q, cache.cache_k, cache.cache_v, 1, None, plan.lengths, plan, None, new_key=k, new_value=v)
+  got = layers.AttentionKernel(env, 1)(q, k, v, None, cache, start=None, end=plan.lengths, ragged_batch_index=plan)
+  assert torch.equal(got.reshape(-1), want.reshape(-1))
+  for stash, row in ((cache.new_ks, k), (cache.new_vs, v)):
+    assert torch.equal(stash[1], row)
+    assert torch.all(stash[0] == 7.0) and torch.all(stash[2] == 7.0)
