@@ -334,18 +334,22 @@ __global__ void __launch_bounds__(kSplitThreads, (split_waves_per_simd<D, KV>())
   // positions of tile t that count (0: the tile of an empty slot)
   auto valid_of = [&](const Seq& s, int t) { return min(kTile, s.len + n_new - t * kTile); };
   // A tile's rows: its own from `base` on, the last of them row `top` (positions past the end repeat
-  // it); in the tile with the position behind the cache's, the new token's row in its place.
+  // it); in the tile with the position behind the cache's, the new token's row in its place.  An empty
+  // slot has no row of its own: all are the token's (without one the tile's products are left out).
+  // What lies past a slot's end may be anything, and 0 times NaN is NaN.
   struct Rows {
     const char *base, *fresh;
     int top, top_fresh;
   };
   auto rows_of = [&](const Seq& s, int t, const void* cache, const void* fresh) {
     const int left = s.len - t * kTile;  // cache rows from the tile's first position on
+    const char* const token = static_cast<const char*>(fresh) + (static_cast<int64_t>(s.slot) * H + s.h) * ST::kRowBytes;
     Rows w;
-    w.base = static_cast<const char*>(cache) +
-             ((static_cast<int64_t>(s.slot) * H + s.h) * S + min(t * kTile, max(s.len - 1, 0))) * ST::kRowBytes;
+    w.base = n_new && s.len == 0 ? token
+                                 : static_cast<const char*>(cache) + ((static_cast<int64_t>(s.slot) * H + s.h) * S +
+                                                                      min(t * kTile, max(s.len - 1, 0))) * ST::kRowBytes;
     w.top = min(max(left, 1), kTile) - 1;
-    w.fresh = n_new && left < kTile ? static_cast<const char*>(fresh) + (static_cast<int64_t>(s.slot) * H + s.h) * ST::kRowBytes : nullptr;
+    w.fresh = n_new && s.len > 0 && left < kTile ? token : nullptr;
     w.top_fresh = left;
     return w;
   };
@@ -573,11 +577,13 @@ __global__ void __launch_bounds__(kSplitThreads, (split_waves_per_simd<D, KV>())
 #pragma unroll
       for (int i = 0; i < 4; ++i) split_pack<KV>(w[2 * i], w[2 * i + 1], hi[i], lo[i]);
       const Op p_hi = as_op<Op>(hi[0], hi[1], hi[2], hi[3]), p_lo = as_op<Op>(lo[0], lo[1], lo[2], lo[3]);
+      if (valid > 0) {
 #pragma unroll
-      for (int j = 0; j < kJ; ++j) {
-        const Op v = tile.v_op(j);
-        acc[j] = T::mfma(v, p_hi, acc[j]);
-        acc[j] = T::mfma(v, p_lo, acc[j]);
+        for (int j = 0; j < kJ; ++j) {
+          const Op v = tile.v_op(j);
+          acc[j] = T::mfma(v, p_hi, acc[j]);
+          acc[j] = T::mfma(v, p_lo, acc[j]);
+        }
       }
       if (T::kBias != 0.f) {
         accw = T::mfma(T::ones(), p_hi, accw);

@@ -73,6 +73,38 @@ def test_lengths(token, d, hq, hkv, s, lens, kind):
   assert torch.equal(o, o2), "the counters are not back at zero, or the order of a sum changed"
 
 
+@pytest.mark.parametrize("kind", ["bf16", "int8_f32", "int8_bf16"])
+@pytest.mark.parametrize("d,hq,hkv,s", [(64, 4, 4, 96), (256, 16, 2, 64), (128, 8, 4, 77)])
+@pytest.mark.parametrize("token", [False, True])
+def test_what_lies_past_a_slots_end_does_not_count(token, d, hq, hkv, s, kind):
+  """Rows from a slot's end on, and their scales, may hold anything: an empty slot, one whose first token
+  this is, and slots that end inside a tile and on its edge."""
+  from jetstream_pt_amd import attention_kernel as ak
+  g = torch.Generator().manual_seed(1050 + d)
+  lens = [0, 1, 31, 32, 33, 0, s]
+  b, hs = len(lens), hkv if kind == "int8_bf16" else 1
+  end = torch.tensor(lens, dtype=torch.int32)
+  q = torch.randn((b, hq, 1, d), generator=g).to(torch.bfloat16)
+  clean = make(g, kind, b, hkv, s, d, hs)
+  new = {}
+  if token:
+    rows = make(g, kind, b, hkv, 1, d, hs)
+    new = {n: x.to(DEV) for n, x in zip(("new_key", "new_value", "new_k_scaler", "new_v_scaler"), rows) if x is not None}
+  outs = []
+  for poison in (False, True):
+    dev = [None if x is None else x.to(DEV) for x in clean]
+    for x in dev if poison else ():
+      if x is not None and x.is_floating_point():
+        for slot, n in enumerate(lens):
+          x[slot, :, n:] = math.nan if slot % 2 == 0 else math.inf
+    o, (m, l) = ak.ragged_mha(q.to(DEV), dev[0], dev[1], 0, None, end.to(DEV), None, None, dev[2], dev[3], **new)
+    outs.append((o, m, l))
+  for clean_out, out in zip(*outs):
+    assert torch.equal(clean_out, out)
+  if not token:
+    assert torch.all(outs[0][0][0] == 0) and torch.all(outs[0][2][0] == 0)
+
+
 @pytest.mark.parametrize("kind", ["bf16", "int8_bf16"])
 @pytest.mark.parametrize("d,hq,hkv,t,s,per_head", [(64, 8, 2, 1, 160, False), (256, 4, 4, 3, 90, True), (128, 8, 4, 2, 77, True), (256, 16, 16, 1, 1024, False)])
 def test_masks(d, hq, hkv, t, s, per_head, kind):
