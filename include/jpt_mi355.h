@@ -335,7 +335,11 @@ int32_t jpt_prefill_insert_prompts(const jpt_prefill_insert_args* args,
  * workspace: device scratch of at least jpt_attn_workspace_bytes(args)
  * bytes, 256-byte aligned.  Its first JPT_ATTN_WS_STATE_BYTES (the state
  * block) must be zero before the first call; calls sharing one workspace
- * must not overlap in time.
+ * must not overlap in time.  Calls of the streaming kernel's shapes (dim 128,
+ * bf16 query, up to 16 query rows a KV head) plan, unless reuse_plan is set, and
+ * leave their plan there.  All others plan nothing; they use the workspace's
+ * end, and a plan it holds stays good if workspace_bytes is at least
+ * jpt_attn_workspace_bytes of the planned call and of the other call together.
  *
  * Errors.  Shape and state errors are refused before anything is enqueued
  * (JPT_E_BADARG; the reference raises on them, attention_kernel.py:525-526,
@@ -431,9 +435,9 @@ int32_t jpt_attn_paged(const jpt_attn_args* args, void* stream);
  * The call allocates nothing (no hipMalloc, no hipFree, no allocating
  * library routine): it plans (unless reuse_plan), attends and merges like
  * jpt_attn_ragged, with identical results.  args->workspace and
- * workspace_bytes are ignored.  Shapes whose workspace
- * (jpt_attn_workspace_bytes) exceeds the array are refused with JPT_E_BADARG.
- * All calls on one GPU share that GPU's array, which keeps the last call's
+ * workspace_bytes are ignored.  Shapes whose plan and partials exceed the
+ * array are refused with JPT_E_BADARG; calls that plan nothing use what it has
+ * room for.  All calls on one GPU share that GPU's array, which keeps the last
  * plan (so reuse_plan works across calls with the same lengths): calls that
  * overlap in time on one GPU race, whatever their streams.
  * jpt_attn_status(NULL, ...) reads its status word on the current device. */

@@ -17,6 +17,13 @@ bool attn_fast_supported(const jpt_attn_args& a, AttnMode mode);
 int32_t attn_fast_launch(const jpt_attn_args& a, AttnMode mode, hipStream_t stream, void* stash_k = nullptr, void* stash_v = nullptr);
 int64_t attn_fast_workspace_bytes(const jpt_attn_args& a);
 int64_t attn_partials_offset(const jpt_attn_args& a);  // in the workspace: behind the plan
+// Where kernels that need no plan put what they need: the last `bytes` of the workspace, from a multiple of
+// 256 on, so that a plan for other calls that the workspace holds stays (bytes from attn_partials_offset(a)
+// on are there to have: a plan for this call's slots and heads lies below it, and one for more of them has
+// its partials, which no launch leaves for the next, between its records and the end).
+inline char* attn_workspace_end(const jpt_attn_args& a, int64_t bytes) {
+  return static_cast<char*>(a.workspace) + (a.workspace_bytes - bytes) / 256 * 256;
+}
 int32_t attn_plan_launch(const jpt_attn_args& a, bool paged, bool fresh, hipStream_t stream);
 
 // Few query rows over caches the streaming kernel is not built for: attn_split.hip.  Needs a workspace
@@ -25,8 +32,8 @@ bool attn_split_supported(const jpt_attn_args& a, AttnMode mode);
 int64_t attn_split_workspace_bytes(const jpt_attn_args& a);
 int32_t attn_split_launch(const jpt_attn_args& a, hipStream_t stream);
 
-// Many query rows (prefill) over bf16 keys and values: attn_prefill.hip.  The workspace it can use lies
-// behind the state block and need not be cleared.
+// Many query rows (prefill) over bf16 keys and values: attn_prefill.hip.  Bytes of workspace it can use,
+// which need not be cleared.
 bool attn_prefill_supported(const jpt_attn_args& a, AttnMode mode);
 int64_t attn_prefill_workspace_bytes(const jpt_attn_args& a);
 int32_t attn_prefill_launch(const jpt_attn_args& a, hipStream_t stream);

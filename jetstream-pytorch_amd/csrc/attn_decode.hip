@@ -720,9 +720,13 @@ int64_t jpt_attn_workspace_bytes(const jpt_attn_args* args) {
     return JPT_ATTN_WS_STATE_BYTES;
   const int64_t planned = jpt::attn_fast_workspace_bytes(*args);
   const int64_t rows = static_cast<int64_t>(args->q_heads) / args->kv_heads * args->q_rows;
-  // (the prefill kernel can do without; jpt_attn_ragged_static takes what its array has room for)
-  if (rows > jpt::kMaxRows) return planned + jpt::attn_prefill_workspace_bytes(*args);
-  if (args->dim != 64 && args->dim != 256) return planned;
+  // (the prefill kernel can do without)
+  if (rows > jpt::kMaxRows) {
+    const int64_t classes = jpt::attn_prefill_workspace_bytes(*args);
+    return classes > 0 ? jpt::attn_partials_offset(*args) + classes : planned;
+  }
+  // (dim 128: the calls the streaming kernel leaves; a planning call says neither dim nor, if paged, seq)
+  if ((args->dim != 64 && args->dim != 128 && args->dim != 256) || args->seq <= 0) return planned;
   const int64_t split = jpt::attn_split_workspace_bytes(*args);
   return split > planned ? split : planned;
 }

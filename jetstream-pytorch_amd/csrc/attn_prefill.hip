@@ -468,8 +468,8 @@ int32_t attn_prefill_launch(const jpt_attn_args& a, hipStream_t stream) {
   if (classes_pay(a)) {
     const Classes c = mask_classes(a);
     // without a workspace (it is the caller's to give) every block is taken to hold anything
-    if (a.workspace != nullptr && a.workspace_bytes >= JPT_ATTN_WS_STATE_BYTES + c.bytes) {
-      uint8_t* classes = static_cast<uint8_t*>(a.workspace) + JPT_ATTN_WS_STATE_BYTES;
+    if (a.workspace != nullptr && a.workspace_bytes >= attn_partials_offset(a) + c.bytes) {
+      uint8_t* classes = reinterpret_cast<uint8_t*>(attn_workspace_end(a, c.bytes));
       p.classes = classes;
       p.row_blocks = c.row_blocks;
       p.col_blocks = c.col_blocks;

@@ -733,7 +733,6 @@ bool attn_split_supported(const jpt_attn_args& a, AttnMode mode) {
   if (a.new_k && (!aligned(a.new_k, 16) || !aligned(a.new_v, 16))) return false;
   // tile numbers fit 32 bits, the sum over the batch before it is multiplied by the heads too
   if (static_cast<int64_t>(a.batch) * (a.seq / kTile + 16) >= (1ll << 31)) return false;
-  // the partials lie where a plan's do, behind its entries: a workspace that holds a plan keeps it
   return a.workspace != nullptr && aligned(a.workspace, 256) && decode::split_groups(a) >= decode::kMinGroups;
 }
 
@@ -747,8 +746,9 @@ int32_t attn_split_launch(const jpt_attn_args& a, hipStream_t stream) {
   p.rep = a.q_heads / a.kv_heads;
   p.rows = p.rep * a.q_rows;
   p.counters = static_cast<int32_t*>(a.workspace) + kStateSplitCounters;
-  p.partials = reinterpret_cast<float*>(static_cast<char*>(a.workspace) + attn_partials_offset(a));
-  const dim3 grid(static_cast<unsigned>(decode::split_groups(a)));
+  const int64_t groups = decode::split_groups(a);
+  p.partials = reinterpret_cast<float*>(attn_workspace_end(a, groups * decode::group_bytes(a)));
+  const dim3 grid(static_cast<unsigned>(groups));
   if (a.dim == 64) decode::launch_split_dim<64>(p, grid, stream);
   else if (a.dim == 128) decode::launch_split_dim<128>(p, grid, stream);
   else decode::launch_split_dim<256>(p, grid, stream);

@@ -40,7 +40,7 @@ def _outputs(case):
   return out, omax, oden, nk, nv, nks, nvs
 
 
-def _run(fn, case, workspace, outputs=None):
+def _run(fn, case, workspace, outputs=None, reuse_plan=0):
   """One launch that quantises and attends the step's token too (every kind of
   scratch use: plan, partials of split slots, status word).  Returns every
   tensor the launch writes (`outputs`, or new ones)."""
@@ -55,7 +55,7 @@ def _run(fn, case, workspace, outputs=None):
       new_v_scale=_ffi.ptr(nvs), new_k_raw=_ffi.ptr(xk), new_v_raw=_ffi.ptr(xv), out=_ffi.ptr(out),
       out_max=_ffi.ptr(omax), out_denom=_ffi.ptr(oden), batch=b, q_heads=hq, kv_heads=hkv, q_rows=1, dim=d,
       seq=s, q_dtype=_ffi.BF16, kv_dtype=_ffi.I8, scale_dtype=_ffi.F32, scale_heads=1,
-      sm_scale=1.0 / d ** 0.5, new_rounding=_ffi.ROUND_TRUNC)
+      sm_scale=1.0 / d ** 0.5, new_rounding=_ffi.ROUND_TRUNC, reuse_plan=reuse_plan)
   if workspace is not None:
     a.workspace, a.workspace_bytes = _ffi.ptr(workspace), workspace.numel()
   _ffi.check(fn(a, _ffi.stream()))
@@ -109,3 +109,37 @@ def test_static_scratch_entry_point_refuses_what_does_not_fit():
   assert _ffi.lib.jpt_attn_workspace_bytes(a) > _ffi.ATTN_STATIC_SCRATCH_BYTES
   with pytest.raises(ValueError, match="workspace of"):
     _ffi.check(_ffi.lib.jpt_attn_ragged_static(a, _ffi.stream()))
+
+
+@pytest.mark.parametrize("static", [False, True])
+@pytest.mark.parametrize("t,d,s", [(128, 128, 512), (300, 64, 4096), (1, 256, 700), (2, 128, 333)])
+def test_a_plan_outlives_calls_that_plan_nothing(t, d, s, static):
+  """A step is planned, other requests' calls (a masked prompt of many query rows, heads or cache lengths
+  of the kernels beside the streaming one) run on the same workspace, and the step's launch reuses the plan:
+  the plan's bytes are as they were, and so are the outputs."""
+  from jetstream_pt_amd import _ffi
+  g = torch.Generator().manual_seed(910)
+  case = _case(g, 96, 32, 8, 1024, [1024, 700, 1, 0, 17, 999] * 16)
+  b, hq, hkv = 96, 32, 8
+  q, k, v = (torch.randn((1, h, n, d), generator=g).to(torch.bfloat16).to(DEV) for h, n in ((hq, t), (hkv, s), (hkv, s)))
+  mask = torch.full((1, 1, t, s), float("-inf"), device=DEV).triu(1 + s - t)
+  out = torch.empty_like(q)
+  end = torch.full((1,), s, dtype=torch.int32, device=DEV)
+  other = _ffi.AttnArgs(
+      q=_ffi.ptr(q), k=_ffi.ptr(k), v=_ffi.ptr(v), mask=_ffi.ptr(mask), mask_stride_t=s, mask_dtype=_ffi.F32, out=_ffi.ptr(out),
+      batch=1, q_heads=hq, kv_heads=hkv, q_rows=t, dim=d, seq=s, q_dtype=_ffi.BF16, kv_dtype=_ffi.BF16, sm_scale=1.0 / d ** 0.5)
+  sizes = _ffi.AttnArgs(batch=b, q_heads=hq, kv_heads=hkv, q_rows=1, seq=1024, dim=128)
+  planned = _ffi.lib.jpt_attn_workspace_bytes(sizes)
+  ws = None if static else torch.zeros(planned + _ffi.lib.jpt_attn_workspace_bytes(other), dtype=torch.uint8, device=DEV)
+  fn = _ffi.lib.jpt_attn_ragged_static if static else _ffi.lib.jpt_attn_ragged
+  want = [x.clone() for x in _run(fn, case, ws)]
+  if ws is not None:
+    other.workspace, other.workspace_bytes = _ffi.ptr(ws), ws.numel()
+    before = ws[:planned].clone()
+  other.lengths = _ffi.ptr(end)
+  _ffi.check(fn(other, _ffi.stream()))
+  if ws is not None:
+    assert torch.equal(ws[:planned], before)
+  got = _run(fn, case, ws, reuse_plan=1)
+  for x, y in zip(got, want):
+    assert torch.equal(x, y)
