@@ -141,7 +141,7 @@ Attended attend(Mode mode, const Tensor& q, const Tensor& keys, const Tensor& va
   need(q.dim() == 4);
   const int64_t b = q.size(0), hq = q.size(1), t = q.size(2), d = q.size(3);
   const Layer k(keys, 4, layer), v(values, 4, layer);
-  need(k.sizes == v.sizes && k.code == v.code && k.sizes[3] == d && b > 0 && hq > 0 && t > 0 && d > 0);
+  need(keys.dim() == values.dim() && k.sizes == v.sizes && k.code == v.code && k.sizes[3] == d && b > 0 && hq > 0 && t > 0 && d > 0);
   jpt_attn_args a{};
   a.q = q.data_ptr();
   a.k = k.data;
@@ -174,8 +174,9 @@ Attended attend(Mode mode, const Tensor& q, const Tensor& keys, const Tensor& va
   }
   need((k_scaler == nullptr) == (v_scaler == nullptr));
   if (k_scaler != nullptr) {
-    // dense (B, Hs, S[, 1]) or stacks of (B, Hs, S, 1); scale pages (Hs, P, ps)
+    // dense (B, Hs, S[, 1]) or stacks of (B, Hs, S, 1) beside stacked keys; scale pages (Hs, P, ps)
     const int dims = mode == kPaged || k_scaler->dim() == 3 ? 3 : 4;
+    need(k_scaler->dim() == v_scaler->dim() && (k_scaler->dim() == dims || keys.dim() == 5));
     const Layer ks(*k_scaler, dims, layer), vs(*v_scaler, dims, layer);
     need(ks.sizes == vs.sizes && ks.code == vs.code && ks.code != JPT_I8 && (dims == 3 || ks.sizes[3] == 1));
     if (mode == kPaged) need(ks.sizes[1] == k.sizes[1] && ks.sizes[2] == k.sizes[2]);

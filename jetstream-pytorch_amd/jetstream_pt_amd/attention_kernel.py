@@ -232,18 +232,19 @@ def _attend(mode, xq, keys, values, *, lengths=None, page_table=None, mask=None,
             k_scaler=None, v_scaler=None, sm_scale=None, new_key=None,
             new_value=None, new_k_scaler=None, new_v_scaler=None, new_key_raw=None,
             new_value_raw=None, new_rounding="trunc", new_key_rope=None, new_to_pages=False,
-            want_stats=False, plan=None, force_generic=False, layer=-1):
-  """xq (B, Hq, T, D); keys/values (B, Hkv, S, D), or stacks of them with `layer`
-  picking one, or pages (Hkv, P, ps, D).
+            want_stats=False, plan=None, force_generic=False, layer=None):
+  """xq (B, Hq, T, D); keys/values (B, Hkv, S, D), or stacks of them (and of their
+  scalers) where `layer` picks one, or pages (Hkv, P, ps, D).
   Returns (o (B, Hq, T, D), max (B, Hq, T) | None, denom (B, Hq, T) | None)."""
   if not force_generic:
-    r = _host.attend(_MODES[mode], xq, keys, values, layer, lengths, page_table, mask, k_scaler, v_scaler, sm_scale,
-                     new_key, new_value, new_k_scaler, new_v_scaler, new_key_raw, new_value_raw,
-                     0 if new_key_raw is None else _rounding_code(new_rounding), new_key_rope, new_to_pages, want_stats, plan)
+    r = _host.attend(_MODES[mode], xq, keys, values, -1 if layer is None else layer, lengths, page_table, mask,
+                     k_scaler, v_scaler, sm_scale, new_key, new_value, new_k_scaler, new_v_scaler,
+                     new_key_raw, new_value_raw, 0 if new_key_raw is None else _rounding_code(new_rounding), new_key_rope, new_to_pages, want_stats, plan)
     if r is not None:
       return r
   # not the ordinary case (contiguous device tensors of the library's dtypes): converted, or refused, here
-  keys, values, k_scaler, v_scaler = _pick_layer(keys, values, layer, k_scaler, v_scaler)
+  if layer is not None:
+    keys, values, k_scaler, v_scaler = _pick_layer(keys, values, layer, k_scaler, v_scaler)
   xq = _ffi.dev(xq, "xq")
   keys, values = _ffi.dev(keys, "keys"), _ffi.dev(values, "values")
   b, hq, t, d = xq.shape

@@ -122,3 +122,28 @@ def test_lazy_bf16_step_leaves_the_token_in_the_stash(b, hq, hkv, d, s):
   for stash, row in ((cache.new_ks, k), (cache.new_vs, v)):
     assert torch.equal(stash[1], row)
     assert torch.all(stash[0] == 7.0) and torch.all(stash[2] == 7.0)
+
+
+def test_stacks_of_layers_are_taken_only_where_a_layer_is_named():
+  """Five-dimensional keys without a layer, and stacks beside tensors of one layer, are refused; a named
+  layer of a stack gives that layer's bits."""
+  from jetstream_pt_amd import attention_kernel as ak
+  g = torch.Generator().manual_seed(12)
+  b, hq, hkv, s, d = 2, 8, 2, 64, 128
+  q = torch.randn((b, hq, 1, d), generator=g).to(torch.bfloat16).to(DEV)
+  k, v = (torch.randn((3, b, hkv, s, d), generator=g).to(torch.bfloat16).to(DEV) for _ in range(2))
+  codes = torch.randint(-127, 128, (3, b, hkv, s, d), generator=g, dtype=torch.int8).to(DEV)
+  scales = torch.rand((3, b, 1, s, 1), generator=g).to(DEV)
+  lens = torch.tensor([64, 5], dtype=torch.int32, device=DEV)
+  refused = [lambda: ak.dense_attention(q, k, v), lambda: ak.dense_attention(q, codes, codes, scales, scales),
+             lambda: ak.flash_attention(q, codes[1], codes[1], 1, scales, scales),
+             lambda: ak.flash_attention(q, codes, codes, 1, scales[1], scales),
+             lambda: ak.ragged_mha(q, k[1], v, 1, None, lens),
+             lambda: ak.call_paged_attention(None, q.squeeze(2), k.reshape(3, hkv, b * 2, s // 2, d), v.reshape(3, hkv, b * 2, s // 2, d), lens,
+                                             torch.zeros((b, 2), dtype=torch.int32, device=DEV))]
+  for call in refused:
+    with pytest.raises(ValueError):
+      call()
+  for a, w in zip(ak.flash_attention(q, codes, codes, 1, scales, scales)[1], ak.flash_attention(q, codes[1], codes[1], 0, scales[1], scales[1])[1]):
+    assert torch.equal(a, w)
+  assert torch.equal(ak.ragged_mha(q, k, v, 2, None, lens)[0], ak.ragged_mha(q, k[2], v[2], 0, None, lens)[0])
