@@ -95,3 +95,15 @@ def no_attention_launch_gave_up(request):
   ak = sys.modules.get("jetstream_pt_amd.attention_kernel")
   if ak is not None:
     ak.check_status()
+
+
+def float32_bound(want, total, units=16):
+  """Bound of |got - want| for a bf16 output whose weights, scores and sums were float32: half an ulp of the
+  output, and `units` times 2^-24 of `total`, the output with every value's magnitude in its place.  For a
+  handful of positions and scores below 4: a score's roundings (product, scale, difference to the maximum)
+  at most 4 units of its weight, the hardware's exp2 and the weight times its scale 3, the sums of weights
+  and of products 2 each, the division and the last product 2."""
+  import torch
+  slack = units * 2.0 ** -24 * total
+  _, e = torch.frexp(want.abs() + slack)
+  return torch.ldexp(torch.ones_like(want), e - 9) + slack

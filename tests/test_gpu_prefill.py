@@ -1,16 +1,15 @@
 """GPU parity: attention of many query rows (prefill) on the matrix cores, against
 the float64 closed form, at the edges of its tiles: 128 query rows and 32 a wave,
 64 positions a tile, mask blocks of 32 rows x 64 positions, heads folded below 128
-rows.  Softmax weights carry 16 bits, so below 2 (where the output's rounding is at
-most 2^-8) the error stays under 6e-3: half an ulp, 2^-8, plus a score's float32
-sums and exp2, far below it."""
+rows.  Below 2, where the output's rounding is at most 2^-8, the error stays under
+6e-3: half an ulp, 2^-8, plus a score's float32 sums and exp2, far below it."""
 
 import math
 
 import pytest
 import torch
 
-from conftest import attention_bound
+from conftest import attention_bound, float32_bound
 from oracle import attention as OA
 
 pytestmark = pytest.mark.gpu
@@ -88,3 +87,32 @@ def test_many_query_rows_with_lengths():
   got, _ = ak.ragged_mha(q.to(DEV), k.to(DEV), v.to(DEV), 0, None, end.to(DEV))
   err = (got.double().cpu().reshape(want.shape) - want).abs()
   assert torch.all(err <= 6e-3), float(err.max())
+
+
+@pytest.mark.parametrize("d", [64, 128, 256])
+@pytest.mark.parametrize("sdt", [None, torch.bfloat16, torch.float32])
+@pytest.mark.parametrize("masked", [False, True])
+def test_weights_are_float32(masked, sdt, d):
+  """Two positions whose values nearly cancel in some column of every row: weights of fewer bits than
+  float32's stand out there."""
+  from jetstream_pt_amd import attention_kernel as ak
+  b, hq, hkv, t = 2, 4, 2, 130
+  s = t if masked else 2
+  q, k, v = torch.zeros((b, hq, t, d)), torch.zeros((b, hkv, s, d)), torch.zeros((b, hkv, s, d))
+  q[..., 0] = (torch.arange(t) + 1) / 64.0
+  k[:, :, 1, 0] = -8.0 - torch.arange(b * hkv).reshape(b, hkv)
+  v[:, :, 0], v[:, :, 1] = -torch.arange(d) / d, 1.0
+  q, k, v = (x.to(torch.bfloat16) for x in (q, k, v))
+  mask = ks = vs = rows = None
+  if masked:
+    mask = torch.full((1, 1, t, s), -math.inf)
+    mask[..., :2] = 0.0
+    rows = mask.expand(b, hq, t, s).reshape(b, hkv, hq // hkv * t, s)
+  if sdt is not None:
+    ks, vs = torch.full((b, 1, s, 1), 0.9).to(sdt), torch.full((b, 1, s, 1), 0.7).to(sdt)
+  want, _, _ = OA.closed_form(q, k, v, mask=rows, k_scale=ks, v_scale=vs)
+  total, _, _ = OA.closed_form(q, k, v.abs(), mask=rows, k_scale=ks, v_scale=vs)
+  dev = [None if x is None else x.to(DEV) for x in (q, k, v, ks, vs, mask)]
+  got = ak.dense_attention(*dev).double().cpu()
+  over = (got - want).abs() / float32_bound(want, total)
+  assert torch.all(over <= 1.0), float(over.max())
