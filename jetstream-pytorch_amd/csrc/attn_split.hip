@@ -17,8 +17,8 @@
 // tiles whatever the sequences' number, and the new token a tile of its own: 60 us for 48 us below.)
 //
 // The arithmetic is that of the streaming kernel (S^T = K . Q^T, O^T = V^T . P^T on 16x16x32 MFMAs,
-// int8 codes as float16 1024 + 128 + code), with softmax weights as the sum of two 16-bit numbers:
-// the matrix cores have the time, and the result keeps only its own rounding to bf16.
+// int8 codes as float16 1024 + 128 + code), with softmax weights as the sum of three 16-bit numbers:
+// the matrix cores have the time, and the weights keep float32's bits.
 //
 // A sequence cut between groups: every group parks a float32 partial past the caches and counts
 // itself; the last one folds them.  No group waits for another.
@@ -143,20 +143,22 @@ struct SplitTile {
   }
 };
 
-// A weight as the sum of two numbers of the operand's type: two packed pairs.
+// A weight as the sum of three numbers of the operand's type, of each what rounding the ones before has
+// left: float32's 24 bits (8 a number as bf16, 11 as float16).  Three packed pairs.
 template <typename KV>
-__device__ __forceinline__ void split_pack(float x, float y, uint32_t& hi, uint32_t& lo) {
-  hi = Tile<KV>::pack(x, y);
-  float hx, hy;
-  if constexpr (sizeof(KV) == 1) {
-    const f16x2 t = __builtin_bit_cast(f16x2, hi);
-    hx = static_cast<float>(t[0]);
-    hy = static_cast<float>(t[1]);
-  } else {
-    hx = __uint_as_float(hi << 16);
-    hy = __uint_as_float(hi & 0xffff0000u);
+__device__ __forceinline__ void split_pack(float x, float y, uint32_t (&part)[3]) {
+#pragma unroll
+  for (int i = 0; i < 3; ++i) {
+    const uint32_t both = part[i] = Tile<KV>::pack(x, y);
+    if constexpr (sizeof(KV) == 1) {
+      const f16x2 t = __builtin_bit_cast(f16x2, both);
+      x -= static_cast<float>(t[0]);
+      y -= static_cast<float>(t[1]);
+    } else {
+      x -= __uint_as_float(both << 16);
+      y -= __uint_as_float(both & 0xffff0000u);
+    }
   }
-  lo = Tile<KV>::pack(x - hx, y - hy);
 }
 
 // Two waves a SIMD, but for bf16 rows of 256, whose tile is 128 registers.
@@ -573,21 +575,23 @@ __global__ void __launch_bounds__(kSplitThreads, (split_waves_per_simd<D, KV>())
         for (int j = 0; j < kJ; ++j) acc[j] *= alpha;
         if (T::kBias != 0.f) accw *= alpha;
       }
-      uint32_t hi[4], lo[4];
+      uint32_t part[4][3];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) split_pack<KV>(w[2 * i], w[2 * i + 1], hi[i], lo[i]);
-      const Op p_hi = as_op<Op>(hi[0], hi[1], hi[2], hi[3]), p_lo = as_op<Op>(lo[0], lo[1], lo[2], lo[3]);
+      for (int i = 0; i < 4; ++i) split_pack<KV>(w[2 * i], w[2 * i + 1], part[i]);
+      Op pw[3];
+#pragma unroll
+      for (int i = 0; i < 3; ++i) pw[i] = as_op<Op>(part[0][i], part[1][i], part[2][i], part[3][i]);
       if (valid > 0) {
 #pragma unroll
         for (int j = 0; j < kJ; ++j) {
           const Op v = tile.v_op(j);
-          acc[j] = T::mfma(v, p_hi, acc[j]);
-          acc[j] = T::mfma(v, p_lo, acc[j]);
+#pragma unroll
+          for (int i = 0; i < 3; ++i) acc[j] = T::mfma(v, pw[i], acc[j]);
         }
       }
       if (T::kBias != 0.f) {
-        accw = T::mfma(T::ones(), p_hi, accw);
-        accw = T::mfma(T::ones(), p_lo, accw);
+#pragma unroll
+        for (int i = 0; i < 3; ++i) accw = T::mfma(T::ones(), pw[i], accw);
       }
       if (more) load_v(nxt, t_next);
       if (!more || nxt.number != cur.number) break;

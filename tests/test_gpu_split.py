@@ -1,15 +1,15 @@
 """GPU parity: decode attention over head dims of 64 and 256 and over cache lengths and masks the
 streaming kernel does not take, against the float64 closed form, where shares and tiles end: slots
 of 0, 1, 31..33 positions, fewer tiles than groups, sequences over many groups, more slots than a
-workgroup has threads.  Softmax weights carry 16 bits and more, so below 2 (where the output's
-rounding is at most 2^-8) the error stays under 6e-3."""
+workgroup has threads.  Below 2, where the output's rounding is at most 2^-8, the error stays under
+6e-3."""
 
 import math
 
 import pytest
 import torch
 
-from conftest import attention_bound
+from conftest import attention_bound, float32_bound
 from oracle import attention as OA
 
 pytestmark = pytest.mark.gpu
@@ -123,3 +123,35 @@ def test_masks(d, hq, hkv, t, s, per_head, kind):
   dev = [None if x is None else x.to(DEV) for x in (q, k, v, ks, vs, mask)]
   o, (m, l) = ak.flash_attention(*dev[:3], 0, dev[3], dev[4], dev[5])
   check(o, want, m, l, wm, wl)
+
+
+def cancelling(d, kind, scale, top):
+  """Slots of two positions whose values, up to `top`, nearly cancel in some column of every row: anything
+  computed in fewer bits than float32's stands out there."""
+  b, hq, hkv, s = 130, 4, 2, 40
+  q, k, v = torch.zeros((b, hq, 1, d)), torch.zeros((b, hkv, s, d)), torch.zeros((b, hkv, s, d))
+  q[..., 0] = (torch.arange(b).reshape(b, 1, 1) + 1) / 64.0
+  k[:, :, 1, 0] = -8.0 - torch.arange(hkv)
+  v[:, :, 0], v[:, :, 1] = -(torch.arange(d) % (top + 1)), top
+  if kind == "bf16":
+    return [x.to(torch.bfloat16) for x in (q, k, v)] + [None, None]
+  sdt = torch.float32 if kind == "int8_f32" else torch.bfloat16
+  return [q.to(torch.bfloat16), k.to(torch.int8), v.to(torch.int8), torch.full((b, 1, s, 1), 0.9).to(sdt),
+          torch.full((b, 1, s, 1), scale).to(sdt)]
+
+
+def check_cancelling(d, kind, scale, top):
+  from jetstream_pt_amd import attention_kernel as ak
+  q, k, v, ks, vs = cancelling(d, kind, scale, top)
+  end = torch.full((q.shape[0],), 2, dtype=torch.int32)
+  want, _, _ = OA.closed_form(q, k, v, lengths=end, k_scale=ks, v_scale=vs)
+  total, _, _ = OA.closed_form(q, k, v.abs(), lengths=end, k_scale=ks, v_scale=vs)
+  dev = [None if x is None else x.to(DEV) for x in (q, k, v, end, ks, vs)]
+  got, _ = ak.ragged_mha(*dev[:3], 0, None, dev[3], None, None, dev[4], dev[5])
+  over = (got.double().cpu().reshape(want.shape) - want).abs() / float32_bound(want, total)
+  assert torch.all(over <= 1.0), float(over.max())
+
+
+@pytest.mark.parametrize("d", [64, 128, 256])
+def test_weights_are_float32(d):
+  check_cancelling(d, "bf16", 1.0, min(d - 1, 127))
