@@ -16,9 +16,11 @@
 // parts.  (With barriers at every sequence's end and its tiles dealt to the waves anew, shares of equal
 // tiles whatever the sequences' number, and the new token a tile of its own: 60 us for 48 us below.)
 //
-// The arithmetic is that of the streaming kernel (S^T = K . Q^T, O^T = V^T . P^T on 16x16x32 MFMAs,
-// int8 codes as float16 1024 + 128 + code), with softmax weights as the sum of three 16-bit numbers:
-// the matrix cores have the time, and the weights keep float32's bits.
+// The arithmetic is the streaming kernel's (S^T = K . Q^T, O^T = V^T . P^T on 16x16x32 MFMAs), but keeps
+// float32's bits: softmax weights are the sum of three 16-bit numbers, and int8 codes go in as float16 numbers
+// of their own, not 1152 too high.  (The constant, carried through float32 sums and taken out at their end,
+// costs ten bits of a sum of small terms: 1.4 % of the outputs of the case below were not the rounded exact
+// value.  A packed subtraction a pair of codes takes it out; four layers of the case below 275 -> 287 us.)
 //
 // A sequence cut between groups: every group parks a float32 partial past the caches and counts
 // itself; the last one folds them.  No group waits for another.
@@ -118,11 +120,16 @@ struct SplitTile {
   }
   using T = Tile<KV>;
   using Op = typename T::Op;
+  // two float16 1152 + code as the codes, exactly
+  static __device__ __forceinline__ uint32_t unbias(uint32_t both) {
+    const f16x2 bias = {static_cast<_Float16>(T::kBias), static_cast<_Float16>(T::kBias)};
+    return __builtin_bit_cast(uint32_t, __builtin_bit_cast(f16x2, both) - bias);
+  }
   __device__ __forceinline__ Op k_op(int half, int s) const {
     if constexpr (sizeof(KV) == 1) {
       const uint4 x = k[half][s >> 1];
       const uint32_t w0 = ((s & 1) ? x.z : x.x) ^ 0x80808080u, w1 = ((s & 1) ? x.w : x.y) ^ 0x80808080u;
-      return as_op<Op>(T::widen(w0, false), T::widen(w0, true), T::widen(w1, false), T::widen(w1, true));
+      return as_op<Op>(unbias(T::widen(w0, false)), unbias(T::widen(w0, true)), unbias(T::widen(w1, false)), unbias(T::widen(w1, true)));
     } else {
       return __builtin_bit_cast(Op, k[half][s]);
     }
@@ -134,7 +141,7 @@ struct SplitTile {
     for (int i = 0; i < 4; ++i) {
       if constexpr (sizeof(KV) == 1) {
         const uint32_t sel = 0x0c000c00u | static_cast<uint32_t>(j & 3) | (static_cast<uint32_t>(4 + (j & 3)) << 16);
-        w[i] = __builtin_amdgcn_perm(v[2 * i + 1][j >> 2], v[2 * i][j >> 2], sel) ^ 0x64806480u;
+        w[i] = unbias(__builtin_amdgcn_perm(v[2 * i + 1][j >> 2], v[2 * i][j >> 2], sel) ^ 0x64806480u);
       } else {
         w[i] = __builtin_amdgcn_perm(v[2 * i + 1][j >> 1], v[2 * i][j >> 1], (j & 1) ? 0x07060302u : 0x05040100u);
       }
@@ -480,7 +487,6 @@ __global__ void __launch_bounds__(kSplitThreads, (split_waves_per_simd<D, KV>())
     Op qop[kQInLds ? 1 : kSteps];
     auto q_at = [&](int s) { return reinterpret_cast<Op*>(&s_q[wave][min(r, R - 1) * D + split_element<KV>(s, g)]); };
     float c2_row = c2;
-    f32x4 s_init = {0.f, 0.f, 0.f, 0.f};
     {
       uint4 raw[kSteps];
 #pragma unroll
@@ -488,7 +494,7 @@ __global__ void __launch_bounds__(kSplitThreads, (split_waves_per_simd<D, KV>())
         raw[s] = *reinterpret_cast<const uint4*>(q_at(s));
       if constexpr (sizeof(KV) == 1) {
         // as float16: the row times the power of two that puts its largest magnitude in [2^13, 2^14)
-        float amax = 0.f, qs = 0.f;
+        float amax = 0.f;
 #pragma unroll
         for (int s = 0; s < kSteps; ++s) {
           const uint32_t w[4] = {raw[s].x, raw[s].y, raw[s].z, raw[s].w};
@@ -507,23 +513,18 @@ __global__ void __launch_bounds__(kSplitThreads, (split_waves_per_simd<D, KV>())
           uint32_t f[4];
 #pragma unroll
           for (int i = 0; i < 4; ++i) {
-            const float u = __uint_as_float(w[i] << 16) * up, y = __uint_as_float(w[i] & 0xffff0000u) * up;
-            qs += u + y;
-            f[i] = pack_f16(u, y);
+            f[i] = pack_f16(__uint_as_float(w[i] << 16) * up, __uint_as_float(w[i] & 0xffff0000u) * up);
           }
           if constexpr (kQInLds) *q_at(s) = as_op<Op>(f[0], f[1], f[2], f[3]);
           else qop[s] = as_op<Op>(f[0], f[1], f[2], f[3]);
         }
-        qs = sum_across_rows(qs);
         c2_row = c2 * ldexpf(1.f, e - 14);
-        const float bias = -T::kBias * qs;
-        s_init = f32x4{bias, bias, bias, bias};
       } else if constexpr (!kQInLds) {
 #pragma unroll
         for (int s = 0; s < kSteps; ++s) qop[s] = __builtin_bit_cast(Op, raw[s]);
       }
     }
-    f32x4 acc[kJ], accw = {0.f, 0.f, 0.f, 0.f};
+    f32x4 acc[kJ];
 #pragma unroll
     for (int j = 0; j < kJ; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
     float m_run = -INFINITY, l_run = 0.f;
@@ -533,7 +534,7 @@ __global__ void __launch_bounds__(kSplitThreads, (split_waves_per_simd<D, KV>())
       x += kSplitWaves;
       more = move_to(x);
       const int t_next = nxt.ta + x - nxt.base;
-      f32x4 sa = s_init, sb = s_init;
+      f32x4 sa = {0.f, 0.f, 0.f, 0.f}, sb = sa;
 #pragma unroll
       for (int s = 0; s < kSteps; ++s) {
         Op q;
@@ -573,7 +574,6 @@ __global__ void __launch_bounds__(kSplitThreads, (split_waves_per_simd<D, KV>())
       if (__any(alpha != 1.f)) {
 #pragma unroll
         for (int j = 0; j < kJ; ++j) acc[j] *= alpha;
-        if (T::kBias != 0.f) accw *= alpha;
       }
       uint32_t part[4][3];
 #pragma unroll
@@ -589,10 +589,6 @@ __global__ void __launch_bounds__(kSplitThreads, (split_waves_per_simd<D, KV>())
           for (int i = 0; i < 3; ++i) acc[j] = T::mfma(v, pw[i], acc[j]);
         }
       }
-      if (T::kBias != 0.f) {
-#pragma unroll
-        for (int i = 0; i < 3; ++i) accw = T::mfma(T::ones(), pw[i], accw);
-      }
       if (more) load_v(nxt, t_next);
       if (!more || nxt.number != cur.number) break;
     }
@@ -604,13 +600,12 @@ __global__ void __launch_bounds__(kSplitThreads, (split_waves_per_simd<D, KV>())
       __builtin_amdgcn_s_sleep(1);
     const float l_row = sum_across_rows(l_run);
     if (r < R) {
-      const float bias = T::kBias * accw[0];
 #pragma unroll
       for (int i = 0; i < 4; ++i)
 #pragma unroll
         for (int j = 0; j < kJ; j += 4)
           *reinterpret_cast<float4*>(&so[buf][wave][r][kJ * (4 * g + i) + j]) =
-              make_float4(acc[j][i] - bias, acc[j + 1][i] - bias, acc[j + 2][i] - bias, acc[j + 3][i] - bias);
+              make_float4(acc[j][i], acc[j + 1][i], acc[j + 2][i], acc[j + 3][i]);
       if (g == 0) {
         s_m[buf][wave][r] = m_run;
         s_l[buf][wave][r] = l_row;

@@ -155,3 +155,9 @@ def check_cancelling(d, kind, scale, top):
 @pytest.mark.parametrize("d", [64, 128, 256])
 def test_weights_are_float32(d):
   check_cancelling(d, "bf16", 1.0, min(d - 1, 127))
+
+
+@pytest.mark.parametrize("kind", ["int8_f32", "int8_bf16"])
+@pytest.mark.parametrize("d,top", [(64, 3), (128, 127), (256, 3)])
+def test_sums_of_small_codes_are_float32(d, top, kind):
+  check_cancelling(d, kind, 1.0, top)
