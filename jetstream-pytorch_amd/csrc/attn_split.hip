@@ -21,6 +21,9 @@
 // of their own, not 1152 too high.  (The constant, carried through float32 sums and taken out at their end,
 // costs ten bits of a sum of small terms: 1.4 % of the outputs of the case below were not the rounded exact
 // value.  A packed subtraction a pair of codes takes it out; four layers of the case below 275 -> 287 us.)
+// A weight times its value's scale is held against the row's largest so far, a power of two that rows carry
+// along as they do their maximum: float16 alone would lose scales below 1e-3 bit by bit (0.3 % of the outputs
+// of the case below, with scales of 0.03; all of them at 1e-7), and overflow above 65504.
 //
 // A sequence cut between groups: every group parks a float32 partial past the caches and counts
 // itself; the last one folds them.  No group waits for another.
@@ -40,6 +43,7 @@ constexpr int kSplitThreads = 64 * kSplitWaves;
 constexpr int kMaxGroups = kSplitCounters;
 constexpr int kLeastPart = 4;  // tiles, see where shares begin
 constexpr int kSeqCost = 1;    // tiles a wave, likewise
+constexpr int kLargestUp = 127 + 124;  // its inverse is a normal number too
 
 struct SplitParams {
   jpt_attn_args a;
@@ -528,6 +532,10 @@ __global__ void __launch_bounds__(kSplitThreads, (split_waves_per_simd<D, KV>())
 #pragma unroll
     for (int j = 0; j < kJ; ++j) acc[j] = f32x4{0.f, 0.f, 0.f, 0.f};
     float m_run = -INFINITY, l_run = 0.f;
+    // int8: the largest weight times value scale so far, and the exponent (biased as float32's) of the power
+    // of two that puts it in [2^14, 2^15): float16's range is too short for what scales may be
+    float w_run = 0.f;
+    int up = kLargestUp;
 
     for (;;) {
       const int valid = valid_of(cur, cur.ta + x - cur.base);
@@ -571,9 +579,22 @@ __global__ void __launch_bounds__(kSplitThreads, (split_waves_per_simd<D, KV>())
       }
       l_run = l_run * alpha + psum;
       m_run = m_new;
-      if (__any(alpha != 1.f)) {
+      float keep = alpha;  // what the products so far are multiplied with
+      if (SCALE) {
+        float w_max = 0.f;
 #pragma unroll
-        for (int j = 0; j < kJ; ++j) acc[j] *= alpha;
+        for (int i = 0; i < 8; ++i) w_max = fmaxf(w_max, fabsf(w[i]));
+        w_run = fmaxf(w_run * alpha, max_across_rows(w_max));
+        const int up_new = min(127 + 14 + 127 - static_cast<int>(__float_as_uint(w_run) >> 23), kLargestUp);
+        keep = ldexpf(alpha, up_new - up);
+        up = up_new;
+        const float by = __uint_as_float(static_cast<uint32_t>(up) << 23);
+#pragma unroll
+        for (int i = 0; i < 8; ++i) w[i] *= by;
+      }
+      if (__any(keep != 1.f)) {
+#pragma unroll
+        for (int j = 0; j < kJ; ++j) acc[j] *= keep;
       }
       uint32_t part[4][3];
 #pragma unroll
@@ -600,12 +621,13 @@ __global__ void __launch_bounds__(kSplitThreads, (split_waves_per_simd<D, KV>())
       __builtin_amdgcn_s_sleep(1);
     const float l_row = sum_across_rows(l_run);
     if (r < R) {
+      const float down = SCALE ? __uint_as_float(static_cast<uint32_t>(254 - up) << 23) : 1.f;
 #pragma unroll
       for (int i = 0; i < 4; ++i)
 #pragma unroll
         for (int j = 0; j < kJ; j += 4)
           *reinterpret_cast<float4*>(&so[buf][wave][r][kJ * (4 * g + i) + j]) =
-              make_float4(acc[j][i], acc[j + 1][i], acc[j + 2][i], acc[j + 3][i]);
+              make_float4(acc[j][i] * down, acc[j + 1][i] * down, acc[j + 2][i] * down, acc[j + 3][i] * down);
       if (g == 0) {
         s_m[buf][wave][r] = m_run;
         s_l[buf][wave][r] = l_row;

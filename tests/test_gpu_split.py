@@ -161,3 +161,32 @@ def test_weights_are_float32(d):
 @pytest.mark.parametrize("d,top", [(64, 3), (128, 127), (256, 3)])
 def test_sums_of_small_codes_are_float32(d, top, kind):
   check_cancelling(d, kind, 1.0, top)
+
+
+@pytest.mark.parametrize("kind", ["int8_f32", "int8_bf16"])
+@pytest.mark.parametrize("d,scale", [(64, 8e-8), (64, 1e3), (128, 1e-5), (256, 1e-6), (256, 1e-3), (256, 1e30)])
+def test_value_scales_of_any_size(d, scale, kind):
+  check_cancelling(d, kind, scale, min(d - 1, 127))
+
+
+@pytest.mark.parametrize("d", [64, 128, 256])
+def test_value_scales_far_apart(d):
+  """Scales of a slot's positions over twelve orders of magnitude, growing, falling and mixed, the large ones
+  on positions whose weights are small too: errors stay float32's beside the sum of the magnitudes."""
+  from jetstream_pt_amd import attention_kernel as ak
+  g = torch.Generator().manual_seed(1200 + d)
+  b, hq, hkv, s = 6, 8, 4, 300
+  q = (torch.randn((b, hq, 1, d), generator=g) * 0.1).to(torch.bfloat16)
+  k, v = (torch.randint(-127, 128, (b, hkv, s, d), generator=g, dtype=torch.int8) for _ in range(2))
+  ks = torch.full((b, 1, s, 1), 0.02)
+  spread = 10.0 ** (torch.rand((b, 1, s, 1), generator=g) * 12 - 7)
+  spread[0], spread[1] = spread[0].sort(1)[0], spread[1].sort(1, descending=True)[0]
+  q[2] *= 40.0  # sharp weights
+  end = torch.tensor([s, s, s, 33, 299, 64], dtype=torch.int32)
+  want, _, _ = OA.closed_form(q, k, v, lengths=end, k_scale=ks, v_scale=spread)
+  total, _, _ = OA.closed_form(q, k, v.abs(), lengths=end, k_scale=ks, v_scale=spread)
+  got, _ = ak.ragged_mha(q.to(DEV), k.to(DEV), v.to(DEV), 0, None, end.to(DEV), None, None, ks.to(DEV), spread.to(DEV))
+  # scores up to 8 (slot 2: 320): a unit of a weight for every 2^-24 of its score, sums of up to 300 terms
+  units = torch.tensor([64, 64, 1024, 64, 64, 64]).reshape(b, 1, 1, 1)
+  over = (got.double().cpu().reshape(want.shape) - want).abs() / float32_bound(want, total, units)
+  assert torch.all(over <= 1.0), over.amax((1, 2, 3))
