@@ -27,8 +27,8 @@
 // tiles are neither loaded nor computed, and all-zero tiles need no mask reads.
 //
 // Measured, causal, 32 query heads over 8 KV heads of 128, a call with its pass over
-// the mask, calls back to back: 1024 rows 46 us (12.3 ms for the shape-generic
-// kernel, one wave a row, scalar dot products), 3500 rows with scales 240 us (171 ms);
+// the mask, calls back to back: 1024 rows 48 us (12.3 ms for the shape-generic
+// kernel, one wave a row, scalar dot products), 3500 rows with scales 241 us (171 ms);
 // with weights of two bf16 numbers, 16 bits, they would be 41 and 199 us.  Outputs
 // that are not the rounded exact value: 0.025 % (shape-generic 0.034 %, 16 bits 0.21 %).
 #include <math.h>
@@ -224,8 +224,11 @@ __global__ void __launch_bounds__(64 * kWavesPerGroup, D == 256 ? 1 : 2) attn_pr
   for (int d = 0; d < kBlocks; ++d)
 #pragma unroll
     for (int i = 0; i < 16; ++i) o[d][i] = 0.f;
-  float m_run = -INFINITY, l_run = 0.f;  // log2 units; this lane's share of the row sum
-  const float c2 = a.sm_scale * kLog2e;
+  float m_run = -INFINITY, l_run = 0.f;  // l_run: this lane's share of the row sum
+  // Scores in log2 units - but where a mask is added, which may be float32's lowest value: that times
+  // log2(e) would be -infinity, and a row masked throughout empty instead of the mean of the values.
+  const float c2 = MASK ? a.sm_scale : a.sm_scale * kLog2e;
+  auto weight_of = [](float above_max) { return fast_exp2(MASK ? above_max * kLog2e : above_max); };
 
   // lane's addresses inside a tile: keys - row n, piece h; values - the transposing
   // read's row 4 h + (lane & 15) / 4 (+ 8 for the second half of a step's positions)
@@ -292,7 +295,7 @@ __global__ void __launch_bounds__(64 * kWavesPerGroup, D == 256 ? 1 : 2) attn_pr
 #pragma unroll
         for (int e = 0; e < 16; ++e) {
           const int at_pos = min(pos0 + 32 * mb + 8 * (e / 4) + e % 4, S - 1);
-          s[mb][e] += kLog2e * load_as_f32(a.mask, mrow + at_pos, MASK == 1 ? JPT_F32 : JPT_BF16);
+          s[mb][e] += load_as_f32(a.mask, mrow + at_pos, MASK == 1 ? JPT_F32 : JPT_BF16);
         }
     }
     if (tile * kCols + kCols > len) {  // the last tile's positions past the end
@@ -310,7 +313,7 @@ __global__ void __launch_bounds__(64 * kWavesPerGroup, D == 256 ? 1 : 2) attn_pr
     tmax = fmaxf(tmax, other_half(tmax));
     const float m_new = fmaxf(m_run, tmax);
     const float m_use = m_new == -INFINITY ? 0.f : m_new;
-    const float alpha = fast_exp2(m_run - m_use);
+    const float alpha = weight_of(m_run - m_use);
     m_run = m_new;
     l_run *= alpha;
     if (__any(alpha != 1.f)) {
@@ -322,7 +325,7 @@ __global__ void __launch_bounds__(64 * kWavesPerGroup, D == 256 ? 1 : 2) attn_pr
       float w[8];
 #pragma unroll
       for (int j = 0; j < 8; ++j) {
-        w[j] = fast_exp2(s[st >> 1][8 * (st & 1) + j] - m_use);
+        w[j] = weight_of(s[st >> 1][8 * (st & 1) + j] - m_use);
         l_run += w[j];
       }
       if (SCALE) {
@@ -376,7 +379,7 @@ __global__ void __launch_bounds__(64 * kWavesPerGroup, D == 256 ? 1 : 2) attn_pr
       *reinterpret_cast<uint2*>(dst + 64 * d + 16 * g) =
           make_uint2(pack_bf16(o[d][4 * g] * inv, o[d][4 * g + 1] * inv), pack_bf16(o[d][4 * g + 2] * inv, o[d][4 * g + 3] * inv));
   if (h == 0) {
-    if (a.out_max) a.out_max[q_row] = m_run * kLn2;
+    if (a.out_max) a.out_max[q_row] = MASK ? m_run : m_run * kLn2;
     if (a.out_denom) a.out_denom[q_row] = l;
   }
 }

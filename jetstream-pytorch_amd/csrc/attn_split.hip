@@ -333,7 +333,10 @@ __global__ void __launch_bounds__(kSplitThreads, (split_waves_per_simd<D, KV>())
   int pos[8];
 #pragma unroll
   for (int i = 0; i < 8; ++i) pos[i] = 4 * g + (i & 3) + 16 * (i >> 2);
-  const float c2 = a.sm_scale * kLog2e;
+  // Scores in log2 units - but where a mask is added, which may be float32's lowest value: that times
+  // log2(e) would be -infinity, and a row masked throughout empty instead of the mean of the values.
+  const float c2 = MASK ? a.sm_scale : a.sm_scale * kLog2e;
+  auto weight_of = [](float above_max) { return fast_exp2(MASK ? above_max * kLog2e : above_max); };
   const uint32_t q_lds = static_cast<uint32_t>(reinterpret_cast<uintptr_t>((lds_ptr)&s_q[wave][0]));
   auto q_row_of = [&](const Seq& s) { return (static_cast<int64_t>(s.slot) * a.q_heads + s.h * p.rep) * a.q_rows; };
   auto stage_q = [&](const Seq& s) {
@@ -418,7 +421,7 @@ __global__ void __launch_bounds__(kSplitThreads, (split_waves_per_simd<D, KV>())
     *reinterpret_cast<uint2*>(static_cast<uint16_t*>(a.out) + q_row * D + d) =
         make_uint2(pack_bf16(o[0] * inv, o[1] * inv), pack_bf16(o[2] * inv, o[3] * inv));
     if (d == 0) {
-      if (a.out_max) a.out_max[q_row] = M * kLn2;
+      if (a.out_max) a.out_max[q_row] = MASK ? M : M * kLn2;
       if (a.out_denom) a.out_denom[q_row] = l;
     }
   };
@@ -447,7 +450,7 @@ __global__ void __launch_bounds__(kSplitThreads, (split_waves_per_simd<D, KV>())
         if (i >= nw) continue;
         const int w = (w0 + i) % kSplitWaves;
         const float mw = s_m[buf][w][row];
-        const float f = mw == -INFINITY ? 0.f : fast_exp2(mw - M);
+        const float f = mw == -INFINITY ? 0.f : weight_of(mw - M);
         l += s_l[buf][w][row] * f;
         o += *reinterpret_cast<const f32x4*>(&so[buf][w][row][d]) * f;
       }
@@ -555,7 +558,7 @@ __global__ void __launch_bounds__(kSplitThreads, (split_waves_per_simd<D, KV>())
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
         sc[i] = (i < 4 ? sa[i] : sb[i - 4]) * (SCALE ? ks[i] * c2_row : c2_row);
-        if (MASK) sc[i] += mk[i] * kLog2e;
+        if (MASK) sc[i] += mk[i];
         if (valid != kTile) sc[i] = pos[i] < valid ? sc[i] : -INFINITY;
       }
       if (more) {
@@ -568,11 +571,11 @@ __global__ void __launch_bounds__(kSplitThreads, (split_waves_per_simd<D, KV>())
       tmax = max_across_rows(tmax);
       const float m_new = fmaxf(m_run, tmax);
       const float m_use = m_new == -INFINITY ? 0.f : m_new;
-      const float alpha = fast_exp2(m_run - m_use);
+      const float alpha = weight_of(m_run - m_use);
       float w[8], psum = 0.f;
 #pragma unroll
       for (int i = 0; i < 8; ++i) {
-        const float pr = fast_exp2(sc[i] - m_use);
+        const float pr = weight_of(sc[i] - m_use);
         psum += pr;
         w[i] = SCALE ? pr * vs[i] : pr;
         if (SCALE && valid != kTile) w[i] = pos[i] < valid ? w[i] : 0.f;  // whatever its scale holds
@@ -680,12 +683,12 @@ __global__ void __launch_bounds__(kSplitThreads, (split_waves_per_simd<D, KV>())
         float Mb = M;
 #pragma unroll
         for (int i = 0; i < 4; ++i) Mb = fmaxf(Mb, st[i][0]);
-        const float keep = M == -INFINITY ? 0.f : fast_exp2(M - Mb);
+        const float keep = M == -INFINITY ? 0.f : weight_of(M - Mb);
         l *= keep;
         o *= keep;
 #pragma unroll
         for (int i = 0; i < 4; ++i) {
-          const float f = c0 + i > g_last || st[i][0] == -INFINITY ? 0.f : fast_exp2(st[i][0] - Mb);
+          const float f = c0 + i > g_last || st[i][0] == -INFINITY ? 0.f : weight_of(st[i][0] - Mb);
           l += st[i][1] * f;
           o += y[i] * f;
         }

@@ -116,3 +116,31 @@ def test_weights_are_float32(masked, sdt, d):
   got = ak.dense_attention(*dev).double().cpu()
   over = (got - want).abs() / float32_bound(want, total)
   assert torch.all(over <= 1.0), float(over.max())
+
+
+LOWEST = [torch.finfo(torch.float32).min, OA.DEFAULT_MASK_VALUE, -2.0 ** 127]
+
+
+@pytest.mark.parametrize("low", LOWEST)
+@pytest.mark.parametrize("d,t,s,dtype", [(64, 20, 100, torch.float32), (128, 200, 300, torch.float32), (256, 20, 64, torch.float32),
+                                         (128, 150, 320, torch.bfloat16)])
+def test_masks_of_the_lowest_finite_value(d, t, s, dtype, low):
+  """A row masked throughout with a finite value attends every position alike; a row with a live position
+  attends only those that are live; beyond them -inf still counts for nothing."""
+  from jetstream_pt_amd import attention_kernel as ak
+  g = torch.Generator().manual_seed(950 + d + t)
+  b, hq, hkv = 2, 4, 2
+  low = max(low, torch.finfo(dtype).min)
+  q, k, v = rnd(g, (b, hq, t, d)), rnd(g, (b, hkv, s, d)), rnd(g, (b, hkv, s, d))
+  mask = torch.full((b, 1, t, s), low).to(dtype)
+  mask[:, :, t // 2:, : s // 3] = 0.0
+  mask[1, :, 0] = -math.inf
+  mask[1, :, :, s - 1] = -math.inf
+  rows = mask.expand(b, hq, t, s).reshape(b, hkv, hq // hkv * t, s)
+  want, wm, wl = OA.closed_form(q, k, v, mask=rows)
+  got, (m, l) = ak.flash_attention(*(x.to(DEV) for x in (q, k, v)), 0, None, None, mask.to(DEV))
+  err = (got.double().cpu() - want).abs()
+  assert torch.all(err <= torch.where(want.abs() < 2.0, torch.full_like(err, 6e-3), attention_bound(want))), float(err.max())
+  live = wl > 0
+  assert torch.allclose(m.double().cpu()[live], wm[live], rtol=1e-3, atol=1e-4)
+  assert torch.allclose(l.double().cpu()[live], wl[live], rtol=1e-3)

@@ -190,3 +190,22 @@ def test_value_scales_far_apart(d):
   units = torch.tensor([64, 64, 1024, 64, 64, 64]).reshape(b, 1, 1, 1)
   over = (got.double().cpu().reshape(want.shape) - want).abs() / float32_bound(want, total, units)
   assert torch.all(over <= 1.0), over.amax((1, 2, 3))
+
+
+@pytest.mark.parametrize("kind", ["bf16", "int8_f32"])
+@pytest.mark.parametrize("low", [torch.finfo(torch.float32).min, OA.DEFAULT_MASK_VALUE])
+@pytest.mark.parametrize("d,s", [(64, 160), (128, 77), (256, 2048)])
+def test_masks_of_the_lowest_finite_value(d, s, low, kind):
+  from jetstream_pt_amd import attention_kernel as ak
+  g = torch.Generator().manual_seed(1300 + d)
+  b, hq, hkv = 3, 4, 2
+  q = torch.randn((b, hq, 1, d), generator=g).to(torch.bfloat16)
+  k, v, ks, vs = make(g, kind, b, hkv, s, d, 1)
+  mask = torch.full((b, 1, 1, s), low)      # slot 0: masked throughout
+  mask[1, ..., : s // 2] = 0.0              # slot 1: a live half
+  mask[2, ..., 5:] = -math.inf              # slot 2: five positions at the lowest value, nothing else
+  rows = mask.expand(b, hq, 1, s).reshape(b, hkv, hq // hkv, s)
+  want, wm, wl = OA.closed_form(q, k, v, mask=rows, k_scale=ks, v_scale=vs)
+  dev = [None if x is None else x.to(DEV) for x in (q, k, v, ks, vs, mask)]
+  o, (m, l) = ak.flash_attention(*dev[:3], 0, dev[3], dev[4], dev[5])
+  check(o, want, m, l, wm, wl)
