@@ -132,13 +132,14 @@ class AttentionKernel:
       return _host.eager_step(xq, xk, xv, mask, cache.cache_k, cache.cache_v, ks, vs, cache.input_pos, env.ring_buffer,
                               rounding, freqs_cis)
     if kind is PageKVCacheGenerate or kind is Int8PageKVCacheGenerate:
-      pam = cache.page_attention_manager
-      lens = getattr(pam, "step_lens", None)
-      if lens is None or not (env.page_attention and self.fuse_new_token) or env.ragged_mha or env.flash_attention:
-        return None
-      pages, table = cache.cache_k, pam.page_indices
-      step_plan = ak.paged_decode_plan(pam, lens, xq.shape[0], xq.shape[1], pages.shape[0], pages.shape[2], table.shape[1])
       int8 = kind is Int8PageKVCacheGenerate
+      pages = cache.cache_k
+      # looked at before anything is planned: where another launch appends, the step is planned for other lengths
+      if not self._will_append_in_launch(xq, cache, pages) or (int8 and xk.dtype != torch.bfloat16):
+        return None
+      pam = cache.page_attention_manager
+      lens, table = pam.step_lens, pam.page_indices
+      step_plan = ak.paged_decode_plan(pam, lens, xq.shape[0], xq.shape[1], pages.shape[0], pages.shape[2], table.shape[1])
       return _host.paged_step(xq, xk, xv, pages, cache.cache_v, cache.k_scaler if int8 else None,
                               cache.v_scaler if int8 else None, lens, table, step_plan, self.sm_scale_paged,
                               _rounding_code(cache.rounding) if int8 else 0, freqs_cis)

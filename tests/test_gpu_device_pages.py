@@ -345,3 +345,37 @@ def test_a_decode_step_without_a_free_page_drops_the_token_and_touches_no_other_
   with pytest.raises(queue.Empty):
     dp.check()
   dp.check()  # the record was cleared
+
+
+@pytest.mark.parametrize("kind,dim,ps", [("bf16", 128, 32), ("int8", 128, 32), ("bf16", 64, 32), ("bf16", 256, 32), ("bf16", 128, 16),
+                                         ("int8", 64, 32), ("int8 f32 rows", 128, 32)])
+def test_a_paged_step_plans_once_whatever_takes_it(kind, dim, ps, monkeypatch):
+  """Calls that the launch which appends does not take are not planned for it: the layers of a step share one
+  plan, as they do where it takes them."""
+  from jetstream_pt_amd import attention_kernel as ak, cache_manager as cm, layers
+  from jetstream_pt_amd.environment import JetEngineEnvironment, JetEngineEnvironmentData
+  from jetstream_pt_amd.page_attention_manager import DevicePageAttentionManager
+  b, hq, hkv, total, n_layers = 3, 8, 2, 24, 3
+  env = JetEngineEnvironment(JetEngineEnvironmentData(batch_size=b, num_layers=n_layers, paged_attention_total_num_pages=total,
+                                                      paged_attention_page_size=ps))
+  pam = DevicePageAttentionManager(b, total, ps, 4, device=DEV)
+  lens = torch.tensor([5, 17, 30], dtype=torch.int32, device=DEV)
+  pam.reserve_pages_insert_many(torch.arange(b, dtype=torch.int32), lens.cpu())
+  int8 = kind.startswith("int8")
+  pages = lambda: torch.zeros((hkv, total, ps, dim), dtype=torch.int8 if int8 else torch.bfloat16, device=DEV)
+  scales = lambda: torch.ones((1, total, ps), device=DEV)
+  if int8:
+    caches = [cm.Int8PageKVCacheGenerate(pages(), pages(), scales(), scales(), pam, None, env=env) for _ in range(n_layers)]
+  else:
+    caches = [cm.PageKVCacheGenerate(pages(), pages(), pam, None, env=env) for _ in range(n_layers)]
+  kernels = [(layers.Int8KVAttentionKernel if int8 else layers.AttentionKernel)(env, l) for l in range(n_layers)]
+  made = []
+  plan = ak.DecodePlan
+  monkeypatch.setattr(ak, "DecodePlan", lambda *a, **k: made.append(a) or plan(*a, **k))
+  q = torch.ones((b, hq, 1, dim), dtype=torch.bfloat16, device=DEV)
+  row = torch.ones((b, hkv, 1, dim), dtype=torch.float32 if kind.endswith("f32 rows") else torch.bfloat16, device=DEV)
+  indices = pam.decode_step(lens)
+  for c, k in zip(caches, kernels):
+    c.page_token_indices = indices
+    k(q, row, row, None, c)
+  assert len(made) == 1
