@@ -116,23 +116,25 @@ class AttentionKernel:
     it then goes the general way below, launch by launch."""
     env = self.env
     kind = type(cache)
-    if kind is KVCacheGenerate or kind is Int8KVCacheGenerate:
-      int8 = kind is Int8KVCacheGenerate
+    int8 = isinstance(self, Int8KVAttentionKernel)
+    if kind is (Int8KVCacheGenerate if int8 else KVCacheGenerate):
       ks, vs, rounding = (cache.k_scaler, cache.v_scaler, _rounding_code(cache.rounding)) if int8 else (None, None, 0)
+      mode = cache.env  # how the cache is updated is the cache's to say
       if env.lazy_cache_update:
-        if not (env.ragged_mha and env.generate_cache_stacked and env.new_cache_stacked and self.fuse_new_token):
+        if not (mode.lazy_cache_update and mode.generate_cache_stacked and mode.new_cache_stacked
+                and env.ragged_mha and self.fuse_new_token):
           return None
         if int8 and not self.fuse_quantize:
           return None
         return _host.lazy_step(xq, xk, xv, cache.cache_k, cache.cache_v, ks, vs, cache.new_ks, cache.new_vs,
                                cache.new_k_scaler if int8 else None, cache.new_v_scaler if int8 else None, self.layer_id,
                                end, plan if isinstance(plan, ak.DecodePlan) else None, rounding, freqs_cis)
-      if env.ragged_mha or env.flash_attention or env.generate_cache_stacked or env.new_cache_stacked:
+      if (mode.lazy_cache_update or mode.generate_cache_stacked or mode.new_cache_stacked
+          or env.ragged_mha or env.flash_attention):
         return None
-      return _host.eager_step(xq, xk, xv, mask, cache.cache_k, cache.cache_v, ks, vs, cache.input_pos, env.ring_buffer,
+      return _host.eager_step(xq, xk, xv, mask, cache.cache_k, cache.cache_v, ks, vs, cache.input_pos, mode.ring_buffer,
                               rounding, freqs_cis)
-    if kind is PageKVCacheGenerate or kind is Int8PageKVCacheGenerate:
-      int8 = kind is Int8PageKVCacheGenerate
+    if kind is (Int8PageKVCacheGenerate if int8 else PageKVCacheGenerate):
       pages = cache.cache_k
       # looked at before anything is planned: where another launch appends, the step is planned for other lengths
       if not self._will_append_in_launch(xq, cache, pages) or (int8 and xk.dtype != torch.bfloat16):

@@ -147,3 +147,49 @@ def test_stacks_of_layers_are_taken_only_where_a_layer_is_named():
   for a, w in zip(ak.flash_attention(q, codes, codes, 1, scales, scales)[1], ak.flash_attention(q, codes[1], codes[1], 0, scales[1], scales[1])[1]):
     assert torch.equal(a, w)
   assert torch.equal(ak.ragged_mha(q, k, v, 2, None, lens)[0], ak.ragged_mha(q, k[2], v[2], 0, None, lens)[0])
+
+
+@pytest.mark.parametrize("int8_kernel", [False, True])
+@pytest.mark.parametrize("mode", ["ring", "lazy", "paged"])
+def test_kernels_and_caches_that_do_not_belong_together_are_refused(mode, int8_kernel):
+  """The bf16 kernel on an int8 cache and the int8 kernel on a bf16 one raise, as they do launch by launch."""
+  from jetstream_pt_amd import attention_kernel as ak, cache_manager as cm, layers
+  from jetstream_pt_amd.environment import JetEngineEnvironment, JetEngineEnvironmentData
+  from jetstream_pt_amd.page_attention_manager import DevicePageAttentionManager
+  b, hq, hkv, s, d, nl = 2, 8, 2, 64, 128, 2
+  env = JetEngineEnvironment(JetEngineEnvironmentData(batch_size=b, num_layers=nl, ring_buffer=mode == "ring",
+                                                      paged_attention_total_num_pages=8 if mode == "paged" else 0, paged_attention_page_size=32))
+  kern = (layers.Int8KVAttentionKernel if int8_kernel else layers.AttentionKernel)(env, 0)
+  lens = torch.tensor([3, 40], dtype=torch.int32, device=DEV)
+  kw = {}
+  if mode == "paged":
+    pam = DevicePageAttentionManager(b, 8, 32, 4, device=DEV)
+    pam.reserve_pages_insert_many(torch.arange(b, dtype=torch.int32), lens.cpu())
+    pages = [torch.zeros((hkv, 8, 32, d), dtype=torch.bfloat16 if int8_kernel else torch.int8, device=DEV) for _ in range(2)]
+    scales = [torch.ones((1, 8, 32), device=DEV) for _ in range(2)]
+    cache = cm.PageKVCacheGenerate(*pages, pam, None, env=env) if int8_kernel else cm.Int8PageKVCacheGenerate(*pages, *scales, pam, None, env=env)
+    cache.page_token_indices = pam.decode_step(lens)
+  else:
+    kind = cm.KVCacheGenerate if int8_kernel else cm.Int8KVCacheGenerate
+    cache = kind.empty((b, hkv, s, d) if mode == "ring" else (nl, b, hkv, s, d), DEV, env)
+    cache.input_pos = torch.tensor([40], dtype=torch.int32, device=DEV) if mode == "ring" else lens
+    if mode == "lazy":
+      plan, _ = ak.precompute_ragged_block_indices(lens, b, hq, hkv, s)
+      kw = dict(start=None, end=plan.lengths, ragged_batch_index=plan)
+  q, k, v = (torch.ones((b, h, 1, d), dtype=torch.bfloat16, device=DEV) for h in (hq, hkv, hkv))
+  with pytest.raises(ValueError, match="unpack"):
+    kern(q, k, v, torch.zeros((b, 1, 1, s), device=DEV) if mode == "ring" else None, cache, **kw)
+
+
+@pytest.mark.parametrize("int8", [False, True])
+def test_how_a_cache_is_updated_is_the_caches_to_say(int8):
+  """A cache that stashes its lines, under a kernel whose environment writes at once: the cache stashes."""
+  from jetstream_pt_amd import cache_manager as cm, layers
+  from jetstream_pt_amd.environment import JetEngineEnvironment, JetEngineEnvironmentData
+  b, hq, hkv, s, d = 2, 8, 2, 64, 128
+  eager, lazy = (JetEngineEnvironment(JetEngineEnvironmentData(batch_size=b, num_layers=1, testing=True, lazy_cache_update=x)) for x in (False, True))
+  cache = (cm.Int8KVCacheGenerate if int8 else cm.KVCacheGenerate).empty((b, hkv, s, d), DEV, lazy)
+  cache.input_pos = torch.tensor([40], dtype=torch.int32, device=DEV)
+  q, k, v = (torch.ones((b, h, 1, d), dtype=torch.bfloat16, device=DEV) for h in (hq, hkv, hkv))
+  (layers.Int8KVAttentionKernel if int8 else layers.AttentionKernel)(eager, 0)(q, k, v, torch.zeros((b, 1, 1, s), device=DEV), cache)
+  assert torch.all(cache.cache_k == 0) and torch.all(cache.new_ks != 0)
