@@ -112,8 +112,9 @@ class AttentionKernel:
     """A decode step's layer in one native call - cache update, attention, the token
     merged - in the modes a serving loop runs: the stacked lazy cache with ragged
     attention, the eagerly written cache under a mask, pages with the device
-    allocator.  None, with nothing returned yet, where the call is anything else:
-    it then goes the general way below, launch by launch."""
+    allocator.  None where the call is anything else - another attention put in the
+    kernel's place for one, too: it then goes the general way below, launch by
+    launch, which writes the token's line again if that was written already."""
     env = self.env
     kind = type(cache)
     int8 = isinstance(self, Int8KVAttentionKernel)
@@ -122,7 +123,7 @@ class AttentionKernel:
       mode = cache.env  # how the cache is updated is the cache's to say
       if env.lazy_cache_update:
         if not (mode.lazy_cache_update and mode.generate_cache_stacked and mode.new_cache_stacked
-                and env.ragged_mha and self.fuse_new_token):
+                and env.ragged_mha and self.fuse_new_token and type(self.ragged_attention_new) is ak.RaggedAttentionKernel):
           return None
         if int8 and not self.fuse_quantize:
           return None
@@ -130,14 +131,15 @@ class AttentionKernel:
                                cache.new_k_scaler if int8 else None, cache.new_v_scaler if int8 else None, self.layer_id,
                                end, plan if isinstance(plan, ak.DecodePlan) else None, rounding, freqs_cis)
       if (mode.lazy_cache_update or mode.generate_cache_stacked or mode.new_cache_stacked
-          or env.ragged_mha or env.flash_attention):
+          or env.ragged_mha or env.flash_attention or self.dense_attention is not ak.dense_attention):
         return None
       return _host.eager_step(xq, xk, xv, mask, cache.cache_k, cache.cache_v, ks, vs, cache.input_pos, mode.ring_buffer,
                               rounding, freqs_cis)
     if kind is (Int8PageKVCacheGenerate if int8 else PageKVCacheGenerate):
       pages = cache.cache_k
       # looked at before anything is planned: where another launch appends, the step is planned for other lengths
-      if not self._will_append_in_launch(xq, cache, pages) or (int8 and xk.dtype != torch.bfloat16):
+      if (not self._will_append_in_launch(xq, cache, pages) or (int8 and xk.dtype != torch.bfloat16)
+          or self.page_attention is not ak.call_paged_attention):
         return None
       pam = cache.page_attention_manager
       lens, table = pam.step_lens, pam.page_indices

@@ -193,3 +193,33 @@ def test_how_a_cache_is_updated_is_the_caches_to_say(int8):
   q, k, v = (torch.ones((b, h, 1, d), dtype=torch.bfloat16, device=DEV) for h in (hq, hkv, hkv))
   (layers.Int8KVAttentionKernel if int8 else layers.AttentionKernel)(eager, 0)(q, k, v, torch.zeros((b, 1, 1, s), device=DEV), cache)
   assert torch.all(cache.cache_k == 0) and torch.all(cache.new_ks != 0)
+
+
+@pytest.mark.parametrize("mode", ["ring", "lazy", "paged"])
+def test_an_attention_put_in_the_kernels_place_is_the_one_that_runs(mode):
+  from jetstream_pt_amd import attention_kernel as ak, cache_manager as cm, layers
+  from jetstream_pt_amd.environment import JetEngineEnvironment, JetEngineEnvironmentData
+  from jetstream_pt_amd.page_attention_manager import DevicePageAttentionManager
+  b, hq, hkv, s, d, nl = 2, 8, 2, 64, 128, 2
+  env = JetEngineEnvironment(JetEngineEnvironmentData(batch_size=b, num_layers=nl, ring_buffer=mode == "ring",
+                                                      paged_attention_total_num_pages=8 if mode == "paged" else 0, paged_attention_page_size=32))
+  kern = layers.AttentionKernel(env, 0)
+  lens = torch.tensor([3, 40], dtype=torch.int32, device=DEV)
+  kw, name = {}, {"ring": "dense_attention", "lazy": "ragged_attention_new", "paged": "page_attention"}[mode]
+  ran = []
+  own = getattr(kern, name)
+  setattr(kern, name, lambda *a, **k: ran.append(name) or own(*a, **k))
+  if mode == "paged":
+    pam = DevicePageAttentionManager(b, 8, 32, 4, device=DEV)
+    pam.reserve_pages_insert_many(torch.arange(b, dtype=torch.int32), lens.cpu())
+    cache = cm.PageKVCacheGenerate(*(torch.zeros((hkv, 8, 32, d), dtype=torch.bfloat16, device=DEV) for _ in range(2)), pam, None, env=env)
+    cache.page_token_indices = pam.decode_step(lens)
+  else:
+    cache = cm.KVCacheGenerate.empty((b, hkv, s, d) if mode == "ring" else (nl, b, hkv, s, d), DEV, env)
+    cache.input_pos = torch.tensor([40], dtype=torch.int32, device=DEV) if mode == "ring" else lens
+    if mode == "lazy":
+      plan, _ = ak.precompute_ragged_block_indices(lens, b, hq, hkv, s)
+      kw = dict(start=None, end=plan.lengths, ragged_batch_index=plan)
+  q, k, v = (torch.ones((b, h, 1, d), dtype=torch.bfloat16, device=DEV) for h in (hq, hkv, hkv))
+  kern(q, k, v, torch.zeros((b, 1, 1, s), device=DEV) if mode == "ring" else None, cache, **kw)
+  assert ran == [name]
