@@ -61,6 +61,24 @@ void check(int32_t status) {
   throw Raised{};
 }
 
+// A call into the library, which knows nothing of Python: other threads run meanwhile (a launch waits where
+// the queue is full).  What the launch reads is held by the caller's arguments, or by copies of the tensors.
+class Unlocked {
+ public:
+  Unlocked() : state_(PyEval_SaveThread()) {}
+  ~Unlocked() { PyEval_RestoreThread(state_); }
+  Unlocked(const Unlocked&) = delete;
+  Unlocked& operator=(const Unlocked&) = delete;
+
+ private:
+  PyThreadState* state_;
+};
+template <typename F, typename... A>
+int32_t unlocked(F fn, A... args) {
+  Unlocked here;
+  return fn(args...);
+}
+
 void* stream() { return c10::hip::getCurrentHIPStream().stream(); }
 
 int dtype_code(const Tensor& t) {
@@ -278,8 +296,8 @@ Attended attend(Mode mode, const Tensor& q, const Tensor& keys, const Tensor& va
     }
     if (a.workspace == nullptr) use_shared(lib.workspace_bytes(&a));
   }
-  if (token != nullptr && token->stash_k != nullptr) check(lib.ragged_stash(&a, token->stash_k, token->stash_v, stream()));
-  else check(lib.attn[mode](&a, stream()));
+  if (token != nullptr && token->stash_k != nullptr) check(unlocked(lib.ragged_stash, &a, token->stash_k, token->stash_v, stream()));
+  else check(unlocked(lib.attn[mode], &a, stream()));
   return r;
 }
 
@@ -452,7 +470,7 @@ PyObject* py_eager_step(PyObject*, PyObject* const* x, Py_ssize_t n) {
       a.scale_heads = static_cast<int32_t>(ks->size(1));
       a.rounding = static_cast<int32_t>(whole(x[10]));
       a.rope = rope_of(opt(x[11]), b, d);
-      check(lib.append_quant(&a, stream()));
+      check(unlocked(lib.append_quant, &a, stream()));
     } else {
       need(ks == nullptr && x[11] == Py_None);
       given_token(line, xk, xv, b, hkv, d, code);
@@ -460,7 +478,7 @@ PyObject* py_eager_step(PyObject*, PyObject* const* x, Py_ssize_t n) {
       jpt_line_tensor t[2]{};
       t[0].dst = ck.data_ptr(); t[0].src = line.k; t[0].heads = heads; t[0].row_bytes = bytes;
       t[1].dst = cv.data_ptr(); t[1].src = line.v; t[1].heads = heads; t[1].row_bytes = bytes;
-      check(lib.scatter_lines(t, 2, at, count, 1, static_cast<int32_t>(b), static_cast<int32_t>(seq), stream()));
+      check(unlocked(lib.scatter_lines, t, 2, at, count, 1, static_cast<int32_t>(b), static_cast<int32_t>(seq), stream()));
     }
     return wrap(attend(kDense, q, ck, cv, -1, nullptr, nullptr, mask, ks, vs, NAN, nullptr, false, nullptr).out);
   });
@@ -524,8 +542,8 @@ PyObject* py_scatter_lines(PyObject*, PyObject* const* x, Py_ssize_t n) {
       t[i].heads = static_cast<int32_t>(heads);
       t[i].row_bytes = static_cast<int32_t>(row * dst.element_size());
     }
-    check(lib.scatter_lines(t, static_cast<int32_t>(m), static_cast<const int32_t*>(pos.data_ptr()), static_cast<int32_t>(count),
-                            static_cast<int32_t>(layers), static_cast<int32_t>(batch), static_cast<int32_t>(seq), stream()));
+    check(unlocked(lib.scatter_lines, t, static_cast<int32_t>(m), static_cast<const int32_t*>(pos.data_ptr()), static_cast<int32_t>(count),
+                   static_cast<int32_t>(layers), static_cast<int32_t>(batch), static_cast<int32_t>(seq), stream()));
     Py_RETURN_TRUE;
   });
 }
@@ -541,16 +559,16 @@ Py_ssize_t count_of(PyObject* o) {
   return PySequence_Fast_GET_SIZE(o);
 }
 // Member `which` of layer `layer`'s pair: a list of pairs, a list of one pair of stacks, or a pair of stacks.
-Layer layer_of(PyObject* caches, Py_ssize_t layer, Py_ssize_t layers, int which) {
+// `held` keeps it: the lists are the caller's to change while the library runs.
+Layer layer_of(PyObject* caches, Py_ssize_t layer, Py_ssize_t layers, int which, std::vector<Tensor>& held) {
   PyObject* first = item(caches, 0);
-  if (PyList_Check(first) || PyTuple_Check(first)) {
-    if (count_of(caches) == 1 && ten(item(first, 0)).dim() == 5) return Layer(ten(item(first, which)), 4, layer);
-    need(count_of(caches) >= layers);
-    const Tensor& t = ten(item(item(caches, layer), which));
-    need(t.dim() == 4);
-    return Layer(t, 4, -1);
-  }
-  return Layer(ten(item(caches, which)), 4, layer);
+  const bool pairs = PyList_Check(first) || PyTuple_Check(first);
+  const bool stacks = !pairs || (count_of(caches) == 1 && ten(item(first, 0)).dim() == 5);
+  if (!stacks) need(count_of(caches) >= layers);
+  const Tensor& t = ten(item(!pairs ? caches : stacks ? first : item(caches, layer), which));
+  need(stacks || t.dim() == 4);
+  if (!stacks || layer == 0) held.push_back(t);
+  return Layer(t, 4, stacks ? layer : -1);
 }
 
 // insert_layers(prefix, caches, scales | None, page_ids | None, slot, start, rounding) -> True | None.
@@ -564,10 +582,14 @@ PyObject* py_insert_layers(PyObject*, PyObject* const* x, Py_ssize_t n) {
     jpt_prefill_insert_args a{};
     std::vector<jpt_insert_layer> table(layers);
     c10::IntArrayRef cache_sizes, prefix_sizes, scale_sizes;
+    std::vector<Tensor> held;
+    held.reserve(6 * layers);
     for (Py_ssize_t l = 0; l < layers; ++l) {
       PyObject* pair = item(x[0], l);
       const Tensor &pk = ten(item(pair, 0)), &pv = ten(item(pair, 1));
-      const Layer k = layer_of(x[1], l, layers, 0), v = layer_of(x[1], l, layers, 1);
+      held.push_back(pk);
+      held.push_back(pv);
+      const Layer k = layer_of(x[1], l, layers, 0, held), v = layer_of(x[1], l, layers, 1, held);
       need(k.sizes == v.sizes && k.code == v.code && pk.sizes() == pv.sizes() && pk.scalar_type() == pv.scalar_type());
       const int in = dtype_code(pk);
       const bool quant = k.code == JPT_I8 && in != JPT_I8;
@@ -583,7 +605,7 @@ PyObject* py_insert_layers(PyObject*, PyObject* const* x, Py_ssize_t n) {
       out.k_scale = out.v_scale = nullptr;
       if (quant) {
         need(!paged && x[2] != Py_None);
-        const Layer ks = layer_of(x[2], l, layers, 0), vs = layer_of(x[2], l, layers, 1);
+        const Layer ks = layer_of(x[2], l, layers, 0, held), vs = layer_of(x[2], l, layers, 1, held);
         need(ks.sizes == vs.sizes && ks.code == vs.code && ks.code != JPT_I8 && ks.sizes[0] == k.sizes[0] && ks.sizes[2] == k.sizes[2]);
         out.k_scale = ks.data;
         out.v_scale = vs.data;
@@ -619,7 +641,7 @@ PyObject* py_insert_layers(PyObject*, PyObject* const* x, Py_ssize_t n) {
       }
       need(k.sizes == cache_sizes && pk.sizes() == prefix_sizes && in == a.in_dtype && k.code == a.dst_dtype);
     }
-    check(lib.insert_layers(&a, table.data(), static_cast<int32_t>(layers), stream()));
+    check(unlocked(lib.insert_layers, &a, table.data(), static_cast<int32_t>(layers), stream()));
     Py_RETURN_TRUE;
   });
 }
@@ -643,7 +665,7 @@ PyObject* py_plan(PyObject*, PyObject* const* x, Py_ssize_t n) {
     const Tensor space = fresh ? at::empty({lib.workspace_bytes(&a)}, lengths.options().dtype(at::kByte)) : ten(x[8]);
     a.workspace = space.data_ptr();
     a.workspace_bytes = space.numel();
-    check(lib.plan[fresh](&a, a.page_size > 0, stream()));
+    check(unlocked(lib.plan[fresh], &a, a.page_size > 0, stream()));
     return wrap(space);
   });
 }
@@ -672,9 +694,9 @@ PyObject* py_insert_state(PyObject*, PyObject* const* x, Py_ssize_t n) {
       need(t->dim() == 1 && t->scalar_type() == at::kInt && slot < t->numel());
       rows[i] = static_cast<int32_t*>(t->data_ptr());
     }
-    check(lib.insert_state(mask, mask_code, seq, rows[0], rows[1], rows[2], static_cast<int32_t>(slot),
-                           static_cast<int32_t>(whole(x[5])), static_cast<int32_t>(whole(x[6])), 1, static_cast<int32_t>(whole(x[7])),
-                           static_cast<int32_t>(whole(x[8])), PyObject_IsTrue(x[9]), stream()));
+    check(unlocked(lib.insert_state, mask, mask_code, seq, rows[0], rows[1], rows[2], static_cast<int32_t>(slot),
+                   static_cast<int32_t>(whole(x[5])), static_cast<int32_t>(whole(x[6])), 1, static_cast<int32_t>(whole(x[7])),
+                   static_cast<int32_t>(whole(x[8])), PyObject_IsTrue(x[9]), stream()));
     Py_RETURN_TRUE;
   });
 }

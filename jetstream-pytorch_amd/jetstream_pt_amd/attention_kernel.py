@@ -142,12 +142,16 @@ def _dense_workspace(index, batch, q_heads, kv_heads, q_rows, seq):
   return ws, planned
 
 
+def _shared_workspace_buf(nbytes, index):
+  return _shared_workspace(nbytes, index).buf
+
+
 def _dense_workspace_buf(*shape):
   ws, planned = _dense_workspace(*shape)
   return ws.buf, planned
 
 
-_host.bind(_ffi.addresses(), _ffi.check, lambda nbytes, index: _shared_workspace(nbytes, index).buf, _dense_workspace_buf)
+_host.bind(_ffi.addresses(), _ffi.check, _shared_workspace_buf, _dense_workspace_buf)
 
 
 class DecodePlan:

@@ -223,3 +223,79 @@ def test_an_attention_put_in_the_kernels_place_is_the_one_that_runs(mode):
   q, k, v = (torch.ones((b, h, 1, d), dtype=torch.bfloat16, device=DEV) for h in (hq, hkv, hkv))
   kern(q, k, v, torch.zeros((b, 1, 1, s), device=DEV) if mode == "ring" else None, cache, **kw)
   assert ran == [name]
+
+
+def test_other_threads_run_while_the_library_does():
+  """Every call into the library is made without the interpreter's lock: in the library's place stands the
+  interpreter's own question whether this thread holds it, whose "no" is the library's OK."""
+  import ctypes
+  from jetstream_pt_amd import _ffi, _host, attention_kernel as ak
+  held = ctypes.cast(ctypes.pythonapi.PyGILState_Check, ctypes.c_void_p).value
+  asked = {name: held if name != "jpt_attn_workspace_bytes" else at for name, at in _ffi.addresses().items()}
+
+  def status(code):
+    raise AssertionError("the interpreter's lock was held")
+
+  b, hq, hkv, s, d, nl, t = 2, 8, 2, 64, 128, 2, 16
+  bf16 = lambda *shape: torch.zeros(shape, dtype=torch.bfloat16, device=DEV)
+  i8 = lambda *shape: torch.zeros(shape, dtype=torch.int8, device=DEV)
+  lens, table = (torch.ones(shape, dtype=torch.int32, device=DEV) for shape in ((b,), (b, 2)))
+  q, row, mask = bf16(b, hq, 1, d), bf16(b, hkv, 1, d), torch.zeros((b, s), device=DEV)
+  stack, lines, one = bf16(nl, b, hkv, s, d), bf16(nl, b, hkv, 1, d), bf16(b, hkv, s, d)
+  scale, new_scale, layer_scale = (torch.ones(shape, device=DEV) for shape in ((nl, b, 1, s, 1), (nl, b, 1, 1, 1), (b, 1, s, 1)))
+  pages, prompt = bf16(hkv, 8, 32, d), [(bf16(1, hkv, t, d), bf16(1, hkv, t, d))] * nl
+  torch.cuda.synchronize()
+  _host.bind(asked, status, ak._shared_workspace_buf, ak._dense_workspace_buf)
+  try:
+    done = [
+        _host.attend(0, q, one, one, -1, lens, None, None, None, None, None, None, None, None, None, None, None, 0, None, False, False, None),
+        _host.lazy_step(q, row, row, stack, stack, None, None, lines, lines, None, None, 0, lens, None, 0, None),
+        _host.lazy_step(q, row, row, stack.char(), stack.char(), scale, scale, lines.char(), lines.char(), new_scale, new_scale, 0, lens, None, 0, None),
+        _host.eager_step(q, row, row, mask[:, None, None], i8(b, hkv, s, d), i8(b, hkv, s, d), layer_scale, layer_scale, lens, False, 0, None),
+        _host.eager_step(q, row, row, mask[:, None, None], one, one, None, None, lens, False, 0, None),
+        _host.paged_step(q, row, row, pages, pages, None, None, lens, table, None, 1.0, 0, None),
+        _host.scatter_lines((stack,), (lines,), lens, b, nl, b, s),
+        _host.insert_layers(prompt, [(stack, stack)], None, None, 0, 0, 1),
+        _host.plan(lens, b, hq, hkv, 1, s, 0, 0, None),
+        _host.insert_state(mask, lens, lens, lens, 0, 0, 1, 0, 1, False),
+    ]
+  finally:
+    _host.bind(_ffi.addresses(), _ffi.check, ak._shared_workspace_buf, ak._dense_workspace_buf)
+  assert all(x is not None for x in done)
+
+
+def test_two_threads_on_streams_of_their_own():
+  """Steps through the native host side from two threads at once, each on its own stream: the bits of the
+  same steps one after the other."""
+  import threading
+  from jetstream_pt_amd import attention_kernel as ak
+  g = torch.Generator().manual_seed(77)
+  b, hq, hkv, s, d = 4, 8, 2, 512, 128
+  work = []
+  for dim in (d, 64):
+    q = torch.randn((b, hq, 1, dim), generator=g).to(torch.bfloat16).to(DEV)
+    k, v = (torch.randn((b, hkv, s, dim), generator=g).to(torch.bfloat16).to(DEV) for _ in range(2))
+    work.append((q, k, v, torch.zeros((b, 1, 1, s), device=DEV)))
+  run = lambda q, k, v, mask: ak.dense_attention(q, k, v, mask=mask)
+  want = [run(*w) for w in work]
+  torch.cuda.synchronize()
+  outs, errors = [[], []], []
+
+  def steps(i):
+    try:
+      with torch.cuda.stream(torch.cuda.Stream()):
+        for n in range(50):
+          outs[i].append(run(*work[(i + n) % 2]))
+        torch.cuda.current_stream().synchronize()
+    except Exception as e:  # pylint: disable=broad-except
+      errors.append(e)
+
+  threads = [threading.Thread(target=steps, args=(i,)) for i in range(2)]
+  for t in threads:
+    t.start()
+  for t in threads:
+    t.join()
+  assert not errors
+  for i in range(2):
+    for n, o in enumerate(outs[i]):
+      assert torch.equal(o, want[(i + n) % 2])
