@@ -560,11 +560,11 @@ Py_ssize_t count_of(PyObject* o) {
 }
 // Member `which` of layer `layer`'s pair: a list of pairs, a list of one pair of stacks, or a pair of stacks.
 // `held` keeps it: the lists are the caller's to change while the library runs.
-Layer layer_of(PyObject* caches, Py_ssize_t layer, Py_ssize_t layers, int which, std::vector<Tensor>& held) {
+Layer layer_of(PyObject* caches, Py_ssize_t layer, Py_ssize_t layers, int which, bool paged, std::vector<Tensor>& held) {
   PyObject* first = item(caches, 0);
   const bool pairs = PyList_Check(first) || PyTuple_Check(first);
   const bool stacks = !pairs || (count_of(caches) == 1 && ten(item(first, 0)).dim() == 5);
-  if (!stacks) need(count_of(caches) >= layers);
+  need(stacks ? !paged : count_of(caches) >= layers);
   const Tensor& t = ten(item(!pairs ? caches : stacks ? first : item(caches, layer), which));
   need(stacks || t.dim() == 4);
   if (!stacks || layer == 0) held.push_back(t);
@@ -572,7 +572,7 @@ Layer layer_of(PyObject* caches, Py_ssize_t layer, Py_ssize_t layers, int which,
 }
 
 // insert_layers(prefix, caches, scales | None, page_ids | None, slot, start, rounding) -> True | None.
-// Dense slots (page_ids None): caches (B, H, S, D); pages: (H, P, ps, D).
+// Dense slots (page_ids None): caches (B, H, S, D), or stacks of them; pages: a list of pairs (H, P, ps, D).
 PyObject* py_insert_layers(PyObject*, PyObject* const* x, Py_ssize_t n) {
   return guarded([&]() -> PyObject* {
     need(n == 7);
@@ -589,12 +589,12 @@ PyObject* py_insert_layers(PyObject*, PyObject* const* x, Py_ssize_t n) {
       const Tensor &pk = ten(item(pair, 0)), &pv = ten(item(pair, 1));
       held.push_back(pk);
       held.push_back(pv);
-      const Layer k = layer_of(x[1], l, layers, 0, held), v = layer_of(x[1], l, layers, 1, held);
+      const Layer k = layer_of(x[1], l, layers, 0, paged, held), v = layer_of(x[1], l, layers, 1, paged, held);
       need(k.sizes == v.sizes && k.code == v.code && pk.sizes() == pv.sizes() && pk.scalar_type() == pv.scalar_type());
       const int in = dtype_code(pk);
       const bool quant = k.code == JPT_I8 && in != JPT_I8;
       need(quant || in == k.code);
-      need(pk.dim() == 3 || (pk.dim() == 4 && pk.size(0) == 1));
+      need((pk.dim() == 3 && !paged) || (pk.dim() == 4 && pk.size(0) == 1));
       const int64_t heads = pk.size(-3), tokens = pk.size(-2), dim = pk.size(-1);
       need(heads == k.sizes[paged ? 0 : 1] && dim == k.sizes[3] && dim % 4 == 0);
       jpt_insert_layer& out = table[l];
@@ -605,7 +605,7 @@ PyObject* py_insert_layers(PyObject*, PyObject* const* x, Py_ssize_t n) {
       out.k_scale = out.v_scale = nullptr;
       if (quant) {
         need(!paged && x[2] != Py_None);
-        const Layer ks = layer_of(x[2], l, layers, 0, held), vs = layer_of(x[2], l, layers, 1, held);
+        const Layer ks = layer_of(x[2], l, layers, 0, paged, held), vs = layer_of(x[2], l, layers, 1, paged, held);
         need(ks.sizes == vs.sizes && ks.code == vs.code && ks.code != JPT_I8 && ks.sizes[0] == k.sizes[0] && ks.sizes[2] == k.sizes[2]);
         out.k_scale = ks.data;
         out.v_scale = vs.data;

@@ -228,7 +228,7 @@ def insert(env, prefix_caches, prefix_seq_len, caches, cache_scales, slot, *, cu
   # the slot's live positions: [lo, hi), or with `over_end` [lo, seq) and [0, hi)
   lo, hi = (cur - prefix_seq_len, cur) if not wrap else (first, current_position)
   over_end = wrap and not current_position > first
-  if _host.insert_state(mask, start, input_pos, lens, slot, first, prefix_seq_len, lo, hi, over_end):
+  if (mask is None or mask.shape[-1] == seq) and _host.insert_state(mask, start, input_pos, lens, slot, first, prefix_seq_len, lo, hi, over_end):
     return first
   if mask is not None:
     x = torch.arange(seq, device=mask.device)

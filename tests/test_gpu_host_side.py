@@ -299,3 +299,28 @@ def test_two_threads_on_streams_of_their_own():
   for i in range(2):
     for n, o in enumerate(outs[i]):
       assert torch.equal(o, want[(i + n) % 2])
+
+
+def test_inserts_refuse_what_they_refused():
+  """Prompts without their batch dimension into pages, stacks of pages, and masks of another length."""
+  from jetstream_pt_amd import insert as pi
+  from jetstream_pt_amd.environment import JetEngineEnvironment, JetEngineEnvironmentData
+  from jetstream_pt_amd.page_attention_manager import PageAttentionManager
+  hkv, t, d, ps, nl = 2, 40, 128, 32, 2
+  bf16 = lambda *shape: torch.ones(shape, dtype=torch.bfloat16, device=DEV)
+  ids = torch.tensor([3, 5], dtype=torch.int32, device=DEV)
+  pages = [(bf16(hkv, 8, ps, d), bf16(hkv, 8, ps, d)) for _ in range(nl)]
+  flat = [(bf16(hkv, t, d) * 2, bf16(hkv, t, d) * 2) for _ in range(nl)]
+  whole = [(k[None], v[None]) for k, v in flat]
+  pam = PageAttentionManager(2, 8, ps, 4)
+  with pytest.raises((ValueError, IndexError)):
+    pam.insert_prefill_cache(flat, pages, ids)
+  with pytest.raises(ValueError):
+    pi.insert_prefix_pages_copy(whole, [(bf16(nl, hkv, 8, ps, d), bf16(nl, hkv, 8, ps, d))], ids)
+  assert all(bool((x == 1).all()) for pair in pages for x in pair)
+  assert pi.insert_prefix_pages_copy(whole, pages, ids) and all(bool((x[:, 3] == 2).all()) for pair in pages for x in pair)
+  env = JetEngineEnvironment(JetEngineEnvironmentData(batch_size=2, num_layers=nl, cache_sequence_length=64, ring_buffer=False))
+  mask = torch.zeros((2, 96), device=DEV)
+  with pytest.raises(RuntimeError):
+    pi.insert(env, whole, t, [(bf16(nl, 2, hkv, 64, d), bf16(nl, 2, hkv, 64, d))], None, 1, mask=mask)
+  assert bool((mask == 0).all())
