@@ -18,7 +18,7 @@
 #include <c10/hip/HIPStream.h>
 
 #include <cmath>
-#include <initializer_list>
+#include <optional>
 #include <vector>
 
 #include "jpt_mi355.h"
@@ -154,7 +154,7 @@ struct Attended {
 
 // attention_kernel._attend.  keys / values may be stacks of layers.
 Attended attend(Mode mode, const Tensor& q, const Tensor& keys, const Tensor& values, int64_t layer, const Tensor* lengths,
-                const Tensor* table, const Tensor* mask, const Tensor* k_scaler, const Tensor* v_scaler, double sm_scale,
+                const Tensor* table, const Tensor* mask, const Tensor* k_scaler, const Tensor* v_scaler, std::optional<double> sm_scale,
                 const Token* token, bool stats, PyObject* plan) {
   need(q.dim() == 4);
   const int64_t b = q.size(0), hq = q.size(1), t = q.size(2), d = q.size(3);
@@ -230,7 +230,7 @@ Attended attend(Mode mode, const Tensor& q, const Tensor& keys, const Tensor& va
     a.new_rounding = token->rounding;
     a.new_to_pages = token->to_pages ? 1 : 0;
   }
-  a.sm_scale = static_cast<float>(std::isnan(sm_scale) ? 1.0 / std::sqrt(static_cast<double>(d)) : sm_scale);
+  a.sm_scale = static_cast<float>(sm_scale ? *sm_scale : 1.0 / std::sqrt(static_cast<double>(d)));
 
   Attended r;
   r.out = at::empty_like(q);
@@ -329,8 +329,8 @@ PyObject* wrap(const Tensor& t) {
   return THPVariable_Wrap(t);
 }
 
-double number(PyObject* o) {
-  if (o == Py_None) return NAN;
+std::optional<double> number(PyObject* o) {
+  if (o == Py_None) return std::nullopt;
   const double x = PyFloat_AsDouble(o);
   if (x == -1.0 && PyErr_Occurred()) throw Raised{};
   return x;
@@ -425,7 +425,7 @@ PyObject* py_lazy_step(PyObject*, PyObject* const* x, Py_ssize_t n) {
       token.stash_v = static_cast<char*>(nv.data_ptr()) + layer * row * 2;
     }
     need(is_int32(end, b));
-    const Attended r = attend(kRagged, q, ck, cv, layer, &end, nullptr, nullptr, ks, vs, NAN, &token, false, x[13]);
+    const Attended r = attend(kRagged, q, ck, cv, layer, &end, nullptr, nullptr, ks, vs, std::nullopt, &token, false, x[13]);
     return wrap(r.out);
   });
 }
@@ -480,7 +480,7 @@ PyObject* py_eager_step(PyObject*, PyObject* const* x, Py_ssize_t n) {
       t[1].dst = cv.data_ptr(); t[1].src = line.v; t[1].heads = heads; t[1].row_bytes = bytes;
       check(unlocked(lib.scatter_lines, t, 2, at, count, 1, static_cast<int32_t>(b), static_cast<int32_t>(seq), stream()));
     }
-    return wrap(attend(kDense, q, ck, cv, -1, nullptr, nullptr, mask, ks, vs, NAN, nullptr, false, nullptr).out);
+    return wrap(attend(kDense, q, ck, cv, -1, nullptr, nullptr, mask, ks, vs, std::nullopt, nullptr, false, nullptr).out);
   });
 }
 

@@ -324,3 +324,13 @@ def test_inserts_refuse_what_they_refused():
   with pytest.raises(RuntimeError):
     pi.insert(env, whole, t, [(bf16(nl, 2, hkv, 64, d), bf16(nl, 2, hkv, 64, d))], None, 1, mask=mask)
   assert bool((mask == 0).all())
+
+
+def test_a_scale_that_is_not_a_number_is_not_the_default():
+  from jetstream_pt_amd import attention_kernel as ak
+  g = torch.Generator().manual_seed(3)
+  q = torch.randn((1, 4, 128), generator=g).to(torch.bfloat16).to(DEV)
+  pages = torch.randn((2, 4, 32, 128), generator=g).to(torch.bfloat16).to(DEV)
+  lens, table = torch.tensor([20], dtype=torch.int32, device=DEV), torch.tensor([[1, 2]], dtype=torch.int32, device=DEV)
+  assert bool(ak.call_paged_attention(None, q, pages, pages, lens, table, sm_scale=float("nan")).isnan().all())
+  assert bool(ak.call_paged_attention(None, q, pages, pages, lens, table, sm_scale=0.1).isfinite().all())
