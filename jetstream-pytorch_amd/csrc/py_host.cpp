@@ -261,7 +261,17 @@ Attended attend(Mode mode, const Tensor& q, const Tensor& keys, const Tensor& va
   if (!streaming) {
     if ((d == 64 || d == 128 || d == 256) && a.q_dtype == JPT_BF16 && mode != kPaged) {
       const int64_t bytes = lib.workspace_bytes(&a);
-      if (bytes > JPT_ATTN_WS_STATE_BYTES) use_shared(bytes);
+      if (hq / hkv * t > 16) {
+        // what is live in a prompt's mask goes from one launch to the next: this call's own memory, for
+        // other threads enqueue on the stream too
+        if (bytes > JPT_ATTN_WS_STATE_BYTES) {
+          space = at::empty({bytes}, q.options().dtype(at::kByte));
+          a.workspace = space.data_ptr();
+          a.workspace_bytes = bytes;
+        }
+      } else if (bytes > JPT_ATTN_WS_STATE_BYTES) {
+        use_shared(bytes);
+      }
     }
   } else {
     if (plan != nullptr && plan != Py_None && lengths != nullptr) {

@@ -355,7 +355,12 @@ def _attend(mode, xq, keys, values, *, lengths=None, page_table=None, mask=None,
     # other kernels, which need no plan: the split kernel's partials, or what is live in a prefill's mask
     if not force_generic and d in _MATRIX_CORE_DIMS and xq.dtype == torch.bfloat16 and mode != "paged":
       nbytes = _ffi.lib.jpt_attn_workspace_bytes(a)
-      if nbytes > _ffi.ATTN_WS_STATE_BYTES:
+      if nbytes > _ffi.ATTN_WS_STATE_BYTES and hq // hkv * t > _FAST_MAX_ROWS:
+        # the mask's contents go from one launch to the next: this call's own memory, for other threads
+        # enqueue on the stream too
+        keep.append(torch.empty(nbytes, dtype=torch.uint8, device=device))
+        a.workspace, a.workspace_bytes = _ffi.ptr(keep[-1]), nbytes
+      elif nbytes > _ffi.ATTN_WS_STATE_BYTES:
         ws = _shared_workspace(nbytes, device)
   elif plan is not None and plan.key == (b, hq, hkv, t, a.seq or None, a.page_size or None,
                                          a.max_pages or None) and lengths is not None \

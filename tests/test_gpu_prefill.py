@@ -144,3 +144,54 @@ def test_masks_of_the_lowest_finite_value(d, t, s, dtype, low):
   live = wl > 0
   assert torch.allclose(m.double().cpu()[live], wm[live], rtol=1e-3, atol=1e-4)
   assert torch.allclose(l.double().cpu()[live], wl[live], rtol=1e-3)
+
+
+def test_prompts_of_two_threads_on_one_stream():
+  """A call is two launches, the mask's pass and the attention: calls that other threads enqueue between
+  them, prompts and decode steps, change nothing."""
+  import threading
+  from jetstream_pt_amd import attention_kernel as ak
+  g = torch.Generator().manual_seed(960)
+  hq, hkv, d, t = 8, 2, 64, 512
+  work = []
+  for i in range(2):
+    q, k, v = rnd(g, (1, hq, t, d)).to(DEV), rnd(g, (1, hkv, t, d)).to(DEV), rnd(g, (1, hkv, t, d)).to(DEV)
+    mask = torch.full((1, 1, t, t), -math.inf, device=DEV).triu(1)
+    if i:  # a mask that leaves in what the other leaves out
+      mask = mask.flip(2, 3).contiguous()
+    work.append((q, k, v, mask))
+  step = [x[:, :, :1].contiguous() if i == 0 else x for i, x in enumerate(work[0][:3])]
+  want = [ak.dense_attention(q, k, v, mask=m) for q, k, v, m in work]
+  torch.cuda.synchronize()
+  outs, errors = [[], []], []
+
+  def prompts(i):
+    try:
+      q, k, v, m = work[i]
+      for _ in range(100):
+        outs[i].append(ak.dense_attention(q, k, v, mask=m))
+        ak.dense_attention(*step, mask=m[:, :, :1].contiguous())
+    except Exception as e:  # pylint: disable=broad-except
+      errors.append(e)
+
+  threads = [threading.Thread(target=prompts, args=(i,)) for i in range(2)]
+  for x in threads:
+    x.start()
+  for x in threads:
+    x.join()
+  torch.cuda.synchronize()
+  assert not errors
+  for i in range(2):
+    assert all(torch.equal(o, want[i]) for o in outs[i])
+
+
+def test_a_prompt_uses_no_memory_that_outlives_its_call(monkeypatch):
+  from jetstream_pt_amd import attention_kernel as ak
+  g = torch.Generator().manual_seed(961)
+  t = 700
+  q, k, v = (rnd(g, (1, h, t, 128)).to(DEV) for h in (4, 2, 2))
+  mask = torch.full((1, 1, t, t), -math.inf, device=DEV).triu(1)
+  monkeypatch.setattr(ak, "_workspaces", {})
+  ak.dense_attention(q, k, v, mask=mask)
+  ak.dense_attention(q, k, v, mask=mask.transpose(2, 3))  # the general way: not contiguous
+  assert not ak._workspaces
