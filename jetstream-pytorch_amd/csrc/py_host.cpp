@@ -43,6 +43,7 @@ struct Library {
 } lib;
 PyObject* check_status = nullptr;      // raises for a status code
 PyObject* shared_workspace = nullptr;  // (bytes, device index) -> uint8 tensor
+PyObject* split_workspace = nullptr;   // the same, for a call of the split kernel
 PyObject* dense_workspace = nullptr;   // (device index, b, hq, hkv, t, seq) -> (uint8 tensor, planned)
 
 struct Fallback {};  // not the ordinary case
@@ -251,8 +252,8 @@ Attended attend(Mode mode, const Tensor& q, const Tensor& keys, const Tensor& va
     a.workspace = space.data_ptr();
     a.workspace_bytes = space.numel();
   };
-  auto use_shared = [&](int64_t bytes) {
-    PyObject* w = PyObject_CallFunction(shared_workspace, "Li", static_cast<long long>(bytes), static_cast<int>(q.get_device()));
+  auto use_from = [&](PyObject* from, int64_t bytes) {
+    PyObject* w = PyObject_CallFunction(from, "Li", static_cast<long long>(bytes), static_cast<int>(q.get_device()));
     if (w == nullptr) throw Raised{};
     use(w);
     Py_DECREF(w);
@@ -270,7 +271,7 @@ Attended attend(Mode mode, const Tensor& q, const Tensor& keys, const Tensor& va
           a.workspace_bytes = bytes;
         }
       } else if (bytes > JPT_ATTN_WS_STATE_BYTES) {
-        use_shared(bytes);
+        use_from(split_workspace, bytes);
       }
     }
   } else {
@@ -304,7 +305,7 @@ Attended attend(Mode mode, const Tensor& q, const Tensor& keys, const Tensor& va
       a.reuse_plan = PyObject_IsTrue(PyTuple_GET_ITEM(w, 1));
       Py_DECREF(w);
     }
-    if (a.workspace == nullptr) use_shared(lib.workspace_bytes(&a));
+    if (a.workspace == nullptr) use_from(shared_workspace, lib.workspace_bytes(&a));
   }
   if (token != nullptr && token->stash_k != nullptr) check(unlocked(lib.ragged_stash, &a, token->stash_k, token->stash_v, stream()));
   else check(unlocked(lib.attn[mode], &a, stream()));
@@ -711,10 +712,10 @@ PyObject* py_insert_state(PyObject*, PyObject* const* x, Py_ssize_t n) {
   });
 }
 
-// bind(addresses: dict, check_status, shared_workspace, dense_workspace)
+// bind(addresses: dict, check_status, shared_workspace, split_workspace, dense_workspace)
 PyObject* py_bind(PyObject*, PyObject* args) {
-  PyObject *addresses, *status, *shared, *dense;
-  if (!PyArg_ParseTuple(args, "O!OOO", &PyDict_Type, &addresses, &status, &shared, &dense)) return nullptr;
+  PyObject *addresses, *status, *shared, *split, *dense;
+  if (!PyArg_ParseTuple(args, "O!OOOO", &PyDict_Type, &addresses, &status, &shared, &split, &dense)) return nullptr;
   auto get = [&](const char* name) -> void* {
     PyObject* o = PyDict_GetItemString(addresses, name);
     if (o == nullptr) {
@@ -737,9 +738,11 @@ PyObject* py_bind(PyObject*, PyObject* args) {
   if (PyErr_Occurred()) return nullptr;
   Py_INCREF(status);
   Py_INCREF(shared);
+  Py_INCREF(split);
   Py_INCREF(dense);
   check_status = status;
   shared_workspace = shared;
+  split_workspace = split;
   dense_workspace = dense;
   Py_RETURN_NONE;
 }

@@ -61,6 +61,7 @@ class _Workspace:
 
 
 _workspaces = {}
+_split_workspaces = {}
 _dense_workspaces = collections.OrderedDict()  # most recently used last
 _MAX_DENSE_WORKSPACES = 8
 _FAST_MAX_ROWS = 16  # query rows per KV head (rep * T) the streaming kernel takes
@@ -109,16 +110,26 @@ def check_status(plan=None):
   return bad & ~(STATUS_GAVE_UP | STATUS_PLAN_OVERFLOW)
 
 
-def _shared_workspace(nbytes, device):
+def _shared_workspace(nbytes, device, of=_workspaces):
   # one per (device, stream): calls that share a workspace must not overlap
   index = device if isinstance(device, int) else torch.device(device).index
   index = torch._C._cuda_getDevice() if index is None else index
   key = (index, torch._C._cuda_getCurrentRawStream(index))
-  ws = _workspaces.get(key)
+  ws = of.get(key)
   if ws is None or ws.nbytes < nbytes:
     ws = _Workspace(nbytes, torch.device("cuda", index))
-    _workspaces[key] = ws
+    of[key] = ws
   return ws
+
+
+def _split_workspace(nbytes, device):
+  """The workspace of a call of the split kernel, which needs it for its one launch only: the stream's - not
+  the one in which a streaming call keeps its plan from one launch to the next, for other threads enqueue
+  on the stream too.  A call that is captured gets one of its own, cleared in the graph: the stream's is
+  replaced when a call needs a larger one, and two graphs captured on it may be replayed side by side."""
+  if torch.cuda.is_current_stream_capturing():
+    return _Workspace(nbytes, device if isinstance(device, torch.device) else torch.device("cuda", device))
+  return _shared_workspace(nbytes, device, _split_workspaces)
 
 
 def _dense_workspace(index, batch, q_heads, kv_heads, q_rows, seq):
@@ -146,12 +157,16 @@ def _shared_workspace_buf(nbytes, index):
   return _shared_workspace(nbytes, index).buf
 
 
+def _split_workspace_buf(nbytes, index):
+  return _split_workspace(nbytes, index).buf
+
+
 def _dense_workspace_buf(*shape):
   ws, planned = _dense_workspace(*shape)
   return ws.buf, planned
 
 
-_host.bind(_ffi.addresses(), _ffi.check, _shared_workspace_buf, _dense_workspace_buf)
+_host.bind(_ffi.addresses(), _ffi.check, _shared_workspace_buf, _split_workspace_buf, _dense_workspace_buf)
 
 
 class DecodePlan:
@@ -361,7 +376,7 @@ def _attend(mode, xq, keys, values, *, lengths=None, page_table=None, mask=None,
         keep.append(torch.empty(nbytes, dtype=torch.uint8, device=device))
         a.workspace, a.workspace_bytes = _ffi.ptr(keep[-1]), nbytes
       elif nbytes > _ffi.ATTN_WS_STATE_BYTES:
-        ws = _shared_workspace(nbytes, device)
+        ws = _split_workspace(nbytes, device)
   elif plan is not None and plan.key == (b, hq, hkv, t, a.seq or None, a.page_size or None,
                                          a.max_pages or None) and lengths is not None \
       and plan.lengths.data_ptr() == lengths.data_ptr():

@@ -245,7 +245,7 @@ def test_other_threads_run_while_the_library_does():
   scale, new_scale, layer_scale = (torch.ones(shape, device=DEV) for shape in ((nl, b, 1, s, 1), (nl, b, 1, 1, 1), (b, 1, s, 1)))
   pages, prompt = bf16(hkv, 8, 32, d), [(bf16(1, hkv, t, d), bf16(1, hkv, t, d))] * nl
   torch.cuda.synchronize()
-  _host.bind(asked, status, ak._shared_workspace_buf, ak._dense_workspace_buf)
+  _host.bind(asked, status, ak._shared_workspace_buf, ak._split_workspace_buf, ak._dense_workspace_buf)
   try:
     done = [
         _host.attend(0, q, one, one, -1, lens, None, None, None, None, None, None, None, None, None, None, None, 0, None, False, False, None),
@@ -260,7 +260,7 @@ def test_other_threads_run_while_the_library_does():
         _host.insert_state(mask, lens, lens, lens, 0, 0, 1, 0, 1, False),
     ]
   finally:
-    _host.bind(_ffi.addresses(), _ffi.check, ak._shared_workspace_buf, ak._dense_workspace_buf)
+    _host.bind(_ffi.addresses(), _ffi.check, ak._shared_workspace_buf, ak._split_workspace_buf, ak._dense_workspace_buf)
   assert all(x is not None for x in done)
 
 

@@ -209,3 +209,47 @@ def test_masks_of_the_lowest_finite_value(d, s, low, kind):
   dev = [None if x is None else x.to(DEV) for x in (q, k, v, ks, vs, mask)]
   o, (m, l) = ak.flash_attention(*dev[:3], 0, dev[3], dev[4], dev[5])
   check(o, want, m, l, wm, wl)
+
+
+@pytest.mark.parametrize("kind", ["bf16", "int8_f32"])
+def test_captured_calls_have_a_workspace_of_their_own(kind):
+  """A captured call replayed after larger calls have come and gone on the stream it was captured on, beside
+  another graph's replay on another stream, and with tensors in the memory that was given back: every replay
+  gives the eager bits."""
+  from jetstream_pt_amd import attention_kernel as ak
+  g = torch.Generator().manual_seed(1400)
+  hq, hkv, d, s = 8, 8, 64, 4096
+  lens = [4096, 17, 0, 2500]
+  inputs = []
+  for i in range(2):
+    k, v, ks, vs = make(g, kind, len(lens), hkv, s, d, 1)
+    q = torch.randn((len(lens), hq, 1, d), generator=g).to(torch.bfloat16)
+    inputs.append([None if x is None else x.to(DEV) for x in (q, k, v, torch.tensor(lens, dtype=torch.int32), ks, vs)])
+  call = lambda x: ak.ragged_mha(*x[:3], 0, None, x[3], None, None, x[4], x[5])[0]
+  want = [call(x) for x in inputs]
+  stream = torch.cuda.Stream()
+  graphs, outs = [], []
+  for x in inputs:
+    graph = torch.cuda.CUDAGraph()
+    with torch.cuda.graph(graph, stream=stream):
+      outs.append(call(x))
+    graphs.append(graph)
+  big = torch.randn((8, 16, 1, 256), generator=g).to(torch.bfloat16).to(DEV)
+  cache = torch.randn((8, 1, 512, 256), generator=g).to(torch.bfloat16).to(DEV)
+  with torch.cuda.stream(stream):  # a larger workspace in the place of the stream's
+    ak.dense_attention(big, cache, cache)
+  torch.cuda.synchronize()
+  others = [torch.full((1 << 20,), 7, dtype=torch.int32, device=DEV) for _ in range(8)]
+  side = [torch.cuda.Stream(), torch.cuda.Stream()]
+  for _ in range(5):
+    for o in outs:
+      o.zero_()
+    torch.cuda.synchronize()
+    for graph, at in zip(graphs, side):
+      with torch.cuda.stream(at):
+        graph.replay()
+    assert torch.equal(call(inputs[0]), want[0])
+    torch.cuda.synchronize()
+    for o, w in zip(outs, want):
+      assert torch.equal(o, w)
+  assert all(bool((x == 7).all()) for x in others)
