@@ -409,6 +409,18 @@ typedef struct {
 } jpt_attn_args;
 
 int64_t jpt_attn_workspace_bytes(const jpt_attn_args* args);
+/* Which kernel takes a call (mode 0 ragged, 1 dense, 2 paged) that has a workspace of
+ * jpt_attn_workspace_bytes, and with it what the workspace is to the call:
+ *   JPT_ATTN_STREAMING  plans into it, or finds its plan there (reuse_plan);
+ *   JPT_ATTN_SPLIT      uses it within its one launch;
+ *   JPT_ATTN_PREFILL    can do without, is faster under masks with one;
+ *   JPT_ATTN_GENERIC    does not use it.
+ * Looks at shapes, types and alignments of args; checks nothing. */
+#define JPT_ATTN_GENERIC 0
+#define JPT_ATTN_STREAMING 1
+#define JPT_ATTN_SPLIT 2
+#define JPT_ATTN_PREFILL 3
+int32_t jpt_attn_kernel(const jpt_attn_args* args, int32_t mode);
 /* Plans the split of every slot's positions into workgroup-sized chunks and
  * stores the plan in args->workspace without running attention; later calls
  * on that workspace with reuse_plan = 1 skip planning.  Only lengths,

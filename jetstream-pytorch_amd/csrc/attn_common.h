@@ -29,6 +29,7 @@ int32_t attn_plan_launch(const jpt_attn_args& a, bool paged, bool fresh, hipStre
 // Few query rows over caches the streaming kernel is not built for: attn_split.hip.  Needs a workspace
 // (its state block zero before the first use; the rest need not be cleared).
 bool attn_split_supported(const jpt_attn_args& a, AttnMode mode);
+bool attn_split_has_room(const jpt_attn_args& a);  // in its workspace
 int64_t attn_split_workspace_bytes(const jpt_attn_args& a);
 int32_t attn_split_launch(const jpt_attn_args& a, hipStream_t stream);
 

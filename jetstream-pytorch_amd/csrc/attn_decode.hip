@@ -731,26 +731,41 @@ int64_t jpt_attn_workspace_bytes(const jpt_attn_args* args) {
   return split > planned ? split : planned;
 }
 
-static int32_t attn_entry(const jpt_attn_args* args, jpt::AttnMode mode, void* stream) {
-  using namespace jpt;
+}  // extern "C"
+
+namespace jpt {
+namespace {
+
+// The attention launch can quantise the step's token itself, but every KV head's item then does
+// the slot's whole token (its scale spans the heads), key rotation included, while the rest of its
+// tiles wait in the ring: batch * kv_heads * kv_heads rows.  A launch of its own in front does each
+// token once and costs a layer about 4 us.  Rotated keys, us a layer in one launch / in two:
+// 32 KV heads, bf16 scales: 96 slots 174 / 139, 32 slots 43 / 39, 8 slots 29 / 28, 4 slots 25 / 25;
+// 16 heads: 192 slots 158 / 138, 8 slots 22 / 25; 8 heads: 384 slots 143 / 133, 128 ragged slots
+// 41 / 38, 16 slots 24 / 25; 4 heads, 384 slots 107 / 106.  Keys that come rotated: one launch is
+// the better one, or as good, throughout (32 heads: 96 slots 139 / 139, 32 slots 34 / 38).
+bool quantise_first(const jpt_attn_args& a, AttnMode mode) {
+  constexpr int64_t kRotateFirst = 8192;
+  if (a.new_k_raw == nullptr) return false;
+  return (a.new_k_rope != nullptr && static_cast<int64_t>(a.batch) * a.kv_heads * a.kv_heads >= kRotateFirst) ||
+         !attn_fast_supported(a, mode);
+}
+
+// The kernel for a call whose token, if it brings one, comes as the launch is to take it.
+int32_t kernel_for(const jpt_attn_args& a, AttnMode mode) {
+  if (attn_fast_supported(a, mode)) return JPT_ATTN_STREAMING;
+  if (attn_split_supported(a, mode)) return JPT_ATTN_SPLIT;
+  if (attn_prefill_supported(a, mode)) return JPT_ATTN_PREFILL;
+  return JPT_ATTN_GENERIC;
+}
+
+int32_t attn_entry(const jpt_attn_args* args, AttnMode mode, void* stream) {
   JPT_REQUIRE(args != nullptr, "args is NULL");
   int32_t st = check_attn_args(*args, mode);
   if (st != JPT_OK) return st;
   hipStream_t s = static_cast<hipStream_t>(stream);
-  // The attention launch can quantise the step's token itself, but every KV head's item then does
-  // the slot's whole token (its scale spans the heads), key rotation included, while the rest of its
-  // tiles wait in the ring: batch * kv_heads * kv_heads rows.  A launch of its own in front does each
-  // token once and costs a layer about 4 us.  Rotated keys, us a layer in one launch / in two:
-  // 32 KV heads, bf16 scales: 96 slots 174 / 139, 32 slots 43 / 39, 8 slots 29 / 28, 4 slots 25 / 25;
-  // 16 heads: 192 slots 158 / 138, 8 slots 22 / 25; 8 heads: 384 slots 143 / 133, 128 ragged slots
-  // 41 / 38, 16 slots 24 / 25; 4 heads, 384 slots 107 / 106.  Keys that come rotated: one launch is
-  // the better one, or as good, throughout (32 heads: 96 slots 139 / 139, 32 slots 34 / 38).
-  constexpr int64_t kRotateFirst = 8192;
-  const bool quantise_first = args->new_k_raw && args->new_k_rope &&
-                              static_cast<int64_t>(args->batch) * args->kv_heads * args->kv_heads >= kRotateFirst;
-  if (!quantise_first && attn_fast_supported(*args, mode)) return attn_fast_launch(*args, mode, s);
   jpt_attn_args a = *args;
-  if (a.new_k_raw) {  // quantise first, then attend the codes
+  if (quantise_first(a, mode)) {  // then the codes are attended
     jpt_quant_append_args q{};
     q.new_k = a.new_k_raw;
     q.new_v = a.new_v_raw;
@@ -771,12 +786,31 @@ static int32_t attn_entry(const jpt_attn_args* args, jpt::AttnMode mode, void* s
     if (st != JPT_OK) return st;
     a.new_k_raw = a.new_v_raw = nullptr;
     a.new_k_rope = nullptr;
-    if (attn_fast_supported(a, mode)) return attn_fast_launch(a, mode, s);
   }
-  JPT_REQUIRE(!a.new_to_pages, "new_to_pages needs head_dim 128, a bf16 query and page_size a multiple of 32");
-  if (attn_split_supported(a, mode)) return attn_split_launch(a, s);
-  if (attn_prefill_supported(a, mode)) return attn_prefill_launch(a, s);
-  return attn_generic_launch(a, mode, s);
+  int32_t kernel = kernel_for(a, mode);
+  JPT_REQUIRE(kernel == JPT_ATTN_STREAMING || !a.new_to_pages,
+              "new_to_pages needs head_dim 128, a bf16 query and page_size a multiple of 32");
+  if (kernel == JPT_ATTN_SPLIT && !attn_split_has_room(a))
+    kernel = attn_prefill_supported(a, mode) ? JPT_ATTN_PREFILL : JPT_ATTN_GENERIC;
+  switch (kernel) {
+    case JPT_ATTN_STREAMING: return attn_fast_launch(a, mode, s);
+    case JPT_ATTN_SPLIT: return attn_split_launch(a, s);
+    case JPT_ATTN_PREFILL: return attn_prefill_launch(a, s);
+    default: return attn_generic_launch(a, mode, s);
+  }
+}
+
+}  // namespace
+}  // namespace jpt
+
+extern "C" {
+
+int32_t jpt_attn_kernel(const jpt_attn_args* args, int32_t mode) {
+  using namespace jpt;
+  if (args == nullptr || args->kv_heads <= 0 || args->q_heads % args->kv_heads != 0 || mode < kRagged || mode > kPaged) return JPT_ATTN_GENERIC;
+  jpt_attn_args a = *args;
+  if (quantise_first(a, static_cast<AttnMode>(mode))) a.new_k_raw = a.new_v_raw = nullptr;
+  return kernel_for(a, static_cast<AttnMode>(mode));
 }
 
 static int32_t plan_entry(const jpt_attn_args* args, int32_t paged, bool fresh, void* stream) {
@@ -892,8 +926,8 @@ int32_t jpt_attn_status(void* workspace, void* stream, int32_t* status) {
   return JPT_OK;
 }
 
-int32_t jpt_attn_ragged(const jpt_attn_args* args, void* stream) { return attn_entry(args, jpt::kRagged, stream); }
-int32_t jpt_attn_dense(const jpt_attn_args* args, void* stream) { return attn_entry(args, jpt::kDense, stream); }
-int32_t jpt_attn_paged(const jpt_attn_args* args, void* stream) { return attn_entry(args, jpt::kPaged, stream); }
+int32_t jpt_attn_ragged(const jpt_attn_args* args, void* stream) { return jpt::attn_entry(args, jpt::kRagged, stream); }
+int32_t jpt_attn_dense(const jpt_attn_args* args, void* stream) { return jpt::attn_entry(args, jpt::kDense, stream); }
+int32_t jpt_attn_paged(const jpt_attn_args* args, void* stream) { return jpt::attn_entry(args, jpt::kPaged, stream); }
 
 }  // extern "C"

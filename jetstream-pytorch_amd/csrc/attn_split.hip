@@ -756,7 +756,10 @@ bool attn_split_supported(const jpt_attn_args& a, AttnMode mode) {
   if (a.k_scale && (!aligned(a.k_scale, 16) || !aligned(a.v_scale, 16))) return false;
   if (a.new_k && (!aligned(a.new_k, 16) || !aligned(a.new_v, 16))) return false;
   // tile numbers fit 32 bits, the sum over the batch before it is multiplied by the heads too
-  if (static_cast<int64_t>(a.batch) * (a.seq / kTile + 16) >= (1ll << 31)) return false;
+  return static_cast<int64_t>(a.batch) * (a.seq / kTile + 16) < (1ll << 31);
+}
+
+bool attn_split_has_room(const jpt_attn_args& a) {
   return a.workspace != nullptr && aligned(a.workspace, 256) && decode::split_groups(a) >= decode::kMinGroups;
 }
 

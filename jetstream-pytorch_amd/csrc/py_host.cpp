@@ -32,6 +32,7 @@ using at::Tensor;
 using AttnFn = int32_t (*)(const jpt_attn_args*, void*);
 struct Library {
   int64_t (*workspace_bytes)(const jpt_attn_args*);
+  int32_t (*kernel)(const jpt_attn_args*, int32_t);
   int32_t (*plan[2])(const jpt_attn_args*, int32_t, void*);  // again, on a fresh workspace
   AttnFn attn[3];  // ragged, dense, paged
   int32_t (*scatter_lines)(const jpt_line_tensor*, int32_t, const int32_t*, int32_t, int32_t, int32_t, int32_t, void*);
@@ -244,7 +245,7 @@ Attended attend(Mode mode, const Tensor& q, const Tensor& keys, const Tensor& va
     a.out_denom = static_cast<float*>(r.denom.data_ptr());
   }
 
-  // ---- workspace: the plan's, the shape's own or the stream's ----
+  // ---- workspace: this call's own, the plan's, the shape's or the stream's ----
   Tensor space;  // keeps it alive across the launch
   auto use = [&](PyObject* o) {
     need(THPVariable_Check(o));
@@ -258,23 +259,19 @@ Attended attend(Mode mode, const Tensor& q, const Tensor& keys, const Tensor& va
     use(w);
     Py_DECREF(w);
   };
-  const bool streaming = hq / hkv * t <= 16 && d == 128 && a.q_dtype == JPT_BF16 && a.kv_dtype != JPT_F32;
-  if (!streaming) {
-    if ((d == 64 || d == 128 || d == 256) && a.q_dtype == JPT_BF16 && mode != kPaged) {
-      const int64_t bytes = lib.workspace_bytes(&a);
-      if (hq / hkv * t > 16) {
-        // what is live in a prompt's mask goes from one launch to the next: this call's own memory, for
-        // other threads enqueue on the stream too
-        if (bytes > JPT_ATTN_WS_STATE_BYTES) {
-          space = at::empty({bytes}, q.options().dtype(at::kByte));
-          a.workspace = space.data_ptr();
-          a.workspace_bytes = bytes;
-        }
-      } else if (bytes > JPT_ATTN_WS_STATE_BYTES) {
-        use_from(split_workspace, bytes);
-      }
+  const int32_t kernel = lib.kernel(&a, mode);
+  if (kernel == JPT_ATTN_SPLIT) {
+    use_from(split_workspace, lib.workspace_bytes(&a));
+  } else if (kernel == JPT_ATTN_PREFILL) {
+    // what is live in a prompt's mask goes from one launch to the next: this call's own memory, for
+    // other threads enqueue on the stream too
+    const int64_t bytes = lib.workspace_bytes(&a);
+    if (bytes > JPT_ATTN_WS_STATE_BYTES) {
+      space = at::empty({bytes}, q.options().dtype(at::kByte));
+      a.workspace = space.data_ptr();
+      a.workspace_bytes = bytes;
     }
-  } else {
+  } else if (kernel == JPT_ATTN_STREAMING) {
     if (plan != nullptr && plan != Py_None && lengths != nullptr) {
       // a DecodePlan made for these lengths and this shape
       PyObject* key = PyObject_GetAttrString(plan, "key");
@@ -725,6 +722,7 @@ PyObject* py_bind(PyObject*, PyObject* args) {
     return PyLong_AsVoidPtr(o);
   };
   lib.workspace_bytes = reinterpret_cast<decltype(lib.workspace_bytes)>(get("jpt_attn_workspace_bytes"));
+  lib.kernel = reinterpret_cast<decltype(lib.kernel)>(get("jpt_attn_kernel"));
   lib.attn[kRagged] = reinterpret_cast<AttnFn>(get("jpt_attn_ragged"));
   lib.attn[kDense] = reinterpret_cast<AttnFn>(get("jpt_attn_dense"));
   lib.attn[kPaged] = reinterpret_cast<AttnFn>(get("jpt_attn_paged"));

@@ -28,6 +28,7 @@ from . import _host  # noqa: E402  (the host side of the hot calls, csrc/py_host
 OK, E_BADARG, E_NOPAGES, E_PAGE_OVERFLOW, E_HIP = 0, -1, -2, -3, -4
 BF16, F32, I8 = 0, 1, 2
 ROUND_TRUNC, ROUND_RNE = 0, 1
+ATTN_GENERIC, ATTN_STREAMING, ATTN_SPLIT, ATTN_PREFILL = 0, 1, 2, 3
 ATTN_WS_STATE_BYTES = 65536
 ATTN_STATIC_SCRATCH_BYTES = 8 << 20
 MAX_LINE_TENSORS = 4
@@ -138,6 +139,7 @@ _sig("jpt_prefill_insert", _i32, _c.POINTER(PrefillInsertArgs), _vp)
 _sig("jpt_prefill_insert_layers", _i32, _c.POINTER(PrefillInsertArgs), _c.POINTER(InsertLayer), _i32, _vp)
 _sig("jpt_prefill_insert_prompts", _i32, _c.POINTER(PrefillInsertArgs), _c.POINTER(InsertPrompt), _i32, _vp)
 _sig("jpt_attn_workspace_bytes", _i64, _c.POINTER(AttnArgs))
+_sig("jpt_attn_kernel", _i32, _c.POINTER(AttnArgs), _i32)
 _sig("jpt_attn_plan", _i32, _c.POINTER(AttnArgs), _i32, _vp)
 _sig("jpt_attn_plan_fresh", _i32, _c.POINTER(AttnArgs), _i32, _vp)
 _sig("jpt_attn_ragged", _i32, _c.POINTER(AttnArgs), _vp)
@@ -176,7 +178,7 @@ EXPORTS = (
     "jpt_dpam_free", "jpt_dpam_decode_step", "jpt_decode_advance", "jpt_rope",
     "jpt_ragged_block_indices", "jpt_prefill_insert_layers", "jpt_prefill_insert_prompts",
     "jpt_attn_status", "jpt_attn_ragged_static", "jpt_attn_plan_fresh", "jpt_kv_stash_lines", "jpt_insert_state",
-    "jpt_attn_ragged_stash",
+    "jpt_attn_ragged_stash", "jpt_attn_kernel",
 )
 
 

@@ -64,15 +64,6 @@ _workspaces = {}
 _split_workspaces = {}
 _dense_workspaces = collections.OrderedDict()  # most recently used last
 _MAX_DENSE_WORKSPACES = 8
-_FAST_MAX_ROWS = 16  # query rows per KV head (rep * T) the streaming kernel takes
-_MATRIX_CORE_DIMS = (64, 128, 256)  # head dims of the kernels beside it
-
-
-def _streaming_kernel_may_run(rows, dim, q_dtype, kv_dtype):
-  """Whether the library's streaming kernel can take this shape at all; other
-  shapes go to its shape-generic kernel, which uses no workspace and no plan."""
-  return (rows <= _FAST_MAX_ROWS and dim == 128 and q_dtype == torch.bfloat16
-          and kv_dtype in (torch.int8, torch.bfloat16))
 
 
 STATUS_GAVE_UP, STATUS_SLOT_FULL, STATUS_PLAN_OVERFLOW = 1, 2, 4
@@ -366,17 +357,18 @@ def _attend(mode, xq, keys, values, *, lengths=None, page_table=None, mask=None,
     a.out_max, a.out_denom = _ffi.ptr(omax), _ffi.ptr(oden)
 
   ws = None
-  if not _streaming_kernel_may_run(hq // hkv * t, d, xq.dtype, keys.dtype) or force_generic:
-    # other kernels, which need no plan: the split kernel's partials, or what is live in a prefill's mask
-    if not force_generic and d in _MATRIX_CORE_DIMS and xq.dtype == torch.bfloat16 and mode != "paged":
-      nbytes = _ffi.lib.jpt_attn_workspace_bytes(a)
-      if nbytes > _ffi.ATTN_WS_STATE_BYTES and hq // hkv * t > _FAST_MAX_ROWS:
-        # the mask's contents go from one launch to the next: this call's own memory, for other threads
-        # enqueue on the stream too
-        keep.append(torch.empty(nbytes, dtype=torch.uint8, device=device))
-        a.workspace, a.workspace_bytes = _ffi.ptr(keep[-1]), nbytes
-      elif nbytes > _ffi.ATTN_WS_STATE_BYTES:
-        ws = _split_workspace(nbytes, device)
+  kernel = _ffi.lib.jpt_attn_kernel(a, _MODES[mode])
+  if kernel == _ffi.ATTN_SPLIT:
+    ws = _split_workspace(_ffi.lib.jpt_attn_workspace_bytes(a), device)
+  elif kernel == _ffi.ATTN_PREFILL:
+    nbytes = _ffi.lib.jpt_attn_workspace_bytes(a)
+    if nbytes > _ffi.ATTN_WS_STATE_BYTES:
+      # the mask's contents go from one launch to the next: this call's own memory, for other threads
+      # enqueue on the stream too
+      keep.append(torch.empty(nbytes, dtype=torch.uint8, device=device))
+      a.workspace, a.workspace_bytes = _ffi.ptr(keep[-1]), nbytes
+  elif kernel == _ffi.ATTN_GENERIC:
+    pass
   elif plan is not None and plan.key == (b, hq, hkv, t, a.seq or None, a.page_size or None,
                                          a.max_pages or None) and lengths is not None \
       and plan.lengths.data_ptr() == lengths.data_ptr():

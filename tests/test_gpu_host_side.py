@@ -231,7 +231,7 @@ def test_other_threads_run_while_the_library_does():
   import ctypes
   from jetstream_pt_amd import _ffi, _host, attention_kernel as ak
   held = ctypes.cast(ctypes.pythonapi.PyGILState_Check, ctypes.c_void_p).value
-  asked = {name: held if name != "jpt_attn_workspace_bytes" else at for name, at in _ffi.addresses().items()}
+  asked = {name: at if name in ("jpt_attn_workspace_bytes", "jpt_attn_kernel") else held for name, at in _ffi.addresses().items()}
 
   def status(code):
     raise AssertionError("the interpreter's lock was held")

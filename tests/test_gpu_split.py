@@ -212,14 +212,15 @@ def test_masks_of_the_lowest_finite_value(d, s, low, kind):
 
 
 @pytest.mark.parametrize("kind", ["bf16", "int8_f32"])
-def test_captured_calls_have_a_workspace_of_their_own(kind):
+@pytest.mark.parametrize("d,s", [(64, 4096), (128, 4090)])
+def test_captured_calls_have_a_workspace_of_their_own(d, s, kind):
   """A captured call replayed after larger calls have come and gone on the stream it was captured on, beside
   another graph's replay on another stream, and with tensors in the memory that was given back: every replay
   gives the eager bits."""
   from jetstream_pt_amd import attention_kernel as ak
   g = torch.Generator().manual_seed(1400)
-  hq, hkv, d, s = 8, 8, 64, 4096
-  lens = [4096, 17, 0, 2500]
+  hq, hkv = 8, 8
+  lens = [s, 17, 0, 2500]
   inputs = []
   for i in range(2):
     k, v, ks, vs = make(g, kind, len(lens), hkv, s, d, 1)

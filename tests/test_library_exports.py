@@ -43,3 +43,19 @@ def test_ops_refuse_cpu_tensors():
   q = torch.zeros((1, 2, 1, 8))
   with pytest.raises(RuntimeError, match="ROCm device only"):
     ak.dense_attention(q, q, q)
+
+
+@pytest.mark.parametrize("change,mode,want", [
+    ({}, 0, "STREAMING"), ({}, 1, "STREAMING"), (dict(seq=96), 1, "STREAMING"), (dict(seq=90), 1, "SPLIT"), (dict(dim=64), 0, "SPLIT"),
+    (dict(dim=256), 1, "SPLIT"), (dict(dim=80), 1, "GENERIC"), (dict(mask=64, mask_stride_h=4), 1, "SPLIT"),
+    (dict(mask=64, mask_dtype=1), 1, "STREAMING"), (dict(mask=64, mask_dtype=0), 1, "SPLIT"), (dict(q_rows=5), 1, "PREFILL"),
+    (dict(q_rows=4), 1, "STREAMING"), (dict(q_rows=500, kv_dtype=2, k_scale=64, v_scale=64, scale_heads=1), 1, "GENERIC"),
+    (dict(kv_dtype=2), 0, "GENERIC"), (dict(kv_dtype=2, k_scale=64, v_scale=64, scale_heads=1), 0, "STREAMING"), (dict(q=8), 0, "GENERIC"),
+    (dict(seq=0, page_size=32), 2, "STREAMING"), (dict(seq=0, page_size=16), 2, "GENERIC"), (dict(seq=0, page_size=32, dim=64), 2, "GENERIC"),
+    (dict(force_generic=1), 0, "GENERIC"), (dict(batch=5000), 1, "SPLIT"), (dict(kv_heads=0), 0, "GENERIC"),
+])
+def test_which_kernel_takes_a_call(change, mode, want):
+  """Addresses are looked at, not followed."""
+  from jetstream_pt_amd import _ffi
+  a = dict(q=64, k=64, v=64, out=64, batch=2, q_heads=8, kv_heads=2, q_rows=1, dim=128, seq=256, q_dtype=_ffi.BF16, kv_dtype=_ffi.BF16)
+  assert _ffi.lib.jpt_attn_kernel(_ffi.AttnArgs(**dict(a, **change)), mode) == getattr(_ffi, "ATTN_" + want)
