@@ -123,6 +123,54 @@ def test_many_rotated_tokens_are_quantised_ahead_of_the_launch(sdt, per_head, b,
   assert torch.equal(out, given) and all(torch.equal(a, w) for a, w in zip(stats, given_stats))
 
 
+@pytest.mark.parametrize("b,hq,hkv", [(8, 32, 32), (33, 16, 16), (128, 32, 8)])
+@pytest.mark.parametrize("sdt,per_head", [(torch.float32, False), (torch.bfloat16, True)])
+def test_many_rotated_tokens_go_to_their_pages(sdt, per_head, b, hq, hkv):
+  """The same over pages, from the same number of rows on: codes and scales lie in the token's page and
+  nothing else changes (an inactive slot and one without a page among them); outputs as with given codes."""
+  from jetstream_pt_amd import attention_kernel as ak
+  from jetstream_pt_amd.quantize import quantize_kv
+  ps, mp, d = 32, 4, 128
+  total, hs = b * mp, hkv if per_head else 1
+  g = torch.Generator().manual_seed(6)
+  xq, xk, xv, freqs = step_inputs(b, hq, hkv, d, 6)
+  lens = torch.randint(1, ps * mp - 1, (b,), generator=g, dtype=torch.int32)
+  lens[0], lens[1], lens[2] = 0, ps, 2 * ps - 1
+  table = torch.randperm(total, generator=g).reshape(b, mp).to(torch.int32)
+  table[3, int(lens[3]) // ps] = -1
+  q, raw_k, raw_v = (x.transpose(1, 2).contiguous().to(DEV) for x in (xq, xk, xv))
+  pool = [torch.randint(-127, 128, (hkv, total, ps, d), generator=g, dtype=torch.int8) for _ in range(2)]
+  pool += [(torch.rand((hs, total, ps), generator=g) * 0.045 + 0.005).to(sdt) for _ in range(2)]
+  codes = quantize_kv(raw_k, raw_v, rounding="trunc", scale_heads=hs, scale_dtype=sdt, freqs_cis=freqs.to(DEV))
+  codes = [c.contiguous() for c in codes]
+  dlens, dtable = lens.to(DEV), table.to(DEV)
+  plan = ak.DecodePlan(dlens, b, hq, hkv, page_size=ps, max_pages=mp)
+  names = ("new_key", "new_value", "new_k_scaler", "new_v_scaler")
+
+  def run(new):
+    pages = [x.to(DEV) for x in pool]
+    out = ak.call_paged_attention(None, q.squeeze(2), *pages[:2], dlens, dtable, sm_scale=0.1, k_scaler=pages[2], v_scaler=pages[3],
+                                  plan=plan, append=new)
+    return [out] + pages
+
+  outputs = [torch.zeros_like(raw_k, dtype=torch.int8) for _ in range(2)] + [torch.zeros((b, hs), dtype=sdt, device=DEV) for _ in range(2)]
+  got = run(dict(zip(names, outputs), new_key_raw=raw_k, new_value_raw=raw_v, new_key_rope=freqs.to(DEV)))
+  want = run(dict(zip(names, codes)))
+  assert all(torch.equal(a.reshape(-1), w.reshape(-1)) for a, w in zip(outputs, codes))
+  for a, w in zip(got, want):
+    assert torch.equal(a, w)
+  written = pool  # what the pages hold with every live slot's token in its place
+  for slot, n in enumerate(lens.tolist()):
+    page = int(table[slot, n // ps])
+    if n > 0 and page >= 0:
+      for x, c in zip(written[:2], codes[:2]):
+        x[:, page, n % ps] = c[slot, :, 0].cpu()
+      for x, c in zip(written[2:], codes[2:]):
+        x[:, page, n % ps] = c.reshape(b, hs)[slot].cpu()
+  for a, w in zip(got[1:], written):
+    assert torch.equal(a.cpu(), w)
+
+
 def test_orchestration_with_unrotated_keys():
   """Int8KVAttentionKernel(freqs_cis=...) on raw keys == the same kernel on keys
   rotated beforehand, in lazy ragged (fused), eager dense and paged int8 modes;
