@@ -9,8 +9,9 @@
 // bf16 pages 30 -> 8; a 32-layer prompt insert 434 -> 27.
 //
 // Every function takes the ordinary case (device tensors, contiguous, of the dtypes the library has)
-// and returns None, having done nothing, for anything else: the Python code then goes the long way,
-// which converts what can be converted and raises the errors the package documents.
+// and returns None for anything else: the Python code then goes the long way, which converts what can
+// be converted and raises the errors the package documents.  Nothing has been done then, but that
+// eager_step may have written the token's line, which the long way writes again.
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
@@ -566,16 +567,34 @@ Py_ssize_t count_of(PyObject* o) {
   need(PyList_Check(o) || PyTuple_Check(o));
   return PySequence_Fast_GET_SIZE(o);
 }
+// Tensors out of lists, which are the caller's to change while the library runs: their objects are held.
+class Held {
+ public:
+  explicit Held(size_t n) { objects_.reserve(n); }
+  ~Held() {
+    for (PyObject* o : objects_) Py_DECREF(o);
+  }
+  Held(const Held&) = delete;
+  Held& operator=(const Held&) = delete;
+  const Tensor& operator()(PyObject* o) {
+    const Tensor& t = ten(o);
+    Py_INCREF(o);
+    objects_.push_back(o);
+    return t;
+  }
+
+ private:
+  std::vector<PyObject*> objects_;
+};
+
 // Member `which` of layer `layer`'s pair: a list of pairs, a list of one pair of stacks, or a pair of stacks.
-// `held` keeps it: the lists are the caller's to change while the library runs.
-Layer layer_of(PyObject* caches, Py_ssize_t layer, Py_ssize_t layers, int which, bool paged, std::vector<Tensor>& held) {
+Layer layer_of(PyObject* caches, Py_ssize_t layer, Py_ssize_t layers, int which, bool paged, Held& held) {
   PyObject* first = item(caches, 0);
   const bool pairs = PyList_Check(first) || PyTuple_Check(first);
   const bool stacks = !pairs || (count_of(caches) == 1 && ten(item(first, 0)).dim() == 5);
   need(stacks ? !paged : count_of(caches) >= layers);
-  const Tensor& t = ten(item(!pairs ? caches : stacks ? first : item(caches, layer), which));
+  const Tensor& t = held(item(!pairs ? caches : stacks ? first : item(caches, layer), which));
   need(stacks || t.dim() == 4);
-  if (!stacks || layer == 0) held.push_back(t);
   return Layer(t, 4, stacks ? layer : -1);
 }
 
@@ -590,13 +609,10 @@ PyObject* py_insert_layers(PyObject*, PyObject* const* x, Py_ssize_t n) {
     jpt_prefill_insert_args a{};
     std::vector<jpt_insert_layer> table(layers);
     c10::IntArrayRef cache_sizes, prefix_sizes, scale_sizes;
-    std::vector<Tensor> held;
-    held.reserve(6 * layers);
+    Held held(6 * layers);
     for (Py_ssize_t l = 0; l < layers; ++l) {
       PyObject* pair = item(x[0], l);
-      const Tensor &pk = ten(item(pair, 0)), &pv = ten(item(pair, 1));
-      held.push_back(pk);
-      held.push_back(pv);
+      const Tensor &pk = held(item(pair, 0)), &pv = held(item(pair, 1));
       const Layer k = layer_of(x[1], l, layers, 0, paged, held), v = layer_of(x[1], l, layers, 1, paged, held);
       need(k.sizes == v.sizes && k.code == v.code && pk.sizes() == pv.sizes() && pk.scalar_type() == pv.scalar_type());
       const int in = dtype_code(pk);
