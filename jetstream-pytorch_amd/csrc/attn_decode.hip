@@ -41,8 +41,10 @@ constexpr int kChunkAlign = 128;
 //               the numbers of work entries and of merge entries in the plan,
 //               words 16, 32, ... 128 the counters that hand out the merge
 //               entries (cleared by every plan, advanced by the same amounts by
-//               every launch)
+//               every launch); its last 4 KiB the arrival counters of the split
+//               kernel (attn_split.hip), zero between launches
 // then          plan entries, arrival counters (batch x kv_heads), partials
+// the end       what kernels that plan nothing need within a call (attn_workspace_end)
 struct Layout {
   int64_t entries, arrivals, partials, total;
   int32_t max_entries;

@@ -14,7 +14,7 @@
 // across the end of a sequence, so that a wave always has half a tile to a whole one in flight.
 // Waves do not wait for each other: the one that delivers the last part of a sequence folds the
 // parts.  (With barriers at every sequence's end and its tiles dealt to the waves anew, shares of equal
-// tiles whatever the sequences' number, and the new token a tile of its own: 60 us for 48 us below.)
+// tiles whatever the sequences' number, and the new token a tile of its own, 60 us where this took 48.)
 //
 // The arithmetic is the streaming kernel's (S^T = K . Q^T, O^T = V^T . P^T on 16x16x32 MFMAs), but keeps
 // float32's bits: softmax weights are the sum of three 16-bit numbers, and int8 codes go in as float16 numbers
@@ -28,8 +28,11 @@
 // A sequence cut between groups: every group parks a float32 partial past the caches and counts
 // itself; the last one folds them.  No group waits for another.
 //
-// Measured, int8, 48 slots of 16..1024 positions, 16 heads of 256 (190 MB a launch): 48 us, 4.0 TB/s;
-// all 48 at 2048 positions 144 us, 5.6 TB/s (2.2 ms on the shape-generic kernel, one wave a query row).
+// Measured, calls back to back on caches that come from memory, int8, 16 heads of 256: 48 slots of 16..1024
+// positions (201 MB a launch) 59 us, 3.4 TB/s; all 48 at 2048 positions 184 us, 4.4 TB/s (2.2 ms on the
+// shape-generic kernel, one wave a query row).  With two-number weights, biased codes and raw scales 55 and
+// 168 us.  A wave spends 54 % of its time waiting, for memory above all, and issues vector instructions in
+// 21 % of it: 568 of them a tile of 32 x 128 int8, where the streaming kernel needs 321.
 #include <algorithm>
 
 #include "attn_decode_impl.h"
@@ -251,8 +254,8 @@ __global__ void __launch_bounds__(kSplitThreads, (split_waves_per_simd<D, KV>())
   if (me >= groups) return;
   // Share w begins at total * w / groups in the sequences laid end to end, each its cost long - but not
   // less than kLeastPart tiles inside a sequence: a cut costs its groups a partial, its count and a
-  // fold.  (Ragged lengths as above: kLeastPart 4 and a sequence's cost of a tile a wave 47.5 us; no
-  // such cost 49.8; kLeastPart 7 48.8 and, all slots at 512 positions, 51.1 for 46.7 us.)
+  // fold.  (Ragged lengths as above, in one run: kLeastPart 4 and a sequence's cost of a tile a wave 47.5 us;
+  // no such cost 49.8; kLeastPart 7 48.8 and, all slots at 512 positions, 51.1 for 46.7 us.)
   auto raw_begin = [&](int w) -> int64_t { return total * w / groups; };
   auto group_of = [&](int64_t at) -> int { return static_cast<int>(((at + 1) * groups - 1) / total); };  // before moving
 #pragma unroll

@@ -41,6 +41,8 @@ def check(got, want, m, l, wm, wl):
     (64, 28, 4, 2048, [2047]),
     (256, 2, 1, 40, [(7 * i) % 41 for i in range(300)]),
     (64, 1, 1, 4, [i % 5 for i in range(4200)]),
+    (256, 32, 2, 700, [700, 33, 0, 31]),
+    (64, 16, 1, 3000, [3000, 1, 2999]),
 ])
 @pytest.mark.parametrize("token", [False, True])
 def test_lengths(token, d, hq, hkv, s, lens, kind):
