@@ -334,3 +334,27 @@ def test_a_scale_that_is_not_a_number_is_not_the_default():
   lens, table = torch.tensor([20], dtype=torch.int32, device=DEV), torch.tensor([[1, 2]], dtype=torch.int32, device=DEV)
   assert bool(ak.call_paged_attention(None, q, pages, pages, lens, table, sm_scale=float("nan")).isnan().all())
   assert bool(ak.call_paged_attention(None, q, pages, pages, lens, table, sm_scale=0.1).isfinite().all())
+
+
+@pytest.mark.parametrize("b,fill", [(5, 255), (5, 1), (4200, 255)])
+def test_a_fresh_plans_workspace_serves_the_kernel_whose_counters_it_holds(b, fill):
+  """At the library's entries: a workspace full of other data, planned as a fresh one, then a call whose
+  kernel counts in the state block (batches beyond the planner's have no plan: the block is cleared)."""
+  from jetstream_pt_amd import _ffi, attention_kernel as ak
+  g = torch.Generator().manual_seed(8)
+  hq, hkv, s, d = 8, 4, 250, 128
+  q = torch.randn((b, hq, 1, d), generator=g).to(torch.bfloat16).to(DEV)
+  k, v = (torch.randn((b, hkv, s, d), generator=g).to(torch.bfloat16).to(DEV) for _ in range(2))
+  end = torch.randint(0, s + 1, (b,), generator=g, dtype=torch.int32).to(DEV)
+  want = ak.ragged_mha(q, k, v, 0, None, end)[0]
+  out = torch.empty_like(q)
+  a = _ffi.AttnArgs(q=_ffi.ptr(q), k=_ffi.ptr(k), v=_ffi.ptr(v), lengths=_ffi.ptr(end), out=_ffi.ptr(out), batch=b, q_heads=hq, kv_heads=hkv,
+                    q_rows=1, dim=d, seq=s, q_dtype=_ffi.BF16, kv_dtype=_ffi.BF16, sm_scale=1.0 / d ** 0.5)
+  assert _ffi.lib.jpt_attn_kernel(a, 0) == _ffi.ATTN_SPLIT
+  ws = torch.full((_ffi.lib.jpt_attn_workspace_bytes(a),), fill, dtype=torch.uint8, device=DEV)
+  a.workspace, a.workspace_bytes = _ffi.ptr(ws), ws.numel()
+  _ffi.check(_ffi.lib.jpt_attn_plan_fresh(a, 0, _ffi.stream()))
+  for _ in range(3):
+    out.zero_()
+    _ffi.check(_ffi.lib.jpt_attn_ragged(a, _ffi.stream()))
+    assert torch.equal(out.reshape(want.shape), want)
