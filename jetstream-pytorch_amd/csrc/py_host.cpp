@@ -368,7 +368,9 @@ PyObject* py_attend(PyObject*, PyObject* const* x, Py_ssize_t n) {
       given_token(token, ten(x[11]), ten(x[12]), b, hkv, d, dtype_code(k));
       if (x[13] != Py_None) {
         const Tensor &nks = ten(x[13]), &nvs = ten(x[14]);
-        need(ks != nullptr && nks.scalar_type() == ks->scalar_type() && nvs.scalar_type() == ks->scalar_type());
+        need(ks != nullptr && nks.scalar_type() == ks->scalar_type() && nvs.scalar_type() == ks->scalar_type() && ks->dim() >= 3);
+        const int64_t heads = mode == kPaged ? ks->size(0) : ks->size(ks->dim() == 3 ? -2 : -3);  // see attend
+        need(nks.numel() == b * heads && nvs.numel() == b * heads);
         token.k_scale = nks.data_ptr();
         token.v_scale = nvs.data_ptr();
       }

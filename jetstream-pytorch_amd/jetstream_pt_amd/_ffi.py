@@ -218,6 +218,19 @@ def dev(t, name="tensor"):
   return t
 
 
+def alike(a, b, what):
+  """Two tensors that a kernel walks side by side, by the first one's shape and dtype."""
+  if a.shape != b.shape or a.dtype != b.dtype:
+    raise ValueError(f"{what} must agree in shape and dtype: {tuple(a.shape)} {a.dtype} and {tuple(b.shape)} {b.dtype}")
+
+
+def holds(t, n, name):
+  """A kernel is about to read or write `n` elements of `t`."""
+  if t.numel() != n:
+    raise ValueError(f"{name} has shape {tuple(t.shape)}, {n} elements are needed")
+  return t
+
+
 def rope_factors(freqs_cis, rows, dim, name="freqs_cis"):
   """The step's rotary factors as a contiguous float32 (rows, dim / 2, 2) device
   tensor of (cos, sin): accepts the reference's complex64 freqs_cis

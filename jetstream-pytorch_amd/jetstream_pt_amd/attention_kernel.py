@@ -290,8 +290,8 @@ def _attend(mode, xq, keys, values, *, lengths=None, page_table=None, mask=None,
   if k_scaler is not None:
     ks, hs = _scale_tensor(k_scaler, mode == "paged")
     vs, _ = _scale_tensor(v_scaler, mode == "paged")
-    if ks.dtype != vs.dtype or ks.shape != vs.shape:
-      raise ValueError("k_scaler and v_scaler must agree in shape and dtype")
+    _ffi.alike(ks, vs, "k_scaler and v_scaler")
+    _ffi.holds(ks, hs * (total * ps if mode == "paged" else b * s), "k_scaler")
     a.k_scale, a.v_scale = _ffi.ptr(ks), _ffi.ptr(vs)
     a.scale_dtype, a.scale_heads = _ffi.dtype_code(ks.dtype), hs
     keep += [ks, vs]
@@ -314,11 +314,13 @@ def _attend(mode, xq, keys, values, *, lengths=None, page_table=None, mask=None,
     nk, nv = _ffi.dev(new_key, "new_key"), _ffi.dev(new_value, "new_value")
     if nk.shape != (b, hkv, 1, d) or nk.dtype != keys.dtype:
       raise ValueError("new_key must be (batch, kv_heads, 1, dim) in the cache dtype")
+    _ffi.alike(nk, nv, "new_key and new_value")
     a.new_k, a.new_v = _ffi.ptr(nk), _ffi.ptr(nv)
     keep += [nk, nv]
     if new_k_scaler is not None:
       nks = _ffi.dev(new_k_scaler, "new_k_scaler").to(ks.dtype)
       nvs = _ffi.dev(new_v_scaler, "new_v_scaler").to(ks.dtype)
+      _ffi.holds(nks, b * hs, "new_k_scaler"), _ffi.holds(nvs, b * hs, "new_v_scaler")
       a.new_k_scale, a.new_v_scale = _ffi.ptr(nks), _ffi.ptr(nvs)
       keep += [nks, nvs]
     if new_key_raw is not None:

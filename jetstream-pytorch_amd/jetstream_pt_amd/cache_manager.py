@@ -68,6 +68,8 @@ def _scatter_lines(pairs, pos, pos_count, n_layers, batch, seq):
     _ffi.dev(dst, "cache"), _ffi.dev(src, "new line")
     if src.dtype != dst.dtype:
       raise ValueError(f"line dtype {src.dtype} does not match cache dtype {dst.dtype}")
+    lines = n_layers * batch * dst.shape[-3] * dst.shape[-1]
+    _ffi.holds(src, lines, "new line"), _ffi.holds(dst, lines * seq, "cache")
     arr[i] = _ffi.LineTensor(_ffi.ptr(dst), _ffi.ptr(src), dst.shape[-3],
                              dst.shape[-1] * dst.element_size())
   _ffi.check(_ffi.lib.jpt_kv_scatter_lines(
@@ -217,12 +219,13 @@ class Int8KVCacheGenerate:
     b, h, t, d = xk.shape
     if t != 1:
       raise ValueError("the decode cache takes one token per update")
+    _ffi.alike(xk, xv, "xk and xv")
     a = _ffi.QuantAppendArgs(
         new_k=_ffi.ptr(xk), new_v=_ffi.ptr(xv), batch=b, heads=h, dim=d, seq=1, pos_count=b,
         in_dtype=_ffi.dtype_code(xk.dtype), scale_dtype=_ffi.dtype_code(self.scale_dtype),
         scale_heads=self.scale_heads, rounding=_rounding_code(self.rounding))
-    for t_ in out:
-      _ffi.dev(t_, "quantiser output")
+    for i, t_ in enumerate(out):
+      _ffi.holds(_ffi.dev(t_, "quantiser output"), b * h * d if i < 2 else b * self.scale_heads, "quantiser output")
     a.out_k, a.out_v, a.out_k_scale, a.out_v_scale = (_ffi.ptr(t_) for t_ in out)
     rope = None
     if freqs_cis is not None:  # xk is unrotated: the launch rotates it first
@@ -230,8 +233,8 @@ class Int8KVCacheGenerate:
       a.rope = _ffi.ptr(rope)
     pos = None
     if cache is not None:
-      for t_ in cache:
-        _ffi.dev(t_, "cache")
+      for i, t_ in enumerate(cache):
+        _ffi.holds(_ffi.dev(t_, "cache"), (b * h * d if i < 2 else b * self.scale_heads) * cache[0].shape[-2], "cache")
       a.cache_k, a.cache_v, a.k_scale, a.v_scale = (_ffi.ptr(t_) for t_ in cache)
       a.seq = cache[0].shape[-2]
       a.pos_count = 1 if ring else b
@@ -363,6 +366,8 @@ class PageKVCacheGenerate:
     heads, total, ps, dim = pk.shape
     key = _ffi.dev(key.to(pk.dtype).contiguous(), "key")
     value = _ffi.dev(value.to(pv.dtype).contiguous(), "value")
+    _ffi.alike(pk, pv, "key and value pages"), _ffi.alike(key, value, "key and value")
+    _ffi.holds(key, key.shape[0] * heads * dim, "key")
     idx = self.page_token_indices
     if isinstance(idx, DeviceTokenIndices):  # column count stays on the device
       _ffi.check(_ffi.lib.jpt_paged_append_dev(
@@ -373,6 +378,7 @@ class PageKVCacheGenerate:
       idx = _ffi.as_i32(idx, pk.device).reshape(3, -1)
       self.page_token_indices = idx
     idx = idx.contiguous()
+    _ffi.holds(idx, 3 * idx.shape[-1], "page_token_indices")
     _ffi.check(_ffi.lib.jpt_paged_append(
         _ffi.ptr(pk), _ffi.ptr(pv), _ffi.ptr(key), _ffi.ptr(value), _ffi.ptr(idx), idx.shape[1],
         key.shape[0], heads, total, ps, dim * pk.element_size(), _ffi.stream()))
@@ -422,6 +428,8 @@ class Int8PageKVCacheGenerate:
     ks, vs = _ffi.dev(self.k_scaler, "k_scale_pages"), _ffi.dev(self.v_scaler, "v_scale_pages")
     heads, total, ps, dim = pk.shape
     key, value = _ffi.dev(key.contiguous(), "key"), _ffi.dev(value.contiguous(), "value")
+    _ffi.alike(pk, pv, "key and value pages"), _ffi.alike(ks, vs, "key and value scale pages"), _ffi.alike(key, value, "key and value")
+    _ffi.holds(key, key.shape[0] * heads * dim, "key"), _ffi.holds(ks, ks.shape[0] * total * ps, "scale pages")
     idx = self.page_token_indices
     n_dev, stride = None, 0
     if isinstance(idx, DeviceTokenIndices):  # column count stays on the device
@@ -430,6 +438,7 @@ class Int8PageKVCacheGenerate:
       idx = _ffi.as_i32(idx, pk.device).reshape(3, -1)
       self.page_token_indices = idx
     idx = idx.contiguous()
+    _ffi.holds(idx, 3 * idx.shape[-1], "page_token_indices")
     a = _ffi.PagedQuantAppendArgs(
         new_k=_ffi.ptr(key), new_v=_ffi.ptr(value), pages_k=_ffi.ptr(pk), pages_v=_ffi.ptr(pv),
         k_scale_pages=_ffi.ptr(ks), v_scale_pages=_ffi.ptr(vs), indices=_ffi.ptr(idx),

@@ -59,12 +59,14 @@ def insert_prefix_caches(prefix_caches, caches, cache_scales, slot, start, *, ro
     if not quant and newk.dtype != k.dtype:
       newk, newv = newk.to(k.dtype), newv.to(v.dtype)
     newk, newv = _ffi.dev(newk.contiguous(), "prefix key"), _ffi.dev(newv.contiguous(), "prefix value")
+    _ffi.alike(k, v, "key and value caches"), _ffi.alike(newk, newv, "prefix key and value")
     if newk.shape != (heads, tokens, dim):
       raise ValueError(f"prefix key {tuple(newk.shape)} does not match cache {tuple(k.shape)}")
     ks = vs = None
     if quant:
       ks, vs = _layer_views(cache_scales, layer, n_layers)
       ks, vs = _ffi.dev(ks, "k_scaler"), _ffi.dev(vs, "v_scaler")
+      _ffi.alike(ks, vs, "key and value scalers"), _ffi.holds(ks, batch * ks.shape[1] * seq, "scalers")
     this = (tuple(k.shape), k.dtype, tuple(newk.shape), newk.dtype, None if ks is None else (ks.dtype, tuple(ks.shape)))
     if shape is not None and this != shape:
       raise ValueError("the layers of one insert must agree in shape and dtype")
@@ -103,6 +105,8 @@ def insert_prefix_pages_int8(prefix_caches, decode_caches, scale_pages, page_ids
     if newk.dim() == 4:
       newk, newv = newk[0], newv[0]
     newk, newv = _ffi.dev(newk.contiguous(), "prefix key"), _ffi.dev(newv.contiguous(), "prefix value")
+    _ffi.alike(pk, pv, "key and value pages"), _ffi.alike(ks, vs, "key and value scale pages"), _ffi.alike(newk, newv, "prefix key and value")
+    _ffi.holds(newk, heads * newk.shape[1] * dim, "prefix key"), _ffi.holds(ks, ks.shape[0] * total * ps, "scale pages")
     this = (tuple(pk.shape), tuple(newk.shape), newk.dtype, ks.dtype, tuple(ks.shape))
     if shape is not None and this != shape:
       raise ValueError("the layers of one insert must agree in shape and dtype")
@@ -133,6 +137,7 @@ def insert_prefix_pages_copy(prefix_caches, decode_caches, page_ids):
       return False
     heads, total, ps, dim = pk.shape
     newk, newv = newk.to(pk.dtype).contiguous(), newv.to(pv.dtype).contiguous()
+    _ffi.alike(pk, pv, "key and value pages"), _ffi.alike(newk, newv, "prefix key and value")
     this = (tuple(pk.shape), pk.dtype, tuple(newk.shape))
     if dim % 4 != 0 or newk.dim() != 4 or newk.shape[0] != 1 or newk.shape[1] != heads or newk.shape[3] != dim \
         or (shape is not None and this != shape) or not newk.is_cuda:
@@ -161,6 +166,8 @@ def insert_prefix_pages_int8_stacked(prefix_k, prefix_v, pages_k, pages_v, k_sca
           newk.stride() == newv.stride()):
     newk, newv = _ffi.dev(newk.contiguous(), "prefix key"), _ffi.dev(newv.contiguous(), "prefix value")
   layers, heads, total, ps, dim = pk.shape
+  _ffi.alike(pk, pv, "key and value pages"), _ffi.alike(ks, vs, "key and value scale pages"), _ffi.alike(newk, newv, "prefix key and value")
+  _ffi.holds(ks, layers * ks.shape[1] * total * ps, "scale pages")
   if newk.shape[0] != layers or newk.shape[1] != heads or newk.shape[3] != dim:
     raise ValueError(f"prefix {tuple(newk.shape)} does not match pages {tuple(pk.shape)}")
   ids = _ffi.as_i32(page_ids, pk.device)
@@ -184,11 +191,14 @@ def insert_prompts_pages_int8_stacked(prefixes, pages_k, pages_v, k_scale_pages,
   pk, pv = _ffi.dev(pages_k, "pages_k"), _ffi.dev(pages_v, "pages_v")
   ks, vs = _ffi.dev(k_scale_pages, "k_scale_pages"), _ffi.dev(v_scale_pages, "v_scale_pages")
   layers, heads, total, ps, dim = pk.shape
+  _ffi.alike(pk, pv, "key and value pages"), _ffi.alike(ks, vs, "key and value scale pages")
+  _ffi.holds(ks, layers * ks.shape[1] * total * ps, "scale pages")
   recs, keep = [], []
   for (newk, newv), ids in zip(prefixes, page_ids):
     if not (newk.is_cuda and newk.stride(3) == 1 and newk.stride(2) == newk.shape[3] and
             newk.stride() == newv.stride()):
       newk, newv = _ffi.dev(newk.contiguous(), "prefix key"), _ffi.dev(newv.contiguous(), "prefix value")
+    _ffi.alike(newk, newv, "prefix key and value")
     if newk.shape[0] != layers or newk.shape[1] != heads or newk.shape[3] != dim or newk.dtype != prefixes[0][0].dtype:
       raise ValueError(f"prefix {tuple(newk.shape)} does not match pages {tuple(pk.shape)}")
     ids = _ffi.as_i32(ids, pk.device)

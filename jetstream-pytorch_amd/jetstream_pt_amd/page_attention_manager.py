@@ -151,6 +151,7 @@ class PageAttentionManager:
       heads, total, ps, dim = pk.shape
       k = _ffi.dev(k.to(pk.dtype).contiguous(), "prefill k")
       v = _ffi.dev(v.to(pv.dtype).contiguous(), "prefill v")
+      _ffi.alike(pk, pv, "key and value pages"), _ffi.alike(k, v, "prefill key and value")
       if k.shape[0] != 1 or k.shape[1] != heads or k.shape[3] != dim:
         raise ValueError(f"prefill cache {tuple(k.shape)} does not match pages {tuple(pk.shape)}")
       _ffi.check(_ffi.lib.jpt_paged_insert(

@@ -32,6 +32,7 @@ def quantize_kv(xk, xv, *, rounding="trunc", scale_heads=1, scale_dtype=None, fr
   b, h, t, d = xk.shape
   if t != 1 or xv.shape != xk.shape:
     raise ValueError(f"expected matching (batch, heads, 1, dim) tensors, got {tuple(xk.shape)} and {tuple(xv.shape)}")
+  _ffi.alike(xk, xv, "xk and xv")
   sdt = scale_dtype or xk.dtype
   kq = torch.empty_like(xk, dtype=torch.int8)
   vq = torch.empty_like(xv, dtype=torch.int8)

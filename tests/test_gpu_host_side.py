@@ -358,3 +358,71 @@ def test_a_fresh_plans_workspace_serves_the_kernel_whose_counters_it_holds(b, fi
     out.zero_()
     _ffi.check(_ffi.lib.jpt_attn_ragged(a, _ffi.stream()))
     assert torch.equal(out.reshape(want.shape), want)
+
+
+def test_rows_that_do_not_belong_together_are_refused():
+  """What a kernel walks side by side, or by another tensor's shape, agrees with it: everything else is
+  refused before a launch (a bf16 value read as the float32 its key is ends past its rows)."""
+  from jetstream_pt_amd import attention_kernel as ak, cache_manager as cm, insert as pi, layers
+  from jetstream_pt_amd.environment import JetEngineEnvironment, JetEngineEnvironmentData
+  from jetstream_pt_amd.page_attention_manager import PageAttentionManager
+  from jetstream_pt_amd.quantize import quantize_kv
+  b, hq, hkv, s, d, ps, total, nl, t = 2, 4, 2, 64, 128, 32, 8, 2, 40
+  z = lambda *shape, dt=torch.bfloat16: torch.zeros(shape, dtype=dt, device=DEV)
+  i8, f32 = torch.int8, torch.float32
+  row, q, wide = z(b, hkv, 1, d), z(b, hq, 1, d), z(b, hkv, 1, d, dt=f32)
+  few = z(b, 1, 1, d)  # a head short
+  ring = JetEngineEnvironment(JetEngineEnvironmentData(batch_size=b, num_layers=nl))
+  lazy = JetEngineEnvironment(JetEngineEnvironmentData(batch_size=b, num_layers=nl, ring_buffer=False))
+  pos, lens, idx = (torch.tensor(x, dtype=torch.int32, device=DEV) for x in ([3], [3, 40], [[1, 2], [3, 8], [0, 1]]))
+  mask = z(b, 1, 1, s, dt=f32)
+
+  def step(env, kind, k, v, **kw):
+    cache = kind.empty((b, hkv, s, d) if env is ring else (nl, b, hkv, s, d), DEV, env, **kw)
+    cache.input_pos = pos if env is ring else lens
+    kern = (layers.Int8KVAttentionKernel if kind is cm.Int8KVCacheGenerate else layers.AttentionKernel)(env, 0)
+    kern(q, k, v, mask if env is ring else None, cache, start=None, end=lens)
+
+  def paged(k, v, int8, scale_shape=(1, total, ps), pages_v=(hkv, total, ps, d)):
+    pam = PageAttentionManager(b, total, ps, 4)
+    dt = i8 if int8 else torch.bfloat16
+    pages = [z(hkv, total, ps, d, dt=dt), z(*pages_v, dt=dt)]
+    scales = [z(*scale_shape, dt=f32), z(*scale_shape, dt=f32)]
+    cache = cm.Int8PageKVCacheGenerate(*pages, *scales, pam, idx) if int8 else cm.PageKVCacheGenerate(*pages, pam, idx)
+    cache.update(k, v)
+
+  prompt, wide_prompt = z(1, hkv, t, d), z(1, hkv, t, d, dt=f32)
+  dense8, dense_scale = lambda: z(b, hkv, s, d, dt=i8), z(b, 1, s, 1, dt=f32)
+  pages8, scale_pages = z(hkv, total, ps, d, dt=i8), z(1, total, ps, dt=f32)
+  stack8, stack_scale, prompts = z(nl, hkv, total, ps, d, dt=i8), z(nl, 1, total, ps, dt=f32), z(nl, hkv, t, d)
+  ids = torch.tensor([1, 2], dtype=torch.int32, device=DEV)
+  codes, scale = z(b, hkv, s, d, dt=i8), z(b, 1, s, 1, dt=f32)
+  refused = [
+      lambda: quantize_kv(row, wide), lambda: quantize_kv(wide, row),
+      lambda: step(ring, cm.Int8KVCacheGenerate, wide, row, scale_dtype=f32), lambda: step(ring, cm.Int8KVCacheGenerate, row, few),
+      lambda: step(ring, cm.Int8KVCacheGenerate, few, few), lambda: step(ring, cm.KVCacheGenerate, row, few),
+      lambda: step(ring, cm.KVCacheGenerate, few, few), lambda: step(lazy, cm.Int8KVCacheGenerate, wide, row, scale_dtype=f32),
+      lambda: step(lazy, cm.Int8KVCacheGenerate, few, few),
+      lambda: paged(wide, row, True), lambda: paged(row, wide, True), lambda: paged(few, few, True), lambda: paged(row, few, True),
+      lambda: paged(row, row, True, scale_shape=(1, total, 1)), lambda: paged(row, row, True, pages_v=(hkv, 2, ps, d)),
+      lambda: paged(row, few, False), lambda: paged(few, few, False), lambda: paged(row, row, False, pages_v=(hkv, 2, ps, d)),
+      lambda: pi.insert_prefix_caches([(wide_prompt, prompt)], [(dense8(), dense8())], [(dense_scale, dense_scale)], 0, 0),
+      lambda: pi.insert_prefix_caches([(prompt, prompt[:, :, :8])], [(dense8(), dense8())], [(dense_scale, dense_scale)], 0, 0),
+      lambda: pi.insert_prefix_caches([(prompt, prompt)], [(dense8(), dense8()[:1])], [(dense_scale, dense_scale)], 0, 0),
+      lambda: pi.insert_prefix_caches([(prompt, prompt)], [(dense8(), dense8())], [(dense_scale[:, :, :8].contiguous(), dense_scale[:, :, :8].contiguous())], 0, 0),
+      lambda: pi.insert_prefix_pages_int8([(wide_prompt, prompt)], [(pages8, pages8)], [(scale_pages, scale_pages)], ids),
+      lambda: pi.insert_prefix_pages_int8([(prompt, prompt)], [(pages8, pages8[:1])], [(scale_pages, scale_pages)], ids),
+      lambda: pi.insert_prefix_pages_int8([(prompt, prompt)], [(pages8, pages8)], [(scale_pages, scale_pages[:, :2])], ids),
+      lambda: pi.insert_prefix_pages_int8_stacked(prompts.float(), prompts, stack8, stack8, stack_scale, stack_scale, ids),
+      lambda: pi.insert_prompts_pages_int8_stacked([(prompts, prompts[:, :, :8])], stack8, stack8, stack_scale, stack_scale, [ids]),
+      lambda: pi.insert_prefix_pages_copy([(prompt, prompt[:, :, :8])] * 2, [(z(hkv, total, ps, d), z(hkv, total, ps, d))] * 2, ids),
+      lambda: PageAttentionManager(b, total, ps, 4).insert_prefill_cache([(prompt, prompt[:, :, :8])], [(z(hkv, total, ps, d), z(hkv, total, ps, d))], ids),
+      lambda: ak.dense_attention(q, codes, codes, scale[:1], scale[:1]), lambda: ak.dense_attention(q, codes, codes, scale[:, :, :8].contiguous(), scale[:, :, :8].contiguous()),
+      lambda: ak.ragged_mha(q, codes, codes, 0, None, lens, None, None, scale, scale, new_key=row.char(), new_value=few.char(),
+                            new_k_scaler=scale[:, :, :1].contiguous(), new_v_scaler=scale[:, :, :1].contiguous()),
+      lambda: ak.ragged_mha(q, codes, codes, 0, None, lens, None, None, scale, scale, new_key=row.char(), new_value=row.char(),
+                            new_k_scaler=scale[:1, :, :1].contiguous(), new_v_scaler=scale[:1, :, :1].contiguous()),
+  ]
+  for call in refused:
+    with pytest.raises(ValueError):
+      call()
