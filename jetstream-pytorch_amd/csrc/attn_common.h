@@ -39,6 +39,17 @@ bool attn_prefill_supported(const jpt_attn_args& a, AttnMode mode);
 int64_t attn_prefill_workspace_bytes(const jpt_attn_args& a);
 int32_t attn_prefill_launch(const jpt_attn_args& a, hipStream_t stream);
 
+// Of the current device (all of a process are alike).
+inline int32_t compute_units() {
+  static const int32_t v = [] {
+    int dev = 0, cus = 256;
+    if (hipGetDevice(&dev) == hipSuccess &&
+        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) cus = 256;
+    return cus;
+  }();
+  return v;
+}
+
 int32_t attn_generic_launch(const jpt_attn_args& a, AttnMode mode, hipStream_t stream);
 
 }  // namespace jpt

@@ -702,16 +702,6 @@ __global__ void __launch_bounds__(kSplitThreads, (split_waves_per_simd<D, KV>())
   }
 }
 
-int32_t compute_units() {
-  static const int32_t v = [] {
-    int dev = 0, cus = 256;
-    if (hipGetDevice(&dev) == hipSuccess &&
-        hipDeviceGetAttribute(&cus, hipDeviceAttributeMultiprocessorCount, dev) != hipSuccess) cus = 256;
-    return cus;
-  }();
-  return v;
-}
-
 constexpr int kMinGroups = 64;
 int64_t group_bytes(const jpt_attn_args& a) {  // two records
   return 2ll * (a.q_heads / a.kv_heads) * a.q_rows * (a.dim + 4) * 4;

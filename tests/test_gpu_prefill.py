@@ -48,6 +48,12 @@ CASES = [  # b, hq, hkv, d, t, s, mask, scale heads (None: no scales), scale dty
     (1, 8, 2, 128, 64, 63, None, 2, torch.bfloat16),
     (1, 2, 2, 64, 1, 77, None, None, None),
     (3, 4, 2, 256, 5, 1, None, None, None),
+    (1, 4, 2, 128, 130, 257, "any", None, None),            # mask rows that no wide load fits
+    (1, 2, 1, 256, 190, 320, "causal", 1, torch.float32),
+    (5, 64, 8, 64, 130, 130, "causal", None, None),         # enough rows for workgroups of 128: no mask pass ...
+    (5, 64, 8, 64, 130, 258, "causal", 1, torch.bfloat16),  # ... with one
+    (40, 8, 1, 128, 129, 192, None, None, None),
+    (11, 32, 4, 256, 129, 257, "causal", None, None),
 ]
 
 
@@ -116,6 +122,45 @@ def test_weights_are_float32(masked, sdt, d):
   got = ak.dense_attention(*dev).double().cpu()
   over = (got - want).abs() / float32_bound(want, total)
   assert torch.all(over <= 1.0), float(over.max())
+
+
+@pytest.mark.parametrize("heads", [2, 336])
+@pytest.mark.parametrize("jump", [2.0, 7.0, 40.0])
+def test_maxima_that_rise(jump, heads):
+  """Scores that climb from tile to tile, by less and by more than what sums are carried over without being
+  rescaled; both ways of dividing a workgroup's waves."""
+  from jetstream_pt_amd import attention_kernel as ak
+  d, t, s = 64, 130, 512
+  g = torch.Generator().manual_seed(945)
+  q, k = torch.zeros((1, heads, t, d)), 0.05 * torch.randn((1, heads, s, d), generator=g)
+  q[..., 0] = math.sqrt(d) * (torch.arange(t) % 3 - 1)  # rows whose scores fall, stay and climb
+  k[..., 0] = (torch.arange(s) // 64) * jump
+  q, k, v = q.to(torch.bfloat16), k.to(torch.bfloat16), rnd(g, (1, heads, s, d))
+  mask = torch.zeros((1, 1, t, s))
+  mask[..., 300:310] = -math.inf
+  for m in (None, mask):
+    want, wm, wl = OA.closed_form(q, k, v, mask=None if m is None else m.expand(1, heads, t, s))
+    got, (gm, gl) = ak.flash_attention(q.to(DEV), k.to(DEV), v.to(DEV), 0, None, None, None if m is None else m.to(DEV))
+    err = (got.double().cpu() - want).abs()
+    assert torch.all(err <= torch.where(want.abs() < 2.0, torch.full_like(err, 6e-3), attention_bound(want))), float(err.max())
+    assert torch.allclose(gm.double().cpu(), wm, rtol=1e-3, atol=1e-4) and torch.allclose(gl.double().cpu(), wl, rtol=1e-3)
+
+
+@pytest.mark.parametrize("scale", [-0.25, 0.0])
+@pytest.mark.parametrize("kind", [None, "causal"])
+def test_scales_that_are_not_positive(kind, scale):
+  from jetstream_pt_amd import attention_kernel as ak
+  b, hq, hkv, d, t, s = 1, 4, 2, 128, 200, 333
+  g = torch.Generator().manual_seed(947)
+  q, k, v = rnd(g, (b, hq, t, d)), rnd(g, (b, hkv, s, d)), rnd(g, (b, hkv, s, d))
+  mask = make_mask(kind, g, b, hq, t, s)
+  rows = None if mask is None else mask.expand(b, hq, t, s).reshape(b, hkv, hq // hkv * t, s)
+  want, wm, wl = OA.closed_form(q, k, v, mask=rows, sm_scale=scale)
+  got, m, l = ak._attend("dense", q.to(DEV), k.to(DEV), v.to(DEV), mask=None if mask is None else mask.to(DEV), sm_scale=scale, want_stats=True)
+  err = (got.double().cpu() - want.reshape(got.shape)).abs()
+  assert torch.all(err <= torch.where(want.reshape(got.shape).abs() < 2.0, torch.full_like(err, 6e-3), attention_bound(want.reshape(got.shape)))), float(err.max())
+  assert torch.allclose(m.double().cpu().reshape(wm.shape), wm, rtol=1e-3, atol=1e-4)
+  assert torch.allclose(l.double().cpu().reshape(wl.shape), wl, rtol=1e-3)
 
 
 LOWEST = [torch.finfo(torch.float32).min, OA.DEFAULT_MASK_VALUE, -2.0 ** 127]
