@@ -13,8 +13,15 @@ int32_t check_attn_args(const jpt_attn_args& a, AttnMode mode);
 // JPT_E_BADARG (without setting the message) when the shape is outside what
 // it handles and the generic kernel must run.
 bool attn_fast_supported(const jpt_attn_args& a, AttnMode mode);
-// stash_k, stash_v: see FastParams
-int32_t attn_fast_launch(const jpt_attn_args& a, AttnMode mode, hipStream_t stream, void* stash_k = nullptr, void* stash_v = nullptr);
+// stash_k, stash_v and the line: see FastParams
+struct StepLine {
+  const void *k = nullptr, *v = nullptr;
+  const int32_t* pos = nullptr;
+  const float* rope = nullptr;
+  int32_t count = 0, rounding = 0;
+};
+int32_t attn_fast_launch(const jpt_attn_args& a, AttnMode mode, hipStream_t stream, void* stash_k = nullptr, void* stash_v = nullptr,
+                         const StepLine& line = StepLine());
 int64_t attn_fast_workspace_bytes(const jpt_attn_args& a);
 int64_t attn_partials_offset(const jpt_attn_args& a);  // in the workspace: behind the plan
 // Where kernels that need no plan put what they need: the last `bytes` of the workspace, from a multiple of

@@ -671,7 +671,7 @@ int32_t attn_plan_launch(const jpt_attn_args& a, bool paged, bool fresh, hipStre
   return launch_status("plan_kernel");
 }
 
-int32_t attn_fast_launch(const jpt_attn_args& a, AttnMode mode, hipStream_t stream, void* stash_k, void* stash_v) {
+int32_t attn_fast_launch(const jpt_attn_args& a, AttnMode mode, hipStream_t stream, void* stash_k, void* stash_v, const StepLine& line) {
   const int rep = a.q_heads / a.kv_heads;
   const int rows = rep * a.q_rows;
   const Layout l = make_layout(a.batch, a.kv_heads, rows);
@@ -691,6 +691,12 @@ int32_t attn_fast_launch(const jpt_attn_args& a, AttnMode mode, hipStream_t stre
   p.status = reinterpret_cast<int32_t*>(ws);
   p.stash_k = stash_k;
   p.stash_v = stash_v;
+  p.line_k = line.k;
+  p.line_v = line.v;
+  p.line_pos = line.pos;
+  p.line_rope = line.rope;
+  p.line_count = line.count;
+  p.line_rounding = line.rounding;
   if (!a.reuse_plan) {
     int32_t st = attn_plan_launch(a, mode == kPaged, false, stream);
     if (st != JPT_OK) return st;
@@ -839,6 +845,71 @@ int32_t jpt_attn_ragged_stash(const jpt_attn_args* args, void* stash_k, void* st
   if (at != JPT_OK) return at;
   const int64_t bytes = static_cast<int64_t>(args->batch) * args->kv_heads * args->dim * 2;
   return jpt_kv_stash_lines(stash_k, args->new_k, stash_v, args->new_v, bytes, stream);
+}
+
+namespace {
+// The launch that attends writes the step's line where it looks through a mask first (see the streaming kernel), and
+// where a row shares no cache line of 128 bytes with its neighbours.
+bool writes_line(const jpt_attn_args& a, const void* line_k, const void* line_v) {
+  using namespace jpt;
+  return attn_fast_supported(a, kDense) && a.mask != nullptr && aligned(a.k, 128) && aligned(a.v, 128) && aligned(line_k, 16) && aligned(line_v, 16);
+}
+int32_t check_line(const jpt_attn_args* args, const void* line_k, const void* line_v, const int32_t* pos, int32_t pos_count) {
+  using namespace jpt;
+  JPT_REQUIRE(args != nullptr && line_k != nullptr && line_v != nullptr && pos != nullptr, "args, the line's rows and pos must not be NULL");
+  JPT_REQUIRE(pos_count == 1 || pos_count == args->batch, "pos must hold 1 or batch entries");
+  JPT_REQUIRE(args->new_k == nullptr && args->lengths == nullptr, "the line is the token, and every position is attended");
+  return check_attn_args(*args, kDense);
+}
+}  // namespace
+
+int32_t jpt_attn_dense_line(const jpt_attn_args* args, const void* line_k, const void* line_v, const int32_t* pos, int32_t pos_count, void* stream) {
+  using namespace jpt;
+  const int32_t st = check_line(args, line_k, line_v, pos, pos_count);
+  if (st != JPT_OK) return st;
+  if (args->kv_dtype == JPT_BF16 && writes_line(*args, line_k, line_v)) {
+    StepLine line;
+    line.k = line_k;
+    line.v = line_v;
+    line.pos = pos;
+    line.count = pos_count;
+    return attn_fast_launch(*args, kDense, static_cast<hipStream_t>(stream), nullptr, nullptr, line);
+  }
+  jpt_line_tensor t[2] = {};
+  t[0].dst = args->k;
+  t[0].src = line_k;
+  t[1].dst = args->v;
+  t[1].src = line_v;
+  t[0].heads = t[1].heads = args->kv_heads;
+  t[0].row_bytes = t[1].row_bytes = args->dim * elem_size(args->kv_dtype);
+  const int32_t wrote = jpt_kv_scatter_lines(t, 2, pos, pos_count, 1, args->batch, args->seq, stream);
+  return wrote != JPT_OK ? wrote : jpt_attn_dense(args, stream);
+}
+
+int32_t jpt_attn_dense_append(const jpt_attn_args* args, const jpt_quant_append_args* append, void* stream) {
+  using namespace jpt;
+  JPT_REQUIRE(append != nullptr, "append is NULL");
+  const jpt_quant_append_args& q = *append;
+  const int32_t st = check_line(args, q.new_k, q.new_v, q.pos, q.pos_count);
+  if (st != JPT_OK) return st;
+  const jpt_attn_args& a = *args;
+  // the same cache, and what the launch can quantise
+  if (a.kv_dtype == JPT_I8 && q.in_dtype == JPT_BF16 && q.cache_k == a.k && q.cache_v == a.v && q.k_scale == a.k_scale &&
+      q.v_scale == a.v_scale && q.batch == a.batch && q.heads == a.kv_heads && q.seq == a.seq && q.dim == a.dim &&
+      q.scale_dtype == a.scale_dtype && q.scale_heads == a.scale_heads && (q.scale_heads == 1 || q.scale_heads == q.heads) &&
+      q.out_k == nullptr && q.out_v == nullptr && (q.rounding == JPT_ROUND_TRUNC || q.rounding == JPT_ROUND_RNE) &&
+      aligned(q.rope, 16) && writes_line(a, q.new_k, q.new_v)) {
+    StepLine line;
+    line.k = q.new_k;
+    line.v = q.new_v;
+    line.pos = q.pos;
+    line.count = q.pos_count;
+    line.rope = q.rope;
+    line.rounding = q.rounding;
+    return attn_fast_launch(a, kDense, static_cast<hipStream_t>(stream), nullptr, nullptr, line);
+  }
+  const int32_t wrote = jpt_kv_append_quant_i8(append, stream);
+  return wrote != JPT_OK ? wrote : jpt_attn_dense(args, stream);
 }
 
 // ---- jpt_attn_ragged_static: the workspace is a device array of this library ----

@@ -87,6 +87,10 @@ constexpr int kMergeSpinLimit = 1 << 16;  // polls of a merge's wait for other w
 constexpr int kStreamOnce = 2;  // the NT bit of the instruction's cache-policy field
 constexpr int kListedItems = 64;     // a worker's first items, read into LDS at start
 constexpr int kStagedPages = 64;     // page ids of an item kept in LDS (later pages are read one by one)
+// Masked calls: a worker's first kMappedItems items have a bit a tile, set where the mask leaves something of it to
+// attend (items of more than kMappedTiles tiles, and later ones, are attended tile by tile).
+constexpr int kMappedItems = 10;
+constexpr int kMappedTiles = 256;
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLn2 = 0.6931471805599453f;
 
@@ -358,6 +362,72 @@ struct Tile<__bf16> {
 };
 
 
+// Quantising a token whose bf16 rows of all heads lie one after another at `rows`: arithmetic and rounding of
+// jpt_kv_append_quant_i8, each step rounded to the scale dtype.  (The consumers' new_absmax and new_encode are the same
+// steps, in LDS; with these in their place the paged launch keeps four more scalars in lanes: 439 -> 443 us a step.)  One wave; head h is coded, two elements a lane.
+// token_absmax leaves them in x0, x1 and returns the lane's share of the absmax, over head h and the first `heads`
+// heads.  `rope`: NULL, or the slot's (cos, sin) factors: the rows are rotated pair by pair first (keys only), rounded
+// to bf16 as the separate rotary op would.
+__device__ __forceinline__ float token_absmax(const char* rows, int h, int heads, const float* rope, int lane, float& x0, float& x1) {
+  auto rotate = [](float& x, float& y, float c, float s) {
+#pragma clang fp contract(off)  // the products are rounded before they are combined
+    const float xc = x * c, ys = y * s, xs = x * s, yc = y * c;
+    const float re = xc - ys;
+    const float im = xs + yc;
+    x = round_to_bf16(re);
+    y = round_to_bf16(im);
+  };
+  const uint32_t pair = *reinterpret_cast<const uint32_t*>(rows + h * (kD * 2) + lane * 4);
+  x0 = __uint_as_float(pair << 16);
+  x1 = __uint_as_float(pair & 0xffff0000u);
+  if (rope) {  // the lane's elements 2 * lane, 2 * lane + 1 of the head are pair number `lane`
+    const float2 cs = *reinterpret_cast<const float2*>(rope + 2 * lane);
+    rotate(x0, x1, cs.x, cs.y);
+  }
+  float m = fmaxf(fabsf(x0), fabsf(x1));
+  for (int at = lane * 32; at < heads * (kD * 2); at += 64 * 32) {
+    const uint4 r0 = *reinterpret_cast<const uint4*>(rows + at);
+    const uint4 r1 = *reinterpret_cast<const uint4*>(rows + at + 16);
+    const uint32_t raw[8] = {r0.x, r0.y, r0.z, r0.w, r1.x, r1.y, r1.z, r1.w};
+    float f[16];
+#pragma unroll
+    for (int i = 0; i < 8; ++i) {
+      f[2 * i] = __uint_as_float(raw[i] << 16);
+      f[2 * i + 1] = __uint_as_float(raw[i] & 0xffff0000u);
+    }
+    if (rope) {  // byte `at` of the rows is element (at % 256) / 2 of its head: eight pairs from there
+      const float4* cs4 = reinterpret_cast<const float4*>(rope + (at % (kD * 2)) / 2);
+#pragma unroll
+      for (int i = 0; i < 4; ++i) {
+        const float4 cs = cs4[i];
+        rotate(f[4 * i], f[4 * i + 1], cs.x, cs.y);
+        rotate(f[4 * i + 2], f[4 * i + 3], cs.z, cs.w);
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < 16; ++i) m = fmaxf(m, fabsf(f[i]));
+  }
+  return m;
+}
+// The two codes of x0 and x1; `scale`: the absmax, becomes the scale.
+template <bool BF16_MATH>
+__device__ __forceinline__ uint16_t token_codes(float x0, float x1, int rounding, float& scale) {
+  auto rnd = [](float x) { return BF16_MATH ? round_to_bf16(x) : x; };
+  if (rounding == JPT_ROUND_RNE) scale = fmaxf(scale, rnd(1e-5f));
+  const float sc = scale = rnd(scale / 127.0f);
+  int c0, c1;
+  if (rounding == JPT_ROUND_TRUNC) {
+    const float q0 = rnd(x0 / sc), q1 = rnd(x1 / sc);
+    c0 = (q0 != q0) ? 0 : static_cast<int>(q0);  // 0/0 -> 0; the cast truncates
+    c1 = (q1 != q1) ? 0 : static_cast<int>(q1);
+  } else {
+    const float inv = rnd(1.0f / sc);
+    c0 = static_cast<int>(fminf(fmaxf(rintf(rnd(x0 * inv)), -128.f), 127.f));
+    c1 = static_cast<int>(fminf(fmaxf(rintf(rnd(x1 * inv)), -128.f), 127.f));
+  }
+  return static_cast<uint16_t>((c0 & 0xff) | ((c1 & 0xff) << 8));
+}
+
 // One work item: a chunk of one slot for one KV head.
 struct Item {
   int slot, start, count, part, n_chunks, h;
@@ -404,6 +474,10 @@ __global__ void __launch_bounds__(kThreads, kWavesPerSimd) attn_decode_kernel(Fa
   __shared__ __attribute__((aligned(16))) int sm_items_all[kGroups][kListedItems][8];
   // page ids of the item being issued and of the next one (paged caches)
   __shared__ int sm_pages_all[PAGED ? kGroups : 1][2][kStagedPages];
+  // masked calls: an item's live tiles, a bit each, and their number; positions of the tile in a ring slot that count
+  __shared__ __attribute__((aligned(16))) uint8_t sm_live_all[MASK ? kGroups : 1][MASK ? kMappedItems : 1][MASK ? kMappedTiles / 8 : 4];
+  __shared__ __attribute__((aligned(16))) int sm_n_live_all[MASK ? kGroups : 1][MASK ? kMappedItems : 1][4];  // counted by each of the four waves
+  __shared__ int sm_valid_all[MASK ? kGroups : 1][C::kSlots];
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int hw_wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform, and known to be
@@ -455,7 +529,7 @@ __global__ void __launch_bounds__(kThreads, kWavesPerSimd) attn_decode_kernel(Fa
   if (wave == kConsumers) {
     const int j = (lane & 1) ? (G - 1 - worker) : worker;
     const int i = lane * G + j;
-    const int entry = ((i >> 3) / a.kv_heads) * 8 + (i & 7);
+    const int entry = MASK ? i / a.kv_heads : ((i >> 3) / a.kv_heads) * 8 + (i & 7);  // see item_index
     const int4* en = reinterpret_cast<const int4*>(p.entries + min(entry, p.total_items / a.kv_heads - 1));
     listed0 = en[0];
     listed1 = en[1];
@@ -481,11 +555,17 @@ __global__ void __launch_bounds__(kThreads, kWavesPerSimd) attn_decode_kernel(Fa
   // (entry, head) with all heads of an entry on ids of equal i % 8: workgroup
   // ids go round-robin over the 8 XCDs, so an entry's scales and page-table
   // row are fetched into one L2 only.  Unused entries give invalid items.
+  // Under a mask the plan does not know how much of an entry there is to do, and a
+  // die with the long slots would be the launch: heads go round the dies there, so
+  // that each has a share of every entry (half of the positions live, us for eight
+  // layers: 8 slots x 32 heads x 1024 bf16 178 -> 159, 64 slots x 8 heads x 2048 int8 359
+  // -> 345).
+  // The two groups of a workgroup still have one head of entries half a round apart.
   auto item_index = [&](int k, int* entry, int* h) -> bool {
     const int j = (k & 1) ? (G - 1 - worker) : worker;
     const int i = k * G + j;
-    const int m = i >> 3;
-    *entry = (m / a.kv_heads) * 8 + (i & 7);
+    const int m = MASK ? i : i >> 3;
+    *entry = MASK ? m / a.kv_heads : (m / a.kv_heads) * 8 + (i & 7);
     *h = m % a.kv_heads;
     return k < n_rounds && i < n_ids && *entry < n_entries;
   };
@@ -505,14 +585,9 @@ __global__ void __launch_bounds__(kThreads, kWavesPerSimd) attn_decode_kernel(Fa
   int* const sm_folded = sm_folded_all[group];
   int (*const sm_items)[8] = sm_items_all[group];
   int (*const sm_pages)[kStagedPages] = sm_pages_all[PAGED ? group : 0];
-  if (wave == kConsumers) {
-    int entry, h;
-    if (!item_index(lane, &entry, &h)) listed0 = make_int4(-1, 0, 0, 0);
-    // slot, start, count, part | n_chunks, head, valid, slot length
-    *reinterpret_cast<int4*>(&sm_items[lane][0]) = listed0;
-    *reinterpret_cast<int4*>(&sm_items[lane][4]) = make_int4(listed1.x, h, listed0.x >= 0 ? 1 : 0, listed1.y);
-  }
-  __syncthreads();
+  auto& sm_live = sm_live_all[MASK ? group : 0];
+  auto& sm_n_live = sm_n_live_all[MASK ? group : 0];
+  int* const sm_valid = sm_valid_all[MASK ? group : 0];
   auto unpack_item = [&](int4 e0, int4 e1) -> Item {
     Item it;
     it.slot = __builtin_amdgcn_readfirstlane(e0.x);
@@ -542,10 +617,99 @@ __global__ void __launch_bounds__(kThreads, kWavesPerSimd) attn_decode_kernel(Fa
   // tiles of an item: its cache positions, plus one for the step's new token
   // on the slot's first chunk (when the token also goes into the pages, an
   // empty slot is an inactive one and has no token)
-  auto cache_tiles = [&](const Item& it) { return (it.count + kTile - 1) / kTile; };
-  auto item_tiles = [&](const Item& it) {
-    return cache_tiles(it) + ((has_new && it.start == 0 && !(to_pages && it.len == 0)) ? (wide_new ? 2 : 1) : 0);
+  auto all_tiles = [&](const Item& it) { return (it.count + kTile - 1) / kTile; };
+  // those that are attended, of the item of round k
+  auto mapped = [&](const Item& it, int k) { return MASK && k < kMappedItems && it.count <= kMappedTiles * kTile; };
+  auto cache_tiles = [&](const Item& it, int k) {
+    if (!mapped(it, k)) return all_tiles(it);
+    const i32x4 live = lds_peek4(&sm_n_live[k][0]);
+    return __builtin_amdgcn_readfirstlane(live[0] + live[1] + live[2] + live[3]);
   };
+  auto item_tiles = [&](const Item& it, int n_cache) {
+    return n_cache + ((has_new && it.start == 0 && !(to_pages && it.len == 0)) ? (wide_new ? 2 : 1) : 0);
+  };
+  if (wave == kConsumers) {
+    int entry, h;
+    if (!item_index(lane, &entry, &h)) listed0 = make_int4(-1, 0, 0, 0);
+    // slot, start, count, part | n_chunks, head, valid, slot length
+    *reinterpret_cast<int4*>(&sm_items[lane][0]) = listed0;
+    *reinterpret_cast<int4*>(&sm_items[lane][4]) = make_int4(listed1.x, h, listed0.x >= 0 ? 1 : 0, listed1.y);
+  }
+  if constexpr (MASK) {
+    // The step's line, where this launch writes it: the rows of the heads and slots whose chunk holds its position,
+    // by the workgroup that then reads them, before it does: consumer 1 the keys', consumer 2 the values', beside the
+    // other two waves' look through the mask.  (Eight layers of 64 slots x 8 heads, int8: 368 us with the quantiser's
+    // launch ahead, 344 so.)
+    const bool lined = NEW == kNewNone && p.line_k != nullptr;
+    if (lined && (wave == 1 || wave == 2)) {
+      const bool is_v = wave == 2;
+      for (int k = 0; k < n_rounds; ++k) {
+        const Item it = fetch(k);
+        if (!it.valid) continue;
+        const int at = load_uniform(p.line_pos + (p.line_count == 1 ? 0 : it.slot));
+        if (at < it.start || at >= it.start + it.count) continue;
+        const int64_t row = static_cast<int64_t>(it.slot) * a.kv_heads + it.h;
+        char* const to = static_cast<char*>(is_v ? a.v : a.k) + (row * a.seq + at) * C::kRowBytes;
+        if constexpr (std::is_same<KV, int8_t>::value) {
+          constexpr bool kBf16Math = SCALE == kScaleBF16;
+          const char* const rows = static_cast<const char*>(is_v ? p.line_v : p.line_k) + static_cast<int64_t>(it.slot) * a.kv_heads * (kD * 2);
+          const float* const rope = p.line_rope && !is_v ? p.line_rope + static_cast<int64_t>(it.slot) * kD : nullptr;
+          float x0, x1;
+          // the scale goes over all heads, or over the head's own elements
+          float scale = rows_max(row_max(token_absmax(rows, it.h, a.scale_heads == 1 ? a.kv_heads : 0, rope, lane, x0, x1)));
+          reinterpret_cast<uint16_t*>(to)[lane] = token_codes<kBf16Math>(x0, x1, p.line_rounding, scale);
+          if (lane == 0)  // one scale for all heads: every head's workgroup writes it, the same, before it reads it
+            store_from_f32(is_v ? a.v_scale : a.k_scale,
+                           (static_cast<int64_t>(it.slot) * a.scale_heads + (a.scale_heads == 1 ? 0 : it.h)) * a.seq + at,
+                           kBf16Math ? JPT_BF16 : JPT_F32, scale);
+        } else {
+          const uint32_t* from = reinterpret_cast<const uint32_t*>(static_cast<const char*>(is_v ? p.line_v : p.line_k) + row * C::kRowBytes);
+          reinterpret_cast<uint32_t*>(to)[lane] = from[lane];
+        }
+      }
+    }
+    // Which tiles of this worker's items the mask leaves anything of: a tile that it leaves nothing of is neither
+    // loaded nor computed.  The mask's rows (L2's after the first head) are looked through by four waves of the group,
+    // two where there is a line, 1024 positions a wave and trip to memory, before the stream starts: the first load goes
+    // out at 4.2 us instead of 2.2.  Attention alone, us, all / half / 15 % of the positions live: 8 slots x 32 heads x
+    // 1024 bf16 25.5 -> 26.5 / 19 / 13, 64 slots x 8 heads x 2048 int8 51 -> 50.5 / 38.5 / 20, 160 slots x 32 heads x 512 bf16
+    // 199 -> 204 / 130 / 59.  What is left is the unit with the longest slots: 1.5 us a tile and consumer.
+    const int n_items = min(n_rounds, kMappedItems);
+    const int lookers = lined ? 2 : 4, looker = !lined ? wave : wave == 0 ? 1 : wave == kConsumers ? 0 : -1;
+    const int per_item = n_items == 1 ? lookers : n_items == 2 ? lookers / 2 : 1;  // waves
+    for (int k = 0; k < n_items; ++k) {
+      int n_live = 0;
+      if (looker >= 0 && k % (lookers / per_item) == looker / per_item) {
+        const Item it = fetch(k);
+        const float* const row = static_cast<const float*>(a.mask) + it.slot * a.mask_stride_b + it.start + 4 * lane;
+        const int blocks = it.valid && mapped(it, k) ? (it.count + 255) / 256 : 0;
+        for (int b0 = looker % per_item; b0 < blocks; b0 += 4 * per_item) {
+          float4 x[4];
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            const int at = 256 * (b0 + u * per_item);  // (a chunk starts at a tile and a row is whole tiles: the four are in it)
+            x[u] = make_float4(-INFINITY, -INFINITY, -INFINITY, -INFINITY);
+            if (at + 4 * lane < it.count) x[u] = *reinterpret_cast<const float4*>(row + at);
+          }
+#pragma unroll
+          for (int u = 0; u < 4; ++u) {
+            const int block = b0 + u * per_item, left = it.count - 256 * block - 4 * lane;  // a NaN counts
+            const uint64_t set = __ballot((left > 0 && x[u].x != -INFINITY) || (left > 1 && x[u].y != -INFINITY) ||
+                                          (left > 2 && x[u].z != -INFINITY) || (left > 3 && x[u].w != -INFINITY));
+            // eight lanes a tile
+            const uint64_t tiles = __ballot(lane < 8 && ((set >> (8 * (lane & 7))) & 0xff) != 0);
+            if (block < blocks) {
+              if (lane == 0) sm_live[k][block] = static_cast<uint8_t>(tiles);
+              n_live += __popcll(tiles);
+            }
+          }
+        }
+      }
+      if (lane == 0) sm_n_live[k][wave] = n_live;
+    }
+    __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));  // the lines are where the loads behind the barrier find them
+  }
+  __syncthreads();
   // A wave gives up: the other waves of the workgroup see the flag at their
   // next wait and leave too, and the host finds the sticky word in the
   // workspace's state block (jpt_attn_status).
@@ -872,6 +1036,7 @@ __global__ void __launch_bounds__(kThreads, kWavesPerSimd) attn_decode_kernel(Fa
           __builtin_amdgcn_global_load_lds((global_ptr)(tv + off), (lds_ptr)(slot + C::kTileBytes + j * 1024), 16, 0, kStreamOnce);
         }
       }
+      if (MASK) lds_poke(&sm_valid[fill_slot], valid);
       char* side = slot + 2 * C::kTileBytes;
       if (SCALE) {
         if (lane < 2 * kHalf) __builtin_amdgcn_global_load_lds((global_ptr)sc, (lds_ptr)side, 4, 0, kStreamOnce);
@@ -897,7 +1062,7 @@ __global__ void __launch_bounds__(kThreads, kWavesPerSimd) attn_decode_kernel(Fa
       }
       if (!cur.valid) continue;
       const int hs = a.scale_heads == 1 ? 0 : cur.h;
-      const int n_cache = cache_tiles(cur), nt = item_tiles(cur);
+      const int n_cache = cache_tiles(cur, k), nt = item_tiles(cur, n_cache);
       // rows of the item's first position in the key/value and scale tensors
       const char *kt = nullptr, *vt = nullptr;
       int64_t srow = 0;
@@ -970,7 +1135,20 @@ __global__ void __launch_bounds__(kThreads, kWavesPerSimd) attn_decode_kernel(Fa
           return;
         }
       }
-      for (int ct = 0; ct < n_cache; ++ct) {
+      uint32_t live_bits = 0;  // masked: of the live tiles from live_next - 32 on, those still to be issued
+      int live_next = 0;
+      for (int nth = 0; nth < n_cache; ++nth) {
+        int ct = nth;
+        if (MASK && mapped(cur, k)) {
+          while (live_bits == 0) {  // (there are n_cache bits in all)
+            live_bits = static_cast<uint32_t>(lds_peek_uniform(reinterpret_cast<const int*>(&sm_live[k][live_next / 8])));
+            const int left = all_tiles(cur) - live_next;  // bytes past the item's end hold nothing
+            if (left < 32) live_bits &= (1u << left) - 1;
+            live_next += 32;
+          }
+          ct = live_next - 32 + __builtin_ctz(live_bits);
+          live_bits &= live_bits - 1;
+        }
         const int t0 = cur.start + ct * kTile;
         const int valid = min(kTile, cur.start + cur.count - t0);
         int64_t ts = srow;
@@ -990,6 +1168,11 @@ __global__ void __launch_bounds__(kThreads, kWavesPerSimd) attn_decode_kernel(Fa
           ts = static_cast<int64_t>(hs) * a.total_pages * a.page_size + in_pool;
         }
         const float* mk = MASK ? static_cast<const float*>(a.mask) + cur.slot * a.mask_stride_b + t0 : nullptr;
+        if (MASK) {
+          const int64_t in_item = static_cast<int64_t>(ct) * kTile;
+          if (!issue_tile(kt + in_item * C::kRowBytes, vt + in_item * C::kRowBytes, scale_lane + (srow + in_item) * kEs, mk, valid, false)) return;
+          continue;
+        }
         if (!issue_tile(kt, vt, scale_lane + ts * kEs, mk, valid, false)) return;
         if (!PAGED) {
           kt += kTile * C::kRowBytes;
@@ -1174,9 +1357,10 @@ __global__ void __launch_bounds__(kThreads, kWavesPerSimd) attn_decode_kernel(Fa
     // One body for every tile: what only the new token's tile or a chunk's last,
     // partly filled tile need sits behind wave-uniform branches, so that the
     // accumulators live in the same registers whichever way a tile goes.
-    const bool partial = valid != kTile;
     const int s = t % C::kSlots;
     if (!wait_for(&sm_filled[s], t / C::kSlots + 1)) return false;
+    if (MASK) valid = __builtin_amdgcn_readfirstlane(sm_valid[s]);  // which of the item's tiles it is, the producer knows
+    const bool partial = valid != kTile;
     char* slot = ring + s * C::kSlotBytes;
     const char* side = slot + 2 * C::kTileBytes;
     JPT_TL(if (tl_first == 0) tl_first = tl_now(); ++tl_tiles;)
@@ -1406,7 +1590,7 @@ __global__ void __launch_bounds__(kThreads, kWavesPerSimd) attn_decode_kernel(Fa
       cur = fetch(k);
     }
     if (!cur.valid) continue;
-    const int n_cache = cache_tiles(cur), nt = item_tiles(cur);
+    const int n_cache = cache_tiles(cur, k), nt = item_tiles(cur, n_cache);
     if (nt > 0) {
       // query rows: staged by the producer ahead of the item's first tile
       if (!wait_for(&sm_filled[base % C::kSlots], base / C::kSlots + 1)) return;
@@ -1453,7 +1637,7 @@ __global__ void __launch_bounds__(kThreads, kWavesPerSimd) attn_decode_kernel(Fa
     for (int ti = (wave + kConsumers - base % kConsumers) % kConsumers; ti < nt; ti += kConsumers) {
       if (wide_new && ti == 1 && nt - n_cache == 2) continue;  // read by the consumer of tile 0
       const bool is_new = ti < nt - n_cache;  // the new token comes first
-      const int valid = is_new ? 1 : min(kTile, cur.count - (ti - (nt - n_cache)) * kTile);
+      const int valid = is_new ? 1 : MASK ? kTile : min(kTile, cur.count - (ti - (nt - n_cache)) * kTile);  // masked: see consume_tile
       if (!consume_tile(base + ti, valid, is_new)) return;
     }
     if (keep) {  // this consumer had the new token's tile

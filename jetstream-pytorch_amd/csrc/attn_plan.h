@@ -48,6 +48,14 @@ struct FastParams {
   int32_t total_items;  // max_entries * kv_heads
   int32_t* status;      // the workspace's state block (kState* words)
   void *stash_k, *stash_v;  // NULL, or where a given bf16 token's rows are left too: (batch, kv_heads, 128)
+  // Masked calls without a new token: NULL, or the step's bf16 rows (batch, kv_heads, 128), which the launch writes to
+  // position line_pos[slot] of their slots (line_pos[0] with a line_count of 1) - int8 caches: quantised, with their
+  // scales, the key rotated first where there are factors - before it attends the cache; a position outside the cache is
+  // no line.
+  const void *line_k, *line_v;
+  const int32_t* line_pos;
+  const float* line_rope;
+  int32_t line_count, line_rounding;
 };
 
 // How the step's new token reaches the streaming kernel (a template argument of it).

@@ -10,8 +10,7 @@
 //
 // Every function takes the ordinary case (device tensors, contiguous, of the dtypes the library has)
 // and returns None for anything else: the Python code then goes the long way, which converts what can
-// be converted and raises the errors the package documents.  Nothing has been done then, but that
-// eager_step may have written the token's line, which the long way writes again.
+// be converted and raises the errors the package documents.  Nothing has been done then.
 #include <torch/csrc/Exceptions.h>
 #include <torch/csrc/autograd/python_variable.h>
 
@@ -37,8 +36,9 @@ struct Library {
   int32_t (*plan[2])(const jpt_attn_args*, int32_t, void*);  // again, on a fresh workspace
   AttnFn attn[3];  // ragged, dense, paged
   int32_t (*scatter_lines)(const jpt_line_tensor*, int32_t, const int32_t*, int32_t, int32_t, int32_t, int32_t, void*);
+  int32_t (*dense_line)(const jpt_attn_args*, const void*, const void*, const int32_t*, int32_t, void*);
+  int32_t (*dense_append)(const jpt_attn_args*, const jpt_quant_append_args*, void*);
   int32_t (*ragged_stash)(const jpt_attn_args*, void*, void*, void*);
-  int32_t (*append_quant)(const jpt_quant_append_args*, void*);
   int32_t (*insert_layers)(const jpt_prefill_insert_args*, const jpt_insert_layer*, int32_t, void*);
   int32_t (*insert_state)(void*, int32_t, int64_t, int32_t*, int32_t*, int32_t*, int32_t, int32_t, int32_t, int32_t, int32_t, int32_t,
                           int32_t, void*);
@@ -151,6 +151,14 @@ struct Token {
   void *stash_k = nullptr, *stash_v = nullptr;  // bf16 rows: where they are left too (kRagged)
 };
 
+// The step's line, which the call writes before it attends the cache (kDense).
+struct Line {
+  const void *k = nullptr, *v = nullptr;
+  const int32_t* pos = nullptr;
+  int32_t count = 0;
+  const jpt_quant_append_args* quantised = nullptr;  // int8 caches: all of it
+};
+
 struct Attended {
   Tensor out, max, denom;
 };
@@ -158,7 +166,7 @@ struct Attended {
 // attention_kernel._attend.  keys / values may be stacks of layers.
 Attended attend(Mode mode, const Tensor& q, const Tensor& keys, const Tensor& values, int64_t layer, const Tensor* lengths,
                 const Tensor* table, const Tensor* mask, const Tensor* k_scaler, const Tensor* v_scaler, std::optional<double> sm_scale,
-                const Token* token, bool stats, PyObject* plan) {
+                const Token* token, bool stats, PyObject* plan, const Line* line = nullptr) {
   need(q.dim() == 4);
   const int64_t b = q.size(0), hq = q.size(1), t = q.size(2), d = q.size(3);
   const Layer k(keys, 4, layer), v(values, 4, layer);
@@ -305,7 +313,9 @@ Attended attend(Mode mode, const Tensor& q, const Tensor& keys, const Tensor& va
     }
     if (a.workspace == nullptr) use_from(shared_workspace, lib.workspace_bytes(&a));
   }
-  if (token != nullptr && token->stash_k != nullptr) check(unlocked(lib.ragged_stash, &a, token->stash_k, token->stash_v, stream()));
+  if (line != nullptr && line->quantised != nullptr) check(unlocked(lib.dense_append, &a, line->quantised, stream()));
+  else if (line != nullptr) check(unlocked(lib.dense_line, &a, line->k, line->v, line->pos, line->count, stream()));
+  else if (token != nullptr && token->stash_k != nullptr) check(unlocked(lib.ragged_stash, &a, token->stash_k, token->stash_v, stream()));
   else check(unlocked(lib.attn[mode], &a, stream()));
   return r;
 }
@@ -481,17 +491,14 @@ PyObject* py_eager_step(PyObject*, PyObject* const* x, Py_ssize_t n) {
       a.scale_heads = static_cast<int32_t>(ks->size(1));
       a.rounding = static_cast<int32_t>(whole(x[10]));
       a.rope = rope_of(opt(x[11]), b, d);
-      check(unlocked(lib.append_quant, &a, stream()));
-    } else {
-      need(ks == nullptr && x[11] == Py_None);
-      given_token(line, xk, xv, b, hkv, d, code);
-      const int32_t bytes = static_cast<int32_t>(d * element_bytes(code)), heads = static_cast<int32_t>(hkv);
-      jpt_line_tensor t[2]{};
-      t[0].dst = ck.data_ptr(); t[0].src = line.k; t[0].heads = heads; t[0].row_bytes = bytes;
-      t[1].dst = cv.data_ptr(); t[1].src = line.v; t[1].heads = heads; t[1].row_bytes = bytes;
-      check(unlocked(lib.scatter_lines, t, 2, at, count, 1, static_cast<int32_t>(b), static_cast<int32_t>(seq), stream()));
+      Line quantised;
+      quantised.quantised = &a;
+      return wrap(attend(kDense, q, ck, cv, -1, nullptr, nullptr, mask, ks, vs, std::nullopt, nullptr, false, nullptr, &quantised).out);
     }
-    return wrap(attend(kDense, q, ck, cv, -1, nullptr, nullptr, mask, ks, vs, std::nullopt, nullptr, false, nullptr).out);
+    need(ks == nullptr && x[11] == Py_None);
+    given_token(line, xk, xv, b, hkv, d, code);
+    const Line rows{line.k, line.v, at, count};
+    return wrap(attend(kDense, q, ck, cv, -1, nullptr, nullptr, mask, ks, vs, std::nullopt, nullptr, false, nullptr, &rows).out);
   });
 }
 
@@ -745,8 +752,9 @@ PyObject* py_bind(PyObject*, PyObject* args) {
   lib.attn[kDense] = reinterpret_cast<AttnFn>(get("jpt_attn_dense"));
   lib.attn[kPaged] = reinterpret_cast<AttnFn>(get("jpt_attn_paged"));
   lib.scatter_lines = reinterpret_cast<decltype(lib.scatter_lines)>(get("jpt_kv_scatter_lines"));
+  lib.dense_line = reinterpret_cast<decltype(lib.dense_line)>(get("jpt_attn_dense_line"));
+  lib.dense_append = reinterpret_cast<decltype(lib.dense_append)>(get("jpt_attn_dense_append"));
   lib.ragged_stash = reinterpret_cast<decltype(lib.ragged_stash)>(get("jpt_attn_ragged_stash"));
-  lib.append_quant = reinterpret_cast<decltype(lib.append_quant)>(get("jpt_kv_append_quant_i8"));
   lib.plan[0] = reinterpret_cast<int32_t (*)(const jpt_attn_args*, int32_t, void*)>(get("jpt_attn_plan"));
   lib.plan[1] = reinterpret_cast<int32_t (*)(const jpt_attn_args*, int32_t, void*)>(get("jpt_attn_plan_fresh"));
   lib.insert_state = reinterpret_cast<decltype(lib.insert_state)>(get("jpt_insert_state"));

@@ -143,6 +143,8 @@ _sig("jpt_attn_kernel", _i32, _c.POINTER(AttnArgs), _i32)
 _sig("jpt_attn_plan", _i32, _c.POINTER(AttnArgs), _i32, _vp)
 _sig("jpt_attn_plan_fresh", _i32, _c.POINTER(AttnArgs), _i32, _vp)
 _sig("jpt_attn_ragged", _i32, _c.POINTER(AttnArgs), _vp)
+_sig("jpt_attn_dense_line", _i32, _c.POINTER(AttnArgs), _vp, _vp, _vp, _i32, _vp)
+_sig("jpt_attn_dense_append", _i32, _c.POINTER(AttnArgs), _c.POINTER(QuantAppendArgs), _vp)
 _sig("jpt_attn_ragged_stash", _i32, _c.POINTER(AttnArgs), _vp, _vp, _vp)
 _sig("jpt_attn_dense", _i32, _c.POINTER(AttnArgs), _vp)
 _sig("jpt_attn_paged", _i32, _c.POINTER(AttnArgs), _vp)
@@ -178,7 +180,7 @@ EXPORTS = (
     "jpt_dpam_free", "jpt_dpam_decode_step", "jpt_decode_advance", "jpt_rope",
     "jpt_ragged_block_indices", "jpt_prefill_insert_layers", "jpt_prefill_insert_prompts",
     "jpt_attn_status", "jpt_attn_ragged_static", "jpt_attn_plan_fresh", "jpt_kv_stash_lines", "jpt_insert_state",
-    "jpt_attn_ragged_stash", "jpt_attn_kernel",
+    "jpt_attn_ragged_stash", "jpt_attn_kernel", "jpt_attn_dense_line", "jpt_attn_dense_append",
 )
 
 

@@ -114,7 +114,7 @@ class AttentionKernel:
     attention, the eagerly written cache under a mask, pages with the device
     allocator.  None where the call is anything else - another attention put in the
     kernel's place for one, too: it then goes the general way below, launch by
-    launch, which writes the token's line again if that was written already."""
+    launch."""
     env = self.env
     kind = type(cache)
     int8 = isinstance(self, Int8KVAttentionKernel)
