@@ -2,18 +2,40 @@
 // into one slot of a dense cache (with ring wrap) or into the slot's pages,
 // either copied or quantised per token to int8 with the insert quantiser.
 //
-// One workgroup per (token, K|V).  HBM-bound data movement: reads the prompt
-// once (the quantising pass re-reads it from cache), writes codes and scales.
+// HBM-bound data movement: the prompt is read once, codes (or rows) and scales
+// are written.  Rows of whole, aligned 16-byte pieces are copied by
+// prefill_copy_kernel and, from bf16, quantised by prefill_insert_rows_kernel;
+// any other dtype, shape or alignment takes prefill_insert_kernel.
 #include "common.h"
 
 namespace jpt {
 namespace {
+
+constexpr int kPieces = 4;
+// How a workgroup's threads are laid out: heads x tokens x 2^lanes_log lanes of a row, `passes` heads a thread.
+struct RowSplit {
+  int lanes_log, tokens_log, passes;
+};
+// False: the shape is not taken (a row is a power of two of pieces up to 64, a token's pieces four a thread).
+bool split_rows(int heads, int dim, RowSplit* s) {
+  const int lanes = dim / 8;
+  if (dim < 8 || dim % 8 != 0 || lanes > 64 || (lanes & (lanes - 1)) != 0 || heads < 1 || heads * lanes > 256 * kPieces) return false;
+  s->lanes_log = 0;
+  while ((1 << s->lanes_log) < lanes) ++s->lanes_log;
+  // as many tokens as leave a thread four heads: long runs of one head
+  for (s->tokens_log = 8 - s->lanes_log;; --s->tokens_log) {
+    const int heads_a_pass = 256 >> (s->tokens_log + s->lanes_log);
+    s->passes = (heads + heads_a_pass - 1) / heads_a_pass;
+    if (s->passes <= kPieces) return true;
+  }
+}
 
 // Layers that are tensors of their own (no common stride) come as a table of
 // pointers inside the kernel arguments.
 constexpr int kTableLayers = 64;
 struct InsertParams {
   jpt_prefill_insert_args a;
+  RowSplit split;  // of the rows kernel
   int32_t use_table;
   const void* src_k[kTableLayers];
   const void* src_v[kTableLayers];
@@ -59,7 +81,7 @@ __device__ __forceinline__ void load4(const void* src, int64_t i, int dtype, flo
   }
 }
 
-// dim % 4 == 0.  The op order of the quantiser is that of
+// A workgroup a (token, K|V, layer).  dim % 4 == 0.  The op order of the quantiser is that of
 // jpt_kv_append_quant_i8 (each op rounded to the scale dtype):
 //   trunc: a = absmax; s = a / 127;             q = x / s;      code = trunc(q)
 //   rne:   a = max(absmax, eps); s = a / 127; r = 1 / s; q = x * r;
@@ -175,150 +197,37 @@ __global__ void __launch_bounds__(256) prefill_insert_kernel(InsertParams p) {
   if (threadIdx.x < groups) store_from_f32(scale_out, scale_index(threadIdx.x), a.scale_dtype, s_scale[threadIdx.x]);
 }
 
-// The common quantising shape - bf16 prompt, heads * dim == 1024 - eight tokens
-// a workgroup, two at a time: 128 threads a token, each keeping its eight
-// elements (one 16-byte load) of four tokens in registers between the absmax
-// pass and the quantise pass, so the prompt is read once, in wide loads that
-// are all issued before the first wait.  Same op order as the general kernel.
-constexpr int kTokensPerBlock = 8;
-// Tokens t0 .. t0 + 7 of the prompt `a` describes (tokens, page_ids, n_pages,
+// bf16 prompts quantised, laid out for memory: a workgroup takes a few consecutive tokens in all heads.  A thread keeps
+// one 16-byte piece of one token's row in up to four heads, so that the lanes of a wave read consecutive rows of one head
+// (1 KiB in one piece at 128 elements a row and four tokens or more) and write contiguous codes, the token's position or
+// page is worked out once, and the prompt is read once: the pieces stay in registers, all asked for before the first wait,
+// between the absmax pass and the quantise pass.  A token's absmax: over the lanes that share its row, then (one scale a
+// token) over the thread's heads and, in LDS, the waves that have the others.  Same op order as the general kernel.
+// Measured, 16 layers into a slot, heads x dim, tokens; prefill_insert_kernel -> this, us a call: 32x128, 1000: 154.5 -> 75
+// (5.2 TB/s read and written); 16x256, 700: 123 -> 68; 8x256, 1200: 106 -> 45; 4x128, 1500: 70.6 -> 23.5; 8x64, 1000: 50
+// -> 18; 1x128, 900: 35.5 -> 9.4.
+// The `block`-th workgroup's tokens of the prompt `a` describes (tokens, page_ids, n_pages,
 // src_head_stride), read from src, written to dst / scale_out.
-template <bool BF16_MATH>
-__device__ __forceinline__ void quant_insert_tokens(const jpt_prefill_insert_args& a, const uint16_t* src, char* dst,
-                                                    void* scale_out, int t0) {
-  constexpr int kPasses = kTokensPerBlock / 2;
-  const int half = threadIdx.x >> 7;  // which of the pass's two tokens
-  const bool paged = a.page_ids != nullptr;
-  const int H = a.heads, D = a.dim;
-  const int rows = paged ? a.n_pages * a.page_size : a.tokens;
-  const int i0 = 8 * (threadIdx.x & 127), h = i0 / D, d = i0 - h * D;
-  const int groups = a.scale_heads;
-  const int64_t head_stride = a.src_head_stride > 0 ? a.src_head_stride : static_cast<int64_t>(a.tokens) * D;
-
-  // every load of the workgroup before anything waits for one (addresses
-  // clamped into the prompt, results masked afterwards); page ids likewise
-  uint4 raw[kPasses];
-#pragma unroll
-  for (int j = 0; j < kPasses; ++j) {
-    const int t = min(t0 + 2 * j + half, a.tokens - 1);
-    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-    const u32x4 w = __builtin_nontemporal_load(
-        reinterpret_cast<const u32x4*>(src + h * head_stride + static_cast<int64_t>(t) * D + d));  // read once
-    raw[j] = make_uint4(w.x, w.y, w.z, w.w);
-  }
-  int page_of[kPasses];
-#pragma unroll
-  for (int j = 0; j < kPasses; ++j)
-    page_of[j] = paged ? a.page_ids[min(t0 + 2 * j + half, rows - 1) / a.page_size] : 0;
-  float x[kPasses][8], m[kPasses];
-  int64_t pool_row[kPasses];  // dense: position in the slot's row; paged: row in the pool; -1: nothing to write
-#pragma unroll
-  for (int j = 0; j < kPasses; ++j) {
-    const int t = t0 + 2 * j + half;
-    pool_row[j] = -1;
-    if (t < rows) {
-      if (paged) {
-        const int page = page_of[j];
-        if (page >= 0 && page < a.total_pages) pool_row[j] = static_cast<int64_t>(page) * a.page_size + t % a.page_size;
-      } else {
-        const int at = (a.start + t) % a.seq;
-        pool_row[j] = at < 0 ? at + a.seq : at;
-      }
-    }
-    const bool live = t < a.tokens;
-    const uint32_t w[4] = {raw[j].x, raw[j].y, raw[j].z, raw[j].w};
-    m[j] = 0.f;
-#pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      x[j][2 * i] = live ? __uint_as_float(w[i] << 16) : 0.f;
-      x[j][2 * i + 1] = live ? __uint_as_float(w[i] & 0xffff0000u) : 0.f;
-      m[j] = fmaxf(m[j], fmaxf(fabsf(x[j][2 * i]), fabsf(x[j][2 * i + 1])));
-    }
-  }
-  __shared__ float s_red[kPasses][4];
-  if (groups == 1) {
-#pragma unroll
-    for (int j = 0; j < kPasses; ++j) {
-      for (int off = 32; off > 0; off >>= 1) m[j] = fmaxf(m[j], __shfl_xor(m[j], off));
-      if ((threadIdx.x & 63) == 0) s_red[j][threadIdx.x >> 6] = m[j];
-    }
-    __syncthreads();
-#pragma unroll
-    for (int j = 0; j < kPasses; ++j) m[j] = fmaxf(s_red[j][2 * half], s_red[j][2 * half + 1]);
-  } else {
-    // a head's D / 8 threads are consecutive; D / 8 is a power of two <= 64
-#pragma unroll
-    for (int j = 0; j < kPasses; ++j)
-      for (int off = D / 16; off > 0; off >>= 1) m[j] = fmaxf(m[j], __shfl_xor(m[j], off));
-  }
-#pragma unroll
-  for (int j = 0; j < kPasses; ++j) {
-    if (pool_row[j] < 0) continue;
-    const int64_t row = paged ? static_cast<int64_t>(h) * a.total_pages * a.page_size + pool_row[j]
-                              : (static_cast<int64_t>(a.slot) * H + h) * a.seq + pool_row[j];
-    uint2* out = reinterpret_cast<uint2*>(dst + row * D + d);
-    if (t0 + 2 * j + half >= a.tokens) {  // paged only: the tail of the last page is zero-filled
-      *out = make_uint2(0u, 0u);
-      continue;
-    }
-    float amax = m[j];
-    if (a.rounding == JPT_ROUND_RNE) amax = fmaxf(amax, rnd<BF16_MATH>(1e-5f));
-    const float s = rnd<BF16_MATH>(amax / 127.0f);
-    uint32_t code[8];
-    if (a.rounding == JPT_ROUND_TRUNC) {
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const float q = rnd<BF16_MATH>(x[j][i] / s);
-        code[i] = static_cast<uint32_t>((q != q) ? 0 : static_cast<int>(q)) & 0xffu;
-      }
-    } else {
-      const float r = rnd<BF16_MATH>(1.0f / s);
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const float q = rnd<BF16_MATH>(x[j][i] * r);
-        code[i] = static_cast<uint32_t>(static_cast<int>(fminf(fmaxf(rintf(q), -128.f), 127.f))) & 0xffu;
-      }
-    }
-    // written once, read by later launches only: keep it out of the way of the prompt being read
-    typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
-    const u32x2 packed = {code[0] | (code[1] << 8) | (code[2] << 16) | (code[3] << 24),
-                          code[4] | (code[5] << 8) | (code[6] << 16) | (code[7] << 24)};
-    __builtin_nontemporal_store(packed, reinterpret_cast<u32x2*>(out));
-    if (groups == 1 ? (threadIdx.x & 127) == 0 : d == 0) {
-      const int g = groups == 1 ? 0 : h;
-      const int64_t idx = paged ? static_cast<int64_t>(g) * a.total_pages * a.page_size + pool_row[j]
-                                : (static_cast<int64_t>(a.slot) * groups + g) * a.seq + pool_row[j];
-      store_from_f32(scale_out, idx, a.scale_dtype, s);
-    }
-  }
-}
-
-// The same for the Llama shape, 8 heads of 128 elements, laid out for memory: a
-// thread keeps one 16-byte piece of one token's row in four heads (passes), so
-// that the 64 lanes of a wave read four consecutive tokens' rows of one head -
-// 1 KiB in one piece - and write 512 contiguous bytes of codes, where the
-// mapping above touches four heads' 256 bytes.  A token's absmax: over the
-// thread's four heads, the 16 lanes that share the token, and (one scale a
-// token) the workgroup's other half, which has the other four heads.
-template <bool BF16_MATH>
-__device__ __forceinline__ void quant_insert_tokens_8x128(const jpt_prefill_insert_args& a, const uint16_t* src, char* dst,
-                                                          void* scale_out, int t0) {
-  constexpr int H = 8, D = 128, kHeadsPerThread = 4;
-  const int piece = threadIdx.x & 15, tq = (threadIdx.x >> 4) & 7, hg = threadIdx.x >> 7;
+template <bool BF16_MATH, int PASSES>
+__device__ __forceinline__ void quant_insert_rows(const jpt_prefill_insert_args& a, const RowSplit split, const int H, const int D,
+                                                  const uint16_t* src, char* dst, void* scale_out, int block) {
+  typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+  typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+  const int lanes = 1 << split.lanes_log, tokens = 1 << split.tokens_log;
   const bool paged = a.page_ids != nullptr;
   const int rows = paged ? a.n_pages * a.page_size : a.tokens;
   const int groups = a.scale_heads;
   const int64_t head_stride = a.src_head_stride > 0 ? a.src_head_stride : static_cast<int64_t>(a.tokens) * D;
-  const int t = t0 + tq, d = 8 * piece;
-  const int t_src = min(t, a.tokens - 1);
-  uint4 raw[kHeadsPerThread];
+  const int piece = threadIdx.x & (lanes - 1), tq = (threadIdx.x >> split.lanes_log) & (tokens - 1);
+  const int h0 = (threadIdx.x >> (split.lanes_log + split.tokens_log)) * PASSES;  // the thread's heads: h0 .. h0 + PASSES - 1
+  const int t = block * tokens + tq, d = 8 * piece;
+
+  // addresses clamped into the prompt, results masked afterwards
+  const uint16_t* const from = src + static_cast<int64_t>(min(t, a.tokens - 1)) * D + d;
+  u32x4 raw[PASSES];
 #pragma unroll
-  for (int j = 0; j < kHeadsPerThread; ++j) {
-    typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
-    const u32x4 w = __builtin_nontemporal_load(
-        reinterpret_cast<const u32x4*>(src + (hg * kHeadsPerThread + j) * head_stride + static_cast<int64_t>(t_src) * D + d));
-    raw[j] = make_uint4(w.x, w.y, w.z, w.w);
-  }
+  for (int j = 0; j < PASSES; ++j)
+    raw[j] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(from + min(h0 + j, H - 1) * head_stride));  // read once
   const int page = paged ? a.page_ids[min(t, rows - 1) / a.page_size] : 0;
   int64_t pool_row = -1;  // dense: position in the slot's row; paged: row in the pool; -1: nothing to write
   if (t < rows) {
@@ -329,83 +238,138 @@ __device__ __forceinline__ void quant_insert_tokens_8x128(const jpt_prefill_inse
       pool_row = at < 0 ? at + a.seq : at;
     }
   }
-  const bool live = t < a.tokens;
-  float x[kHeadsPerThread][8], m[kHeadsPerThread];
+  float m[PASSES];
 #pragma unroll
-  for (int j = 0; j < kHeadsPerThread; ++j) {
-    const uint32_t w[4] = {raw[j].x, raw[j].y, raw[j].z, raw[j].w};
+  for (int j = 0; j < PASSES; ++j) {
     m[j] = 0.f;
 #pragma unroll
-    for (int i = 0; i < 4; ++i) {
-      x[j][2 * i] = live ? __uint_as_float(w[i] << 16) : 0.f;
-      x[j][2 * i + 1] = live ? __uint_as_float(w[i] & 0xffff0000u) : 0.f;
-      m[j] = fmaxf(m[j], fmaxf(fabsf(x[j][2 * i]), fabsf(x[j][2 * i + 1])));
-    }
-    for (int off = 8; off > 0; off >>= 1) m[j] = fmaxf(m[j], __shfl_xor(m[j], off));  // the head's 16 pieces
+    for (int i = 0; i < 4; ++i)
+      m[j] = fmaxf(m[j], fmaxf(fabsf(__uint_as_float(raw[j][i] << 16)), fabsf(__uint_as_float(raw[j][i] & 0xffff0000u))));
   }
-  __shared__ float s_half[2][kTokensPerBlock];
+  __shared__ float s_max[256];  // by (the threads' heads, token)
   if (groups == 1) {
-    const float mine = fmaxf(fmaxf(m[0], m[1]), fmaxf(m[2], m[3]));
-    if (piece == 0) s_half[hg][tq] = mine;
-    __syncthreads();
-    const float all = fmaxf(s_half[0][tq], s_half[1][tq]);
+    // (a head clamped above is one that counts anyway)
 #pragma unroll
-    for (int j = 0; j < kHeadsPerThread; ++j) m[j] = all;
+    for (int j = 1; j < PASSES; ++j) m[0] = fmaxf(m[0], m[j]);
+    for (int off = lanes / 2; off > 0; off >>= 1) m[0] = fmaxf(m[0], __shfl_xor(m[0], off));
+    if (piece == 0) s_max[threadIdx.x >> split.lanes_log] = m[0];
+    __syncthreads();
+    for (int i = tq; i < (256 >> split.lanes_log); i += tokens) m[0] = fmaxf(m[0], s_max[i]);
+#pragma unroll
+    for (int j = 1; j < PASSES; ++j) m[j] = m[0];
+  } else {
+#pragma unroll
+    for (int j = 0; j < PASSES; ++j)
+      for (int off = lanes / 2; off > 0; off >>= 1) m[j] = fmaxf(m[j], __shfl_xor(m[j], off));
   }
   if (pool_row < 0) return;
+  const int64_t head_rows = paged ? static_cast<int64_t>(a.total_pages) * a.page_size : a.seq;
+  const int64_t row0 = (paged ? 0 : static_cast<int64_t>(a.slot) * H * a.seq) + pool_row;
 #pragma unroll
-  for (int j = 0; j < kHeadsPerThread; ++j) {
-    const int h = hg * kHeadsPerThread + j;
-    const int64_t row = paged ? static_cast<int64_t>(h) * a.total_pages * a.page_size + pool_row
-                              : (static_cast<int64_t>(a.slot) * H + h) * a.seq + pool_row;
-    uint2* out = reinterpret_cast<uint2*>(dst + row * D + d);
-    if (!live) {  // paged only: the tail of the last page is zero-filled
-      *out = make_uint2(0u, 0u);
+  for (int j = 0; j < PASSES; ++j) {
+    const int h = h0 + j;
+    if (h >= H) break;
+    u32x2* out = reinterpret_cast<u32x2*>(dst + (row0 + h * head_rows) * D + d);
+    if (t >= a.tokens) {  // paged only: the tail of the last page is zero-filled
+      *out = u32x2{0u, 0u};
       continue;
     }
     float amax = m[j];
     if (a.rounding == JPT_ROUND_RNE) amax = fmaxf(amax, rnd<BF16_MATH>(1e-5f));
     const float s = rnd<BF16_MATH>(amax / 127.0f);
     uint32_t code[8];
-    if (a.rounding == JPT_ROUND_TRUNC) {
+    const float inv = a.rounding == JPT_ROUND_TRUNC ? 0.f : rnd<BF16_MATH>(1.0f / s);
 #pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const float q = rnd<BF16_MATH>(x[j][i] / s);
+    for (int i = 0; i < 8; ++i) {
+      const float x = __uint_as_float((i & 1) ? raw[j][i / 2] & 0xffff0000u : raw[j][i / 2] << 16);
+      if (a.rounding == JPT_ROUND_TRUNC) {
+        const float q = rnd<BF16_MATH>(x / s);
         code[i] = static_cast<uint32_t>((q != q) ? 0 : static_cast<int>(q)) & 0xffu;
-      }
-    } else {
-      const float r = rnd<BF16_MATH>(1.0f / s);
-#pragma unroll
-      for (int i = 0; i < 8; ++i) {
-        const float q = rnd<BF16_MATH>(x[j][i] * r);
+      } else {
+        const float q = rnd<BF16_MATH>(x * inv);
         code[i] = static_cast<uint32_t>(static_cast<int>(fminf(fmaxf(rintf(q), -128.f), 127.f))) & 0xffu;
       }
     }
-    typedef uint32_t u32x2 __attribute__((ext_vector_type(2)));
+    // written once, read by later launches only: keep it out of the way of the prompt being read
     const u32x2 packed = {code[0] | (code[1] << 8) | (code[2] << 16) | (code[3] << 24),
                           code[4] | (code[5] << 8) | (code[6] << 16) | (code[7] << 24)};
-    __builtin_nontemporal_store(packed, reinterpret_cast<u32x2*>(out));
-    if (piece == 0 && (groups == 1 ? (hg == 0 && j == 0) : true)) {
-      const int g = groups == 1 ? 0 : h;
-      const int64_t idx = paged ? static_cast<int64_t>(g) * a.total_pages * a.page_size + pool_row
-                                : (static_cast<int64_t>(a.slot) * groups + g) * a.seq + pool_row;
+    __builtin_nontemporal_store(packed, out);
+    if (d == 0 && (groups != 1 || h == 0)) {
+      const int64_t idx = (paged ? 0 : static_cast<int64_t>(a.slot) * groups * a.seq) + (groups == 1 ? 0 : h) * head_rows + pool_row;
       store_from_f32(scale_out, idx, a.scale_dtype, s);
     }
   }
 }
 
-template <bool BF16_MATH>
-__global__ void __launch_bounds__(256) prefill_insert_quant4_kernel(InsertParams p) {
+// LLAMA: 8 heads of 128 elements.  Numbers that the compiler knows, in a kernel of their own:
+// 1500 tokens, 16 layers 50.6 us a call, 52.8 through the other branch.
+template <bool BF16_MATH, bool LLAMA>
+__device__ __forceinline__ void quant_insert_block(const jpt_prefill_insert_args& a, const RowSplit& split, const uint16_t* src,
+                                                   char* dst, void* scale_out, int block) {
+  if constexpr (LLAMA) {
+    quant_insert_rows<BF16_MATH, 4>(a, RowSplit{4, 3, 4}, 8, 128, src, dst, scale_out, block);
+  } else {
+    if (split.passes == 4) quant_insert_rows<BF16_MATH, 4>(a, split, a.heads, a.dim, src, dst, scale_out, block);
+    else if (split.passes == 3) quant_insert_rows<BF16_MATH, 3>(a, split, a.heads, a.dim, src, dst, scale_out, block);
+    else if (split.passes == 2) quant_insert_rows<BF16_MATH, 2>(a, split, a.heads, a.dim, src, dst, scale_out, block);
+    else quant_insert_rows<BF16_MATH, 1>(a, split, a.heads, a.dim, src, dst, scale_out, block);
+  }
+}
+
+template <bool BF16_MATH, bool LLAMA>
+__global__ void __launch_bounds__(256) prefill_insert_rows_kernel(InsertParams p) {
   const jpt_prefill_insert_args& a = p.a;
   const bool is_v = blockIdx.y == 1;
   const void* src;
   char* dst;
   void* scale_out;
   layer_tensors(p, blockIdx.z, is_v, 2, 1, a.scale_dtype == JPT_F32 ? 4 : 2, &src, &dst, &scale_out);
-  if (a.heads == 8 && a.dim == 128)
-    quant_insert_tokens_8x128<BF16_MATH>(a, static_cast<const uint16_t*>(src), dst, scale_out, blockIdx.x * kTokensPerBlock);
-  else
-    quant_insert_tokens<BF16_MATH>(a, static_cast<const uint16_t*>(src), dst, scale_out, blockIdx.x * kTokensPerBlock);
+  quant_insert_block<BF16_MATH, LLAMA>(a, p.split, static_cast<const uint16_t*>(src), dst, scale_out, blockIdx.x);
+}
+
+// Rows copied as they are, 16 bytes a piece: a workgroup takes 1024 consecutive pieces of one head's rows (16 KiB: 64
+// rows of 128 bf16), four a thread, asked for before the first is written.  The ordinary kernel
+// moves 2 KiB a workgroup with one load in flight a thread.  Measured, 16 layers of bf16 rows, us a call, before -> now:
+// pages of 64, 8x128, 1500 tokens 75 -> 56; pages of 32, 8x128, 4000 tokens 158 -> 113 (4.6 TB/s); 1x128, 2000 tokens 69
+// -> 23; 32x128, 1500 tokens 166 -> 165 (4.8 TB/s before, too); a slot, 8x128, 1000 tokens 34.5 -> 27.
+__global__ void __launch_bounds__(256) prefill_copy_kernel(InsertParams p, int esz, int pieces_a_row) {
+  typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
+  const jpt_prefill_insert_args& a = p.a;
+  const int h = blockIdx.y >> 1;
+  const void* src;
+  char* dst;
+  void* scale;
+  layer_tensors(p, blockIdx.z, blockIdx.y & 1, esz, esz, 0, &src, &dst, &scale);
+  const bool paged = a.page_ids != nullptr;
+  const int rows = paged ? a.n_pages * a.page_size : a.tokens;
+  const int64_t row_bytes = 16ll * pieces_a_row;
+  const int64_t head_bytes = a.src_head_stride > 0 ? a.src_head_stride * esz : a.tokens * row_bytes;
+  const char* const from = static_cast<const char*>(src) + h * head_bytes;
+  u32x4 x[kPieces];
+  int t[kPieces], off[kPieces], page[kPieces];
+#pragma unroll
+  for (int j = 0; j < kPieces; ++j) {
+    const int i = (static_cast<int>(blockIdx.x) * kPieces + j) * 256 + static_cast<int>(threadIdx.x);
+    t[j] = i / pieces_a_row;
+    off[j] = 16 * (i - t[j] * pieces_a_row);
+    // pieces of the zero-filled tail, and past it, read nothing
+    x[j] = u32x4{0u, 0u, 0u, 0u};
+    if (t[j] < a.tokens) x[j] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(from + t[j] * row_bytes + off[j]));
+  }
+#pragma unroll
+  for (int j = 0; j < kPieces; ++j) page[j] = paged ? a.page_ids[min(t[j], rows - 1) / a.page_size] : 0;
+#pragma unroll
+  for (int j = 0; j < kPieces; ++j) {
+    if (t[j] >= rows || (paged && (page[j] < 0 || page[j] >= a.total_pages))) continue;
+    int64_t row;
+    if (paged) {
+      row = (static_cast<int64_t>(h) * a.total_pages + page[j]) * a.page_size + t[j] % a.page_size;
+    } else {
+      const int at = (a.start + t[j]) % a.seq;
+      row = (static_cast<int64_t>(a.slot) * a.heads + h) * a.seq + (at < 0 ? at + a.seq : at);
+    }
+    __builtin_nontemporal_store(x[j], reinterpret_cast<u32x4*>(dst + row * row_bytes + off[j]));
+  }
 }
 
 // Several prompts into the pages of one stacked pool in one launch: the
@@ -413,13 +377,14 @@ __global__ void __launch_bounds__(256) prefill_insert_quant4_kernel(InsertParams
 // first_block[r] on), layers along z by the layer strides.
 constexpr int kLaunchPrompts = 32;
 struct PromptsParams {
+  RowSplit split;
   jpt_prefill_insert_args a;  // destination, geometry, dtypes; its source and page fields are unused
   int32_t n_prompts;
   int32_t first_block[kLaunchPrompts + 1];
   jpt_insert_prompt prompt[kLaunchPrompts];
 };
 
-template <bool BF16_MATH>
+template <bool BF16_MATH, bool LLAMA>
 __global__ void __launch_bounds__(256) prefill_insert_prompts_kernel(PromptsParams p) {
   int r = 0;
   while (r + 1 < p.n_prompts && static_cast<int>(blockIdx.x) >= p.first_block[r + 1]) ++r;
@@ -435,9 +400,7 @@ __global__ void __launch_bounds__(256) prefill_insert_prompts_kernel(PromptsPara
   char* dst = static_cast<char*>(is_v ? a.dst_v : a.dst_k) + layer * a.dst_layer_stride;
   const int esz_scale = a.scale_dtype == JPT_F32 ? 4 : 2;
   void* scale_out = static_cast<char*>(is_v ? a.v_scale : a.k_scale) + layer * a.scale_layer_stride * esz_scale;
-  const int t0 = (static_cast<int>(blockIdx.x) - p.first_block[r]) * kTokensPerBlock;
-  if (a.heads == 8 && a.dim == 128) quant_insert_tokens_8x128<BF16_MATH>(a, src, dst, scale_out, t0);
-  else quant_insert_tokens<BF16_MATH>(a, src, dst, scale_out, t0);
+  quant_insert_block<BF16_MATH, LLAMA>(a, p.split, src, dst, scale_out, static_cast<int>(blockIdx.x) - p.first_block[r]);
 }
 
 }  // namespace
@@ -466,7 +429,7 @@ int32_t insert_launch(const jpt_prefill_insert_args& a, const jpt_insert_layer* 
   }
   InsertParams p{};
   p.a = a;
-  bool wide_ok = true;  // every tensor is aligned for the wide quantising kernel
+  bool wide_ok = true, pieces_ok = true;  // every tensor is aligned for the wide quantising kernel, for 16-byte copies
   auto check_layer = [&](const void* sk, const void* sv, const void* dk, const void* dv, const void* ks,
                          const void* vs) -> int32_t {
     JPT_REQUIRE(sk && sv && dk && dv, "NULL tensor argument");
@@ -474,6 +437,7 @@ int32_t insert_launch(const jpt_prefill_insert_args& a, const jpt_insert_layer* 
     JPT_REQUIRE(aligned(dk, 4 * esz_out) && aligned(dv, 4 * esz_out), "destination must be aligned to four elements");
     if (quant) JPT_REQUIRE(ks && vs, "k_scale/v_scale are NULL");
     wide_ok = wide_ok && aligned(sk, 16) && aligned(sv, 16) && aligned(dk, 8) && aligned(dv, 8);
+    pieces_ok = pieces_ok && aligned(sk, 16) && aligned(sv, 16) && aligned(dk, 16) && aligned(dv, 16);
     return JPT_OK;
   };
   if (layers) {
@@ -495,6 +459,7 @@ int32_t insert_launch(const jpt_prefill_insert_args& a, const jpt_insert_layer* 
     if (p.a.n_layers <= 0) p.a.n_layers = 1;
     JPT_REQUIRE(p.a.n_layers <= 65535, "n_layers out of range");
     wide_ok = wide_ok && a.src_layer_stride % 8 == 0 && a.dst_layer_stride % 8 == 0;
+    pieces_ok = pieces_ok && a.src_layer_stride * esz % 16 == 0 && a.dst_layer_stride * esz % 16 == 0;
   }
   int32_t rows = a.tokens;
   if (a.page_ids) {
@@ -506,17 +471,23 @@ int32_t insert_launch(const jpt_prefill_insert_args& a, const jpt_insert_layer* 
     JPT_REQUIRE(a.tokens <= a.seq, "%d tokens do not fit a cache of %d positions", a.tokens, a.seq);
   }
   if (rows == 0) return JPT_OK;
-  const int d8 = a.dim / 8;  // threads a head in the wide kernel
-  const bool four = quant && wide_ok && a.tokens > 0 && a.in_dtype == JPT_BF16 && a.heads * a.dim == 1024 &&
-                    a.dim % 8 == 0 && (a.scale_heads == 1 || (d8 <= 64 && (d8 & (d8 - 1)) == 0)) &&
-                    (a.src_head_stride == 0 || a.src_head_stride % 8 == 0);
-  if (four) {
-    dim3 grid4((rows + kTokensPerBlock - 1) / kTokensPerBlock, 2, p.a.n_layers);
-    if (a.scale_dtype == JPT_BF16)
-      hipLaunchKernelGGL(prefill_insert_quant4_kernel<true>, grid4, dim3(256), 0, static_cast<hipStream_t>(stream), p);
-    else
-      hipLaunchKernelGGL(prefill_insert_quant4_kernel<false>, grid4, dim3(256), 0, static_cast<hipStream_t>(stream), p);
-    return launch_status("prefill_insert_quant4_kernel");
+  if (quant && wide_ok && a.tokens > 0 && a.in_dtype == JPT_BF16 && split_rows(a.heads, a.dim, &p.split) &&
+      (a.src_head_stride == 0 || a.src_head_stride % 8 == 0)) {
+    const int tb = 1 << p.split.tokens_log;
+    const dim3 blocks((rows + tb - 1) / tb, 2, p.a.n_layers);
+    const bool llama = a.heads == 8 && a.dim == 128;
+    auto kernel = llama ? prefill_insert_rows_kernel<true, true> : prefill_insert_rows_kernel<true, false>;
+    if (a.scale_dtype == JPT_F32) kernel = llama ? prefill_insert_rows_kernel<false, true> : prefill_insert_rows_kernel<false, false>;
+    hipLaunchKernelGGL(kernel, blocks, dim3(256), 0, static_cast<hipStream_t>(stream), p);
+    return launch_status("prefill_insert_rows_kernel");
+  }
+  // rows of whole 16-byte pieces, all of them aligned, in numbers that 32 bits and a grid count: never slower above
+  const int64_t row_pieces = static_cast<int64_t>(a.dim) * esz / 16;
+  if (!quant && pieces_ok && a.dim * esz % 16 == 0 && a.src_head_stride * esz % 16 == 0 &&
+      rows * row_pieces < (1ll << 31) - 256 * kPieces && a.heads < 32768) {
+    const dim3 blocks(static_cast<unsigned>((rows * row_pieces + 256 * kPieces - 1) / (256 * kPieces)), 2 * a.heads, p.a.n_layers);
+    hipLaunchKernelGGL(prefill_copy_kernel, blocks, dim3(256), 0, static_cast<hipStream_t>(stream), p, esz, static_cast<int>(row_pieces));
+    return launch_status("prefill_copy_kernel");
   }
   dim3 grid(rows, 2, p.a.n_layers);
   if (quant && a.scale_dtype == JPT_BF16)
@@ -557,10 +528,10 @@ int32_t jpt_prefill_insert_prompts(const jpt_prefill_insert_args* args, const jp
   JPT_REQUIRE(n_prompts >= 1, "n_prompts must be positive");
   const jpt_prefill_insert_args& a = *args;
   const int n_layers = a.n_layers > 0 ? a.n_layers : 1;
-  const int d8 = a.dim / 8;
-  // the shape the one-launch kernel takes; anything else goes prompt by prompt
-  bool wide = a.dst_dtype == JPT_I8 && a.in_dtype == JPT_BF16 && a.heads * a.dim == 1024 && a.dim % 8 == 0 &&
-              a.heads > 0 && (a.scale_heads == 1 || (a.scale_heads == a.heads && d8 <= 64 && (d8 & (d8 - 1)) == 0)) &&
+  // the shapes the one-launch kernel takes; anything else goes prompt by prompt
+  RowSplit split;
+  bool wide = a.dst_dtype == JPT_I8 && a.in_dtype == JPT_BF16 && split_rows(a.heads, a.dim, &split) &&
+              (a.scale_heads == 1 || (a.scale_heads == a.heads && (a.scale_heads <= 64 || a.heads * a.dim == 1024))) &&
               a.dst_k && a.dst_v && a.k_scale && a.v_scale && aligned(a.dst_k, 8) && aligned(a.dst_v, 8) &&
               a.dst_layer_stride % 8 == 0 && a.total_pages > 0 && a.page_size > 0 && n_layers <= 65535 &&
               (a.scale_dtype == JPT_BF16 || a.scale_dtype == JPT_F32) &&
@@ -591,20 +562,22 @@ int32_t jpt_prefill_insert_prompts(const jpt_prefill_insert_args* args, const jp
   for (int32_t r0 = 0; r0 < n_prompts; r0 += kLaunchPrompts) {
     PromptsParams p{};
     p.a = a;
+    p.split = split;
     p.a.n_layers = n_layers;
     p.n_prompts = n_prompts - r0 < kLaunchPrompts ? n_prompts - r0 : kLaunchPrompts;
+    const int tb = 1 << split.tokens_log;
     int blocks = 0;
     for (int r = 0; r < p.n_prompts; ++r) {
       p.prompt[r] = prompts[r0 + r];
       p.first_block[r] = blocks;
-      blocks += (prompts[r0 + r].n_pages * a.page_size + kTokensPerBlock - 1) / kTokensPerBlock;
+      blocks += (prompts[r0 + r].n_pages * a.page_size + tb - 1) / tb;
     }
     p.first_block[p.n_prompts] = blocks;
     const dim3 grid(blocks, 2, n_layers);
-    if (a.scale_dtype == JPT_BF16)
-      hipLaunchKernelGGL(prefill_insert_prompts_kernel<true>, grid, dim3(256), 0, static_cast<hipStream_t>(stream), p);
-    else
-      hipLaunchKernelGGL(prefill_insert_prompts_kernel<false>, grid, dim3(256), 0, static_cast<hipStream_t>(stream), p);
+    const bool llama = a.heads == 8 && a.dim == 128;
+    auto kernel = llama ? prefill_insert_prompts_kernel<true, true> : prefill_insert_prompts_kernel<true, false>;
+    if (a.scale_dtype == JPT_F32) kernel = llama ? prefill_insert_prompts_kernel<false, true> : prefill_insert_prompts_kernel<false, false>;
+    hipLaunchKernelGGL(kernel, grid, dim3(256), 0, static_cast<hipStream_t>(stream), p);
     const int32_t st = launch_status("prefill_insert_prompts_kernel");
     if (st != JPT_OK) return st;
   }
