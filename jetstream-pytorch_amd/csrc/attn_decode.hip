@@ -89,6 +89,9 @@ Layout make_layout(int batch, int kv_heads, int rows) {
   return l;
 }
 
+// Bytes of LDS the planning kernel needs by size: a word a slot twice, a word a record twice.
+unsigned plan_lds_bytes(int batch, int max_entries) { return 4u * (2u * batch + 2u * max_entries); }
+
 // ---- planning kernel -----------------------------------------------------------
 // One workgroup.  chunk = max(128, total positions * kv_heads / target items,
 // rounded up to 128); a slot longer than that is cut into ceil(len / chunk)
@@ -99,6 +102,13 @@ Layout make_layout(int batch, int kv_heads, int rows) {
 // then the chunks of the other cut slots, then whole slots; after the last
 // place one merge entry for every slot cut in three or more; places nobody was
 // put on are marked unused.  The arrival counters are cleared.
+//
+// What bounds it: one workgroup's chain of barriers, LDS round trips and one trip to memory each way.  So the records stay
+// words in LDS (slot, chunk, kind) through deal and reorderings and are written out once, at the end (moved about in
+// memory, every round of a bin cost a trip); a sum goes through a wave's shuffles before LDS; the keys are scanned four a
+// thread; a slot's equal chunks take their ranks with one atomic.  Measured, us a launch, before -> now: 1 slot of 700
+// positions 15.0 -> 10.9, 96 ragged slots of up to 2048 16.4 -> 12.6, of 1024 each 11.9 -> 8.7, 8 of up to 32768 22.1 ->
+// 16.8, 4000 of up to 256 55 -> 53 (whose launch needs 141 KB of LDS; 96 slots 28).
 // Exclusive prefix sum of `x` over the 256 threads of the planning workgroup;
 // *total gets the sum.
 __device__ __forceinline__ int plan_exclusive_scan(int x, int* total) {
@@ -200,41 +210,65 @@ __device__ __forceinline__ void deal_longest_first(int first, int n, int per_rou
   }
 }
 
-// The same deal, many entries a step (at most 64 bins, one a lane).  The bins are
-// sorted by (tiles, bin) across the wave; entry i + j goes to the j-th lightest bin
-// for as long as that bin is lighter than every bin already given an entry of this
-// step is afterwards - exactly the choices of the one-by-one deal, which picks bin
-// j for entry i + j if and only if bin j's key is below the new keys of bins
-// 0..j-1.  Entries come in levels (every bin gets one of the long entries before
-// any gets a second), so a step usually places dozens: a sort of 21 exchanges and
-// a running minimum instead of a minimum per entry.  When a step places fewer than
-// eight (short entries on uneven bins), the rest is dealt one by one.  Returns the
+// The same deal, many entries a step.  The bins are sorted by (tiles, bin) across the wave, PER_LANE of them a lane;
+// entry i + j goes to the j-th lightest bin for as long as that bin is lighter than every bin already given an entry of
+// this step is afterwards - exactly the choices of the one-by-one deal, which picks bin j for entry i + j if and only if
+// bin j's key is below the new keys of bins 0..j-1.  Entries come in levels (every bin gets one of the long entries before
+// any gets a second), so a step usually places dozens: a sort of 21 exchanges (64 bins) and a running minimum instead of a
+// minimum per entry.  When a step places fewer than eight (short entries on uneven bins), it is the last.  Returns the
 // first rank that is still to be dealt.
-__device__ __forceinline__ unsigned plan_sort_wave(unsigned key, int lane) {
+// (One KV head has 512 bins.  Ragged 64 slots of up to 2048 positions, the plan's launch: 316 us one by one, 26 so.)
+template <int PER_LANE>
+__device__ __forceinline__ void plan_sort_wave(unsigned (&key)[PER_LANE], int lane) {  // the bin `i` of a lane: PER_LANE * lane + i
 #pragma unroll
-  for (int k = 2; k <= 64; k <<= 1) {
+  for (int k = 2; k <= 64 * PER_LANE; k <<= 1) {
 #pragma unroll
     for (int j = k >> 1; j > 0; j >>= 1) {
-      const unsigned other = static_cast<unsigned>(__shfl_xor(static_cast<int>(key), j));
-      const bool up = (lane & k) == 0, lower = (lane & j) == 0;
-      key = (lower == up) ? min(key, other) : max(key, other);
+      if (j >= PER_LANE) {
+        const int across = j / PER_LANE;
+        const bool lower = (lane & across) == 0;
+#pragma unroll
+        for (int i = 0; i < PER_LANE; ++i) {
+          const bool up = ((PER_LANE * lane + i) & k) == 0;
+          const unsigned other = static_cast<unsigned>(__shfl_xor(static_cast<int>(key[i]), across));
+          key[i] = (lower == up) ? min(key[i], other) : max(key[i], other);
+        }
+      } else {
+#pragma unroll
+        for (int i = 0; i < PER_LANE; ++i) {
+          if (i & j) continue;
+          const bool up = ((PER_LANE * lane + i) & k) == 0;
+          const unsigned x = key[i], y = key[i | j];
+          key[i] = up ? min(x, y) : max(x, y);
+          key[i | j] = up ? max(x, y) : min(x, y);
+        }
+      }
     }
   }
-  return key;
 }
-__device__ __forceinline__ int deal_longest_first_in_steps(int n, int per_round, int max_rounds, int* bin_load,
+template <int PER_LANE>
+__device__ __forceinline__ int deal_longest_first_in_steps(int first, int n, int per_round, int max_rounds, int* bin_load,
                                                            int* bin_rounds, const int* rank_tiles, int* rank_place) {
   const int lane = threadIdx.x;
-  int first = 0;
   while (first < n) {
-    unsigned key = ~0u;  // a bin with no free round is out of the running
-    if (lane < per_round && bin_rounds[lane] < max_rounds) key = (static_cast<unsigned>(bin_load[lane]) << 10) | static_cast<unsigned>(lane);
-    key = plan_sort_wave(key, lane);
-    const bool has_entry = first + lane < n && key != ~0u;
-    const unsigned tiles = has_entry ? static_cast<unsigned>(rank_tiles[first + lane]) : 0u;
-    const unsigned after = has_entry ? key + (tiles << 10) : ~0u;
-    // the lightest of the bins before this lane once they have their entries (exclusive running minimum)
-    unsigned before = after;
+    unsigned key[PER_LANE];
+#pragma unroll
+    for (int i = 0; i < PER_LANE; ++i) {
+      const int x = lane + 64 * i;  // (any order will do before the sort)
+      // a bin with no free round is out of the running
+      key[i] = x < per_round && bin_rounds[x] < max_rounds ? (static_cast<unsigned>(bin_load[x]) << 10) | static_cast<unsigned>(x) : ~0u;
+    }
+    plan_sort_wave<PER_LANE>(key, lane);
+    unsigned tiles[PER_LANE], lightest = ~0u;  // the lightest of the lane's bins once they have their entries
+    bool has_entry[PER_LANE];
+#pragma unroll
+    for (int i = 0; i < PER_LANE; ++i) {
+      const int rank = first + PER_LANE * lane + i;
+      has_entry[i] = rank < n && key[i] != ~0u;
+      tiles[i] = has_entry[i] ? static_cast<unsigned>(rank_tiles[rank]) : 0u;
+      lightest = min(lightest, has_entry[i] ? key[i] + (tiles[i] << 10) : ~0u);
+    }
+    unsigned before = lightest;  // ... of the bins before this lane's (exclusive running minimum)
 #pragma unroll
     for (int off = 1; off < 64; off <<= 1) {
       const unsigned y = static_cast<unsigned>(__shfl_up(static_cast<int>(before), off));
@@ -242,15 +276,25 @@ __device__ __forceinline__ int deal_longest_first_in_steps(int n, int per_round,
     }
     before = static_cast<unsigned>(__shfl_up(static_cast<int>(before), 1));
     if (lane == 0) before = ~0u;
-    const bool ok = has_entry && key < before;
-    const unsigned long long bad = ~__ballot(ok);  // lanes whose entry is not this step's
-    const int placed = bad == 0 ? 64 : __ffsll(static_cast<long long>(bad)) - 1;
-    if (lane < placed) {
-      const int x = static_cast<int>(key & 1023u);
-      const int round = bin_rounds[x];
-      rank_place[first + lane] = round * per_round + ((round & 1) ? per_round - 1 - x : x);
-      bin_rounds[x] = round + 1;
-      bin_load[x] = static_cast<int>(key >> 10) + static_cast<int>(tiles);
+    int good = 0;  // of the lane's entries, those before the first that is not this step's
+#pragma unroll
+    for (int i = 0; i < PER_LANE; ++i) {
+      if (good == i && has_entry[i] && key[i] < before) ++good;
+      before = min(before, has_entry[i] ? key[i] + (tiles[i] << 10) : ~0u);
+    }
+    const unsigned long long stops = __ballot(good < PER_LANE);
+    const int stop = stops == 0 ? 64 : __ffsll(static_cast<long long>(stops)) - 1;  // the lane with the first such
+    const int placed = stop == 64 ? 64 * PER_LANE : PER_LANE * stop + __builtin_amdgcn_readlane(good, stop);
+#pragma unroll
+    for (int i = 0; i < PER_LANE; ++i) {
+      const int j = PER_LANE * lane + i;
+      if (j < placed) {
+        const int x = static_cast<int>(key[i] & 1023u);
+        const int round = bin_rounds[x];
+        rank_place[first + j] = round * per_round + ((round & 1) ? per_round - 1 - x : x);
+        bin_rounds[x] = round + 1;
+        bin_load[x] = static_cast<int>(key[i] >> 10) + static_cast<int>(tiles[i]);
+      }
     }
     __builtin_amdgcn_wave_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
@@ -260,6 +304,22 @@ __device__ __forceinline__ int deal_longest_first_in_steps(int n, int per_round,
   return first;
 }
 
+// The deal of ranks 0 .. n - 1: in steps, and 64 one by one where a step places few (or there are few: a step takes as
+// long as ten of them).
+template <int PER_LANE>
+__device__ __forceinline__ void deal(int n, int per_round, int max_rounds, int* bin_load, int* bin_rounds, const int* rank_tiles,
+                                     int* rank_place) {
+  int dealt = 0;
+  while (dealt < n) {
+    if (n - dealt >= 10) dealt = deal_longest_first_in_steps<PER_LANE>(dealt, n, per_round, max_rounds, bin_load, bin_rounds, rank_tiles, rank_place);
+    const int some = min(dealt + 64, n);
+    deal_longest_first<PER_LANE>(dealt, some, per_round, max_rounds, bin_load, bin_rounds, rank_tiles, rank_place);
+    __builtin_amdgcn_wave_barrier();
+    __builtin_amdgcn_fence(__ATOMIC_ACQ_REL, "wavefront");
+    dealt = some;
+  }
+}
+
 __global__ void __launch_bounds__(256)
 plan_kernel(const int32_t* lengths, int batch, int seq_cap, int kv_heads, int target, int workers,
             PlanEntry* entries, int32_t* arrivals, int max_entries, int32_t* status, int fresh) {
@@ -267,10 +327,13 @@ plan_kernel(const int32_t* lengths, int batch, int seq_cap, int kv_heads, int ta
   // (make_layout) is sized so that this cannot happen, and if it ever does the launch says so.
   auto overflow = [&]() { atomicOr(status, JPT_ATTN_STATUS_PLAN_OVERFLOW); };
   constexpr int kKeys = 3 * 257;  // tile count; + 257: chunks of slots cut in three or more; + 514: in two, paired
-  __shared__ int s_len[kMaxPlanBatch];
-  __shared__ int s_first[kMaxPlanBatch];
-  __shared__ long long s_total;
-  __shared__ int s_chunk, s_entries, s_merges, s_pairs, s_positions, s_sizes;
+  extern __shared__ int s_by_size[];  // plan_lds_bytes
+  int* const s_len = s_by_size;
+  int* const s_first = s_len + batch;
+  int* const s_place = s_first + batch;       // by place: who is there (see id_of), -1: nobody
+  int* const s_rank = s_place + max_entries;  // the same by rank, of entries that are not a pair's
+  __shared__ long long s_total[4];
+  __shared__ int s_merges, s_pairs, s_positions, s_sizes;
   __shared__ int s_hist[kKeys];
   __shared__ int s_base[kKeys];
   __shared__ int s_bin_load[kMaxBins];       // tiles dealt to a bin (the workers that take one entry's heads)
@@ -280,8 +343,8 @@ plan_kernel(const int32_t* lengths, int batch, int seq_cap, int kv_heads, int ta
   __shared__ int s_rank_tiles[kDealtOneByOne];
   __shared__ int s_rank_place[kDealtOneByOne];
   const int tid = threadIdx.x;
+  const int first_length = lengths && tid < batch ? lengths[tid] : seq_cap;  // on its way while LDS is cleared
   if (tid == 0) {
-    s_total = 0;
     s_merges = 0;
     s_positions = 0;
     s_pairs = 0;
@@ -294,29 +357,26 @@ plan_kernel(const int32_t* lengths, int batch, int seq_cap, int kv_heads, int ta
   }
   for (int i = tid; i < kKeys; i += blockDim.x) s_hist[i] = 0;
   for (int i = tid; i < batch * kv_heads; i += blockDim.x) arrivals[i] = 0;
-  for (int i = tid; i < max_entries; i += blockDim.x) entries[i] = PlanEntry{-1, 0, 0, 0, 0, 0, {0, 0}};
-  __syncthreads();
+  for (int i = tid; i < max_entries; i += blockDim.x) s_place[i] = -1;
   long long mine = 0;
   bool full = false;  // a slot with no room left for the step's token
   for (int b = tid; b < batch; b += blockDim.x) {
-    int n = lengths ? lengths[b] : seq_cap;
+    int n = b == tid ? first_length : lengths ? lengths[b] : seq_cap;
     full = full || (lengths && n >= seq_cap);
     n = n < 0 ? 0 : (n > seq_cap ? seq_cap : n);
     s_len[b] = n;
     mine += n;
   }
   if (full) atomicOr(status, JPT_ATTN_STATUS_SLOT_FULL);
-  atomicAdd(reinterpret_cast<unsigned long long*>(&s_total), static_cast<unsigned long long>(mine));
+#pragma unroll
+  for (int off = 32; off > 0; off >>= 1) mine += __shfl_xor(mine, off);
+  if ((tid & 63) == 0) s_total[tid >> 6] = mine;
   __syncthreads();
-  if (tid == 0) {
-    long long c = (s_total * kv_heads + target - 1) / target;
-    const long long floor_c = (seq_cap + kMaxChunksPerSlot - 1) / kMaxChunksPerSlot;
-    c = c < floor_c ? floor_c : c;  // at most kMaxChunksPerSlot chunks per slot
-    c = (c + kChunkAlign - 1) / kChunkAlign * kChunkAlign;
-    s_chunk = c < kChunkAlign ? kChunkAlign : static_cast<int>(c);
-  }
-  __syncthreads();
-  const int chunk = s_chunk;
+  const long long positions = s_total[0] + s_total[1] + s_total[2] + s_total[3];
+  long long in_chunk = (positions * kv_heads + target - 1) / target;
+  // at most kMaxChunksPerSlot chunks per slot
+  in_chunk = max(in_chunk, static_cast<long long>((seq_cap + kMaxChunksPerSlot - 1) / kMaxChunksPerSlot));
+  const int chunk = max(static_cast<int>((in_chunk + kChunkAlign - 1) / kChunkAlign * kChunkAlign), kChunkAlign);
   auto chunks_of = [&](int b) { return s_len[b] == 0 ? 1 : (s_len[b] + chunk - 1) / chunk; };
   // positions of one chunk of slot b: the slot cut evenly, in whole tiles
   auto chunk_len = [&](int b) {
@@ -332,19 +392,6 @@ plan_kernel(const int32_t* lengths, int batch, int seq_cap, int kv_heads, int ta
   const int per_round = workers / kv_heads;
   const bool pairing = per_round <= kMaxBins && kv_heads * 16 <= workers && (workers / 16) % kv_heads == 0;
   auto paired = [&](int b) { return pairing && chunks_of(b) == 2; };
-  // a slot's first partial record: running sum of the chunk counts, 256 slots a pass
-  {
-    int base = 0;
-    for (int b0 = 0; b0 < batch; b0 += static_cast<int>(blockDim.x)) {
-      const int b = b0 + tid;
-      int total;
-      const int before = plan_exclusive_scan(b < batch ? chunks_of(b) : 0, &total);
-      if (b < batch) s_first[b] = base + before;
-      base += total;
-    }
-    if (tid == 0) s_entries = base;
-  }
-  __syncthreads();
   // sort keys: paired slots (one key a slot, by its chunk's tiles), then the
   // chunks of the other cut slots, then whole slots, each longest first
   auto key_of = [&](int count, int kind) {
@@ -357,22 +404,40 @@ plan_kernel(const int32_t* lengths, int batch, int seq_cap, int kv_heads, int ta
       atomicAdd(&s_hist[key_of(cl, 2)], 1);
       atomicAdd(&s_pairs, 1);
     } else {
-      for (int c = 0; c < nc; ++c) atomicAdd(&s_hist[key_of(min(cl, s_len[b] - c * cl), nc > 1 ? 1 : 0)], 1);
+      // all chunks but the last are equally long
+      if (nc > 1) atomicAdd(&s_hist[key_of(cl, 1)], nc - 1);
+      atomicAdd(&s_hist[key_of(s_len[b] - (nc - 1) * cl, nc > 1 ? 1 : 0)], 1);
     }
   }
-  __syncthreads();
-  // how many different sizes the entries that are not a pair's have
-  for (int key = tid; key < 2 * 257; key += blockDim.x)
-    if (s_hist[key] > 0) atomicAdd(&s_sizes, 1);
+  // a slot's first partial record: running sum of the chunk counts, 256 slots a pass
+  int n_entries = 0;
+  for (int b0 = 0; b0 < batch; b0 += static_cast<int>(blockDim.x)) {
+    const int b = b0 + tid;
+    int total;
+    const int before = plan_exclusive_scan(b < batch ? chunks_of(b) : 0, &total);
+    if (b < batch) s_first[b] = n_entries + before;
+    n_entries += total;
+  }
+  // (the scan's barriers stand between the histogram and this)  Where each key's entries start, largest key first -
+  // thread t has four keys, from kKeys - 1 - 4 t down - and how many different sizes the entries that are not a pair's have
   {
-    // where each key's entries start, largest key first: thread t of pass i has key kKeys - 1 - (256 i + t)
-    int base = 0;
-    for (int k0 = 0; k0 < kKeys; k0 += static_cast<int>(blockDim.x)) {
-      const int key = kKeys - 1 - (k0 + tid);
-      int total;
-      const int before = plan_exclusive_scan(key >= 0 ? s_hist[key] : 0, &total);
-      if (key >= 0) s_base[key] = base + before;
-      base += total;
+    int n[4], sum = 0, sizes = 0;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int key = kKeys - 1 - (4 * tid + j);
+      n[j] = key >= 0 ? s_hist[key] : 0;
+      sum += n[j];
+      sizes += __popcll(__ballot(n[j] > 0 && key < 2 * 257));
+    }
+    static_assert(4 * 256 >= kKeys, "four keys a thread");
+    if ((tid & 63) == 0 && sizes > 0) atomicAdd(&s_sizes, sizes);
+    int total;
+    int before = plan_exclusive_scan(sum, &total);
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {
+      const int key = kKeys - 1 - (4 * tid + j);
+      if (key >= 0) s_base[key] = before;
+      before += n[j];
     }
   }
   __syncthreads();
@@ -387,7 +452,7 @@ plan_kernel(const int32_t* lengths, int batch, int seq_cap, int kv_heads, int ta
   // deal_longest_first).  `regular`: the walk has whole entries per round, i.e.
   // bins exist; otherwise entries lie in sorted order.
   const bool regular = per_round >= 1 && per_round <= kMaxBins && workers % 8 == 0 && (workers / 8) % kv_heads == 0;
-  const int n_others = s_entries - 2 * n_pairs;
+  const int n_others = n_entries - 2 * n_pairs;
   // (when all of them are equally long there is nothing to even out: they go round the bins)
   const int candidates = regular && s_sizes > 1 ? min(n_others, kDealtOneByOne) : 0;
   auto bin_of_place = [&](int round, int x) { return (round & 1) ? per_round - 1 - x : x; };
@@ -401,28 +466,58 @@ plan_kernel(const int32_t* lengths, int batch, int seq_cap, int kv_heads, int ta
     }
     if (tid == 0) s_snake_max = s_snake_sum = 0;
     __syncthreads();
-    // tiles of the entries by rank (a key is a tile count; ranks go down the keys), pairs' loads and rounds
-    for (int rank = tid; rank < n_pairs + candidates; rank += blockDim.x) {
-      int lo = 0, hi = kKeys - 1;  // the smallest key whose entries start at or before this rank
-      while (lo < hi) {
-        const int mid = (lo + hi) >> 1;
-        if (s_base[mid] <= rank) hi = mid; else lo = mid + 1;
-      }
-      const int tiles = lo % 257;
-      if (rank < n_pairs) {  // a pair: both its bins get the chunk's tiles
-        const int round = rank / half, x = rank % half;
+  }
+  // An entry in one word: slot, which of its chunks, whether it is all of the slot, whether it is one of a pair.
+  static_assert(kMaxPlanBatch <= 1 << 12 && kMaxChunksPerSlot <= 1 << 8, "slot and chunk of an id");
+  constexpr int kWhole = 1 << 20, kPaired = 1 << 21;
+  auto id_of = [&](int b, int c, int kind) { return b | (c << 12) | kind; };
+  auto slot_of = [&](int id) { return id & ((1 << 12) - 1); };
+  int last_place = 0;  // one past the last place this thread put an entry on
+  auto put = [&](int place, int id) {
+    if (place < max_entries) {
+      s_place[place] = id;
+      last_place = max(last_place, place + 1);
+    } else {
+      overflow();
+    }
+  };
+  // Every entry takes its rank; pairs have their places by it, and charge their bins, the others come up for the deal
+  // (ranks go down the keys, and a key is a tile count).
+  for (int b = tid; b < batch; b += blockDim.x) {
+    const int nc = chunks_of(b), cl = chunk_len(b);
+    if (paired(b)) {
+      const int key = key_of(cl, 2), q = atomicAdd(&s_base[key], 1), round = q / half, x = q - round * half;
+      const int at = round * per_round + x;
+      put(at + half < max_entries ? at : max_entries, id_of(b, 0, kPaired));
+      put(at + half, id_of(b, 1, kPaired));
+      if (regular) {  // both its bins get the chunk's tiles
+        const int tiles = key - 2 * 257;
         atomicAdd(&s_bin_load[bin_of_place(round, x)], tiles);
         atomicAdd(&s_bin_load[bin_of_place(round, x + half)], tiles);
         atomicMax(&s_bin_rounds[bin_of_place(round, x)], round + 1);
         atomicMax(&s_bin_rounds[bin_of_place(round, x + half)], round + 1);
-      } else {
+      }
+      continue;
+    }
+    const int key = key_of(cl, nc > 1 ? 1 : 0), last = key_of(s_len[b] - (nc - 1) * cl, nc > 1 ? 1 : 0);
+    const int rank = nc > 1 ? atomicAdd(&s_base[key], nc - 1) - n_pairs : 0, rank_of_last = atomicAdd(&s_base[last], 1) - n_pairs;
+    for (int c = 0; c < nc; ++c) {
+      const int i = c < nc - 1 ? rank + c : rank_of_last;
+      if (i >= max_entries) {
+        overflow();
+        continue;
+      }
+      s_rank[i] = id_of(b, c, nc == 1 ? kWhole : 0);
+      if (i < candidates) {
+        const int tiles = (c < nc - 1 ? key : last) - (nc > 1 ? 257 : 0), lap = i / per_round, x = i - lap * per_round;
         // (and what the plain snake deal - entry i to bin i, 2E-1-i, 2E+i, ... - would give each bin)
-        const int i = rank - n_pairs, lap = i / per_round;
         s_rank_tiles[i] = tiles;
-        atomicAdd(&s_snake_load[(lap & 1) ? per_round - 1 - i % per_round : i % per_round], tiles);
+        atomicAdd(&s_snake_load[bin_of_place(lap, x)], tiles);
       }
     }
-    __syncthreads();
+  }
+  __syncthreads();
+  if (regular) {
     // bins the pairs left behind start at the pairs' last full round, so that every round before a pair's is full
     if (pairing && n_pairs > 0)
       for (int x = tid; x < per_round; x += blockDim.x) s_bin_rounds[x] = max(s_bin_rounds[x], n_pairs / half);
@@ -457,14 +552,10 @@ plan_kernel(const int32_t* lengths, int batch, int seq_cap, int kv_heads, int ta
     const int laps_after = (n_others - one_by_one + per_round - 1) / per_round;
     if (tid < 64 && one_by_one > 0) {
       const int cap = max(max_rounds - laps_after, 1);
-      if (per_round <= 64) {
-        const int dealt = deal_longest_first_in_steps(one_by_one, per_round, cap, s_bin_load, s_bin_rounds, s_rank_tiles, s_rank_place);
-        deal_longest_first<1>(dealt, one_by_one, per_round, cap, s_bin_load, s_bin_rounds, s_rank_tiles, s_rank_place);
-      } else if (per_round <= 256) {
-        deal_longest_first<4>(0, one_by_one, per_round, cap, s_bin_load, s_bin_rounds, s_rank_tiles, s_rank_place);
-      } else {
-        deal_longest_first<16>(0, one_by_one, per_round, cap, s_bin_load, s_bin_rounds, s_rank_tiles, s_rank_place);
-      }
+      if (per_round <= 64) deal<1>(one_by_one, per_round, cap, s_bin_load, s_bin_rounds, s_rank_tiles, s_rank_place);
+      else if (per_round <= 256) deal<4>(one_by_one, per_round, cap, s_bin_load, s_bin_rounds, s_rank_tiles, s_rank_place);
+      else if (per_round <= 512) deal<8>(one_by_one, per_round, cap, s_bin_load, s_bin_rounds, s_rank_tiles, s_rank_place);
+      else deal<16>(one_by_one, per_round, cap, s_bin_load, s_bin_rounds, s_rank_tiles, s_rank_place);
     }
     __syncthreads();
   }
@@ -476,33 +567,7 @@ plan_kernel(const int32_t* lengths, int batch, int seq_cap, int kv_heads, int ta
     const int round = s_bin_rounds[x] + lap;  // one entry a bin and lap
     return round * per_round + bin_of_place(round, x);
   };
-  int last_place = 0;  // one past the last place this thread wrote
-  for (int b = tid; b < batch; b += blockDim.x) {
-    const int nc = chunks_of(b), cl = chunk_len(b), first = s_first[b];
-    if (paired(b)) {
-      const int q = atomicAdd(&s_base[key_of(cl, 2)], 1);
-      const int at = (q / half) * per_round + q % half;
-      // part = -1: folded with its partner through LDS, no partial record
-      if (at + half < max_entries) {
-        entries[at] = PlanEntry{b, 0, cl, -1, 2, s_len[b], {0, 0}};
-        entries[at + half] = PlanEntry{b, cl, s_len[b] - cl, -1, 2, s_len[b], {0, 0}};
-        last_place = max(last_place, at + half + 1);
-      } else {
-        overflow();
-      }
-      continue;
-    }
-    for (int c = 0; c < nc; ++c) {
-      const int count = min(cl, s_len[b] - c * cl);
-      const int at = place_of(atomicAdd(&s_base[key_of(count, nc > 1 ? 1 : 0)], 1) - n_pairs);
-      if (at < max_entries) {
-        entries[at] = PlanEntry{b, c * cl, count, first + c, nc, s_len[b], {0, 0}};
-        last_place = max(last_place, at + 1);
-      } else {
-        overflow();
-      }
-    }
-  }
+  for (int i = tid; i < min(n_others, max_entries); i += blockDim.x) put(place_of(i), s_rank[i]);
 #pragma unroll
   for (int off = 32; off > 0; off >>= 1) last_place = max(last_place, __shfl_xor(last_place, off));
   if ((tid & 63) == 0) atomicMax(&s_positions, last_place);
@@ -525,26 +590,23 @@ plan_kernel(const int32_t* lengths, int batch, int seq_cap, int kv_heads, int ta
   // tensors: the headline workload's launch 34.3 -> 33.6 us.)  Chunks of cut slots keep
   // their places: pairs must share a round, partials must be parked early.
   if (regular) {
-    __threadfence_block();
-    __syncthreads();
     const int rounds_used = (n_places + per_round - 1) / per_round;
     for (int x = tid; x < per_round; x += blockDim.x) {
-      int first = -1, before = -1;
-      PlanEntry longest{};
+      int first = -1, before = -1, longest = -1;
       for (int r = 0; r < rounds_used; ++r) {
         const int at = r * per_round + bin_of_place(r, x);
         if (at >= n_places) continue;
-        const PlanEntry e = entries[at];
-        if (e.slot < 0 || e.n_chunks != 1) continue;
+        const int e = s_place[at];
+        if (e < 0 || !(e & kWhole)) continue;
         if (first < 0) {
           first = at;
           longest = e;
         } else {
-          entries[before] = e;  // every later whole slot moves up one
+          s_place[before] = e;  // every later whole slot moves up one
         }
         before = at;
       }
-      if (first >= 0 && before != first) entries[before] = longest;
+      if (first >= 0 && before != first) s_place[before] = longest;
     }
     // ... and where a workgroup's two bins hold a paired chunk each and, after it, equally many
     // whole slots and nothing else, the pair goes last as well - it is the longest item of both
@@ -553,56 +615,63 @@ plan_kernel(const int32_t* lengths, int batch, int seq_cap, int kv_heads, int ta
     // slots longest first before the pair, or the pair in the middle, gain nothing.)  The pair
     // stays on one round in both walks with every earlier round of the two bins taken, which is
     // what the kernel's fold of the two groups' parts needs.  Only with one round of pairs, and
-    // with as many bins as the staging area holds (the slots' lengths are no longer needed: their
-    // LDS takes both bins' entries of eight rounds for 32 pairs of bins).
+    // with as many bins as the staging area holds (the dealt ranks' places are no longer needed:
+    // they take both bins' entries of eight rounds for 32 pairs of bins).
     constexpr int kMostWhole = 8;
-    constexpr int kStagedBins = static_cast<int>(sizeof(s_len) / (2 * kMostWhole * sizeof(PlanEntry)));
+    constexpr int kStagedBins = kDealtOneByOne / (2 * kMostWhole);
     if (pairing && n_pairs > 0 && n_pairs <= half && half <= kStagedBins) {
-      PlanEntry* const stage = reinterpret_cast<PlanEntry*>(s_len);
-      __threadfence_block();
       __syncthreads();
       for (int x = tid; x < half; x += blockDim.x) {
         const int y = x + half;  // round 0: place = bin
         if (rounds_used - 1 > kMostWhole) continue;
-        // both bins' entries of the first rounds, asked for all at once (one trip to memory, not one a round)
-        const PlanEntry px = entries[x], py = entries[y];
-        PlanEntry* const wx = stage + x * 2 * kMostWhole;
-        PlanEntry* const wy = wx + kMostWhole;
-#pragma unroll
-        for (int r = 1; r <= kMostWhole; ++r) {
-          const int ax = r * per_round + bin_of_place(r, x), ay = r * per_round + bin_of_place(r, y);
-          wx[r - 1] = r < rounds_used && ax < n_places ? entries[ax] : PlanEntry{-1, 0, 0, 0, 0, 0, {0, 0}};
-          wy[r - 1] = r < rounds_used && ay < n_places ? entries[ay] : PlanEntry{-1, 0, 0, 0, 0, 0, {0, 0}};
-        }
-        if (px.slot < 0 || px.n_chunks != 2 || px.part != -1 || py.slot != px.slot || py.n_chunks != 2 || py.part != -1) continue;
+        const int px = s_place[x], py = s_place[y];
+        if (px < 0 || !(px & kPaired) || py < 0 || !(py & kPaired) || slot_of(px) != slot_of(py)) continue;
+        int* const wx = s_rank_place + x * 2 * kMostWhole;
+        int* const wy = wx + kMostWhole;
         int m = 0;  // whole slots after the pair, in both bins: rounds 1 .. m and nothing behind them
         bool fits = true;
 #pragma unroll
-        for (int r = 0; r < kMostWhole; ++r) {
-          const bool hx = wx[r].slot >= 0, hy = wy[r].slot >= 0;
-          if (!hx && !hy) continue;
-          fits = fits && hx && hy && r == m && wx[r].n_chunks == 1 && wy[r].n_chunks == 1;
+        for (int r = 1; r <= kMostWhole; ++r) {
+          const int ax = r * per_round + bin_of_place(r, x), ay = r * per_round + bin_of_place(r, y);
+          const int ex = r < rounds_used && ax < n_places ? s_place[ax] : -1;
+          const int ey = r < rounds_used && ay < n_places ? s_place[ay] : -1;
+          wx[r - 1] = ex;
+          wy[r - 1] = ey;
+          if (ex < 0 && ey < 0) continue;
+          fits = fits && ex >= 0 && ey >= 0 && r == m + 1 && (ex & ey & kWhole);
           ++m;
         }
         if (!fits || m == 0) continue;
         // after the rotation above the whole slots stand as w2, w3, ..., wm, w1 (w1 the longest)
         for (int r = 0; r < m; ++r) {
           const int from = r == m - 1 ? m - 1 : m - 2 - r;
-          entries[r * per_round + bin_of_place(r, x)] = wx[from];
-          entries[r * per_round + bin_of_place(r, y)] = wy[from];
+          s_place[r * per_round + bin_of_place(r, x)] = wx[from];
+          s_place[r * per_round + bin_of_place(r, y)] = wy[from];
         }
-        entries[m * per_round + bin_of_place(m, x)] = px;
-        entries[m * per_round + bin_of_place(m, y)] = py;
+        s_place[m * per_round + bin_of_place(m, x)] = px;
+        s_place[m * per_round + bin_of_place(m, y)] = py;
       }
     }
   }
   __syncthreads();
+  const int n_records = min(n_places + s_merges, max_entries);
+  for (int at = tid; at < max_entries; at += blockDim.x) {
+    if (at >= n_places && at < n_records) continue;  // a merge entry
+    const int id = at < n_places ? s_place[at] : -1;
+    PlanEntry e{-1, 0, 0, 0, 0, 0, {0, 0}};
+    if (id >= 0) {
+      const int b = slot_of(id), c = (id >> 12) & 255, cl = chunk_len(b);
+      // part = -1: folded with its partner through LDS, no partial record
+      e = PlanEntry{b, c * cl, min(cl, s_len[b] - c * cl), (id & kPaired) ? -1 : s_first[b] + c, chunks_of(b), s_len[b], {0, 0}};
+    }
+    entries[at] = e;
+  }
   if (tid < kHandOutCounters) status[kStateHandOut + tid * kStateHandOutStride] = 0;
   if (tid == 0) {
     status[kStateEntries] = n_places;
     status[kStateArrivalsAt] = static_cast<int32_t>(arrivals - status);
     status[kStateArrivalsCount] = batch * kv_heads;
-    status[kStateMerges] = max(min(n_places + s_merges, max_entries) - n_places, 0);
+    status[kStateMerges] = n_records - n_places;
   }
 }
 
@@ -664,7 +733,7 @@ int32_t attn_plan_launch(const jpt_attn_args& a, bool paged, bool fresh, hipStre
   char* ws = static_cast<char*>(a.workspace);
   const int cap = paged ? a.max_pages * a.page_size : a.seq;
   JPT_REQUIRE(cap > 0, "sequence capacity must be positive");
-  hipLaunchKernelGGL(plan_kernel, dim3(1), dim3(256), 0, stream, a.lengths, a.batch, cap,
+  hipLaunchKernelGGL(plan_kernel, dim3(1), dim3(256), plan_lds_bytes(a.batch, l.max_entries), stream, a.lengths, a.batch, cap,
                      a.kv_heads, target_items(), persistent_blocks(), reinterpret_cast<PlanEntry*>(ws + l.entries),
                      reinterpret_cast<int32_t*>(ws + l.arrivals), l.max_entries,
                      reinterpret_cast<int32_t*>(ws), fresh ? 1 : 0);
