@@ -161,7 +161,7 @@ def test_int8_paged_insert_all_layers_in_one_launch():
 @pytest.mark.parametrize("block", range(3))
 def test_random_dense_inserts(block):
   """Randomly drawn insert shapes - stacked and per-layer caches, ring wrap,
-  copy and both quantiser kernels (heads * dim == 1024 takes the wide one),
+  copy and quantiser kernels,
   one to five layers in one launch - bit for bit against the oracle."""
   import numpy as np
   for it in range(10):
@@ -186,8 +186,7 @@ def test_random_dense_inserts(block):
 @pytest.mark.parametrize("heads,dim", [(8, 128), (2, 8)])
 def test_int8_paged_insert_of_several_prompts_in_one_launch(heads, dim):
   """Prompts of different lengths into one stacked pool with one call: the
-  pool must equal prompt-by-prompt inserts bit for bit.  (8, 128) takes the
-  one-launch kernel, (2, 8) the library's prompt-by-prompt route."""
+  pool must equal prompt-by-prompt inserts bit for bit."""
   import numpy as np
   from jetstream_pt_amd import insert as gins
   layers, total, ps = 3, 40, 32

@@ -60,10 +60,11 @@ def test_copied_pages(heads, dim, ps, tokens, dtype, shift):
       assert torch.equal(dpools[layer][which].cpu(), want)
 
 
-@pytest.mark.parametrize("heads,dim,scale_heads", [(3, 64, 3), (24, 128, 1), (64, 128, 64), (2, 512, 2)])
+@pytest.mark.parametrize("heads,dim,scale_heads", [(3, 64, 3), (24, 128, 1), (64, 128, 64), (2, 512, 2), (4, 96, 1)])
 def test_quantised_pages(heads, dim, scale_heads):
   """One scale a token and one a (token, head), several prompts in one launch
-  and one by one: the same pool, and the codes the oracle's quantiser gives."""
+  and one by one: the same pool, and the codes the oracle's quantiser gives.
+  (4, 96): the library's prompt-by-prompt route."""
   from jetstream_pt_amd import insert as gins
   layers, total, ps = 2, 12, 16
   g = torch.Generator().manual_seed(heads)
