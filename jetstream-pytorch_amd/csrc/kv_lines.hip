@@ -197,11 +197,14 @@ __global__ void __launch_bounds__(256) quant_append_kernel(QuantParams p) {
   }
 }
 
-// The same computation for the common shapes: bf16 input, heads * dim ==
-// M * 1024; a thread keeps M runs of four elements in registers between the
-// absmax pass and the quantise pass, and stores codes four at a time.
-template <bool BF16_MATH, int M>
-__global__ void __launch_bounds__(256) quant_append_vec_kernel(QuantParams p) {
+// The same computation for bf16 input of up to 4096 elements a token: a thread keeps four elements in registers between the
+// absmax pass and the quantise pass, and stores their codes at once.  A launch of one step's tokens is a chain of
+// latencies - arguments, loads, shuffles, a barrier, divisions, stores - so a thread has one run of the chain, not four.
+// Measured in a step, us a launch, 256 threads with four runs each -> one run a thread: 32 heads of 128 and 16 of 256,
+// 48 to 64 slots, 6.75 -> 5.10.
+constexpr int kMostRuns = 1024;
+template <bool BF16_MATH>
+__global__ void __launch_bounds__(kMostRuns) quant_append_vec_kernel(QuantParams p) {
   const jpt_quant_append_args& a = p.a;
   const bool paged = p.indices != nullptr;
   const int tok = blockIdx.x;
@@ -230,86 +233,74 @@ __global__ void __launch_bounds__(256) quant_append_vec_kernel(QuantParams p) {
     at = a.pos ? a.pos[a.pos_count == 1 ? 0 : b] : 0;
     write_cache = write_cache && at >= 0 && at < a.seq;
   }
-  // run c of this thread: elements i0 .. i0 + 3, all of one head
-  float x[M][4], m[M];
-#pragma unroll
-  for (int c = 0; c < M; ++c) {
-    const int i0 = 4 * (threadIdx.x + 256 * c);
+  const int i0 = 4 * threadIdx.x;  // all four of one head
+  const bool live = i0 < HD;       // the last wave may have no elements left
+  const int h = i0 / D, d = i0 - h * D;
+  float x[4] = {0.f, 0.f, 0.f, 0.f};
+  if (live) {
     const uint2 raw = *reinterpret_cast<const uint2*>(src + src_base + i0);
-    x[c][0] = __uint_as_float(raw.x << 16);
-    x[c][1] = __uint_as_float(raw.x & 0xffff0000u);
-    x[c][2] = __uint_as_float(raw.y << 16);
-    x[c][3] = __uint_as_float(raw.y & 0xffff0000u);
+    x[0] = __uint_as_float(raw.x << 16);
+    x[1] = __uint_as_float(raw.x & 0xffff0000u);
+    x[2] = __uint_as_float(raw.y << 16);
+    x[3] = __uint_as_float(raw.y & 0xffff0000u);
     if (!is_v && a.rope) {  // the run's two pairs: elements d, d + 1 and d + 2, d + 3 of the head
-      const int d = i0 % D;
       const float4 cs = *reinterpret_cast<const float4*>(a.rope + (static_cast<int64_t>(b) * (D / 2) + d / 2) * 2);
-      rotate_pair(x[c][0], x[c][1], cs.x, cs.y, true);
-      rotate_pair(x[c][2], x[c][3], cs.z, cs.w, true);
+      rotate_pair(x[0], x[1], cs.x, cs.y, true);
+      rotate_pair(x[2], x[3], cs.z, cs.w, true);
     }
-    m[c] = fmaxf(fmaxf(fabsf(x[c][0]), fabsf(x[c][1])), fmaxf(fabsf(x[c][2]), fabsf(x[c][3])));
   }
+  float am = fmaxf(fmaxf(fabsf(x[0]), fabsf(x[1])), fmaxf(fabsf(x[2]), fabsf(x[3])));
 
-  __shared__ float s_red[4];
-  float amax[M];
+  __shared__ float s_red[kMostRuns / 64];
   if (groups == 1) {
-    float all = m[0];
-#pragma unroll
-    for (int c = 1; c < M; ++c) all = fmaxf(all, m[c]);
-    for (int off = 32; off > 0; off >>= 1) all = fmaxf(all, __shfl_xor(all, off));
-    if ((threadIdx.x & 63) == 0) s_red[threadIdx.x >> 6] = all;
-    __syncthreads();
-    all = fmaxf(fmaxf(s_red[0], s_red[1]), fmaxf(s_red[2], s_red[3]));
-#pragma unroll
-    for (int c = 0; c < M; ++c) amax[c] = all;
+    for (int off = 32; off > 0; off >>= 1) am = fmaxf(am, __shfl_xor(am, off));
+    const int waves = blockDim.x >> 6;
+    if (waves > 1) {
+      if ((threadIdx.x & 63) == 0) s_red[threadIdx.x >> 6] = am;
+      __syncthreads();
+      am = s_red[0];
+      for (int w = 1; w < waves; ++w) am = fmaxf(am, s_red[w]);
+    }
   } else {
-    // a head's D / 4 threads of a run are consecutive; D / 4 is a power of two <= 64
+    // a head's D / 4 threads are consecutive; D / 4 is a power of two <= 64
+    for (int off = D / 8; off > 0; off >>= 1) am = fmaxf(am, __shfl_xor(am, off));
+  }
+  if (!live) return;
+  if (a.rounding == JPT_ROUND_RNE) am = fmaxf(am, rnd<BF16_MATH>(1e-5f));
+  const float s = rnd<BF16_MATH>(am / 127.0f);
+  int code[4];
+  if (a.rounding == JPT_ROUND_TRUNC) {
 #pragma unroll
-    for (int c = 0; c < M; ++c) {
-      for (int off = D / 8; off > 0; off >>= 1) m[c] = fmaxf(m[c], __shfl_xor(m[c], off));
-      amax[c] = m[c];
+    for (int i = 0; i < 4; ++i) {
+      const float q = rnd<BF16_MATH>(x[i] / s);
+      code[i] = (q != q) ? 0 : static_cast<int>(q);  // 0/0 -> 0; cast truncates
+    }
+  } else {
+    const float r = rnd<BF16_MATH>(1.0f / s);
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float q = rnd<BF16_MATH>(x[i] * r);
+      code[i] = static_cast<int>(fminf(fmaxf(rintf(q), -128.f), 127.f));
     }
   }
-#pragma unroll
-  for (int c = 0; c < M; ++c) {
-    const int i0 = 4 * (threadIdx.x + 256 * c);
-    const int h = i0 / D, d = i0 - h * D;
-    float am = amax[c];
-    if (a.rounding == JPT_ROUND_RNE) am = fmaxf(am, rnd<BF16_MATH>(1e-5f));
-    const float s = rnd<BF16_MATH>(am / 127.0f);
-    int code[4];
-    if (a.rounding == JPT_ROUND_TRUNC) {
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float q = rnd<BF16_MATH>(x[c][i] / s);
-        code[i] = (q != q) ? 0 : static_cast<int>(q);  // 0/0 -> 0; cast truncates
-      }
-    } else {
-      const float r = rnd<BF16_MATH>(1.0f / s);
-#pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const float q = rnd<BF16_MATH>(x[c][i] * r);
-        code[i] = static_cast<int>(fminf(fmaxf(rintf(q), -128.f), 127.f));
-      }
-    }
-    const uint32_t packed = (static_cast<uint32_t>(code[0]) & 0xffu) | ((static_cast<uint32_t>(code[1]) & 0xffu) << 8) |
-                            ((static_cast<uint32_t>(code[2]) & 0xffu) << 16) | (static_cast<uint32_t>(code[3]) << 24);
-    if (stash) *reinterpret_cast<uint32_t*>(stash + src_base + i0) = packed;
-    if (write_cache) {
-      const int64_t row = paged
-          ? (static_cast<int64_t>(h) * p.total_pages + page) * p.page_size + at
-          : (static_cast<int64_t>(b) * H + h) * a.seq + at;
-      *reinterpret_cast<uint32_t*>(cache + row * D + d) = packed;
-    }
-    // one thread per scale group writes the scale
-    if (groups == 1 ? (c == 0 && threadIdx.x == 0) : d == 0) {
-      const int g = groups == 1 ? 0 : h;
-      if (stash_scale) store_from_f32(stash_scale, static_cast<int64_t>(b) * groups + g, a.scale_dtype, s);
-      if (write_cache && scale_out) {
-        const int64_t idx = paged
-            ? (static_cast<int64_t>(g) * p.total_pages + page) * p.page_size + at
-            : (static_cast<int64_t>(b) * groups + g) * a.seq + at;
-        store_from_f32(scale_out, idx, a.scale_dtype, s);
-      }
+  const uint32_t packed = (static_cast<uint32_t>(code[0]) & 0xffu) | ((static_cast<uint32_t>(code[1]) & 0xffu) << 8) |
+                          ((static_cast<uint32_t>(code[2]) & 0xffu) << 16) | (static_cast<uint32_t>(code[3]) << 24);
+  if (stash) *reinterpret_cast<uint32_t*>(stash + src_base + i0) = packed;
+  if (write_cache) {
+    const int64_t row = paged
+        ? (static_cast<int64_t>(h) * p.total_pages + page) * p.page_size + at
+        : (static_cast<int64_t>(b) * H + h) * a.seq + at;
+    *reinterpret_cast<uint32_t*>(cache + row * D + d) = packed;
+  }
+  // one thread per scale group writes the scale
+  if (groups == 1 ? threadIdx.x == 0 : d == 0) {
+    const int g = groups == 1 ? 0 : h;
+    if (stash_scale) store_from_f32(stash_scale, static_cast<int64_t>(b) * groups + g, a.scale_dtype, s);
+    if (write_cache && scale_out) {
+      const int64_t idx = paged
+          ? (static_cast<int64_t>(g) * p.total_pages + page) * p.page_size + at
+          : (static_cast<int64_t>(b) * groups + g) * a.seq + at;
+      store_from_f32(scale_out, idx, a.scale_dtype, s);
     }
   }
 }
@@ -349,21 +340,17 @@ int32_t launch_quant(const QuantParams& p, int32_t tokens, hipStream_t stream) {
   dim3 grid(tokens, 2);
   const jpt_quant_append_args& a = p.a;
   const int d4 = a.dim / 4;
-  const int runs = a.heads * a.dim / 1024;  // runs of four elements per thread
-  const bool vec = a.in_dtype == JPT_BF16 && a.heads * a.dim % 1024 == 0 && (runs == 1 || runs == 2 || runs == 4) &&
-                   a.dim % 4 == 0 &&
+  const int64_t runs = static_cast<int64_t>(a.heads) * d4;  // of four elements, one a thread
+  const bool vec = a.in_dtype == JPT_BF16 && a.dim % 4 == 0 && runs <= kMostRuns &&
                    (a.scale_heads == 1 || (d4 <= 64 && (d4 & (d4 - 1)) == 0)) &&
                    aligned(a.new_k, 8) && aligned(a.new_v, 8) && aligned(a.out_k, 4) && aligned(a.out_v, 4) &&
                    aligned(a.cache_k, 4) && aligned(a.cache_v, 4) && aligned(a.rope, 16);
   if (vec) {
-    const bool bf = a.scale_dtype == JPT_BF16;
-#define JPT_LAUNCH_VEC(M)                                                                          \
-  if (bf) hipLaunchKernelGGL((quant_append_vec_kernel<true, M>), grid, dim3(256), 0, stream, p);   \
-  else hipLaunchKernelGGL((quant_append_vec_kernel<false, M>), grid, dim3(256), 0, stream, p)
-    if (runs == 1) { JPT_LAUNCH_VEC(1); }
-    else if (runs == 2) { JPT_LAUNCH_VEC(2); }
-    else { JPT_LAUNCH_VEC(4); }
-#undef JPT_LAUNCH_VEC
+    const dim3 block(static_cast<unsigned>((runs + 63) / 64 * 64));
+    if (a.scale_dtype == JPT_BF16)
+      hipLaunchKernelGGL(quant_append_vec_kernel<true>, grid, block, 0, stream, p);
+    else
+      hipLaunchKernelGGL(quant_append_vec_kernel<false>, grid, block, 0, stream, p);
     return launch_status("quant_append_vec_kernel");
   }
   if (p.a.scale_dtype == JPT_BF16)
