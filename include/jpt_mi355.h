@@ -264,7 +264,8 @@ int32_t jpt_prefill_insert_layers(const jpt_prefill_insert_args* args,
  * elements (src_head_stride 0 = tokens * dim), the DEVICE array of its n_pages
  * page ids and its token count.  Equivalent to one jpt_prefill_insert a prompt
  * (and done that way for shapes the one-launch kernel does not take: it
- * needs bf16 prompts, int8 pages, heads * dim == 1024). */
+ * needs bf16 prompts, int8 pages, dim / 8 a power of two up to 64 and
+ * heads * dim <= 8192). */
 typedef struct {
   const void* src_k;
   const void* src_v;
