@@ -474,10 +474,9 @@ __global__ void __launch_bounds__(kThreads, kWavesPerSimd) attn_decode_kernel(Fa
   __shared__ __attribute__((aligned(16))) int sm_items_all[kGroups][kListedItems][8];
   // page ids of the item being issued and of the next one (paged caches)
   __shared__ int sm_pages_all[PAGED ? kGroups : 1][2][kStagedPages];
-  // masked calls: an item's live tiles, a bit each, and their number; positions of the tile in a ring slot that count
+  // masked calls: an item's live tiles, a bit each, and their number
   __shared__ __attribute__((aligned(16))) uint8_t sm_live_all[MASK ? kGroups : 1][MASK ? kMappedItems : 1][MASK ? kMappedTiles / 8 : 4];
   __shared__ __attribute__((aligned(16))) int sm_n_live_all[MASK ? kGroups : 1][MASK ? kMappedItems : 1][4];  // counted by each of the four waves
-  __shared__ int sm_valid_all[MASK ? kGroups : 1][C::kSlots];
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int hw_wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform, and known to be
@@ -520,6 +519,7 @@ __global__ void __launch_bounds__(kThreads, kWavesPerSimd) attn_decode_kernel(Fa
   // are equal mod 8 when the grid is a multiple of 8.
   const int G = kGroups * static_cast<int>(gridDim.x);
   const int worker = static_cast<int>(blockIdx.x) + group * static_cast<int>(gridDim.x);
+  const bool round_dies = MASK && (G / 8) % a.kv_heads == 0;  // see item_index
   // Work entries of the plan (its merge entries follow them; see the producer).
   // The producer wave asks for its first kListedItems records before anything
   // looks at this count (the index is kept inside the entry array): count and
@@ -529,7 +529,7 @@ __global__ void __launch_bounds__(kThreads, kWavesPerSimd) attn_decode_kernel(Fa
   if (wave == kConsumers) {
     const int j = (lane & 1) ? (G - 1 - worker) : worker;
     const int i = lane * G + j;
-    const int entry = MASK ? i / a.kv_heads : ((i >> 3) / a.kv_heads) * 8 + (i & 7);  // see item_index
+    const int entry = round_dies ? i / a.kv_heads : ((i >> 3) / a.kv_heads) * 8 + (i & 7);  // see item_index
     const int4* en = reinterpret_cast<const int4*>(p.entries + min(entry, p.total_items / a.kv_heads - 1));
     listed0 = en[0];
     listed1 = en[1];
@@ -560,12 +560,14 @@ __global__ void __launch_bounds__(kThreads, kWavesPerSimd) attn_decode_kernel(Fa
   // that each has a share of every entry (half of the positions live, us for eight
   // layers: 8 slots x 32 heads x 1024 bf16 178 -> 159, 64 slots x 8 heads x 2048 int8 359
   // -> 345).
-  // The two groups of a workgroup still have one head of entries half a round apart.
+  // The two groups of a workgroup still have one head of entries half a round apart, and a worker the items of the
+  // same entries, in the same order, that it would have had - where a round is whole entries; elsewhere the order is
+  // the other one.
   auto item_index = [&](int k, int* entry, int* h) -> bool {
     const int j = (k & 1) ? (G - 1 - worker) : worker;
     const int i = k * G + j;
-    const int m = MASK ? i : i >> 3;
-    *entry = MASK ? m / a.kv_heads : (m / a.kv_heads) * 8 + (i & 7);
+    const int m = round_dies ? i : i >> 3;
+    *entry = round_dies ? m / a.kv_heads : (m / a.kv_heads) * 8 + (i & 7);
     *h = m % a.kv_heads;
     return k < n_rounds && i < n_ids && *entry < n_entries;
   };
@@ -587,7 +589,6 @@ __global__ void __launch_bounds__(kThreads, kWavesPerSimd) attn_decode_kernel(Fa
   int (*const sm_pages)[kStagedPages] = sm_pages_all[PAGED ? group : 0];
   auto& sm_live = sm_live_all[MASK ? group : 0];
   auto& sm_n_live = sm_n_live_all[MASK ? group : 0];
-  int* const sm_valid = sm_valid_all[MASK ? group : 0];
   auto unpack_item = [&](int4 e0, int4 e1) -> Item {
     Item it;
     it.slot = __builtin_amdgcn_readfirstlane(e0.x);
@@ -1036,7 +1037,6 @@ __global__ void __launch_bounds__(kThreads, kWavesPerSimd) attn_decode_kernel(Fa
           __builtin_amdgcn_global_load_lds((global_ptr)(tv + off), (lds_ptr)(slot + C::kTileBytes + j * 1024), 16, 0, kStreamOnce);
         }
       }
-      if (MASK) lds_poke(&sm_valid[fill_slot], valid);
       char* side = slot + 2 * C::kTileBytes;
       if (SCALE) {
         if (lane < 2 * kHalf) __builtin_amdgcn_global_load_lds((global_ptr)sc, (lds_ptr)side, 4, 0, kStreamOnce);
@@ -1357,10 +1357,9 @@ __global__ void __launch_bounds__(kThreads, kWavesPerSimd) attn_decode_kernel(Fa
     // One body for every tile: what only the new token's tile or a chunk's last,
     // partly filled tile need sits behind wave-uniform branches, so that the
     // accumulators live in the same registers whichever way a tile goes.
+    const bool partial = valid != kTile;
     const int s = t % C::kSlots;
     if (!wait_for(&sm_filled[s], t / C::kSlots + 1)) return false;
-    if (MASK) valid = __builtin_amdgcn_readfirstlane(sm_valid[s]);  // which of the item's tiles it is, the producer knows
-    const bool partial = valid != kTile;
     char* slot = ring + s * C::kSlotBytes;
     const char* side = slot + 2 * C::kTileBytes;
     JPT_TL(if (tl_first == 0) tl_first = tl_now(); ++tl_tiles;)
@@ -1578,6 +1577,7 @@ __global__ void __launch_bounds__(kThreads, kWavesPerSimd) attn_decode_kernel(Fa
   };
 
   int base = 0;   // stream number of the current item's tile 0
+  int whole = 0;  // the same were every tile in the stream (masked calls: which consumer's a tile is)
   int q_seq = 0;  // items with tiles so far
   int seq = 0;    // valid items so far
   for (int k = 0; k < n_rounds; ++k) {
@@ -1633,12 +1633,44 @@ __global__ void __launch_bounds__(kThreads, kWavesPerSimd) attn_decode_kernel(Fa
     accw = f32x4{0.f, 0.f, 0.f, 0.f};
     m_run = -INFINITY;
     l_run = 0.f;
-    // this consumer's tiles: stream numbers congruent to its index
-    for (int ti = (wave + kConsumers - base % kConsumers) % kConsumers; ti < nt; ti += kConsumers) {
-      if (wide_new && ti == 1 && nt - n_cache == 2) continue;  // read by the consumer of tile 0
-      const bool is_new = ti < nt - n_cache;  // the new token comes first
-      const int valid = is_new ? 1 : MASK ? kTile : min(kTile, cur.count - (ti - (nt - n_cache)) * kTile);  // masked: see consume_tile
-      if (!consume_tile(base + ti, valid, is_new)) return;
+    if constexpr (MASK) {
+      // This consumer's tiles: those of the item's, live or not, whose number in the stream of all tiles is congruent to
+      // its index.  Leaving tiles out so changes no bit: each of those left meets the running maximum that it would have
+      // met (a tile that a mask leaves nothing of moves neither maximum nor sums), and a ring's live tiles, which are
+      // consecutive, still go round the consumers.
+      const int first = (wave + kConsumers - whole % kConsumers) % kConsumers, n_new = nt - n_cache, n_all = all_tiles(cur);
+      const bool map = mapped(cur, k);
+      int at = 0, before = n_new;    // cache tiles [at - 32, at) are under work; live ones before them, and the new token's
+      uint32_t live = 0, mine = 0;   // of them, those that are attended; those of these that are this consumer's and left
+      bool is_new = first < n_new && !(wide_new && first == 1);  // the new token comes first; its second tile is read by the consumer of its first
+      for (;;) {
+        int t = base + first, valid = 1;
+        if (!is_new) {
+          while (mine == 0 && at < n_all) {
+            before += __builtin_popcount(live);
+            live = map ? static_cast<uint32_t>(lds_peek_uniform(reinterpret_cast<const int*>(&sm_live[k][at / 8]))) : ~0u;
+            if (n_all - at < 32) live &= (1u << (n_all - at)) - 1;
+            mine = live & (0x49249249u << ((first + 2 * (n_new + at)) % kConsumers));  // every third bit, from the first such tile on
+            at += 32;
+          }
+          if (mine == 0) break;
+          const int bit = __builtin_ctz(mine);
+          mine &= mine - 1;
+          t = base + before + __builtin_popcount(live & ((1u << bit) - 1));
+          valid = min(kTile, cur.count - (at - 32 + bit) * kTile);
+        }
+        if (!consume_tile(t, valid, is_new)) return;
+        is_new = false;
+      }
+      whole += item_tiles(cur, n_all);
+    } else {
+      // this consumer's tiles: stream numbers congruent to its index
+      for (int ti = (wave + kConsumers - base % kConsumers) % kConsumers; ti < nt; ti += kConsumers) {
+        if (wide_new && ti == 1 && nt - n_cache == 2) continue;  // read by the consumer of tile 0
+        const bool is_new = ti < nt - n_cache;  // the new token comes first
+        const int valid = is_new ? 1 : min(kTile, cur.count - (ti - (nt - n_cache)) * kTile);
+        if (!consume_tile(base + ti, valid, is_new)) return;
+      }
     }
     if (keep) {  // this consumer had the new token's tile
       keep = false;

@@ -69,6 +69,38 @@ def test_what_a_mask_leaves_out_is_left_out(b, hq, hkv, s, kind, mask):
   assert torch.all(got.cpu()[few][(~live).expand_as(want)] == 0) and torch.all(gl.cpu()[few][~live] == 0) and torch.all(torch.isneginf(gm.cpu()[few][~live]))
 
 
+@pytest.mark.parametrize("mask", ["window", "single", "edges", "sparse"])
+@pytest.mark.parametrize("b,hq,hkv,s,kind", [
+    (8, 32, 32, 1024, "bf16"), (64, 32, 8, 2048, "int8_f32"), (5, 32, 4, 2080, "int8_bf16"), (40, 20, 5, 512, "bf16"), (200, 12, 12, 256, "int8_bf16"),
+    (3, 8, 8, 9216, "int8_f32"), (200, 32, 32, 96, "bf16")])
+def test_leaving_tiles_out_changes_no_bit(b, hq, hkv, s, kind, mask):
+  """float32's lowest value at one position of a tile makes it a tile that is read, whose weights are all 0: the same
+  outputs and statistics as where nothing of it is left and it is not read."""
+  from jetstream_pt_amd import attention_kernel as ak
+  g = torch.Generator().manual_seed(b * s + hkv)
+  k, v, ks, vs = (None if x is None else x.repeat((b // 4 + 1, 1, 1, 1))[:b].to(DEV) for x in caches(g, min(b, 4), hkv, s, kind))
+  q = torch.randn((b, hq, 1, 128), generator=g).to(torch.bfloat16).to(DEV)
+  left_out = masks(g, mask, b, s)
+  read = left_out.clone()
+  tiles = read.view(b, s // 32, 32)
+  tiles[..., 7][torch.isneginf(tiles).all(-1)] = torch.finfo(torch.float32).min
+  assert not torch.equal(left_out, read)
+  got, want = (ak.flash_attention(q, k, v, 0, ks, vs, m.reshape(b, 1, 1, s).to(DEV)) for m in (left_out, read))
+  assert torch.equal(got[0].view(torch.int16), want[0].view(torch.int16))
+  assert torch.equal(got[1][0], want[1][0]) and torch.equal(got[1][1], want[1][1])
+
+
+@pytest.mark.parametrize("b,hq,hkv,s", [(90, 5, 5, 1120), (200, 12, 12, 256), (64, 32, 8, 2048)])
+def test_a_mask_of_zeros_changes_no_bit(b, hq, hkv, s):
+  """... nor does the order of the heads under a mask."""
+  from jetstream_pt_amd import attention_kernel as ak
+  g = torch.Generator().manual_seed(b + s)
+  k, v = (x.repeat((b // 4 + 1, 1, 1, 1))[:b].to(DEV) for x in caches(g, 4, hkv, s, "bf16")[:2])
+  q = torch.randn((b, hq, 1, 128), generator=g).to(torch.bfloat16).to(DEV)
+  got, want = (ak.flash_attention(q, k, v, 0, None, None, m) for m in (torch.zeros((b, 1, 1, s), device=DEV), None))
+  assert torch.equal(got[0], want[0]) and torch.equal(got[1][1], want[1][1])
+
+
 def test_a_tile_with_a_nan_is_not_left_out():
   from jetstream_pt_amd import attention_kernel as ak
   g = torch.Generator().manual_seed(5)
