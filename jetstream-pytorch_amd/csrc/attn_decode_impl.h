@@ -519,7 +519,6 @@ __global__ void __launch_bounds__(kThreads, kWavesPerSimd) attn_decode_kernel(Fa
   // are equal mod 8 when the grid is a multiple of 8.
   const int G = kGroups * static_cast<int>(gridDim.x);
   const int worker = static_cast<int>(blockIdx.x) + group * static_cast<int>(gridDim.x);
-  const bool round_dies = MASK && (G / 8) % a.kv_heads == 0;  // see item_index
   // Work entries of the plan (its merge entries follow them; see the producer).
   // The producer wave asks for its first kListedItems records before anything
   // looks at this count (the index is kept inside the entry array): count and
@@ -529,7 +528,7 @@ __global__ void __launch_bounds__(kThreads, kWavesPerSimd) attn_decode_kernel(Fa
   if (wave == kConsumers) {
     const int j = (lane & 1) ? (G - 1 - worker) : worker;
     const int i = lane * G + j;
-    const int entry = round_dies ? i / a.kv_heads : ((i >> 3) / a.kv_heads) * 8 + (i & 7);  // see item_index
+    const int entry = ((i >> 3) / a.kv_heads) * 8 + (i & 7);
     const int4* en = reinterpret_cast<const int4*>(p.entries + min(entry, p.total_items / a.kv_heads - 1));
     listed0 = en[0];
     listed1 = en[1];
@@ -555,19 +554,11 @@ __global__ void __launch_bounds__(kThreads, kWavesPerSimd) attn_decode_kernel(Fa
   // (entry, head) with all heads of an entry on ids of equal i % 8: workgroup
   // ids go round-robin over the 8 XCDs, so an entry's scales and page-table
   // row are fetched into one L2 only.  Unused entries give invalid items.
-  // Under a mask the plan does not know how much of an entry there is to do, and a
-  // die with the long slots would be the launch: heads go round the dies there, so
-  // that each has a share of every entry (half of the positions live, us for eight
-  // layers: 8 slots x 32 heads x 1024 bf16 178 -> 159, 64 slots x 8 heads x 2048 int8 359
-  // -> 345).
-  // The two groups of a workgroup still have one head of entries half a round apart, and a worker the items of the
-  // same entries, in the same order, that it would have had - where a round is whole entries; elsewhere the order is
-  // the other one.
   auto item_index = [&](int k, int* entry, int* h) -> bool {
     const int j = (k & 1) ? (G - 1 - worker) : worker;
     const int i = k * G + j;
-    const int m = round_dies ? i : i >> 3;
-    *entry = round_dies ? m / a.kv_heads : (m / a.kv_heads) * 8 + (i & 7);
+    const int m = i >> 3;
+    *entry = (m / a.kv_heads) * 8 + (i & 7);
     *h = m % a.kv_heads;
     return k < n_rounds && i < n_ids && *entry < n_entries;
   };
