@@ -88,9 +88,13 @@ constexpr int kStreamOnce = 2;  // the NT bit of the instruction's cache-policy 
 constexpr int kListedItems = 64;     // a worker's first items, read into LDS at start
 constexpr int kStagedPages = 64;     // page ids of an item kept in LDS (later pages are read one by one)
 // Masked calls: a worker's first kMappedItems items have a bit a tile, set where the mask leaves something of it to
-// attend (items of more than kMappedTiles tiles, and later ones, are attended tile by tile).
+// attend (items of more than kMappedTiles tiles, and later ones, are attended tile by tile).  LDS sets the number: the
+// maps of ten items leave the int8 kernel of 5 to 16 rows 0.4 KB of its 160, and an item more is 72 bytes.
 constexpr int kMappedItems = 10;
-constexpr int kMappedTiles = 256;
+constexpr int kMappedTiles = 256;  // (32 bytes of map: 8192 positions, more than a chunk of most batches)
+// Tiles of the first item that are asked for before its map is there: what a worker gets of the memory's rate until then.
+constexpr int kEarlyTiles = 2;
+constexpr int kLooks = 2;          // blocks of 256 mask values a wave asks for at a time (4 and 8: no faster, and more code ahead of the stream)
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLn2 = 0.6931471805599453f;
 
@@ -476,7 +480,8 @@ __global__ void __launch_bounds__(kThreads, kWavesPerSimd) attn_decode_kernel(Fa
   __shared__ int sm_pages_all[PAGED ? kGroups : 1][2][kStagedPages];
   // masked calls: an item's live tiles, a bit each, and their number
   __shared__ __attribute__((aligned(16))) uint8_t sm_live_all[MASK ? kGroups : 1][MASK ? kMappedItems : 1][MASK ? kMappedTiles / 8 : 4];
-  __shared__ __attribute__((aligned(16))) int sm_n_live_all[MASK ? kGroups : 1][MASK ? kMappedItems : 1][4];  // counted by each of the four waves
+  __shared__ int sm_n_live_all[MASK ? kGroups : 1][MASK ? kMappedItems : 1];
+  __shared__ int sm_looked_all[MASK ? kGroups : 1];  // waves that have done their part of records, line and maps
 
   const int tid = threadIdx.x, lane = tid & 63;
   const int hw_wave = __builtin_amdgcn_readfirstlane(tid >> 6);  // wave-uniform, and known to be
@@ -502,6 +507,10 @@ __global__ void __launch_bounds__(kThreads, kWavesPerSimd) attn_decode_kernel(Fa
   if (tid < kGroups * C::kQBufs) (&sm_qtaken_all[0][0])[tid] = 0;
 
   if (tid == 0) sm_abort = 0;
+  if constexpr (MASK) {
+    if (tid < kGroups * kMappedItems) (&sm_n_live_all[0][0])[tid] = 0;
+    if (tid < kGroups) sm_looked_all[tid] = 0;
+  }
   JPT_TL(
   int* const tl_rec = reinterpret_cast<int*>(reinterpret_cast<char*>(p.status) + 1024) +
       ((static_cast<int>(blockIdx.x) * kGroups + group) * 4 + (wave == kConsumers ? 0 : wave + 1)) * 4;
@@ -525,7 +534,7 @@ __global__ void __launch_bounds__(kThreads, kWavesPerSimd) attn_decode_kernel(Fa
   // records are in flight together, one memory latency for both.
   const int n_entries = load_uniform(p.status + kStateEntries);
   int4 listed0 = make_int4(-1, 0, 0, 0), listed1 = make_int4(0, 0, 0, 0);
-  if (wave == kConsumers) {
+  if (MASK || wave == kConsumers) {
     const int j = (lane & 1) ? (G - 1 - worker) : worker;
     const int i = lane * G + j;
     const int entry = ((i >> 3) / a.kv_heads) * 8 + (i & 7);
@@ -614,94 +623,23 @@ __global__ void __launch_bounds__(kThreads, kWavesPerSimd) attn_decode_kernel(Fa
   auto mapped = [&](const Item& it, int k) { return MASK && k < kMappedItems && it.count <= kMappedTiles * kTile; };
   auto cache_tiles = [&](const Item& it, int k) {
     if (!mapped(it, k)) return all_tiles(it);
-    const i32x4 live = lds_peek4(&sm_n_live[k][0]);
-    return __builtin_amdgcn_readfirstlane(live[0] + live[1] + live[2] + live[3]);
+    return lds_peek_uniform(&sm_n_live[k]);
   };
   auto item_tiles = [&](const Item& it, int n_cache) {
     return n_cache + ((has_new && it.start == 0 && !(to_pages && it.len == 0)) ? (wide_new ? 2 : 1) : 0);
   };
-  if (wave == kConsumers) {
+  if (MASK) __syncthreads();  // the counters are clear: the records follow as the maps below do
+  if (MASK || wave == kConsumers) {
     int entry, h;
     if (!item_index(lane, &entry, &h)) listed0 = make_int4(-1, 0, 0, 0);
+    listed1.z = h;
+  }
+  if (wave == kConsumers) {
     // slot, start, count, part | n_chunks, head, valid, slot length
     *reinterpret_cast<int4*>(&sm_items[lane][0]) = listed0;
-    *reinterpret_cast<int4*>(&sm_items[lane][4]) = make_int4(listed1.x, h, listed0.x >= 0 ? 1 : 0, listed1.y);
+    *reinterpret_cast<int4*>(&sm_items[lane][4]) = make_int4(listed1.x, listed1.z, listed0.x >= 0 ? 1 : 0, listed1.y);
   }
-  if constexpr (MASK) {
-    // The step's line, where this launch writes it: the rows of the heads and slots whose chunk holds its position,
-    // by the workgroup that then reads them, before it does: consumer 1 the keys', consumer 2 the values', beside the
-    // other two waves' look through the mask.  (Eight layers of 64 slots x 8 heads, int8: 368 us with the quantiser's
-    // launch ahead, 344 so.)
-    const bool lined = NEW == kNewNone && p.line_k != nullptr;
-    if (lined && (wave == 1 || wave == 2)) {
-      const bool is_v = wave == 2;
-      for (int k = 0; k < n_rounds; ++k) {
-        const Item it = fetch(k);
-        if (!it.valid) continue;
-        const int at = load_uniform(p.line_pos + (p.line_count == 1 ? 0 : it.slot));
-        if (at < it.start || at >= it.start + it.count) continue;
-        const int64_t row = static_cast<int64_t>(it.slot) * a.kv_heads + it.h;
-        char* const to = static_cast<char*>(is_v ? a.v : a.k) + (row * a.seq + at) * C::kRowBytes;
-        if constexpr (std::is_same<KV, int8_t>::value) {
-          constexpr bool kBf16Math = SCALE == kScaleBF16;
-          const char* const rows = static_cast<const char*>(is_v ? p.line_v : p.line_k) + static_cast<int64_t>(it.slot) * a.kv_heads * (kD * 2);
-          const float* const rope = p.line_rope && !is_v ? p.line_rope + static_cast<int64_t>(it.slot) * kD : nullptr;
-          float x0, x1;
-          // the scale goes over all heads, or over the head's own elements
-          float scale = rows_max(row_max(token_absmax(rows, it.h, a.scale_heads == 1 ? a.kv_heads : 0, rope, lane, x0, x1)));
-          reinterpret_cast<uint16_t*>(to)[lane] = token_codes<kBf16Math>(x0, x1, p.line_rounding, scale);
-          if (lane == 0)  // one scale for all heads: every head's workgroup writes it, the same, before it reads it
-            store_from_f32(is_v ? a.v_scale : a.k_scale,
-                           (static_cast<int64_t>(it.slot) * a.scale_heads + (a.scale_heads == 1 ? 0 : it.h)) * a.seq + at,
-                           kBf16Math ? JPT_BF16 : JPT_F32, scale);
-        } else {
-          const uint32_t* from = reinterpret_cast<const uint32_t*>(static_cast<const char*>(is_v ? p.line_v : p.line_k) + row * C::kRowBytes);
-          reinterpret_cast<uint32_t*>(to)[lane] = from[lane];
-        }
-      }
-    }
-    // Which tiles of this worker's items the mask leaves anything of: a tile that it leaves nothing of is neither
-    // loaded nor computed.  The mask's rows (L2's after the first head) are looked through by four waves of the group,
-    // two where there is a line, 1024 positions a wave and trip to memory, before the stream starts: the first load goes
-    // out at 4.2 us instead of 2.2.  Attention alone, us, all / half / 15 % of the positions live: 8 slots x 32 heads x
-    // 1024 bf16 25.5 -> 26.5 / 19 / 13, 64 slots x 8 heads x 2048 int8 51 -> 50.5 / 38.5 / 20, 160 slots x 32 heads x 512 bf16
-    // 199 -> 204 / 130 / 59.  What is left is the unit with the longest slots: 1.5 us a tile and consumer.
-    const int n_items = min(n_rounds, kMappedItems);
-    const int lookers = lined ? 2 : 4, looker = !lined ? wave : wave == 0 ? 1 : wave == kConsumers ? 0 : -1;
-    const int per_item = n_items == 1 ? lookers : n_items == 2 ? lookers / 2 : 1;  // waves
-    for (int k = 0; k < n_items; ++k) {
-      int n_live = 0;
-      if (looker >= 0 && k % (lookers / per_item) == looker / per_item) {
-        const Item it = fetch(k);
-        const float* const row = static_cast<const float*>(a.mask) + it.slot * a.mask_stride_b + it.start + 4 * lane;
-        const int blocks = it.valid && mapped(it, k) ? (it.count + 255) / 256 : 0;
-        for (int b0 = looker % per_item; b0 < blocks; b0 += 4 * per_item) {
-          float4 x[4];
-#pragma unroll
-          for (int u = 0; u < 4; ++u) {
-            const int at = 256 * (b0 + u * per_item);  // (a chunk starts at a tile and a row is whole tiles: the four are in it)
-            x[u] = make_float4(-INFINITY, -INFINITY, -INFINITY, -INFINITY);
-            if (at + 4 * lane < it.count) x[u] = *reinterpret_cast<const float4*>(row + at);
-          }
-#pragma unroll
-          for (int u = 0; u < 4; ++u) {
-            const int block = b0 + u * per_item, left = it.count - 256 * block - 4 * lane;  // a NaN counts
-            const uint64_t set = __ballot((left > 0 && x[u].x != -INFINITY) || (left > 1 && x[u].y != -INFINITY) ||
-                                          (left > 2 && x[u].z != -INFINITY) || (left > 3 && x[u].w != -INFINITY));
-            // eight lanes a tile
-            const uint64_t tiles = __ballot(lane < 8 && ((set >> (8 * (lane & 7))) & 0xff) != 0);
-            if (block < blocks) {
-              if (lane == 0) sm_live[k][block] = static_cast<uint8_t>(tiles);
-              n_live += __popcll(tiles);
-            }
-          }
-        }
-      }
-      if (lane == 0) sm_n_live[k][wave] = n_live;
-    }
-    __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));  // the lines are where the loads behind the barrier find them
-  }
-  __syncthreads();
+  if (!MASK) __syncthreads();
   // A wave gives up: the other waves of the workgroup see the flag at their
   // next wait and leave too, and the host finds the sticky word in the
   // workspace's state block (jpt_attn_status).
@@ -722,6 +660,105 @@ __global__ void __launch_bounds__(kThreads, kWavesPerSimd) attn_decode_kernel(Fa
     }
     return true;
   };
+
+  // Masked calls: the step's line, where this launch writes it, and which tiles of this worker's first items the mask
+  // leaves anything of.  A tile that it leaves nothing of is neither loaded nor computed - but the first kEarlyTiles of the
+  // first item, which the producer asks for at once, while the mask's rows (L2's after the first head) are on their way to
+  // the consumers, who have nothing to do yet.  (A launch that writes a line has no early tiles, and its producer looks
+  // too.)  Attention alone, us, all tiles read -> so, with all / half / 15 % of the positions live: 8 slots x 32 heads x 1024
+  // bf16 25.0 -> 25.6 / 19.6 / 11.2, 64 x 8 x 2048 int8 49.5 -> 51.0 / 39.9 / 23.4, 160 x 32 x 512 bf16 203 -> 205 / 130 / 59,
+  // 96 x 32 x 1024 int8 125 -> 127 / 85 / 42, 4 x 8 x 2048 bf16 20.8 -> 20.6 / 20.8 / 19.3.  What is left is the unit with the
+  // longest slots.
+  const bool lined = MASK && NEW == kNewNone && p.line_k != nullptr;
+  // (a line is written before any group of the workgroup reads: both groups count on one counter)
+  int* const sm_looked = &sm_looked_all[MASK && !lined ? group : 0];
+  const int looking = lined ? kGroups * kGroupWaves : kGroupWaves;
+  auto early_tiles = [&](int count) { return lined ? 0 : min(kEarlyTiles, (count + kTile - 1) / kTile); };
+  if constexpr (MASK) {
+    // lane k has item k's record
+    const bool listed = listed0.x >= 0;
+    const int slot = listed ? listed0.x : 0, start = listed0.y, count = listed ? listed0.z : 0;
+    // The line: the rows of the heads and slots whose chunk holds its position, by the workgroup that then reads them,
+    // before it does: consumer 1 the keys', consumer 2 the values', beside the other two waves' look through the mask.
+    // All records and all positions are asked for at once.
+    if (lined && (wave == 1 || wave == 2)) {
+      const bool is_v = wave == 2;
+      const int places = listed ? p.line_pos[p.line_count == 1 ? 0 : slot] : -1;
+      const uint64_t here = __ballot(listed && places >= start && places < start + count);
+      for (int k = 0; k < n_rounds; ++k) {
+        int of, h, at;
+        if (k < kListedItems) {
+          if (((here >> k) & 1) == 0) continue;
+          of = __builtin_amdgcn_readlane(slot, k);
+          h = __builtin_amdgcn_readlane(listed1.z, k);
+          at = __builtin_amdgcn_readlane(places, k);
+        } else {
+          const Item it = fetch(k);
+          of = it.slot;
+          h = it.h;
+          at = it.valid ? load_uniform(p.line_pos + (p.line_count == 1 ? 0 : of)) : -1;
+          if (!it.valid || at < it.start || at >= it.start + it.count) continue;
+        }
+        const int64_t row = static_cast<int64_t>(of) * a.kv_heads + h;
+        char* const to = static_cast<char*>(is_v ? a.v : a.k) + (row * a.seq + at) * C::kRowBytes;
+        if constexpr (std::is_same<KV, int8_t>::value) {
+          constexpr bool kBf16Math = SCALE == kScaleBF16;
+          const char* const rows = static_cast<const char*>(is_v ? p.line_v : p.line_k) + static_cast<int64_t>(of) * a.kv_heads * (kD * 2);
+          const float* const rope = p.line_rope && !is_v ? p.line_rope + static_cast<int64_t>(of) * kD : nullptr;
+          float x0, x1;
+          // the scale goes over all heads, or over the head's own elements
+          float scale = rows_max(row_max(token_absmax(rows, h, a.scale_heads == 1 ? a.kv_heads : 0, rope, lane, x0, x1)));
+          reinterpret_cast<uint16_t*>(to)[lane] = token_codes<kBf16Math>(x0, x1, p.line_rounding, scale);
+          if (lane == 0)  // one scale for all heads: every head's workgroup writes it, the same, before it reads it
+            store_from_f32(is_v ? a.v_scale : a.k_scale,
+                           (static_cast<int64_t>(of) * a.scale_heads + (a.scale_heads == 1 ? 0 : h)) * a.seq + at,
+                           kBf16Math ? JPT_BF16 : JPT_F32, scale);
+        } else {
+          const uint32_t* from = reinterpret_cast<const uint32_t*>(static_cast<const char*>(is_v ? p.line_v : p.line_k) + row * C::kRowBytes);
+          reinterpret_cast<uint32_t*>(to)[lane] = from[lane];
+        }
+      }
+    }
+    if (lined ? wave == 0 || wave == kConsumers : wave != kConsumers) {
+      // a wave takes every `step`-th of all items' blocks of 256 positions, kLooks a trip to memory
+      const int looker = lined ? (wave == 0 ? 0 : 1) : wave, step = lined ? 2 : kConsumers;
+      const int n_items = min(n_rounds, kMappedItems);
+      const int early = early_tiles(__builtin_amdgcn_readfirstlane(count));
+      const int looked_at = lane < n_items && count <= kMappedTiles * kTile ? count : 0, blocks = (looked_at + 255) / 256;
+      const int most = __builtin_amdgcn_readfirstlane(static_cast<int>(row_max(static_cast<float>(blocks))));  // (the items are in the first row of lanes)
+      const int log_most = most > 1 ? 32 - __builtin_clz(most - 1) : 0;
+      const int n_blocks = most > 0 ? n_items << log_most : 0;
+      for (int i0 = looker; i0 < n_blocks; i0 += kLooks * step) {
+        f32x4 x[kLooks];
+#pragma unroll
+        for (int u = 0; u < kLooks; ++u) {
+          const int i = i0 + u * step, k = i >> log_most, at = (i & ((1 << log_most) - 1)) * 256 + 4 * lane;
+          x[u] = f32x4{-INFINITY, -INFINITY, -INFINITY, -INFINITY};
+          // (a chunk starts at a tile and a row is whole tiles: the four are in it)
+          if (i < n_blocks && at < __builtin_amdgcn_readlane(looked_at, k))
+            x[u] = *reinterpret_cast<const f32x4*>(static_cast<const float*>(a.mask) + __builtin_amdgcn_readlane(slot, k) * a.mask_stride_b +
+                                                   __builtin_amdgcn_readlane(start, k) + at);
+        }
+#pragma unroll
+        for (int u = 0; u < kLooks; ++u) {
+          const int i = i0 + u * step, k = i >> log_most, block = i & ((1 << log_most) - 1);
+          if (i >= n_blocks || block >= __builtin_amdgcn_readlane(blocks, k)) continue;
+          const int left = __builtin_amdgcn_readlane(looked_at, k) - 256 * block - 4 * lane;  // a NaN counts
+          const uint64_t set = __ballot((left > 0 && x[u][0] != -INFINITY) || (left > 1 && x[u][1] != -INFINITY) ||
+                                        (left > 2 && x[u][2] != -INFINITY) || (left > 3 && x[u][3] != -INFINITY));
+          // eight lanes a tile
+          unsigned tiles = static_cast<unsigned>(__ballot(lane < 8 && ((set >> (8 * (lane & 7))) & 0xff) != 0));
+          if (i == 0) tiles |= (1u << early) - 1;
+          if (lane == 0) {
+            sm_live[k][block] = static_cast<uint8_t>(tiles);
+            __hip_atomic_fetch_add(&sm_n_live[k], __builtin_popcount(tiles), __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_WORKGROUP);
+          }
+        }
+      }
+    }
+    if (lined) __builtin_amdgcn_s_waitcnt(vmcnt_imm(0));  // the lines are where the loads behind this find them
+    if (lane == 0) __hip_atomic_fetch_add(sm_looked, 1, __ATOMIC_RELEASE, __HIP_MEMORY_SCOPE_WORKGROUP);
+  }
 
   // Partials travel between workgroups on different XCDs, each behind an L2 of
   // its own, without a device-wide fence: they are written through to memory and
@@ -1043,7 +1080,9 @@ __global__ void __launch_bounds__(kThreads, kWavesPerSimd) attn_decode_kernel(Fa
     };
 
     int q_seq = 0;  // items with tiles so far: only those have their query rows staged
-    for (int k = 0; k < n_rounds; ++k) {
+    bool looked = !MASK;  // the maps are there, and the step's line
+    bool ahead = false;   // the first item's early tiles are what this turn is for: the next is for the rest of it
+    for (int k = 0; k < n_rounds; k += ahead ? 0 : 1) {
       Item cur;
       if (k < kListedItems) {
         const i32x4 e0 = lds_peek4(&sm_items[k][0]), e1 = lds_peek4(&sm_items[k][4]);
@@ -1051,9 +1090,13 @@ __global__ void __launch_bounds__(kThreads, kWavesPerSimd) attn_decode_kernel(Fa
       } else {
         cur = fetch(k);
       }
+      const int early = MASK && k == 0 && cur.valid ? early_tiles(cur.count) : 0;
+      ahead = early > 0 && !looked && !ahead;
+      if (!looked && !ahead && !(looked = wait_counter(sm_looked, looking, 0))) return;
       if (!cur.valid) continue;
       const int hs = a.scale_heads == 1 ? 0 : cur.h;
-      const int n_cache = cache_tiles(cur, k), nt = item_tiles(cur, n_cache);
+      const int n_cache = ahead ? early : cache_tiles(cur, k), nt = item_tiles(cur, n_cache);
+      const int first = ahead ? 0 : early;  // query rows and the new token go with the early tiles
       // rows of the item's first position in the key/value and scale tensors
       const char *kt = nullptr, *vt = nullptr;
       int64_t srow = 0;
@@ -1083,7 +1126,7 @@ __global__ void __launch_bounds__(kThreads, kWavesPerSimd) attn_decode_kernel(Fa
       }
       // an item's query rows travel ahead of its first tile: loads complete
       // in order, so they are in LDS when any of its tiles is handed over
-      if (nt > 0 && !issue_q(cur, q_seq++)) return;
+      if (nt > 0 && first == 0 && !issue_q(cur, q_seq++)) return;
       if (PAGED && k + 1 < n_rounds) {
         // page ids of the next item, so that they have landed when it starts
         Item nxt;
@@ -1102,7 +1145,7 @@ __global__ void __launch_bounds__(kThreads, kWavesPerSimd) attn_decode_kernel(Fa
       }
       // The step's new token is the item's first tile: the consumer that gets it
       // has the rest of the item to make up for the extra work it can carry.
-      if (nt > n_cache) {
+      if (nt > n_cache && first == 0) {
         const int64_t row = static_cast<int64_t>(cur.slot) * a.kv_heads + cur.h;
         const char* tk = static_cast<const char*>(a.new_k) + row * C::kRowBytes;
         const char* tv = static_cast<const char*>(a.new_v) + row * C::kRowBytes;
@@ -1126,15 +1169,19 @@ __global__ void __launch_bounds__(kThreads, kWavesPerSimd) attn_decode_kernel(Fa
           return;
         }
       }
-      uint32_t live_bits = 0;  // masked: of the live tiles from live_next - 32 on, those still to be issued
+      const float* const mask_at = MASK ? static_cast<const float*>(a.mask) + cur.slot * a.mask_stride_b + cur.start : nullptr;
+      const bool map = !ahead && mapped(cur, k);
+      int from = 0;            // masked: the tile that kt and the like are at
+      uint32_t live_bits = 0;  // of the live tiles from live_next - 32 on, those still to be issued
       int live_next = 0;
-      for (int nth = 0; nth < n_cache; ++nth) {
+      for (int nth = first; nth < n_cache; ++nth) {
         int ct = nth;
-        if (MASK && mapped(cur, k)) {
+        if (MASK && map) {
           while (live_bits == 0) {  // (there are n_cache bits in all)
             live_bits = static_cast<uint32_t>(lds_peek_uniform(reinterpret_cast<const int*>(&sm_live[k][live_next / 8])));
             const int left = all_tiles(cur) - live_next;  // bytes past the item's end hold nothing
             if (left < 32) live_bits &= (1u << left) - 1;
+            if (live_next == 0) live_bits &= ~0u << first;
             live_next += 32;
           }
           ct = live_next - 32 + __builtin_ctz(live_bits);
@@ -1158,14 +1205,15 @@ __global__ void __launch_bounds__(kThreads, kWavesPerSimd) attn_decode_kernel(Fa
           vt = static_cast<const char*>(a.v) + row0 * C::kRowBytes;
           ts = static_cast<int64_t>(hs) * a.total_pages * a.page_size + in_pool;
         }
-        const float* mk = MASK ? static_cast<const float*>(a.mask) + cur.slot * a.mask_stride_b + t0 : nullptr;
-        if (MASK) {
-          const int64_t in_item = static_cast<int64_t>(ct) * kTile;
-          if (!issue_tile(kt + in_item * C::kRowBytes, vt + in_item * C::kRowBytes, scale_lane + (srow + in_item) * kEs, mk, valid, false)) return;
-          continue;
+        if (MASK) {  // on to tile ct
+          const uint32_t by = static_cast<uint32_t>(ct - from);
+          from = ct;
+          kt += by * C::kTileBytes;
+          vt += by * C::kTileBytes;
+          ts = srow += by * kTile;
         }
-        if (!issue_tile(kt, vt, scale_lane + ts * kEs, mk, valid, false)) return;
-        if (!PAGED) {
+        if (!issue_tile(kt, vt, scale_lane + ts * kEs, MASK ? mask_at + ct * kTile : nullptr, valid, false)) return;
+        if (!PAGED && !MASK) {
           kt += kTile * C::kRowBytes;
           vt += kTile * C::kRowBytes;
           srow += kTile;
@@ -1567,6 +1615,7 @@ __global__ void __launch_bounds__(kThreads, kWavesPerSimd) attn_decode_kernel(Fa
     return true;
   };
 
+  if (MASK && !wait_for(sm_looked, looking)) return;
   int base = 0;   // stream number of the current item's tile 0
   int whole = 0;  // the same were every tile in the stream (masked calls: which consumer's a tile is)
   int q_seq = 0;  // items with tiles so far
@@ -1630,28 +1679,20 @@ __global__ void __launch_bounds__(kThreads, kWavesPerSimd) attn_decode_kernel(Fa
       // met (a tile that a mask leaves nothing of moves neither maximum nor sums), and a ring's live tiles, which are
       // consecutive, still go round the consumers.
       const int first = (wave + kConsumers - whole % kConsumers) % kConsumers, n_new = nt - n_cache, n_all = all_tiles(cur);
+      // the new token comes first; its second tile is read by the consumer of its first
+      if (has_new && first < n_new && !(wide_new && first == 1) && !consume_tile(base + first, 1, true)) return;
       const bool map = mapped(cur, k);
-      int at = 0, before = n_new;    // cache tiles [at - 32, at) are under work; live ones before them, and the new token's
-      uint32_t live = 0, mine = 0;   // of them, those that are attended; those of these that are this consumer's and left
-      bool is_new = first < n_new && !(wide_new && first == 1);  // the new token comes first; its second tile is read by the consumer of its first
-      for (;;) {
-        int t = base + first, valid = 1;
-        if (!is_new) {
-          while (mine == 0 && at < n_all) {
-            before += __builtin_popcount(live);
-            live = map ? static_cast<uint32_t>(lds_peek_uniform(reinterpret_cast<const int*>(&sm_live[k][at / 8]))) : ~0u;
-            if (n_all - at < 32) live &= (1u << (n_all - at)) - 1;
-            mine = live & (0x49249249u << ((first + 2 * (n_new + at)) % kConsumers));  // every third bit, from the first such tile on
-            at += 32;
-          }
-          if (mine == 0) break;
+      const int in_last = cur.count - (n_all - 1) * kTile;
+      int third = (first + 2 * n_new) % kConsumers;  // of the item's cache tiles, the first that is this consumer's
+      for (int at = 0, before = base + n_new; at < n_all; at += 32) {
+        uint32_t live = map ? static_cast<uint32_t>(lds_peek_uniform(reinterpret_cast<const int*>(&sm_live[k][at / 8]))) : ~0u;
+        if (n_all - at < 32) live &= (1u << (n_all - at)) - 1;
+        for (uint32_t mine = live & (0x49249249u << third); mine != 0; mine &= mine - 1) {  // every third bit
           const int bit = __builtin_ctz(mine);
-          mine &= mine - 1;
-          t = base + before + __builtin_popcount(live & ((1u << bit) - 1));
-          valid = min(kTile, cur.count - (at - 32 + bit) * kTile);
+          if (!consume_tile(before + __builtin_popcount(live & ((1u << bit) - 1)), at + bit == n_all - 1 ? in_last : kTile, false)) return;
         }
-        if (!consume_tile(t, valid, is_new)) return;
-        is_new = false;
+        before += __builtin_popcount(live);
+        third = third == 2 ? 0 : third + 1;  // 32 is one less than a multiple of three
       }
       whole += item_tiles(cur, n_all);
     } else {
