@@ -442,12 +442,14 @@ int32_t jpt_attn_dense(const jpt_attn_args* args, void* stream);
 /* jpt_kv_scatter_lines of one layer's K and V - the step's rows line_k, line_v, (batch, kv_heads, 1,
  * dim) in the cache's dtype, to position pos[b] of their slots (pos[0] with a pos_count of 1; a
  * position outside the cache is not written) - followed by jpt_attn_dense, in one launch where the
- * streaming kernel takes the call under a mask.  args->new_k and args->lengths must be NULL. */
+ * streaming kernel takes the call under a mask and that is the faster way (up to batch * kv_heads of
+ * 2048).  args->new_k and args->lengths must be NULL. */
 int32_t jpt_attn_dense_line(const jpt_attn_args* args, const void* line_k, const void* line_v, const int32_t* pos,
                             int32_t pos_count, void* stream);
 /* jpt_kv_append_quant_i8 of the step's token (append, with a cache to write to) followed by
- * jpt_attn_dense, in one launch where the streaming kernel takes the call under a mask and both are
- * of one int8 cache.  args->new_k and args->lengths must be NULL. */
+ * jpt_attn_dense, in one launch where the streaming kernel takes the call under a mask, both are
+ * of one int8 cache and that is the faster way (up to batch * kv_heads^2 of 32768; of 8192 where the
+ * key is rotated).  args->new_k and args->lengths must be NULL. */
 int32_t jpt_attn_dense_append(const jpt_attn_args* args, const jpt_quant_append_args* append, void* stream);
 int32_t jpt_attn_paged(const jpt_attn_args* args, void* stream);
 /* jpt_attn_ragged with the workspace inside the library: a device array of

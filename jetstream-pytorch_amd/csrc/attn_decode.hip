@@ -917,10 +917,21 @@ int32_t jpt_attn_ragged_stash(const jpt_attn_args* args, void* stash_k, void* st
 }
 
 namespace {
-// The launch that attends writes the step's line where it looks through a mask first (see the streaming kernel), and
-// where a row shares no cache line of 128 bytes with its neighbours.
-bool writes_line(const jpt_attn_args& a, const void* line_k, const void* line_v) {
+// The launch that attends writes the step's line where it looks through a mask first (see the streaming kernel), where
+// a row shares no cache line of 128 bytes with its neighbours, and where that is the faster way: a worker writes the
+// lines of its items one after the other before its stream starts, and an int8 one takes the scale over the whole token
+// once for every KV head (batch * kv_heads^2 rows, the key's rotated too).  us a layer under a ring's mask, half of 1024
+// (from 2048 items on: of 512) positions live, in one launch / with the line's own ahead -
+//   rows:                  8 slots x 32 heads 20.7 / 22.5, 64 x 32 113.0 / 113.6, 96 x 16 78.8 / 78.9, 160 x 16 74.6 / 69.0;
+//   int8:                  8 x 32 16.0 / 19.5, 32 x 32 40.0 / 42.1, 96 x 16 51.0 / 53.7, 160 x 16 48.1 / 47.6, 96 x 32 54.6 / 51.6,
+//                          160 x 32 88.9 / 80.2;
+//   int8, keys rotated:    8 x 32 19.1 / 20.1, 32 x 16 26.2 / 27.9, 48 x 16 41.8 / 41.3, 160 x 8 50.5 / 50.6, 32 x 32 46.9 / 42.7,
+//                          160 x 32 125 / 81.
+// (A scale a head is less work; it goes by the same line.)
+bool writes_line(const jpt_attn_args& a, const void* line_k, const void* line_v, bool rotated) {
   using namespace jpt;
+  const int64_t items = static_cast<int64_t>(a.batch) * a.kv_heads;
+  if (a.kv_dtype == JPT_BF16 ? items > 2048 : items * a.kv_heads > (rotated ? 8192 : 32768)) return false;
   return attn_fast_supported(a, kDense) && a.mask != nullptr && aligned(a.k, 128) && aligned(a.v, 128) && aligned(line_k, 16) && aligned(line_v, 16);
 }
 int32_t check_line(const jpt_attn_args* args, const void* line_k, const void* line_v, const int32_t* pos, int32_t pos_count) {
@@ -936,7 +947,7 @@ int32_t jpt_attn_dense_line(const jpt_attn_args* args, const void* line_k, const
   using namespace jpt;
   const int32_t st = check_line(args, line_k, line_v, pos, pos_count);
   if (st != JPT_OK) return st;
-  if (args->kv_dtype == JPT_BF16 && writes_line(*args, line_k, line_v)) {
+  if (args->kv_dtype == JPT_BF16 && writes_line(*args, line_k, line_v, false)) {
     StepLine line;
     line.k = line_k;
     line.v = line_v;
@@ -967,7 +978,7 @@ int32_t jpt_attn_dense_append(const jpt_attn_args* args, const jpt_quant_append_
       q.v_scale == a.v_scale && q.batch == a.batch && q.heads == a.kv_heads && q.seq == a.seq && q.dim == a.dim &&
       q.scale_dtype == a.scale_dtype && q.scale_heads == a.scale_heads && (q.scale_heads == 1 || q.scale_heads == q.heads) &&
       q.out_k == nullptr && q.out_v == nullptr && (q.rounding == JPT_ROUND_TRUNC || q.rounding == JPT_ROUND_RNE) &&
-      aligned(q.rope, 16) && writes_line(a, q.new_k, q.new_v)) {
+      aligned(q.rope, 16) && writes_line(a, q.new_k, q.new_v, q.rope != nullptr)) {
     StepLine line;
     line.k = q.new_k;
     line.v = q.new_v;

@@ -115,11 +115,14 @@ def test_a_tile_with_a_nan_is_not_left_out():
 @pytest.mark.parametrize("count", ["one", "each"])
 @pytest.mark.parametrize("b,hq,hkv,s,kind,hs,rounding,rope", [
     (8, 32, 32, 1024, "bf16", 1, None, False), (3, 8, 2, 96, "bf16", 1, None, False), (200, 32, 32, 64, "bf16", 1, None, False),
+    (64, 32, 32, 64, "bf16", 1, None, False), (65, 32, 32, 64, "bf16", 1, None, False), (128, 16, 16, 64, "int8_bf16", 1, "rne", False),
+    (129, 16, 16, 64, "int8_f32", 1, "trunc", False), (128, 8, 8, 96, "int8_f32", 1, "trunc", True), (129, 8, 8, 96, "int8_bf16", 1, "rne", True),
     (5, 32, 8, 2048, "int8_f32", 1, "trunc", False), (5, 32, 8, 2048, "int8_bf16", 1, "rne", True), (3, 28, 4, 4096, "int8_bf16", 4, "trunc", True),
     (33, 64, 8, 512, "int8_f32", 8, "rne", False), (40, 32, 32, 64, "int8_bf16", 1, "trunc", True), (1, 8, 8, 32, "int8_bf16", 1, "rne", False)])
 def test_the_launch_that_attends_writes_the_line(b, hq, hkv, s, kind, hs, rounding, rope, count):
   """Cache, scales and output are those of the line's own launch followed by attention, bit for bit - at every place of a
-  tile and of a chunk, and outside the cache, where nothing is written."""
+  tile and of a chunk, and outside the cache, where nothing is written.  One launch up to 2048 bf16 items, to 32768
+  batch * kv_heads^2 int8, to 8192 with the key rotated; with 2048 items a worker has four records."""
   from jetstream_pt_amd import _ffi
   from jetstream_pt_amd import attention_kernel as ak
   g = torch.Generator().manual_seed(b * s + hq)
