@@ -265,7 +265,8 @@ int32_t jpt_prefill_insert_layers(const jpt_prefill_insert_args* args,
  * page ids and its token count.  Equivalent to one jpt_prefill_insert a prompt
  * (and done that way for shapes the one-launch kernel does not take: it
  * needs bf16 prompts, int8 pages, dim / 8 a power of two up to 64 and
- * heads * dim <= 8192). */
+ * heads * dim <= 8192, or one head of 1024).  A scale a head: up to 64
+ * heads, as in jpt_prefill_insert, or, here only, heads * dim == 1024. */
 typedef struct {
   const void* src_k;
   const void* src_v;

@@ -12,13 +12,21 @@ namespace jpt {
 namespace {
 
 constexpr int kPieces = 4;
-// How a workgroup's threads are laid out: heads x tokens x 2^lanes_log lanes of a row, `passes` heads a thread.
+// How a workgroup's threads are laid out: heads x tokens x 2^lanes_log lanes of a row, `passes` heads a thread; `along`:
+// `passes` tokens a thread instead, of the one head.
 struct RowSplit {
   int lanes_log, tokens_log, passes;
+  bool along = false;
+  constexpr int tokens_a_block() const { return (along ? passes : 1) << tokens_log; }
 };
+constexpr RowSplit kLlamaRows = {4, 3, 4}, kOneWideRow = {7, 1, kPieces, true};  // 8 heads of 128 elements; one of 1024
 // False: the shape is not taken (a row is a power of two of pieces up to 64, a token's pieces four a thread).
 bool split_rows(int heads, int dim, RowSplit* s) {
   const int lanes = dim / 8;
+  if (heads == 1 && lanes == 128 && dim % 8 == 0) {
+    *s = kOneWideRow;
+    return true;
+  }
   if (dim < 8 || dim % 8 != 0 || lanes > 64 || (lanes & (lanes - 1)) != 0 || heads < 1 || heads * lanes > 256 * kPieces) return false;
   s->lanes_log = 0;
   while ((1 << s->lanes_log) < lanes) ++s->lanes_log;
@@ -208,7 +216,7 @@ __global__ void __launch_bounds__(256) prefill_insert_kernel(InsertParams p) {
 // -> 18; 1x128, 900: 35.5 -> 9.4.
 // The `block`-th workgroup's tokens of the prompt `a` describes (tokens, page_ids, n_pages,
 // src_head_stride), read from src, written to dst / scale_out.
-template <bool BF16_MATH, int PASSES>
+template <bool BF16_MATH, int PASSES, bool ALONG = false>
 __device__ __forceinline__ void quant_insert_rows(const jpt_prefill_insert_args& a, const RowSplit split, const int H, const int D,
                                                   const uint16_t* src, char* dst, void* scale_out, int block) {
   typedef uint32_t u32x4 __attribute__((ext_vector_type(4)));
@@ -219,23 +227,33 @@ __device__ __forceinline__ void quant_insert_rows(const jpt_prefill_insert_args&
   const int groups = a.scale_heads;
   const int64_t head_stride = a.src_head_stride > 0 ? a.src_head_stride : static_cast<int64_t>(a.tokens) * D;
   const int piece = threadIdx.x & (lanes - 1), tq = (threadIdx.x >> split.lanes_log) & (tokens - 1);
-  const int h0 = (threadIdx.x >> (split.lanes_log + split.tokens_log)) * PASSES;  // the thread's heads: h0 .. h0 + PASSES - 1
-  const int t = block * tokens + tq, d = 8 * piece;
+  const int d = 8 * piece;
+  // the thread's heads: h0 .. h0 + PASSES - 1, of one token; ALONG: its tokens, of one head
+  const int h0 = (threadIdx.x >> (split.lanes_log + split.tokens_log)) * (ALONG ? 1 : PASSES);
+  constexpr int kTokens = ALONG ? PASSES : 1;
+  int t[kTokens];
+#pragma unroll
+  for (int j = 0; j < kTokens; ++j) t[j] = (block * kTokens + j) * tokens + tq;
 
   // addresses clamped into the prompt, results masked afterwards
-  const uint16_t* const from = src + static_cast<int64_t>(min(t, a.tokens - 1)) * D + d;
   u32x4 raw[PASSES];
 #pragma unroll
-  for (int j = 0; j < PASSES; ++j)
-    raw[j] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(from + min(h0 + j, H - 1) * head_stride));  // read once
-  const int page = paged ? a.page_ids[min(t, rows - 1) / a.page_size] : 0;
-  int64_t pool_row = -1;  // dense: position in the slot's row; paged: row in the pool; -1: nothing to write
-  if (t < rows) {
-    if (paged) {
-      if (page >= 0 && page < a.total_pages) pool_row = static_cast<int64_t>(page) * a.page_size + t % a.page_size;
-    } else {
-      const int at = (a.start + t) % a.seq;
-      pool_row = at < 0 ? at + a.seq : at;
+  for (int j = 0; j < PASSES; ++j) {
+    const uint16_t* const from = src + static_cast<int64_t>(min(t[ALONG ? j : 0], a.tokens - 1)) * D + d;
+    raw[j] = __builtin_nontemporal_load(reinterpret_cast<const u32x4*>(from + min(ALONG ? h0 : h0 + j, H - 1) * head_stride));  // read once
+  }
+  int64_t pool_row[kTokens];  // dense: position in the slot's row; paged: row in the pool; -1: nothing to write
+#pragma unroll
+  for (int j = 0; j < kTokens; ++j) {
+    const int page = paged ? a.page_ids[min(t[j], rows - 1) / a.page_size] : 0;
+    pool_row[j] = -1;
+    if (t[j] < rows) {
+      if (paged) {
+        if (page >= 0 && page < a.total_pages) pool_row[j] = static_cast<int64_t>(page) * a.page_size + t[j] % a.page_size;
+      } else {
+        const int at = (a.start + t[j]) % a.seq;
+        pool_row[j] = at < 0 ? at + a.seq : at;
+      }
     }
   }
   float m[PASSES];
@@ -246,8 +264,17 @@ __device__ __forceinline__ void quant_insert_rows(const jpt_prefill_insert_args&
     for (int i = 0; i < 4; ++i)
       m[j] = fmaxf(m[j], fmaxf(fabsf(__uint_as_float(raw[j][i] << 16)), fabsf(__uint_as_float(raw[j][i] & 0xffff0000u))));
   }
-  __shared__ float s_max[256];  // by (the threads' heads, token)
-  if (groups == 1) {
+  __shared__ float s_max[256];  // by (the threads' heads, token); ALONG: by (pass, token, wave of the row)
+  if constexpr (ALONG) {  // a row is two waves'
+#pragma unroll
+    for (int j = 0; j < PASSES; ++j) {
+      for (int off = 32; off > 0; off >>= 1) m[j] = fmaxf(m[j], __shfl_xor(m[j], off));
+      if ((piece & 63) == 0) s_max[4 * j + (threadIdx.x >> 6)] = m[j];
+    }
+    __syncthreads();
+#pragma unroll
+    for (int j = 0; j < PASSES; ++j) m[j] = fmaxf(s_max[4 * j + 2 * tq], s_max[4 * j + 2 * tq + 1]);
+  } else if (groups == 1) {
     // (a head clamped above is one that counts anyway)
 #pragma unroll
     for (int j = 1; j < PASSES; ++j) m[0] = fmaxf(m[0], m[j]);
@@ -262,15 +289,16 @@ __device__ __forceinline__ void quant_insert_rows(const jpt_prefill_insert_args&
     for (int j = 0; j < PASSES; ++j)
       for (int off = lanes / 2; off > 0; off >>= 1) m[j] = fmaxf(m[j], __shfl_xor(m[j], off));
   }
-  if (pool_row < 0) return;
+  if (!ALONG && pool_row[0] < 0) return;
   const int64_t head_rows = paged ? static_cast<int64_t>(a.total_pages) * a.page_size : a.seq;
-  const int64_t row0 = (paged ? 0 : static_cast<int64_t>(a.slot) * H * a.seq) + pool_row;
+  const int64_t row0 = paged ? 0 : static_cast<int64_t>(a.slot) * H * a.seq;
 #pragma unroll
   for (int j = 0; j < PASSES; ++j) {
-    const int h = h0 + j;
-    if (h >= H) break;
-    u32x2* out = reinterpret_cast<u32x2*>(dst + (row0 + h * head_rows) * D + d);
-    if (t >= a.tokens) {  // paged only: the tail of the last page is zero-filled
+    const int h = ALONG ? h0 : h0 + j, i_t = ALONG ? j : 0;
+    if (!ALONG && h >= H) break;
+    if (ALONG && (h >= H || pool_row[j] < 0)) continue;
+    u32x2* out = reinterpret_cast<u32x2*>(dst + (row0 + pool_row[i_t] + h * head_rows) * D + d);
+    if (t[i_t] >= a.tokens) {  // paged only: the tail of the last page is zero-filled
       *out = u32x2{0u, 0u};
       continue;
     }
@@ -295,19 +323,23 @@ __device__ __forceinline__ void quant_insert_rows(const jpt_prefill_insert_args&
                           code[4] | (code[5] << 8) | (code[6] << 16) | (code[7] << 24)};
     __builtin_nontemporal_store(packed, out);
     if (d == 0 && (groups != 1 || h == 0)) {
-      const int64_t idx = (paged ? 0 : static_cast<int64_t>(a.slot) * groups * a.seq) + (groups == 1 ? 0 : h) * head_rows + pool_row;
+      const int64_t idx = (paged ? 0 : static_cast<int64_t>(a.slot) * groups * a.seq) + (groups == 1 ? 0 : h) * head_rows + pool_row[i_t];
       store_from_f32(scale_out, idx, a.scale_dtype, s);
     }
   }
 }
 
-// LLAMA: 8 heads of 128 elements.  Numbers that the compiler knows, in a kernel of their own:
-// 1500 tokens, 16 layers 50.6 us a call, 52.8 through the other branch.
-template <bool BF16_MATH, bool LLAMA>
+// Two shapes have numbers that the compiler knows, in kernels of their own.  kLlama: 1500 tokens, 16 layers 50.6 us a call,
+// 52.8 through the other branch.  kOneWide, whose threads would have one piece each: 900 and 3000 tokens, 16 layers 30 and
+// 79 us (prefill_insert_kernel 57 and 176; this layout in the other branch 36 and 93, which cost that branch's shapes 3 % too).
+enum RowShape { kAnyShape, kLlama, kOneWide };
+template <bool BF16_MATH, RowShape SHAPE>
 __device__ __forceinline__ void quant_insert_block(const jpt_prefill_insert_args& a, const RowSplit& split, const uint16_t* src,
                                                    char* dst, void* scale_out, int block) {
-  if constexpr (LLAMA) {
-    quant_insert_rows<BF16_MATH, 4>(a, RowSplit{4, 3, 4}, 8, 128, src, dst, scale_out, block);
+  if constexpr (SHAPE == kLlama) {
+    quant_insert_rows<BF16_MATH, 4>(a, kLlamaRows, 8, 128, src, dst, scale_out, block);
+  } else if constexpr (SHAPE == kOneWide) {
+    quant_insert_rows<BF16_MATH, kPieces, true>(a, kOneWideRow, 1, 1024, src, dst, scale_out, block);
   } else {
     if (split.passes == 4) quant_insert_rows<BF16_MATH, 4>(a, split, a.heads, a.dim, src, dst, scale_out, block);
     else if (split.passes == 3) quant_insert_rows<BF16_MATH, 3>(a, split, a.heads, a.dim, src, dst, scale_out, block);
@@ -315,8 +347,11 @@ __device__ __forceinline__ void quant_insert_block(const jpt_prefill_insert_args
     else quant_insert_rows<BF16_MATH, 1>(a, split, a.heads, a.dim, src, dst, scale_out, block);
   }
 }
+RowShape row_shape(const jpt_prefill_insert_args& a, const RowSplit& split) {
+  return split.along ? kOneWide : a.heads == 8 && a.dim == 128 ? kLlama : kAnyShape;
+}
 
-template <bool BF16_MATH, bool LLAMA>
+template <bool BF16_MATH, RowShape SHAPE>
 __global__ void __launch_bounds__(256) prefill_insert_rows_kernel(InsertParams p) {
   const jpt_prefill_insert_args& a = p.a;
   const bool is_v = blockIdx.y == 1;
@@ -324,7 +359,7 @@ __global__ void __launch_bounds__(256) prefill_insert_rows_kernel(InsertParams p
   char* dst;
   void* scale_out;
   layer_tensors(p, blockIdx.z, is_v, 2, 1, a.scale_dtype == JPT_F32 ? 4 : 2, &src, &dst, &scale_out);
-  quant_insert_block<BF16_MATH, LLAMA>(a, p.split, static_cast<const uint16_t*>(src), dst, scale_out, blockIdx.x);
+  quant_insert_block<BF16_MATH, SHAPE>(a, p.split, static_cast<const uint16_t*>(src), dst, scale_out, blockIdx.x);
 }
 
 // Rows copied as they are, 16 bytes a piece: a workgroup takes 1024 consecutive pieces of one head's rows (16 KiB: 64
@@ -384,7 +419,7 @@ struct PromptsParams {
   jpt_insert_prompt prompt[kLaunchPrompts];
 };
 
-template <bool BF16_MATH, bool LLAMA>
+template <bool BF16_MATH, RowShape SHAPE>
 __global__ void __launch_bounds__(256) prefill_insert_prompts_kernel(PromptsParams p) {
   int r = 0;
   while (r + 1 < p.n_prompts && static_cast<int>(blockIdx.x) >= p.first_block[r + 1]) ++r;
@@ -400,7 +435,7 @@ __global__ void __launch_bounds__(256) prefill_insert_prompts_kernel(PromptsPara
   char* dst = static_cast<char*>(is_v ? a.dst_v : a.dst_k) + layer * a.dst_layer_stride;
   const int esz_scale = a.scale_dtype == JPT_F32 ? 4 : 2;
   void* scale_out = static_cast<char*>(is_v ? a.v_scale : a.k_scale) + layer * a.scale_layer_stride * esz_scale;
-  quant_insert_block<BF16_MATH, LLAMA>(a, p.split, src, dst, scale_out, static_cast<int>(blockIdx.x) - p.first_block[r]);
+  quant_insert_block<BF16_MATH, SHAPE>(a, p.split, src, dst, scale_out, static_cast<int>(blockIdx.x) - p.first_block[r]);
 }
 
 }  // namespace
@@ -473,11 +508,13 @@ int32_t insert_launch(const jpt_prefill_insert_args& a, const jpt_insert_layer* 
   if (rows == 0) return JPT_OK;
   if (quant && wide_ok && a.tokens > 0 && a.in_dtype == JPT_BF16 && split_rows(a.heads, a.dim, &p.split) &&
       (a.src_head_stride == 0 || a.src_head_stride % 8 == 0)) {
-    const int tb = 1 << p.split.tokens_log;
+    const int tb = p.split.tokens_a_block();
     const dim3 blocks((rows + tb - 1) / tb, 2, p.a.n_layers);
-    const bool llama = a.heads == 8 && a.dim == 128;
-    auto kernel = llama ? prefill_insert_rows_kernel<true, true> : prefill_insert_rows_kernel<true, false>;
-    if (a.scale_dtype == JPT_F32) kernel = llama ? prefill_insert_rows_kernel<false, true> : prefill_insert_rows_kernel<false, false>;
+    using Kernel = decltype(&prefill_insert_rows_kernel<true, kAnyShape>);
+    static constexpr Kernel kernels[2][3] = {
+        {prefill_insert_rows_kernel<false, kAnyShape>, prefill_insert_rows_kernel<false, kLlama>, prefill_insert_rows_kernel<false, kOneWide>},
+        {prefill_insert_rows_kernel<true, kAnyShape>, prefill_insert_rows_kernel<true, kLlama>, prefill_insert_rows_kernel<true, kOneWide>}};
+    const Kernel kernel = kernels[a.scale_dtype != JPT_F32][row_shape(a, p.split)];
     hipLaunchKernelGGL(kernel, blocks, dim3(256), 0, static_cast<hipStream_t>(stream), p);
     return launch_status("prefill_insert_rows_kernel");
   }
@@ -531,6 +568,7 @@ int32_t jpt_prefill_insert_prompts(const jpt_prefill_insert_args* args, const jp
   // the shapes the one-launch kernel takes; anything else goes prompt by prompt
   RowSplit split;
   bool wide = a.dst_dtype == JPT_I8 && a.in_dtype == JPT_BF16 && split_rows(a.heads, a.dim, &split) &&
+              // (more than 64 scales a token: what this call has always taken beside what jpt_prefill_insert takes)
               (a.scale_heads == 1 || (a.scale_heads == a.heads && (a.scale_heads <= 64 || a.heads * a.dim == 1024))) &&
               a.dst_k && a.dst_v && a.k_scale && a.v_scale && aligned(a.dst_k, 8) && aligned(a.dst_v, 8) &&
               a.dst_layer_stride % 8 == 0 && a.total_pages > 0 && a.page_size > 0 && n_layers <= 65535 &&
@@ -565,7 +603,7 @@ int32_t jpt_prefill_insert_prompts(const jpt_prefill_insert_args* args, const jp
     p.split = split;
     p.a.n_layers = n_layers;
     p.n_prompts = n_prompts - r0 < kLaunchPrompts ? n_prompts - r0 : kLaunchPrompts;
-    const int tb = 1 << split.tokens_log;
+    const int tb = split.tokens_a_block();
     int blocks = 0;
     for (int r = 0; r < p.n_prompts; ++r) {
       p.prompt[r] = prompts[r0 + r];
@@ -574,9 +612,11 @@ int32_t jpt_prefill_insert_prompts(const jpt_prefill_insert_args* args, const jp
     }
     p.first_block[p.n_prompts] = blocks;
     const dim3 grid(blocks, 2, n_layers);
-    const bool llama = a.heads == 8 && a.dim == 128;
-    auto kernel = llama ? prefill_insert_prompts_kernel<true, true> : prefill_insert_prompts_kernel<true, false>;
-    if (a.scale_dtype == JPT_F32) kernel = llama ? prefill_insert_prompts_kernel<false, true> : prefill_insert_prompts_kernel<false, false>;
+    using Kernel = decltype(&prefill_insert_prompts_kernel<true, kAnyShape>);
+    static constexpr Kernel kernels[2][3] = {
+        {prefill_insert_prompts_kernel<false, kAnyShape>, prefill_insert_prompts_kernel<false, kLlama>, prefill_insert_prompts_kernel<false, kOneWide>},
+        {prefill_insert_prompts_kernel<true, kAnyShape>, prefill_insert_prompts_kernel<true, kLlama>, prefill_insert_prompts_kernel<true, kOneWide>}};
+    const Kernel kernel = kernels[a.scale_dtype != JPT_F32][row_shape(a, split)];
     hipLaunchKernelGGL(kernel, grid, dim3(256), 0, static_cast<hipStream_t>(stream), p);
     const int32_t st = launch_status("prefill_insert_prompts_kernel");
     if (st != JPT_OK) return st;

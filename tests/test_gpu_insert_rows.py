@@ -11,10 +11,10 @@ from test_gpu_insert import DEV, run_both
 pytestmark = pytest.mark.gpu
 
 
-# one head; heads that do not fill a pass; three passes; a row of one piece and of 64; the most heads a token may have,
+# one head; heads that do not fill a pass; three passes; a row of one piece, of 64 and, of one head, of 128; the most heads a token may have,
 # one more than that, and rows that are no power of two (both: the general kernel)
 @pytest.mark.parametrize("heads,dim", [(1, 128), (3, 64), (5, 256), (24, 128), (40, 128), (64, 128), (65, 128), (16, 512),
-                                       (7, 8), (60, 8), (4, 96), (16, 64), (4, 256)])
+                                       (7, 8), (60, 8), (4, 96), (16, 64), (4, 256), (1, 1024), (3, 1024), (8, 1024), (9, 1024), (1, 2048)])
 @pytest.mark.parametrize("ring,position,prompt,scale_dtype", [(False, 0, 17, torch.bfloat16), (True, 5, 40, torch.float32)])
 def test_quantised_rows(heads, dim, ring, position, prompt, scale_dtype):
   run_both(ring, True, (2, heads, 64, dim, 2), prompt=prompt, seq_len=prompt - 3, slot=1, current_position=position,
@@ -60,7 +60,7 @@ def test_copied_pages(heads, dim, ps, tokens, dtype, shift):
       assert torch.equal(dpools[layer][which].cpu(), want)
 
 
-@pytest.mark.parametrize("heads,dim,scale_heads", [(3, 64, 3), (24, 128, 1), (64, 128, 64), (2, 512, 2), (4, 96, 1)])
+@pytest.mark.parametrize("heads,dim,scale_heads", [(3, 64, 3), (24, 128, 1), (64, 128, 64), (2, 512, 2), (4, 96, 1), (1, 1024, 1), (4, 1024, 1), (2, 1024, 2)])
 def test_quantised_pages(heads, dim, scale_heads):
   """One scale a token and one a (token, head), several prompts in one launch
   and one by one: the same pool, and the codes the oracle's quantiser gives.
