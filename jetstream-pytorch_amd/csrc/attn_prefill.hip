@@ -28,7 +28,7 @@
 // tiles that a mask changes, the diagonal of a causal one, come last and are done one
 // step after the other.  3500 rows: matrix pipe busy in 55 % of the SIMD time (38 % one
 // step after the other), at a clock of 1.9 GHz that the load leaves.
-// Outputs are rescaled only when a row's maximum has grown by 2^8 since they last were.
+// Outputs are rescaled only when a row's maximum has grown by 2^4 since they last were (kAhead).
 // What a causal mask leaves out is not computed: a pass over the mask (read
 // once, not once a head) first writes down, for every 32 rows x 64 positions,
 // whether anything there is live and whether anything there is not zero; dead
@@ -67,7 +67,10 @@ constexpr int kMaxTiles = 1024;  // tiles that fit the list in LDS: 65536 positi
 constexpr float kLog2e = 1.4426950408889634f;
 constexpr float kLn2 = 0.6931471805599453f;
 constexpr int64_t kL2Bytes = 4 << 20;  // of an XCD
-constexpr float kSlack = 8.f;
+// Weights and sums are relative to a reference that starts 2^kAhead above a row's maximum and moves when the maximum has
+// passed it: seldom (every step's move at heads of 256, 2000 rows: 84 -> 111 us; 4 -> 8: 85 -> 83), and no weight is ever above
+// 1, so that sums over large values overflow no earlier than relative to the maximum itself.
+constexpr float kAhead = 4.f;
 constexpr float kFarBelow = -1e37f;  // times log2(e) finite
 
 // what a mask block (32 rows x 64 positions) holds
@@ -300,7 +303,8 @@ __global__ void __launch_bounds__(64 * kWavesPerGroup, D == 256 ? 1 : 2) attn_pr
 #pragma unroll
     for (int i = 0; i < 16; ++i) o[d][i] = 0.f;
   // The row's maximum so far in log2 units, and as the scores are (what a mask may hold does not fit log2 units);
-  // what weights and sums are relative to: an earlier maximum, until the row's is 2^kSlack times that.
+  // what weights and sums are relative to: 2^kAhead times an earlier maximum, until the row's is above that (rows whose
+  // maximum is far below: the maximum).
   float ml_run = -INFINITY, m_run = -INFINITY, ml_ref = -INFINITY, m_ref = -INFINITY;
   float l_run = 0.f;  // this lane's share of the row sum
   const float c2 = fabsf(a.sm_scale), c2l = c2 * kLog2e;
@@ -466,9 +470,9 @@ __global__ void __launch_bounds__(64 * kWavesPerGroup, D == 256 ? 1 : 2) attn_pr
     ml_run = fmaxf(ml_run, tmax * c2l);
     if (MASK) m_run = fmaxf(m_run, tmax * c2);
     // (a loop of one turn: behind a branch the compiler would have o in two places, and move it at every tile)
-    for (int turn = __any(ml_run > ml_ref + kSlack) ? 1 : 0; turn; turn = nothing()) {
-      const float alpha = fast_exp2(ml_ref - (ml_run == -INFINITY ? 0.f : ml_run));
-      ml_ref = ml_run;
+    for (int turn = __any(ml_run > ml_ref) ? 1 : 0; turn; turn = nothing()) {
+      const float alpha = fast_exp2(ml_ref - (ml_run == -INFINITY ? 0.f : ml_run + kAhead));
+      ml_ref = ml_run + kAhead;
       m_ref = m_run;
       l_run *= alpha;
 #pragma unroll
@@ -543,15 +547,15 @@ __global__ void __launch_bounds__(64 * kWavesPerGroup, D == 256 ? 1 : 2) attn_pr
     tmax = fmaxf(tmax, other_half(tmax));
     ml_run = fmaxf(ml_run, tmax * kLog2e);
     float ml_use = ml_ref == -INFINITY ? 0.f : ml_ref, to_log2 = kLog2e;
-    bool move = ml_run > ml_ref + kSlack;
+    bool move = ml_run > ml_ref;
     if (MASK) {
       m_run = fmaxf(m_run, tmax);
       move = move || m_run < kFarBelow;
     }
     if (__any(move)) {
-      ml_use = ml_run == -INFINITY ? 0.f : ml_run;
+      ml_use = ml_run == -INFINITY ? 0.f : ml_run + kAhead;
       float alpha = fast_exp2(ml_ref - ml_use);
-      ml_ref = ml_run;
+      ml_ref = ml_run + kAhead;
       if (MASK) {
         // Rows whose largest score is near float32's lowest value (a mask may hold that): times log2(e) it may be
         // -infinity, and a row masked throughout would be empty instead of the mean of the values.

@@ -146,6 +146,27 @@ def test_maxima_that_rise(jump, heads):
     assert torch.allclose(gm.double().cpu(), wm, rtol=1e-3, atol=1e-4) and torch.allclose(gl.double().cpu(), wl, rtol=1e-3)
 
 
+@pytest.mark.parametrize("heads", [2, 336])
+@pytest.mark.parametrize("d", [64, 128, 256])
+@pytest.mark.parametrize("up", [3.0, 5.0, 7.5])
+def test_large_values_under_a_maximum_that_rises(up, d, heads):
+  """A value near bfloat16's largest whose score comes late and is 2^up times the weight of the others: its weight is at
+  most 1 in the sums, which so stay finite.  One bfloat16 rounding of the result."""
+  from jetstream_pt_amd import attention_kernel as ak
+  t, s, late = 130, 320, 200
+  q, k, v = torch.zeros((1, heads, t, d)), torch.zeros((1, heads, s, d)), torch.ones((1, heads, s, d))
+  q[..., 0] = 1.0
+  k[..., late, 0] = up * math.log(2) * math.sqrt(d)
+  v[..., late, ::3] = 2.0 ** 127
+  q, k, v = (x.to(torch.bfloat16) for x in (q, k, v))
+  mask = torch.zeros((1, 1, t, s))
+  mask[..., 300:310] = -math.inf
+  for m in (None, mask):
+    want, _, _ = OA.closed_form(q[:, :1], k[:, :1], v[:, :1], mask=None if m is None else m.expand(1, 1, t, s))
+    got = ak.dense_attention(q.to(DEV), k.to(DEV), v.to(DEV), mask=None if m is None else m.to(DEV)).double().cpu()
+    assert torch.all((got - want).abs() <= 2.0 ** -8 * want.abs())
+
+
 @pytest.mark.parametrize("scale", [-0.25, 0.0])
 @pytest.mark.parametrize("kind", [None, "causal"])
 def test_scales_that_are_not_positive(kind, scale):
