@@ -26,8 +26,8 @@
 // positions: 64 matrix instructions of 32 clocks each, 450 vector ones of 4 or,
 // exponentials, 16).  That holds for plain tiles, which all rows attend as they are;
 // tiles that a mask changes, the diagonal of a causal one, come last and are done one
-// step after the other.  3500 rows: matrix pipe busy in 55 % of the SIMD time (38 % one
-// step after the other), at a clock of 1.9 GHz that the load leaves.
+// step after the other.  3500 rows: matrix pipe busy in 46 % of the SIMD time (38 % one
+// step after the other).
 // Outputs are rescaled only when a row's maximum has grown by 2^4 since they last were (kAhead).
 // What a causal mask leaves out is not computed: a pass over the mask (read
 // once, not once a head) first writes down, for every 32 rows x 64 positions,
@@ -35,11 +35,11 @@
 // tiles are neither loaded nor computed, and all-zero tiles need no mask reads.
 //
 // Measured, causal, 32 query heads over 8 KV heads of 128, a call with its pass over
-// the mask, calls back to back, one step after the other -> side by side: 256 rows 20 ->
-// 13 us, 1024 rows 48 -> 31, 2048 rows 94 -> 82, 3500 rows with scales 245 -> 216; 16 heads of
-// 256, 2000 rows 169 -> 105 (12.3 ms for 1024 rows on the shape-generic kernel, one wave a
-// row, scalar dot products).  Outputs that are not the rounded exact value: 0.017-0.039 % over these
-// sizes, 0.017-0.041 % before.
+// the mask, calls back to back, one step after the other -> side by side: 256 rows 21 ->
+// 14 us, 1024 rows 46 -> 31, 2048 rows 93 -> 78, 3500 rows with scales 240 -> 218; 16 heads of
+// 256, 2000 rows 157 -> 85 (12.3 ms for 1024 rows on the shape-generic kernel, one wave a
+// row, scalar dot products).  Outputs that are not the rounded exact value: 0.021-0.042 % over eight
+// shapes, 0.018-0.046 % before.
 #include <math.h>
 
 #include <type_traits>
@@ -785,13 +785,26 @@ bool classes_pay(const jpt_attn_args& a) {
 }
 
 // Four waves over 128 query rows, or two and two over 64 rows and the halves of a tile's positions: twice the
-// workgroups, each half as long.  With enough workgroups of 128 rows for every compute unit's two places and a half
-// more the first reads keys and values half as often; with fewer the longest workgroup is the launch.  us a causal
-// call, 1 / 2 key waves: 32 query heads over 8 of 128 256 rows 16.6 / 13.4, 512 23.3 / 18.6, 1024 (256 workgroups of 128
-// rows) 38 / 31, 2048 (512) 81 / 84, 3500 (896) 193 / 201; 32 heads over 32 2100 rows (544) 116 / 112; 96 heads over 96
-// 700 rows (576) 52 / 50; 16 heads over 16 of 256 2000 rows (256) 127 / 105.  One block of 32 positions has no halves.
+// workgroups, each half as long, but keys and values are read twice as often.  That is the faster way where workgroups of
+// 128 would leave places empty (two a compute unit, one at heads of 256), or be a few more than there are: the longest
+// workgroup, or the second round of them, is the launch.  Under a mask workgroups are of unequal length, and halves pay
+// for longer.  us a call, 1 / 2 key waves, by workgroups of 128 over 256 compute units -
+//   128, mask (causal): 128 23.7 / 18.9, 256 37.6 / 30.8, 384 55.3 / 53.5, 448 66.6 / 66.8 and 116.7 / 113.9 (8 and 16 KV
+//     heads), 480 73.6 / 72.2, 512 79.1 / 80.5 (all places, once), 544 88.3 / 87.8 and 99 / 90 (8 and 32), 576 95.2 / 96.9 and
+//     106.4 / 103.0, 608 111.3 / 113.2, 640 112 / 116;
+//   128, none: 128 19.3 / 15.5, 256 39.7 / 40.6, 384 78.5 / 78.1, 448 94 / 109, 512 116 / 130, 544 164 / 162, 608 184 / 184;
+//   64, mask: 256 28.9 / 23.0, 448 44.4 / 39.7, 512 53.5 / 49.7, 576 63.1 / 59.2, 640 72.5 / 69.2, 768 95.7 / 94.6;
+//   64, none: 128 13.7 / 11.0, 384 50.8 / 46.7, 448 59.7 / 65.9, 512 70.8 / 76.4, 576 109 / 100, 640 122 / 114, 768 153 / 161;
+//   256, mask: 128 58.4 / 41.8, 256 105 / 86, 288 118 / 116, 320 131 / 136, 448 205 / 232;
+//   256, none: 128 56.2 / 41.1, 192 84 / 101, 256 121 / 138, 288 228 / 213, 320 252 / 235, 448 363 / 434.
+// One block of 32 positions has no halves.
 int32_t key_waves_for(const jpt_attn_args& a, int64_t workgroups) {
-  return a.seq > 32 && 2 * workgroups < 5 * compute_units() ? 2 : 1;
+  const int64_t places = static_cast<int64_t>(a.dim == 256 ? 1 : 2) * compute_units();
+  bool halves;
+  if (workgroups > places) halves = a.dim == 128 ? 8 * workgroups <= 9 * places : 4 * workgroups <= 5 * places;
+  else if (a.mask != nullptr) halves = a.dim != 128 || workgroups < places;
+  else halves = a.dim == 256 ? 2 * workgroups <= places : 4 * workgroups <= 3 * places;
+  return a.seq > 32 && halves ? 2 : 1;
 }
 
 template <int D, int SCALE, int MASK>

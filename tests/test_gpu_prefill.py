@@ -54,6 +54,12 @@ CASES = [  # b, hq, hkv, d, t, s, mask, scale heads (None: no scales), scale dty
     (5, 64, 8, 64, 130, 258, "causal", 1, torch.bfloat16),  # ... with one
     (40, 8, 1, 128, 129, 192, None, None, None),
     (11, 32, 4, 256, 129, 257, "causal", None, None),
+    (6, 64, 8, 64, 130, 130, "causal", None, None),         # either side of the limits between the two kinds of workgroups
+    (6, 64, 8, 64, 130, 258, "causal", 1, torch.bfloat16),
+    (28, 8, 4, 128, 130, 258, "causal", None, None),
+    (34, 8, 4, 128, 130, 130, None, 1, torch.float32),
+    (32, 8, 8, 128, 130, 200, None, None, None),
+    (12, 8, 8, 256, 130, 200, None, None, None),
 ]
 
 
