@@ -52,7 +52,7 @@ struct Layout {
 
 constexpr int kMaxPlanBatch = 4096;
 constexpr int kMaxChunksPerSlot = 256;
-constexpr int kMaxBins = 1024;         // entries of one round of the workers' walk: workers / kv_heads
+constexpr int kMaxBins = 512;          // entries of one round of the workers' walk: workers / kv_heads, two workers a unit
 constexpr int kDealtOneByOne = 512;  // entries dealt to the lightest bin one by one (about 0.12 us each)
 
 // Workers of the streaming kernel: two groups of waves on every compute unit.
@@ -108,7 +108,7 @@ unsigned plan_lds_bytes(int batch, int max_entries) { return 4u * (2u * batch + 
 // memory, every round of a bin cost a trip); a sum goes through a wave's shuffles before LDS; the keys are scanned four a
 // thread; a slot's equal chunks take their ranks with one atomic.  Measured, us a launch, before -> now: 1 slot of 700
 // positions 15.0 -> 10.9, 96 ragged slots of up to 2048 16.4 -> 12.6, of 1024 each 11.9 -> 8.7, 8 of up to 32768 22.1 ->
-// 16.8, 4000 of up to 256 55 -> 53 (whose launch needs 141 KB of LDS; 96 slots 28).
+// 16.8, 4000 of up to 256 55 -> 53 (whose launch needs 135 KB of LDS with one KV head; 96 slots with eight 22).
 // Exclusive prefix sum of `x` over the 256 threads of the planning workgroup;
 // *total gets the sum.
 __device__ __forceinline__ int plan_exclusive_scan(int x, int* total) {
@@ -554,8 +554,7 @@ plan_kernel(const int32_t* lengths, int batch, int seq_cap, int kv_heads, int ta
       const int cap = max(max_rounds - laps_after, 1);
       if (per_round <= 64) deal<1>(one_by_one, per_round, cap, s_bin_load, s_bin_rounds, s_rank_tiles, s_rank_place);
       else if (per_round <= 256) deal<4>(one_by_one, per_round, cap, s_bin_load, s_bin_rounds, s_rank_tiles, s_rank_place);
-      else if (per_round <= 512) deal<8>(one_by_one, per_round, cap, s_bin_load, s_bin_rounds, s_rank_tiles, s_rank_place);
-      else deal<16>(one_by_one, per_round, cap, s_bin_load, s_bin_rounds, s_rank_tiles, s_rank_place);
+      else deal<8>(one_by_one, per_round, cap, s_bin_load, s_bin_rounds, s_rank_tiles, s_rank_place);
     }
     __syncthreads();
   }
