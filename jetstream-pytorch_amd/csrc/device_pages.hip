@@ -96,7 +96,7 @@ dpam_reserve_insert_kernel(jpt_dpam d, const int32_t* slots, const int32_t* seq_
       len = seq_lens ? seq_lens[r0 + tid] : len_imm;
     }
     const bool bad = slot < 0 || slot >= d.batch || len < 0;
-    const int pages = bad ? -1 : (len + d.page_size - 1) / d.page_size;
+    const int pages = bad ? -1 : len / d.page_size + (len % d.page_size != 0);  // of any length
     s_slot[tid] = slot;
     s_len[tid] = len;
     s_n[tid] = pages > d.max_pages ? -1 : pages;

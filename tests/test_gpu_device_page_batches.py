@@ -48,3 +48,15 @@ def test_a_batch_equals_its_requests_one_by_one(batch, total, mp, n_req, kind):
     for s in slots:
       one.free_pages_resource_many(i32([s]))
     same(many, one)
+
+
+@pytest.mark.parametrize("n", [41, 2 ** 31 - 4, 2 ** 31 - 1])
+def test_lengths_that_no_slot_holds_are_refused(n):
+  """... up to the largest: the count of their pages does not wrap round."""
+  from jetstream_pt_amd import _ffi
+  from jetstream_pt_amd.page_attention_manager import DevicePageAttentionManager
+  pam = DevicePageAttentionManager(4, 64, 4, 10, device=DEV)
+  before = pam.page_indices.clone(), pam.lengths.clone(), pam.unused_page_ids().tolist()
+  pam.reserve_pages_insert_many(i32([1]), i32([n]))
+  assert torch.equal(pam.page_indices, before[0]) and torch.equal(pam.lengths, before[1]) and pam.unused_page_ids().tolist() == before[2]
+  assert pam.status() == _ffi.DPAM_OVERFLOW
