@@ -26,7 +26,7 @@
 // positions: 64 matrix instructions of 32 clocks each, 450 vector ones of 4 or,
 // exponentials, 16).  That holds for plain tiles, which all rows attend as they are;
 // tiles that a mask changes, the diagonal of a causal one, come last and are done one
-// step after the other.  3500 rows: matrix pipe busy in 46 % of the SIMD time (38 % one
+// step after the other.  3500 rows: matrix pipe busy in 47 % of the SIMD time (38 % one
 // step after the other).
 // Outputs are rescaled only when a row's maximum has grown by 2^4 since they last were (kAhead).
 // What a causal mask leaves out is not computed: a pass over the mask (read
