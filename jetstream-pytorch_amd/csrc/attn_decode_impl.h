@@ -780,30 +780,24 @@ __global__ void __launch_bounds__(kThreads, kWavesPerSimd) attn_decode_kernel(Fa
       asm volatile("global_store_dwordx2 %0, %1, off offset:512 sc0 sc1" : : "v"(row), "v"(st) : "memory");
     }
   };
-  // Rows of four partials at once (one memory latency for all); the caller's
+  // Rows of two partials at once (one memory latency for both); the caller's
   // wave has no other loads in flight.
   struct PartRow {
     f32x4 q0, q1;
     __attribute__((ext_vector_type(2))) float st;
   };
-  auto get_rows = [](const float* const (&row)[4], int lane_in_row, PartRow (&r)[4]) {
-    const float *at0 = row[0] + 4 * lane_in_row, *at1 = row[1] + 4 * lane_in_row, *at2 = row[2] + 4 * lane_in_row, *at3 = row[3] + 4 * lane_in_row;
-    asm volatile("global_load_dwordx4 %0, %12, off sc0 sc1\n\t"
-                 "global_load_dwordx4 %1, %12, off offset:256 sc0 sc1\n\t"
-                 "global_load_dwordx2 %2, %16, off offset:512 sc0 sc1\n\t"
-                 "global_load_dwordx4 %3, %13, off sc0 sc1\n\t"
-                 "global_load_dwordx4 %4, %13, off offset:256 sc0 sc1\n\t"
-                 "global_load_dwordx2 %5, %17, off offset:512 sc0 sc1\n\t"
-                 "global_load_dwordx4 %6, %14, off sc0 sc1\n\t"
-                 "global_load_dwordx4 %7, %14, off offset:256 sc0 sc1\n\t"
-                 "global_load_dwordx2 %8, %18, off offset:512 sc0 sc1\n\t"
-                 "global_load_dwordx4 %9, %15, off sc0 sc1\n\t"
-                 "global_load_dwordx4 %10, %15, off offset:256 sc0 sc1\n\t"
-                 "global_load_dwordx2 %11, %19, off offset:512 sc0 sc1\n\t"
+  auto get_rows = [](const float* row_a, const float* row_b, int lane_in_row, PartRow& ra, PartRow& rb) {
+    const float* at_a = row_a + 4 * lane_in_row;
+    const float* at_b = row_b + 4 * lane_in_row;
+    asm volatile("global_load_dwordx4 %0, %6, off sc0 sc1\n\t"
+                 "global_load_dwordx4 %1, %6, off offset:256 sc0 sc1\n\t"
+                 "global_load_dwordx2 %2, %7, off offset:512 sc0 sc1\n\t"
+                 "global_load_dwordx4 %3, %8, off sc0 sc1\n\t"
+                 "global_load_dwordx4 %4, %8, off offset:256 sc0 sc1\n\t"
+                 "global_load_dwordx2 %5, %9, off offset:512 sc0 sc1\n\t"
                  "s_waitcnt vmcnt(0)"
-                 : "=&v"(r[0].q0), "=&v"(r[0].q1), "=&v"(r[0].st), "=&v"(r[1].q0), "=&v"(r[1].q1), "=&v"(r[1].st), "=&v"(r[2].q0),
-                   "=&v"(r[2].q1), "=&v"(r[2].st), "=&v"(r[3].q0), "=&v"(r[3].q1), "=&v"(r[3].st)
-                 : "v"(at0), "v"(at1), "v"(at2), "v"(at3), "v"(row[0]), "v"(row[1]), "v"(row[2]), "v"(row[3])
+                 : "=&v"(ra.q0), "=&v"(ra.q1), "=&v"(ra.st), "=&v"(rb.q0), "=&v"(rb.q1), "=&v"(rb.st)
+                 : "v"(at_a), "v"(row_a), "v"(at_b), "v"(row_b)
                  : "memory");
   };
   // writes rows of outputs: 16 lanes a row, eight outputs a lane, the statistics by the row's first lane
@@ -845,25 +839,20 @@ __global__ void __launch_bounds__(kThreads, kWavesPerSimd) attn_decode_kernel(Fa
       const float* src = p.partials + (static_cast<int64_t>(it.part) * a.kv_heads + it.h) * rec + row * kPartFloats;
       float M = -INFINITY, L = 0.f;
       float o[8] = {0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f, 0.f};
-      for (int c0 = 0; c0 < it.n_chunks; c0 += 4) {  // four chunks a trip to memory (two: 1 slot of 8000 positions in 63 chunks 30.7 us for 26.8)
-        const float* from[4];
-#pragma unroll
-        for (int c = 0; c < 4; ++c) from[c] = src + min(c0 + c, it.n_chunks - 1) * step;
-        PartRow x[4];
-        get_rows(from, lane & 15, x);
-        float m[4], Mb = M;
-#pragma unroll
-        for (int c = 0; c < 4; ++c) {
-          m[c] = c0 + c < it.n_chunks ? x[c].st[0] : -INFINITY;
-          Mb = fmaxf(Mb, m[c]);
-        }
+      for (int c0 = 0; c0 < it.n_chunks; c0 += 2) {  // two chunks a trip to memory
+        const bool two = c0 + 1 < it.n_chunks;
+        PartRow x[2];
+        get_rows(src + c0 * step, src + (two ? c0 + 1 : c0) * step, lane & 15, x[0], x[1]);
+        const float m0 = x[0].st[0], m1 = two ? x[1].st[0] : -INFINITY;
+        const float Mb = fmaxf(M, fmaxf(m0, m1));
         const float keep_old = M == -INFINITY ? 0.f : fast_exp2(M - Mb);
         L *= keep_old;
 #pragma unroll
         for (int i = 0; i < 8; ++i) o[i] *= keep_old;
 #pragma unroll
-        for (int c = 0; c < 4; ++c) {
-          const float f = m[c] == -INFINITY ? 0.f : fast_exp2(m[c] - Mb);
+        for (int c = 0; c < 2; ++c) {
+          const float mc = c == 0 ? m0 : m1;
+          const float f = mc == -INFINITY ? 0.f : fast_exp2(mc - Mb);
           L += x[c].st[1] * f;
 #pragma unroll
           for (int i = 0; i < 4; ++i) {

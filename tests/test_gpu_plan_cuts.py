@@ -1,9 +1,6 @@
-"""How many chunks the planner cuts a slot in: never three where two groups of one workgroup can fold two, two up to 512
-positions, about 0.18 sqrt(positions) beyond - fewer where chunks rounded up to whole tiles cover the slot sooner - and by
-the batch's mean alone where the workgroups' groups do not pair.  Every plan has the properties the streaming kernel relies
-on and the host model's deal."""
-import math
-
+"""How many chunks the planner cuts a slot in: as many as the batch's mean chunk asks for and no fewer, whatever a merge costs
+- a consumer's largest softmax weight is exact, and a slot in fewer chunks has fewer of them.  Every plan has the properties
+the streaming kernel relies on and the host model's deal."""
 import numpy as np
 import pytest
 import torch
@@ -20,25 +17,19 @@ def chunks_of(lengths, kv_heads, seq):
   return [int(next(e for e in places if e[0] == slot)[4]) for slot in range(len(lengths))]
 
 
-def rule(n, chunk, pairing):
-  if n <= chunk:
-    return 1
-  nc = -(-n // chunk)
-  if pairing and nc > 2:
-    most = 2 if nc == 3 or n <= 512 else math.ceil(np.float32(0.18) * np.sqrt(np.float32(n)))
-    nc = min(nc, most)
-  tiles = -(-(-(-n // 32)) // nc)
-  return -(-n // (32 * tiles))
+def rule(lengths, kv_heads, seq):
+  mean = -(-sum(lengths) * kv_heads // (workers() * 5 // 4))
+  chunk = max(-(-max(mean, -(-seq // 256)) // 128) * 128, 128)
+  return [max(-(-n // chunk), 1) for n in lengths]
 
 
 @pytest.mark.parametrize("kv_heads", [1, 3, 8, 32])
 @pytest.mark.parametrize("n", [1, 128, 129, 256, 257, 384, 385, 512, 513, 640, 780, 781, 1200, 2047, 4000, 8191, 65536])
 def test_one_slot(n, kv_heads):
   check_plan([n], kv_heads, 65536)
-  w = workers()
-  pairing = w // kv_heads <= 512 and kv_heads * 16 <= w and (w // 16) % kv_heads == 0
-  chunk = max(-(-max(-(-n * kv_heads // (w * 5 // 4)), 256) // 128) * 128, 128)
-  assert chunks_of([n], kv_heads, 65536) == [rule(n, chunk, pairing)]
+  check_plan([n], kv_heads, 8192)
+  for seq in (65536, 8192):  # the shorter one: chunks of 128
+    assert chunks_of([min(n, seq)], kv_heads, seq) == rule([min(n, seq)], kv_heads, seq)
 
 
 @pytest.mark.parametrize("kv_heads,count", [(8, 32), (8, 3), (16, 24), (1, 160), (4, 118)])
@@ -46,4 +37,20 @@ def test_batches(kv_heads, count):
   rng = np.random.default_rng(count)
   lengths = rng.integers(1, 4096, size=count).tolist() + [700] * 5
   check_plan(lengths, kv_heads, 4096)
-  assert 3 not in chunks_of(lengths, kv_heads, 4096)
+  assert chunks_of(lengths, kv_heads, 4096) == rule(lengths, kv_heads, 4096)
+
+
+def test_a_mean_just_above_a_whole_number():
+  """One position more than 26240 an item, of more positions than float32 counts: chunks of 26368, and a slot between the two
+  is not cut."""
+  target = workers() * 5 // 4
+  lengths = [26300] + [24000] * 690
+  rest = target * 26240 + 1 - sum(lengths)
+  lengths += [20000] * (rest // 20000) + [rest % 20000]
+  assert rest > 0 and chunks_of(lengths, 1, 65536) == [1] * len(lengths)
+
+
+def test_the_largest_batch():
+  """Every slot's words and every record's are in LDS: 4096 slots with one KV head ask for the most."""
+  lengths = [(7 * i) % 300 for i in range(4096)]
+  assert chunks_of(lengths, 1, 512) == rule(lengths, 1, 512)
