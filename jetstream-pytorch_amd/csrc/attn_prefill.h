@@ -10,8 +10,6 @@ namespace prefill {
 typedef __attribute__((ext_vector_type(8))) __bf16 bf16x8;
 typedef __attribute__((ext_vector_type(4))) __bf16 bf16x4;
 typedef __attribute__((ext_vector_type(2))) __bf16 bf16x2;
-typedef __attribute__((ext_vector_type(8))) _Float16 f16x8;
-typedef __attribute__((ext_vector_type(2))) _Float16 f16x2;
 typedef __attribute__((ext_vector_type(16))) float f32x16;
 typedef __attribute__((address_space(3))) char* lds_char_ptr;
 
@@ -30,19 +28,6 @@ constexpr int64_t kL2Bytes = 4 << 20;  // of an XCD
 constexpr float kAhead = 4.f;
 constexpr float kFarBelow = -1e37f;  // times log2(e) finite
 
-// Values as float16: a tile's largest lies in [2^(kTop - 1), 2^kTop), and a weight of 1 goes in as 2^kWeightTop, so that
-// the largest of a row's, 2^-kAhead or more, keeps its second number among float16's normal ones.  (2^14 would leave more
-// room and cost more: the exponents' own rounding, at 14, was 20 % more outputs that are not the rounded exact value.)
-constexpr int kTop = 15;
-constexpr int kWeightTop = 6;
-// Outputs so far are in units of the tiles' exponents: a tile up to kSlack below them takes its weights that much lower,
-// at any other the outputs change units.  No exponents further apart than kApart: sums stay far from float32's ends.
-constexpr int kSlack = 2;
-constexpr int kApart = 40;
-constexpr int kTiny = -1000, kInexact = 1000, kFarExponent = 90;
-constexpr int kNoExp = -128;
-__device__ __forceinline__ int short_exp(int e) { return e < -kFarExponent || e > kFarExponent ? kNoExp : e; }
-
 // what a mask block (32 rows x 64 positions) holds
 constexpr int kLive = 1;     // some value that is not -inf
 constexpr int kNonZero = 2;  // some value that is not 0
@@ -60,11 +45,6 @@ struct PrefillParams {
   int32_t by_rows;          // workgroups in the order of their rows: the longest first
   int32_t xcd_units;        // compute units of an XCD, where two workgroups share one; or else more than there are
   int32_t mask_runs;        // runs of four mask values are aligned
-  // NULL, or the values as float16 numbers, and of every tile of them the power of two that they were divided by
-  // (kTiny: all zero; kInexact: some of them are not such numbers); see value_tile
-  const char* v16;
-  const int32_t* v_exp;
-  int32_t v_tiles;          // tiles a KV head
 };
 
 // Defined in attn_prefill_<D>.hip.

@@ -1,10 +1,12 @@
-"""GPU parity: prompts whose attention multiplies float16 copies of the values (enough workgroups of 128 rows, heads of
-64 and 128, no scales), against the float64 closed form.  A tile's values are copied relative to a power of two of their
-own, so the values here differ between tiles, within them and from any such number.
+"""GPU parity of prompts with enough workgroups of 128 rows to take every place (heads of 64 and 128, no scales), against the
+float64 closed form: values whose units differ between tiles and within them, and rows whose small weights meet many
+positions, or large values, so that they matter as much as the largest one does.
 
 Bound: half an ulp of the bf16 output, and in units of 2^-24 of the output with every value's magnitude in its place: a
 sum's roundings, one a position at most, and 32 for the score (below 8: its product, scale and difference to the maximum),
-exp2, the weight's two float16 numbers (2^-22) and the division."""
+exp2, the weight and the division.  Where weights are small by construction the units are the same for all sizes, 4096: 2^-12
+of the output, an eighth of half its ulp, and as many roundings as a row of 6000 positions has (3000 in a lane's sum of weights,
+1125 in the products' sums)."""
 
 import math
 
@@ -84,3 +86,46 @@ def test_float16_values_of_slots_of_their_own_lengths():
   got, _ = ak.ragged_mha(q.to(DEV), k.to(DEV), v.to(DEV), 0, None, end.to(DEV))
   over = (got.double().cpu().reshape(want.shape) - want).abs() / float32_bound(want, total, s + 32)
   assert torch.all(over <= 1.0), float(over.max())
+
+
+def check(q, k, v, causal, units=4096):
+  from jetstream_pt_amd import attention_kernel as ak
+  t, s = q.shape[2], k.shape[2]
+  mask = torch.full((1, 1, t, s), -math.inf).triu(1 + s - t).to(torch.bfloat16) if causal else None
+  got, _ = ak.flash_attention(q.to(DEV), k.to(DEV), v.to(DEV), 0, None, None, None if mask is None else mask.to(DEV), normalize_var=False)
+  hkv, rep = k.shape[1], q.shape[1] // k.shape[1]
+  # (a slot and a query head of each KV head: the closed form is slow)
+  q1, rows = q[:1, ::rep], None if mask is None else mask.expand(1, hkv, t, s)
+  want, _, _ = OA.closed_form(q1, k[:1], v[:1], mask=rows, sm_scale=1.0)
+  total, _, _ = OA.closed_form(q1, k[:1], v[:1].abs(), mask=rows, sm_scale=1.0)
+  over = (got[:1, ::rep].double().cpu() - want).abs() / float32_bound(want, total, units)
+  assert torch.all(over <= 1.0), float(over.max())
+
+
+@pytest.mark.parametrize("causal", [False, True])
+@pytest.mark.parametrize("gap", [8.0, 11.0, 14.0, 18.0])
+@pytest.mark.parametrize("b,hq,hkv,d,s", [(8, 64, 8, 64, 6000), (40, 8, 4, 128, 3500)])
+def test_a_sink_and_a_flat_rest(b, hq, hkv, d, s, gap, causal):
+  """One position has all but the whole weight and no value in half of the outputs, which are then the others' alone."""
+  g = torch.Generator().manual_seed(int(gap))
+  q, k = torch.zeros((b, hq, 130, d)), torch.zeros((b, hkv, s, d))
+  q[..., 0] = 8.0
+  k[:, :, 0, 0] = gap / 8
+  v = torch.rand((b, hkv, s, d), generator=g) + 0.5
+  v[:, :, 0, : d // 2] = 0.0
+  check(q.to(torch.bfloat16), k.to(torch.bfloat16), v.to(torch.bfloat16), causal)
+
+
+@pytest.mark.parametrize("one_tile", [False, True])
+@pytest.mark.parametrize("x", [1.5625, 1.75, 2.125, 2.4375, 3.0])  # e^-8x: 2^-18, 2^-20.2, 2^-24.5, 2^-28.1, 2^-34.6
+def test_small_weights_of_large_values(x, one_tile):
+  b, hq, hkv, d, s = 8, 64, 8, 64, 320
+  g = torch.Generator().manual_seed(11)
+  q, k = torch.zeros((b, hq, 130, d)), torch.zeros((b, hkv, s, d))
+  at = torch.arange(s)
+  large = at % 2 == 0 if one_tile else at // 64 % 2 == 0
+  q[..., 0] = 8.0
+  k[:, :, ~large, 0] = x
+  v = 1.0 + torch.rand((b, hkv, s, d), generator=g)
+  v[:, :, large] *= 2.0 ** round(8 * x / math.log(2))
+  check(q.to(torch.bfloat16), k.to(torch.bfloat16), v.to(torch.bfloat16), False)
