@@ -267,3 +267,26 @@ def test_a_prompt_uses_no_memory_that_outlives_its_call(monkeypatch):
   ak.dense_attention(q, k, v, mask=mask)
   ak.dense_attention(q, k, v, mask=mask.transpose(2, 3))  # the general way: not contiguous
   assert not ak._workspaces
+
+
+@pytest.mark.parametrize("t,d,masked", [(40, 64, False), (300, 128, True), (130, 256, False)])
+def test_outputs_that_lie_on_8_bytes(t, d, masked):
+  """The same bits as on 16, and nothing before or behind them."""
+  from jetstream_pt_amd import _ffi
+  g = torch.Generator().manual_seed(t)
+  q, k, v = (torch.randn((2, h, t, d), generator=g).to(torch.bfloat16).to(DEV) for h in (4, 2, 2))
+  mask = torch.full((t, t), -math.inf, device=DEV).triu(1) if masked else None
+  a = _ffi.AttnArgs(q=_ffi.ptr(q), k=_ffi.ptr(k), v=_ffi.ptr(v), batch=2, q_heads=4, kv_heads=2, q_rows=t, seq=t, dim=d,
+                    q_dtype=_ffi.BF16, kv_dtype=_ffi.BF16, sm_scale=d ** -0.5)
+  if masked:
+    a.mask, a.mask_dtype, a.mask_stride_t = _ffi.ptr(mask), _ffi.F32, t
+  outs = []
+  for shift in (8, 4):  # elements: 16 bytes, 8 bytes
+    room = torch.full((q.numel() + 16,), 7.0, dtype=torch.bfloat16, device=DEV)
+    a.out = room.data_ptr() + 2 * shift
+    assert a.out % 16 == 2 * shift % 16 and _ffi.lib.jpt_attn_kernel(a, 1) == _ffi.ATTN_PREFILL
+    _ffi.check(_ffi.lib.jpt_attn_dense(a, _ffi.stream()))
+    torch.cuda.synchronize()
+    assert torch.all(room[:shift] == 7.0) and torch.all(room[shift + q.numel():] == 7.0)
+    outs.append(room[shift:shift + q.numel()].clone())
+  assert torch.equal(outs[0], outs[1]) and torch.isfinite(outs[0]).all()
