@@ -497,6 +497,7 @@ int32_t insert_launch(const jpt_prefill_insert_args& a, const jpt_insert_layer* 
   JPT_REQUIRE(a.in_dtype == JPT_BF16 || a.in_dtype == JPT_F32 || a.in_dtype == JPT_I8, "bad in_dtype");
   const bool quant = a.dst_dtype == JPT_I8 && a.in_dtype != JPT_I8;
   JPT_REQUIRE(quant || a.dst_dtype == a.in_dtype, "dst_dtype must be in_dtype (copy) or int8 (quantise)");
+  if (quant && host_ids) return 1;  // the quantising kernels read ids from the device
   const int esz = a.in_dtype == JPT_F32 ? 4 : a.in_dtype == JPT_BF16 ? 2 : 1;
   const int esz_out = quant ? 1 : esz;
   JPT_REQUIRE(a.src_head_stride == 0 || (a.src_head_stride >= static_cast<int64_t>(a.tokens) * a.dim && a.src_head_stride % 4 == 0),

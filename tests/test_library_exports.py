@@ -59,3 +59,17 @@ def test_which_kernel_takes_a_call(change, mode, want):
   from jetstream_pt_amd import _ffi
   a = dict(q=64, k=64, v=64, out=64, batch=2, q_heads=8, kv_heads=2, q_rows=1, dim=128, seq=256, q_dtype=_ffi.BF16, kv_dtype=_ffi.BF16)
   assert _ffi.lib.jpt_attn_kernel(_ffi.AttnArgs(**dict(a, **change)), mode) == getattr(_ffi, "ATTN_" + want)
+
+
+def test_page_ids_on_the_host_are_for_copies():
+  """A quantising call is left to the entry that takes its ids on the device: 1, and nothing done."""
+  from jetstream_pt_amd import _ffi
+  address = 4096  # looked at, not followed
+  layer = (_ffi.InsertLayer * 1)(_ffi.InsertLayer(*([address] * 6)))
+  ids = (ctypes.c_int32 * 4)(0, 1, 2, 3)
+  fn = _ffi.lib.jpt_prefill_insert_layers_host_pages
+  fn.restype, fn.argtypes = ctypes.c_int32, [ctypes.c_void_p] * 3 + [ctypes.c_int32, ctypes.c_void_p]
+  for scale_dtype in (_ffi.BF16, _ffi.F32):
+    a = _ffi.PrefillInsertArgs(tokens=100, heads=8, dim=128, n_pages=4, total_pages=8, page_size=32, in_dtype=_ffi.BF16, dst_dtype=_ffi.I8,
+                               scale_dtype=scale_dtype, scale_heads=1)
+    assert fn(ctypes.byref(a), ids, layer, 1, None) == 1
