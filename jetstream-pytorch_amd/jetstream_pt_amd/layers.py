@@ -24,6 +24,8 @@ from .cache_manager import Int8KVCacheGenerate, Int8PageKVCacheGenerate, KVCache
 from .quantize import _rounding_code
 from .scopes import scoped
 
+_PREFILL_UPDATE = KVCachePrefill.update
+
 
 def apply_rotary_emb(xq, xk, freqs_cis):
   """The reference's apply_rotary_emb (jetstream_pt/layers.py:368-379) as one small
@@ -198,9 +200,9 @@ class Int8KVAttentionKernel(AttentionKernel):
       xk = apply_rotary_emb(None, xk.transpose(1, 2), freqs_cis)[1].transpose(1, 2)
       freqs_cis = None
     if (seqlen > 1 and type(cache) is KVCachePrefill and cache.kv_quantize and not scopes.ENABLED
-        and self.dense_attention is ak.dense_attention):
+        and self.dense_attention is ak.dense_attention and getattr(cache.update, "__func__", None) is _PREFILL_UPDATE):
       # A prompt's keys and values are attended as they are: the scales that cache.update() gives with them are ones,
-      # which the kernel would be launched to fill, to load and to multiply with.
+      # which the kernel would be launched to fill, to load and to multiply with.  (A caller's own update() is called.)
       cache.cache_k, cache.cache_v = xk, xv
       return self._attend(xq, xk, xv, None, None, mask, cache, start, end, ragged_batch_index, ragged_block_index)[0]
     rope_kw = {} if freqs_cis is None else {"freqs_cis": freqs_cis}
